@@ -1,0 +1,536 @@
+"""What a program that uses this package has it do, as measurable cases.
+
+Each case is one kind of call on an operator that the program already holds
+(an `OperatorBorn` plan, or an `OperatorBatch` of them):
+
+* `pair`: one iteration of an image reconstruction, the forward u = A gamma
+  and the adjoint A^H u on device tensors, in every numeric form, 2-D and 3-D,
+  one or several right-hand sides, identity or mixed receive signals;
+* `gradient`: the data misfit of several uneven instances in one batch and
+  its gradients through autograd;
+* `host`: the solver contract `op_A` on FP64 host arrays with time gain
+  compensation in both directions;
+* `columns`: columns of A for a greedy pursuit's new support;
+* `energy`, `energy_tgc`: received energies of every measurement, which the
+  solvers normalize the columns with, without and with time gain compensation;
+* `signals`: compensated spectra and their time-domain voltage signals.
+
+The linear arrays have the pitch of the named 2-D workloads (0.3048 mm), the
+matrix arrays 0.3 mm; media, pulses and filters are the package's defaults.
+`exact` restates the model in complex128 torch from the same numbers.
+"""
+import math
+
+import numpy as np
+import torch
+
+from comp_ui_toolbox_amd import OperatorBatch, OperatorBorn
+from comp_ui_toolbox_amd import configs as C
+from comp_ui_toolbox_amd.autograd import born_batch_apply
+from comp_ui_toolbox_amd.tgc import exponential_kernels
+
+DEV = "cuda:0"
+
+
+# ---------------------------------------------------------------- the cases
+def _case(kind, elements, nx, nz, ppp, nf, waves, precision="fp32", rhs=1, mixes=0, elements_y=0, ny=0, points=0):
+    """elements(_y) along the array axes, nx x (ny x) nz grid points, ppp grid
+    points per pitch, nf frequencies, mixes = 0: every element is received."""
+    return {"kind": kind, "elements": elements, "elements_y": elements_y, "nx": nx, "ny": ny, "nz": nz, "ppp": ppp,
+            "nf": nf, "waves": waves, "rhs": rhs, "mixes": mixes, "precision": precision, "points": points}
+
+
+def listed():
+    return [
+        # the smallest named workload: one plane wave, an interactive preview of one frame
+        dict(_case("pair", 64, 256, 256, 4, 65, 1), name="pair_one_wave"),
+        # the package's main workload: 11 compounded plane waves on a 128-element array, in its default fast form ...
+        dict(_case("pair", 128, 512, 512, 4, 257, 11, "split_bf16"), name="pair_compound_bf16"),
+        # ... and in plain FP32, as solvers that iterate to small residuals take it
+        dict(_case("pair", 128, 512, 512, 4, 257, 11, "fp32"), name="pair_compound_fp32"),
+        # compressed acquisition: 32 random waves, 16 mixed receive signals each, the accurate fast form
+        dict(_case("pair", 128, 512, 512, 4, 257, 32, "split_fp16", mixes=16), name="pair_random_fp16"),
+        # a region of interest of odd size on part of the array, coarse grid
+        dict(_case("pair", 100, 301, 411, 2, 97, 7, "fp32"), name="pair_odd_fp32"),
+        # a volume under a matrix array, four right-hand sides at once
+        dict(_case("pair", 32, 64, 64, 2, 33, 3, "split_bf16", rhs=4, elements_y=32, ny=64), name="pair_volume_bf16"),
+        # training or variational reconstruction: four uneven instances, gradient of the data misfit
+        dict(_case("gradient", 128, 512, 512, 4, 129, 9), name="gradient_batch"),
+        # a solver written against the toolbox's op_A: host arrays, time gain compensation on
+        dict(_case("host", 128, 512, 512, 4, 129, 5, "split_bf16"), name="host_tgc"),
+        # orthogonal matching pursuit / CoSaMP: a batch of candidate columns
+        dict(_case("columns", 128, 512, 512, 4, 257, 11, points=256), name="columns"),
+        # column norms of a whole sequence
+        dict(_case("energy", 128, 384, 384, 4, 129, 5), name="energy"),
+        # the same under time gain compensation
+        dict(_case("energy_tgc", 64, 192, 192, 4, 65, 2), name="energy_tgc"),
+        # simulated echoes: compensated spectra to time-domain signals
+        dict(_case("signals", 128, 128, 128, 4, 257, 11, rhs=4), name="signals"),
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return max(lo, min(hi, int(round(math.exp(rng.uniform(math.log(lo), math.log(hi + 0.49)))))))
+
+
+def draw(rng):
+    """Sizes over the ranges between and around the listed cases, odd ones among them."""
+    while True:
+        kind = rng.choice(["pair"] * 6 + ["volume", "gradient", "host", "columns", "energy", "energy_tgc", "signals"])
+        ppp = rng.choice([2, 4, 4])
+        ne = _log_int(rng, 17, 128)
+        nx, nz = _log_int(rng, 64, 512), _log_int(rng, 64, 512)
+        nf, waves = _log_int(rng, 17, 257), _log_int(rng, 1, 32)
+        if kind == "pair":
+            precision = rng.choice(["fp32", "fp32", "split_bf16", "split_fp16"])
+            if precision == "fp32" and rng.random() < 0.25:
+                ne, ppp = _log_int(rng, 4, 128), rng.choice([1, 3, 4])
+            c = _case(kind, ne, nx, nz, ppp, nf, waves, precision, rhs=rng.choice([1, 1, 1, 2, 3, 8]),
+                      mixes=rng.choice([0, 0, 0, 5, 16]))
+        elif kind == "volume":
+            c = _case("pair", rng.choice([16, 20, 32]), _log_int(rng, 24, 72), _log_int(rng, 16, 64), 2,
+                      _log_int(rng, 5, 33), _log_int(rng, 1, 5), rng.choice(["fp32", "split_bf16"]), rhs=rng.choice([1, 2, 4]),
+                      elements_y=rng.choice([8, 16, 32]), ny=_log_int(rng, 24, 72))
+            if c["elements"] < 17:
+                c["precision"] = "fp32"
+        elif kind == "gradient":
+            c = _case(kind, 128, nx, nz, 4, _log_int(rng, 33, 129), _log_int(rng, 2, 9))
+        elif kind == "host":
+            c = _case(kind, ne, nx, nz, ppp, _log_int(rng, 33, 129), _log_int(rng, 1, 5),
+                      rng.choice(["fp32", "split_bf16", "split_fp16"]))
+        elif kind == "columns":
+            c = _case(kind, ne, nx, nz, ppp, nf, _log_int(rng, 1, 11), mixes=rng.choice([0, 0, 16]), points=_log_int(rng, 1, 256))
+        elif kind == "energy":
+            c = _case(kind, ne, _log_int(rng, 64, 384), _log_int(rng, 64, 384), ppp, _log_int(rng, 17, 129),
+                      _log_int(rng, 1, 5), mixes=rng.choice([0, 0, 4]))
+        elif kind == "energy_tgc":
+            c = _case(kind, _log_int(rng, 17, 64), _log_int(rng, 64, 192), _log_int(rng, 64, 192), ppp,
+                      _log_int(rng, 17, 65), _log_int(rng, 1, 2), mixes=rng.choice([0, 0, 4]))
+        else:
+            c = _case(kind, ne, _log_int(rng, 64, 128), _log_int(rng, 64, 128), ppp, _log_int(rng, 33, 257),
+                      _log_int(rng, 1, 11), mixes=rng.choice([0, 0, 16]), rhs=_log_int(rng, 1, 4))
+        n_pts = c["nx"] * c["nz"] * max(1, c["ny"])
+        pairs = c["nf"] * c["waves"]
+        macs = pairs * n_pts * c["rhs"] * c["elements"] * max(1, c["elements_y"])
+        if macs <= 257 * 11 * 512 * 512 * 128 and pairs * n_pts * c["rhs"] <= 257 * 11 * 512 * 512:
+            return c
+
+
+# ---------------------------------------------------------------- the model
+C_REF, T_CLK = 1500.0, 1.0 / 80e6
+
+
+def _instances(case):
+    """The sizes of the instances: one, or the four uneven ones of a batch
+    (sides, frequencies and waves in fixed proportions, odd remainders)."""
+    if case["kind"] != "gradient":
+        return [case]
+    out = []
+    for k, (s, f, w) in enumerate(((4, 4, 1), (3, 2, 5), (2, 3, 9), (1, 4, 3))):
+        out.append(dict(case, nx=max(32, case["nx"] * s // 4), nz=max(32, case["nz"] * s // 4),
+                        nf=max(9, case["nf"] * f // 4), waves=max(1, case["waves"] * w // 9), part=k))
+    return out
+
+
+def _model(case, seed):
+    """Plain numbers of one sequence: geometry, frequencies, waves, mixes."""
+    volume = case["elements_y"] > 0
+    pitch = 0.3e-3 if volume else 0.3048e-3
+    rng = np.random.Generator(np.random.PCG64([seed, 11]))
+    m = {"volume": volume, "pitch": pitch, "width": 0.27e-3, "delta": pitch / case["ppp"], "ppp": case["ppp"],
+         "ne": (case["elements"], max(1, case["elements_y"])), "n": (case["nx"], max(1, case["ny"]), case["nz"]),
+         "z0": 3e-3 if volume else 2e-3}
+    nf = case["nf"]
+    if volume:
+        m["f"] = np.linspace(2.5e6, 5.5e6, nf)
+    elif case["kind"] in ("signals", "host", "energy_tgc"):
+        m["f"] = 2e6 + 31.25e3 * np.arange(nf)      # a recorded spectrum: integer multiples of the spacing
+    else:
+        m["f"] = np.linspace(2e6, 10e6 if nf > 65 else 6e6, nf)
+    ex = (np.arange(m["ne"][0]) - (m["ne"][0] - 1) / 2.0) * pitch
+    ey = (np.arange(m["ne"][1]) - (m["ne"][1] - 1) / 2.0) * pitch
+    xe, ye = np.tile(ex, m["ne"][1]), np.repeat(ey, m["ne"][0])   # x fastest
+    m["waves"] = []
+    tilt = rng.uniform(-0.05, 0.05)             # the fan of steering angles or sources, turned a little
+    for w in range(case["waves"]):
+        frac = tilt + (2.0 * w / (case["waves"] - 1) - 1.0 if case["waves"] > 1 else 0.0)
+        apod = np.ones(len(xe))
+        if volume:      # diverging waves from virtual sources 10 mm behind the array
+            tau = np.sqrt((xe - 6e-3 * frac) ** 2 + ye ** 2 + 10e-3 ** 2) / C_REF
+        elif case["mixes"]:   # random waves
+            apod = np.where(rng.random(len(xe)) < 0.5, -1.0, 1.0)
+            tau = rng.uniform(0.0, 5e-6, len(xe))
+        else:
+            tau = xe * math.sin(math.radians(10.0 * frac)) / C_REF
+        m["waves"].append((apod, tau - tau.min()))
+    m["mixes"] = [[np.where(rng.random(len(xe)) < 0.5, -1.0, 1.0) for _ in range(case["mixes"])]
+                  for _ in range(case["waves"])]
+    return m
+
+
+def _spec(m):
+    dims = (0, 1) if m["volume"] else (0,)
+    arr = C.ArraySpec(tuple(m["ne"][d] for d in dims), (m["pitch"],) * len(dims), (m["width"],) * len(dims),
+                      (4,) * len(dims))
+    n = m["n"] if m["volume"] else (m["n"][0], m["n"][2])
+    fov = C.FovSpec(tuple(n), (m["delta"],) * len(n), m["z0"])
+    e = np.arange(arr.N_elements)
+    waves = [C.WaveSpec(e, a, t) for a, t in m["waves"]]
+    mixes = [[C.MixSpec(e, w) for w in ws] if ws else C.identity_mixes(arr.N_elements) for ws in m["mixes"]]
+    return C.SequenceSpec("case", arr, C.MediumSpec(), fov, m["f"], waves, mixes)
+
+
+def _n_obs(case):
+    n = case["mixes"] or case["elements"] * max(1, case["elements_y"])
+    return case["waves"] * n * case["nf"]
+
+
+def _spectrum(f):
+    """The pulse: a Gaussian-windowed 4 MHz burst of two periods."""
+    sigma = (2.0 / 4e6) / (2.0 * math.sqrt(2.0 * math.log(2.0)))
+    g = lambda x: np.exp(-2.0 * (math.pi * sigma * x) ** 2)  # noqa: E731
+    return sigma * math.sqrt(2.0 * math.pi) / 2.0 * (g(f - 4e6) + g(f + 4e6))
+
+
+def _image(case, seed):
+    """Speckle with anechoic disks and a few bright points: (rhs, points) float32."""
+    gen = torch.Generator(device=DEV).manual_seed(1000 + seed)
+    n_pts = case["nx"] * max(1, case["ny"]) * case["nz"]
+    g = torch.randn(case["rhs"], n_pts, generator=gen, device=DEV)
+    ix = torch.arange(n_pts, device=DEV)
+    x, z = ix % case["nx"], ix // (case["nx"] * max(1, case["ny"]))
+    at = torch.rand(6, 2, generator=gen, device=DEV)
+    for a in at:
+        r2 = ((x - a[0] * case["nx"]) ** 2 + (z - a[1] * case["nz"]) ** 2).float()
+        g = torch.where(r2 <= (0.05 * (case["nx"] + case["nz"])) ** 2, 0.05 * g, g)
+    g[:, torch.randint(0, n_pts, (20,), generator=gen, device=DEV)] = 10.0
+    return g
+
+
+def _voltages(case, m, seed):
+    """Received spectra: complex noise under the pulse's spectrum, (rhs, observations) complex64."""
+    gen = torch.Generator(device=DEV).manual_seed(2000 + seed)
+    n_obs = _n_obs(case)
+    v = torch.randn(case["rhs"], n_obs, 2, generator=gen, device=DEV)
+    amp = torch.tensor(_spectrum(m["f"]) / _spectrum(m["f"]).max(), dtype=torch.float32, device=DEV)
+    return torch.view_as_complex(v).reshape(case["rhs"], -1, case["nf"]).mul(amp).reshape(case["rhs"], n_obs)
+
+
+TGC_RATE, TGC_DECAY = 1.2e5, -40.0
+
+
+def _tgc_interval(m):
+    return (0.0, 0.9 / (m["f"][1] - m["f"][0]))
+
+
+def _candidates(case, seed):
+    """Distinct candidate grid points of a pursuit step (0-based)."""
+    rng = np.random.Generator(np.random.PCG64([seed, 12]))
+    return rng.choice(case["nx"] * case["nz"], size=min(case["points"], case["nx"] * case["nz"]), replace=False)
+
+
+# ---------------------------------------------------------------- a pass
+def prepare(case, seed):
+    kind = case["kind"]
+    s = {"case": case, "parts": []}
+    for k, part in enumerate(_instances(case)):
+        m = _model(part, seed)
+        p = {"m": m, "op": OperatorBorn.from_sequence(_spec(m), precision=part["precision"])}
+        if kind in ("host", "signals", "energy_tgc"):
+            n = sum(len(w) or int(np.prod(m["ne"])) for w in m["mixes"])
+            p["op"].set_tgc(exponential_kernels(TGC_RATE, np.tile(_tgc_interval(m), (n, 1)), m["f"][1] - m["f"][0],
+                                                TGC_DECAY))
+        if kind in ("pair", "host", "gradient"):
+            p["g"] = _image(part, seed + 100 * k)
+            p["u"] = _voltages(part, m, seed + 100 * k)
+            if kind == "pair":
+                p["g"] = p["g"].to(torch.complex64)
+            if kind == "host":
+                p["g"] = p["g"][0].cpu().numpy().astype(np.complex128)
+                p["u"] = p["u"][0].cpu().numpy().astype(np.complex128)
+            if kind == "gradient":
+                p["g"], p["u"] = p["g"][0].requires_grad_(True), p["u"][0] * 1e-15
+        elif kind == "signals":
+            p["u"] = _voltages(part, m, seed)
+        elif kind == "columns":
+            p["points"] = _candidates(case, seed)
+        s["parts"].append(p)
+    if kind == "gradient":
+        s["batch"] = OperatorBatch([p["op"] for p in s["parts"]])
+    return s
+
+
+def run(s):
+    kind, p = s["case"]["kind"], s["parts"][0]
+    op = p["op"]
+    if kind == "pair":
+        return {"u": op.forward_dev(p["g"]), "gamma": op.adjoint_dev(p["u"])}
+    if kind == "host":
+        return {"u": op.op_A(p["g"], 1, tgc=True), "gamma": op.op_A(p["u"], 2, tgc=True)}
+    if kind == "columns":
+        return op.columns_dev(p["points"])
+    if kind == "energy" or kind == "energy_tgc":
+        return [op.energy_rx_dev(m, tgc=kind == "energy_tgc") for m in range(s["case"]["waves"])]
+    if kind == "signals":
+        u = op.tgc_dev(p["u"])
+        rf, _ = op.time_signals(u, p["m"]["f"])
+        return {"u": u, "rf": rf}
+    gs = [q["g"] for q in s["parts"]]
+    us = born_batch_apply(s["batch"], gs)
+    loss = sum((1e15 * (u - q["u"])).abs().square().mean() for u, q in zip(us, s["parts"]))
+    return {"loss": loss.detach(), "grad": list(torch.autograd.grad(loss, gs))}
+
+
+# ---------------------------------------------------------------- the least work
+def work(case):
+    """Tables (transfer function and incident fields, single precision
+    complex), inputs and outputs once per direction; the operations of the
+    lateral correlations by fast transforms where these are fewer than the
+    direct products."""
+    bytes_, flops = 0.0, 0.0
+    for c in _instances(case):
+        ne = c["elements"] * max(1, c["elements_y"])
+        n_pts = c["nx"] * max(1, c["ny"]) * c["nz"]
+        span_x = c["nx"] + (c["elements"] - 1) * c["ppp"]
+        span_y = c["ny"] + (c["elements_y"] - 1) * c["ppp"] if c["ny"] else 1
+        h_pts = n_pts if c["nx"] > (c["elements"] - 1) * c["ppp"] and not c["ny"] else span_x * span_y * c["nz"]
+        pairs, n_obs = c["nf"] * c["waves"], _n_obs(c)
+        tables = 8.0 * (c["nf"] * h_pts + pairs * n_pts)
+        span = span_x * span_y
+        apply = pairs * c["rhs"] * c["nz"] * min(8.0 * ne * c["nx"] * max(1, c["ny"]),
+                                                 10.0 * span * math.log2(span) + 8.0 * span)
+        mixing = 8.0 * c["rhs"] * n_obs * (ne if c["mixes"] else 1)
+        kind = c["kind"]
+        if kind in ("pair", "gradient", "host"):
+            host = 2.0 if kind == "host" else 1.0
+            bytes_ += 2.0 * (tables + host * 8.0 * c["rhs"] * (n_pts + n_obs))
+            flops += 2.0 * (apply + mixing + 6.0 * pairs * c["rhs"] * n_pts)
+        elif kind == "columns":
+            n = min(c["points"], n_pts)
+            bytes_ += 8.0 * n * (n_obs + c["nf"] * ne + pairs)
+            flops += n * (6.0 * n_obs + (8.0 * n_obs * ne if c["mixes"] else 6.0 * n_obs))
+        elif kind in ("energy", "energy_tgc"):
+            bytes_ += 8.0 * (c["waves"] * (c["nf"] * n_pts + n_pts) + pairs * n_pts)
+            rows = pairs * n_pts * (c["mixes"] or ne)
+            per_row = 8.0 * ne if c["mixes"] else (6.0 if kind == "energy_tgc" else 4.0)
+            if kind == "energy_tgc":
+                per_row += 20.0 * math.log2(2 * c["nf"])
+            flops += rows * per_row
+        else:
+            n_sig = n_obs // c["nf"]
+            n_t = 2 * (64 + c["nf"] - 1)
+            bytes_ += c["rhs"] * (16.0 * n_obs + 4.0 * n_sig * n_t)
+            flops += c["rhs"] * n_sig * (20.0 * c["nf"] * math.log2(2 * c["nf"]) + 2.5 * n_t * math.log2(n_t))
+    return {"bytes": bytes_, "flops": flops}
+
+
+# ---------------------------------------------------------------- in 64 bits
+def _wavenumber(f):
+    """Time-causal power law with exponent 1: 0.5 dB / (MHz cm), reference 4 MHz."""
+    a = 0.5 * math.log(10.0) / (0.2 * 1e6)
+    return 2.0 * math.pi * f / C_REF - 2.0 * a * f * math.log(f / 4e6) / math.pi - 1j * a * f
+
+
+def _hankel(z):
+    """H0 of the second kind by its large-argument expansion (DLMF 10.17.6; |z| > 16 here)."""
+    s = torch.ones_like(z)
+    term = torch.ones_like(z)
+    iz = 1.0 / z
+    for k in range(1, 26):
+        term = term * iz * (1j * (2 * k - 1) ** 2 / (8.0 * k))
+        s = s + term
+    return torch.sqrt(2.0 / (math.pi * z)) * torch.exp(-1j * (z - math.pi / 4)) * s
+
+
+def _transfer(m, f):
+    """The transfer function over all lateral offsets of a point from an
+    element: (nz, y offsets, x offsets) complex128, offset index
+    i - e * ppp + (ne - 1) * ppp along each lateral axis."""
+    k = _wavenumber(f)
+    n, ne, ppp = m["n"], m["ne"], m["ppp"]
+    off = []
+    for d in range(2):
+        i = torch.arange(-(ne[d] - 1) * ppp, n[d], device=DEV, dtype=torch.float64)
+        off.append((i - (n[d] - 1) / 2.0) * m["delta"] + (ne[d] - 1) / 2.0 * m["pitch"])
+    if not m["volume"]:
+        off[1] = torch.zeros(1, device=DEV, dtype=torch.float64)
+    z = (m["z0"] + m["delta"] * torch.arange(n[2], device=DEV, dtype=torch.float64))[:, None, None]
+    x, y = off[0][None, None, :], off[1][None, :, None]
+    face = (np.arange(4) - 1.5) * (m["width"] / 4)
+    acc = 0
+    for yf in face if m["volume"] else (0.0,):
+        for xf in face:
+            r = torch.sqrt((x - xf) ** 2 + (y - yf) ** 2 + z ** 2)
+            if m["volume"]:
+                acc = acc - torch.exp(-1j * k * r) / (4.0 * math.pi * r)
+            else:
+                acc = acc + 0.25j * _hankel(k * r)
+    acc = -2.0 * (m["width"] / 4) ** (2 if m["volume"] else 1) * acc
+    r = torch.sqrt(x ** 2 + y ** 2 + z ** 2)
+    for d, c in ((0, x), (1, y)):
+        if ne[d] > 1:   # raised cosine over the upper half of the band
+            q = (k.real * m["pitch"] * c.abs() / r - 0.5 * math.pi) / (0.5 * math.pi)
+            acc = acc * (0.5 * (1.0 + torch.cos(math.pi * q.clamp(0.0, 1.0))))
+    return acc
+
+
+def _elements(m, h, ey):
+    """Transfer functions of the elements of y row ey: (nz, ny, ne_x, nx)."""
+    n, ne, ppp = m["n"], m["ne"], m["ppp"]
+    ny = n[1] if m["volume"] else 1
+    y0 = (ne[1] - 1 - ey) * ppp if m["volume"] else 0
+    b = h[:, y0:y0 + ny]
+    w = b.as_strided((n[2], ny, ne[0], n[0]), (h.stride(0), h.stride(1), ppp, 1), b.storage_offset())
+    return w.flip(2).contiguous()    # window e' starts at e' * ppp: element ne - 1 - e'
+
+
+def _velocities(m, f):
+    v = [a * _spectrum(f) * np.exp(-2j * math.pi * f * np.round(t / T_CLK) * T_CLK) for a, t in m["waves"]]
+    return torch.tensor(np.array(v), device=DEV).to(torch.complex128)   # (waves, elements)
+
+
+def _weights(m, f):
+    """Receive weights per wave: None (every element) or (waves, mixes, elements) ones."""
+    pref = -(m["delta"] ** (3 if m["volume"] else 2)) * _wavenumber(f) ** 2
+    if not m["mixes"][0]:
+        return pref, None
+    return pref, torch.tensor(np.array(m["mixes"]), device=DEV).to(torch.complex128)
+
+
+def _incident(m, h, f):
+    """Incident fields (waves, nz, ny, nx)."""
+    v = _velocities(m, f).reshape(-1, m["ne"][1], m["ne"][0])
+    p = 0
+    for ey in range(m["ne"][1]):
+        p = p + torch.matmul(v[:, ey], _elements(m, h, ey))   # (nz, ny, waves, nx)
+    return p.permute(2, 0, 1, 3).contiguous()
+
+
+def _exact_forward(m, g):
+    """g (rhs, points) -> u (rhs, waves, signals, frequencies)."""
+    out = []
+    for f in m["f"]:
+        h = _transfer(m, f)
+        p = _incident(m, h, f)
+        b = p[:, None] * g.reshape(1, g.shape[0], p.shape[1], p.shape[2], p.shape[3])      # (waves, rhs, nz, ny, nx)
+        b = b.reshape(-1, *p.shape[1:]).permute(1, 2, 3, 0).contiguous()                   # (nz, ny, nx, columns)
+        v = torch.stack([torch.matmul(_elements(m, h, ey), b).sum(dim=(0, 1)) for ey in range(m["ne"][1])])
+        v = v.reshape(-1, p.shape[0], g.shape[0])                                          # (elements, waves, rhs)
+        pref, w = _weights(m, f)
+        out.append(pref * (v.permute(2, 1, 0) if w is None else torch.einsum("wke,ewr->rwk", w, v)))
+    return torch.stack(out, dim=-1)
+
+
+def _exact_adjoint(m, u):
+    """u (rhs, waves, signals, frequencies) -> gamma (rhs, points)."""
+    acc = 0
+    for i, f in enumerate(m["f"]):
+        h = _transfer(m, f)
+        p = _incident(m, h, f)
+        pref, w = _weights(m, f)
+        x = u[..., i] * np.conj(pref)
+        if w is not None:
+            x = torch.einsum("wke,rwk->rwe", w.conj(), x)
+        x = x.reshape(u.shape[0], u.shape[1], m["ne"][1], m["ne"][0]).conj()
+        y = 0
+        for ey in range(m["ne"][1]):
+            y = y + torch.matmul(x[:, :, ey].reshape(-1, m["ne"][0]), _elements(m, h, ey))   # (nz, ny, columns, nx)
+        y = y.permute(2, 0, 1, 3).reshape(u.shape[0], u.shape[1], *p.shape[1:])
+        acc = acc + (p[None] * y).sum(dim=1).conj()
+    return acc.reshape(u.shape[0], -1)
+
+
+def _tgc_matrix(m):
+    """The compensation of one signal as the (nf, nf) band matrix of its kernel."""
+    t0, t1 = _tgc_interval(m)
+    period, nf = 1.0 / (m["f"][1] - m["f"][0]), len(m["f"])
+    a, T = TGC_RATE, t1 - t0
+    e = math.exp(-a * T)
+    edge = a * math.sqrt(((1.0 + e) * 10.0 ** (-TGC_DECAY / 20.0) / (1.0 - e)) ** 2 - 1.0) / (2.0 * math.pi)
+    k = np.arange(int(math.ceil(edge * period)) + 1) / period
+    den = a - 2j * math.pi * k
+    c = np.exp(-2j * math.pi * k * t0) * (np.exp(den * T) - 1.0) / (den * period)
+    d = np.arange(nf)[:, None] - np.arange(nf)[None, :]
+    band = np.where(np.abs(d) < len(c), c[np.minimum(np.abs(d), len(c) - 1)], 0.0)
+    return torch.tensor(np.where(d >= 0, band, np.conj(band)), device=DEV)
+
+
+def _exact_energy(m, tgc):
+    """(waves, points): squared norms of the columns of each measurement's rows."""
+    nf, ne = len(m["f"]), m["ne"][0]
+    n_pts = m["n"][0] * m["n"][2]
+    n_sig = len(m["mixes"][0]) or ne
+    out = []
+    hs = [_transfer(m, f) for f in m["f"]]
+    ps = [_incident(m, h, f).reshape(-1, n_pts) for h, f in zip(hs, m["f"])]
+    C_ = _tgc_matrix(m) if tgc else None
+    for wave in range(len(m["waves"])):
+        E = torch.zeros(n_pts, dtype=torch.float64, device=DEV)
+        if not tgc:
+            for f, h, p in zip(m["f"], hs, ps):
+                pref, w = _weights(m, f)
+                q = _elements(m, h, 0)[:, 0]                                   # (nz, ne, nx)
+                q = q if w is None else torch.matmul(w[wave], q)
+                E += (pref * p[wave]).abs() ** 2 * (q.abs() ** 2).sum(dim=1).reshape(-1)
+        else:
+            for sig in range(n_sig):
+                rows = []
+                for f, h, p in zip(m["f"], hs, ps):
+                    pref, w = _weights(m, f)
+                    if w is None:
+                        x0 = (ne - 1 - sig) * m["ppp"]
+                        q = h[:, 0, x0:x0 + m["n"][0]].reshape(-1)
+                    else:
+                        q = torch.matmul(w[wave, sig][None], _elements(m, h, 0)[:, 0]).reshape(-1)
+                    rows.append(pref * p[wave] * q)
+                E += (torch.matmul(C_, torch.stack(rows)).abs() ** 2).sum(dim=0)
+        out.append(E)
+    assert nf == len(hs)
+    return out
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    parts = _instances(case)
+    m = _model(parts[0], seed)
+    if kind in ("pair", "host"):
+        g = _image(case, seed).to(torch.complex64).to(torch.complex128)
+        u = _voltages(case, m, seed).to(torch.complex128).reshape(case["rhs"], case["waves"], -1, case["nf"])
+        if kind == "host":
+            B = _tgc_matrix(m)
+            return {"u": torch.matmul(_exact_forward(m, g), B.T).reshape(-1),
+                    "gamma": _exact_adjoint(m, torch.matmul(u, B.conj())).reshape(-1)}
+        return {"u": _exact_forward(m, g).reshape(case["rhs"], -1), "gamma": _exact_adjoint(m, u)}
+    if kind == "gradient":
+        loss, grads = 0.0, []
+        for k, part in enumerate(parts):
+            mk = _model(part, seed)
+            g = _image(part, seed + 100 * k).to(torch.complex128)
+            u = (_voltages(part, mk, seed + 100 * k) * 1e-15).to(torch.complex128).reshape(1, part["waves"], -1, part["nf"])
+            r = _exact_forward(mk, g) - u
+            loss = loss + 1e30 * (r.abs() ** 2).mean()
+            grads.append((2e30 / r.numel()) * _exact_adjoint(mk, r)[0].real)
+        return {"loss": loss, "grad": grads}
+    if kind == "columns":
+        pts = torch.tensor(_candidates(case, seed), device=DEV)
+        ix, iz = pts % case["nx"], pts // case["nx"]
+        ne = case["elements"]
+        e = torch.arange(ne, device=DEV)
+        cols = []
+        for f in m["f"]:
+            h = _transfer(m, f)
+            q = h[iz[:, None], 0, ix[:, None] + (ne - 1 - e[None, :]) * case["ppp"]]       # (points, elements)
+            p = _velocities(m, f) @ q.T                                                    # (waves, points)
+            pref, w = _weights(m, f)
+            r = q[:, None, :] if w is None else torch.einsum("wke,pe->pwk", w, q)
+            cols.append(pref * p.T[:, :, None] * r)
+        return torch.stack(cols, dim=-1).reshape(len(pts), -1)
+    if kind in ("energy", "energy_tgc"):
+        return _exact_energy(m, kind == "energy_tgc")
+    u = _voltages(case, m, seed).to(torch.complex128).reshape(case["rhs"], -1, case["nf"])
+    u = torch.matmul(u, _tgc_matrix(m).T)
+    q = 64 + torch.arange(case["nf"], device=DEV)
+    n_t = 2 * (64 + case["nf"] - 1)
+    spectrum = torch.zeros(*u.shape[:2], n_t // 2 + 1, dtype=torch.complex128, device=DEV)
+    spectrum[..., q] = u
+    return {"u": u.reshape(case["rhs"], -1), "rf": torch.fft.irfft(spectrum, n=n_t) * n_t}
