@@ -265,12 +265,15 @@ def run(s):
     op = p["op"]
     if kind == "pair":
         return {"u": op.forward_dev(p["g"]), "gamma": op.adjoint_dev(p["u"])}
-    if kind == "host":
-        return {"u": op.op_A(p["g"], 1, tgc=True), "gamma": op.op_A(p["u"], 2, tgc=True)}
+    if kind == "host":      # the doubles hold single-precision sums: the program keeps them as such
+        return {"u": op.op_A(p["g"], 1, tgc=True).astype(np.complex64),
+                "gamma": op.op_A(p["u"], 2, tgc=True).astype(np.complex64)}
     if kind == "columns":
         return op.columns_dev(p["points"])
-    if kind == "energy" or kind == "energy_tgc":
-        return [op.energy_rx_dev(m, tgc=kind == "energy_tgc") for m in range(s["case"]["waves"])]
+    if kind == "energy":
+        return [op.energy_rx_dev(m) for m in range(s["case"]["waves"])]
+    if kind == "energy_tgc":    # single-precision products: kept as weights of single-precision vectors
+        return [op.energy_rx_dev(m, tgc=True).float() for m in range(s["case"]["waves"])]
     if kind == "signals":
         u = op.tgc_dev(p["u"])
         rf, _ = op.time_signals(u, p["m"]["f"])
