@@ -115,6 +115,10 @@ static void free_workspace(Plan& P) {
   dfree(P.d_pexp);
   dfree(P.d_ones);
   dfree(P.d_fvpart);
+  dfree(P.fft.d_gs);
+  dfree(P.fft.d_vp);
+  dfree(P.fft.d_wt);
+  dfree(P.fft.d_gp);
   P.fwd_expand = false;
   P.fwd_table_expanded = false;
   P.fchunks.clear();
@@ -136,6 +140,11 @@ Plan::~Plan() {
   dfree(na.ls.d_inst);
   dfree(ls.d_inst);
   dfree(ls_fwd.d_inst);
+  dfree(fft.d_H);
+  dfree(fft.d_slot);
+  dfree(fft.d_col);
+  dfree(fft.d_tw);
+  dfree(fft.set.d_inst);
   dfree(d_fscale);
   dfree(d_f16max);
   dfree(d_f16part);
@@ -405,6 +414,120 @@ static void detect_structure(Plan& P) {
 }
 
 static bool use_structured(const Plan& P) { return P.structured && !P.force_general; }
+// 2-D structured plans apply both directions by fast lateral correlation in
+// every numeric form (the split forms gain accuracy); the allocation-free
+// apply keeps the MFMA layout.
+static bool use_fft(const Plan& P) { return use_structured(P) && P.fft.ok && !P.in_noalloc; }
+
+// Tables of the fast lateral correlation, built once per plan: the slots
+// (row, segment, phase), the columns by frequency and the spectra of h_ref.
+// The spectra take about twice the space of h_ref; a plan whose spectra do
+// not fit in the free memory with 1 GiB to spare stays on the MFMA kernels.
+static void build_fft(Plan& P) {
+  Plan::Fft& F = P.fft;
+  F.ok = false;
+  if (P.nd != 2 || !P.structured) return;
+  F.shape = fft_shape(P.Nx, P.Np, P.N_e);
+  if (F.shape.TL == 0) return;
+  const int FPW = 64 / F.shape.TL;
+  const int64_t n_slots = (int64_t)P.n_rows * F.shape.nseg * P.Np;
+  if (n_slots > INT32_MAX - 64) return;
+  F.n_slots = (int)n_slots;
+  F.n_ws = (F.n_slots + FPW - 1) / FPW;
+  const size_t n = (size_t)P.N_fu * F.n_ws * 1024;
+  size_t free_b = 0, total_b = 0;
+  HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+  if (n * sizeof(float2) + ((size_t)1 << 30) > free_b) return;
+  std::vector<int2> slot((size_t)F.n_ws * FPW, make_int2(0, 0));
+  for (int s = 0; s < F.n_slots; ++s) {
+    const int phi = s % P.Np, rs = s / P.Np;
+    const int seg = rs % F.shape.nseg, row = rs / F.shape.nseg;
+    const int first = P.Np * seg * F.shape.Sv + phi;
+    const int left = first < P.Nx ? (P.Nx - first + P.Np - 1) / P.Np : 0;
+    slot[s] = left > 0 ? make_int2(row * P.Nx + first, std::min(left, F.shape.Sv)) : make_int2(0, 0);
+  }
+  std::vector<int2> col(P.N_pairs);
+  for (int c = 0; c < P.N_pairs; ++c) col[c] = make_int2(P.fg_pairs[c], P.pair_fg[P.fg_pairs[c]]);
+  std::vector<float2> tw;
+  fft_twiddles(F.shape.TL, tw);
+  F.d_slot = dupload(slot, P.stream);
+  F.d_col = dupload(col, P.stream);
+  F.d_tw = dupload(tw, P.stream);
+  F.d_H = dalloc<float2>(n);
+  launch_fft_table(P, P.stream);
+  HIP_CHECK(hipGetLastError());
+  F.ok = true;
+}
+
+// Work split of a plan's fast-correlation launches: forward waves of at least
+// 4 steps (a wave's final transform costs about two) and at most 64, about
+// 24576 of them; adjoint workgroups of 4 waves with at least 8 columns each,
+// about 12288 waves.
+static void fft_blocking(Plan& P, int N_rhs) {
+  Plan::Fft& F = P.fft;
+  const int64_t cols = (int64_t)P.N_pairs * N_rhs;
+  F.ZR = (int)std::max<int64_t>(4, std::min<int64_t>(64, cols * F.n_ws / 24576));
+  F.ZR = std::min(F.ZR, F.n_ws);
+  F.NZB = (F.n_ws + F.ZR - 1) / F.ZR;
+  const int64_t wg = (int64_t)F.n_ws * N_rhs;
+  F.FG = (int)std::max<int64_t>(1, std::min<int64_t>({(3072 + wg - 1) / wg, P.N_pairs / 32, 64}));
+}
+
+static FftInst make_fft_inst(const Plan& P, int N_rhs) {
+  const Plan::Fft& F = P.fft;
+  FftInst I;
+  std::memset(&I, 0, sizeof(I));
+  I.H = (decltype(I.H))F.d_H;
+  I.P = (decltype(I.P))P.d_p;
+  I.slot = (decltype(I.slot))F.d_slot;
+  I.col = (decltype(I.col))F.d_col;
+  I.gs = (decltype(I.gs))F.d_gs;
+  I.wt = (decltype(I.wt))F.d_wt;
+  I.vp = (decltype(I.vp))F.d_vp;
+  I.gp = (decltype(I.gp))F.d_gp;
+  I.N_pts = P.N_pts;
+  I.N_e = P.N_e;
+  I.Np = P.Np;
+  I.nq = F.shape.nq;
+  I.n_ws = F.n_ws;
+  I.n_cols = P.N_pairs;
+  I.N_rhs = N_rhs;
+  I.NZB = F.NZB;
+  I.ZR = F.ZR;
+  I.FG = F.FG;
+  return I;
+}
+
+// Workgroup ranges of the set's instances and their device copy.
+static void finalize_fft_set(FftSet& S) {
+  int64_t f = 0, a = 0;
+  for (FftInst& I : S.inst) {
+    I.wg_f = (int)f;
+    f += ((int64_t)I.n_cols * I.N_rhs * I.NZB + 3) / 4;
+    I.wg_a = (int)a;
+    a += (int64_t)I.n_ws * I.N_rhs * I.FG;
+    if (f > INT32_MAX - 64 || a > INT32_MAX - 64)
+      throw Error(BORN_ERR_UNSUPPORTED, "too many right-hand sides for one launch");
+  }
+  S.n_wg_f = (int)f;
+  S.n_wg_a = (int)a;
+  if (!S.d_inst) S.d_inst = dalloc<FftInst>(MAX_BATCH);
+  HIP_CHECK(hipMemcpy(S.d_inst, S.inst.data(), S.inst.size() * sizeof(FftInst), hipMemcpyHostToDevice));
+}
+
+static void build_fft_workspace(Plan& P, int N_rhs) {
+  Plan::Fft& F = P.fft;
+  fft_blocking(P, N_rhs);
+  F.d_gs = dalloc<float2>((size_t)N_rhs * F.n_ws * (F.shape.nq <= 8 ? 8 : 16) * 64);
+  F.d_vp = dalloc<float2>((size_t)F.NZB * N_rhs * P.N_pairs * P.N_e);
+  F.d_wt = dalloc<float2>((size_t)P.N_pairs * N_rhs * 16 * F.shape.TL);
+  if (F.FG > 1) F.d_gp = dalloc<float2>((size_t)F.FG * N_rhs * P.N_pts);
+  F.set.inst.assign(1, make_fft_inst(P, N_rhs));
+  F.set.d_tw = F.d_tw;
+  F.set.TL = F.shape.TL;
+  F.set.half = F.shape.nq <= 8;
+  finalize_fft_set(F.set);
+}
 
 static void materialize_shift(Plan& P);
 
@@ -774,7 +897,7 @@ static void build_workspace(Plan& P, int N_rhs);
 // could not get its workspace holds none.
 static void ensure_workspace(Plan& P, int N_rhs) {
   const bool split = P.precision != BORN_PRECISION_FP32;
-  if (P.ws_rhs == N_rhs && (N_rhs == 1 || P.ws_split == split)) return;
+  if (P.ws_rhs == N_rhs && (N_rhs == 1 || P.fft.ok || P.ws_split == split)) return;
   free_workspace(P);
   P.ws_split = split;
   try {
@@ -788,6 +911,16 @@ static void ensure_workspace(Plan& P, int N_rhs) {
 static void build_workspace(Plan& P, int N_rhs) {
   P.chunks.clear();
   P.col_pair.clear();
+  if (P.fft.ok) {   // V, W and the masked input also serve the general path
+    P.d_V = dalloc<double2>((size_t)P.N_pairs * P.N_e * N_rhs);
+    P.d_W = dalloc<float2>((size_t)P.N_pairs * P.N_e * N_rhs);
+    P.d_gm = dalloc<float2>((size_t)N_rhs * P.N_pts);
+    build_fft_workspace(P, N_rhs);
+    HIP_CHECK(hipDeviceSynchronize());
+    P.ws_rhs = N_rhs;
+    ++P.ws_gen;
+    return;
+  }
   std::vector<int> pr_chunk((size_t)P.N_pairs * N_rhs, -1), pr_pos((size_t)P.N_pairs * N_rhs, -1);
   for (int r = 0; r < N_rhs; ++r)
     for (int fg = 0; fg < P.N_fu; ++fg) {
@@ -982,10 +1115,12 @@ struct NoAllocView {
   explicit NoAllocView(Plan& P_) : P(P_), timing(P_.timing) {
     swap_all();
     P.timing = false;
+    P.in_noalloc = true;
   }
   ~NoAllocView() {
     swap_all();
     P.timing = timing;
+    P.in_noalloc = false;
   }
   void swap_all() {
     Plan::NoAlloc& A = P.na;
@@ -1065,6 +1200,7 @@ static void finish_plan(Plan& P, bool structure_known = false) {
   set_max_lds_split(160 * 1024);
   set_max_lds_split3(160 * 1024);
   set_max_lds_fc(160 * 1024);
+  build_fft(P);
   build_noalloc_layout(P);
   HIP_CHECK(hipStreamSynchronize(P.stream));
 }
@@ -1378,7 +1514,21 @@ static int fwd_blocks(const LaunchSet& L, int precision, const Inst& I) {
   return fc_path(L, precision) || precision == BORN_PRECISION_FP32 ? I.NZB : I.NZB_s * I.nseg_s;
 }
 
-static void forward_device(Plan& P, const float2* gm, int N_rhs, void* u, bool out_f64, hipStream_t s) {
+// gm: the input, masked by the occupancy rule unless `mask` (fast-correlation
+// plans apply the rule as they reorder the input).
+static void forward_device(Plan& P, const float2* gm, int N_rhs, void* u, bool out_f64, hipStream_t s,
+                           bool mask = false) {
+  if (use_fft(P)) {
+    launch_fft_gamma(P, gm, N_rhs, mask, s);
+    {
+      TimedLaunch t(P, s, 0);
+      launch_fft_fwd(P.fft.set, s);
+    }
+    launch_fft_reduce(P, N_rhs, s);
+    launch_fwd_mix(P, N_rhs, u, out_f64, s);
+    HIP_CHECK(hipGetLastError());
+    return;
+  }
   if (use_structured(P)) {
     P.ls.f16 = P.ls_fwd.f16 = P.precision == BORN_PRECISION_SPLIT_FP16;
     fp16_scales(P, true, N_rhs, s);
@@ -1407,6 +1557,16 @@ static void forward_device(Plan& P, const float2* gm, int N_rhs, void* u, bool o
 }
 
 static void adjoint_device(Plan& P, const float2* u, int N_rhs, float2* g, hipStream_t s) {
+  if (use_fft(P)) {
+    launch_fft_weights(P, u, N_rhs, s);
+    TimedLaunch t(P, s, 1);
+    OutPtrs outs;
+    outs.p[0] = g;
+    launch_fft_adj(P.fft.set, outs, s);
+    launch_fft_adj_reduce(P, N_rhs, g, s);
+    HIP_CHECK(hipGetLastError());
+    return;
+  }
   launch_adj_unmix(P, u, N_rhs, use_structured(P), s);
   if (use_structured(P)) {
     P.ls.f16 = P.precision == BORN_PRECISION_SPLIT_FP16;
@@ -1566,6 +1726,10 @@ struct Batch {
   LaunchSet sets[N_SETS];
   std::vector<int> set_of;         // per plan: its launch set
   std::vector<int> slot;           // per plan: its index in its launch set
+  // plans on the fast lateral correlation: a launch per transform length and
+  // half-full form (set_of = -1 - index)
+  static constexpr int N_FSETS = 6;
+  FftSet fsets[N_FSETS];
   Chunk* d_chunks[N_SETS] = {};
   int* d_chunk_pairs[N_SETS] = {};
   LaunchSet& set(int k) { return sets[k]; }
@@ -1606,6 +1770,7 @@ Batch::~Batch() {
     dfree(d_chunks[k]);
     dfree(d_chunk_pairs[k]);
   }
+  for (FftSet& S : fsets) dfree(S.d_inst);
   if (ev_in) hipEventDestroy(ev_in);
   if (ev_out) hipEventDestroy(ev_out);
   if (own) {
@@ -1667,6 +1832,12 @@ static void build_batch_launch(Batch& B) {
   B.slot.assign(B.plans.size(), 0);
   for (size_t i = 0; i < B.plans.size(); ++i) {
     const Plan& P = *B.plans[i];
+    if (P.fft.ok) {
+      const int k = (P.fft.shape.TL == 16 ? 0 : (P.fft.shape.TL == 8 ? 2 : 4)) + (P.fft.shape.nq <= 8 ? 0 : 1);
+      B.set_of[i] = -1 - k;
+      B.gen.push_back(P.ws_gen);
+      continue;
+    }
     const int w = fewcol_width(chunk_max_cols(P.chunks));
     // (the split forms run few-column sets on the vector kernels only for at
     // most two columns, so their 3-4-column plans join the MFMA set)
@@ -1679,12 +1850,30 @@ static void build_batch_launch(Batch& B) {
     B.gen.push_back(P.ws_gen);
   }
   for (int k = 0; k < Batch::N_SETS; ++k) build_batch_set(B, k);
+  for (int k = 0; k < Batch::N_FSETS; ++k) {
+    FftSet& S = B.fsets[k];
+    S.inst.clear();
+    for (size_t i = 0; i < B.plans.size(); ++i) {
+      if (B.set_of[i] != -1 - k) continue;
+      const Plan& P = *B.plans[i];
+      B.slot[i] = (int)S.inst.size();
+      S.inst.push_back(make_fft_inst(P, 1));
+      S.d_tw = P.fft.d_tw;
+      S.TL = P.fft.shape.TL;
+      S.half = P.fft.shape.nq <= 8;
+    }
+    if (!S.inst.empty()) finalize_fft_set(S);
+  }
   for (auto& c : B.cap) drop_graph(c);
 }
 
 static void batch_forward_enqueue(Batch& B, const void* const* in, void* const* out, hipStream_t s) {
   for (size_t i = 0; i < B.plans.size(); ++i) {
     Plan& P = *B.plans[i];
+    if (B.set_of[i] < 0) {
+      launch_fft_gamma(P, (const float2*)in[i], 1, true, s);
+      continue;
+    }
     launch_mask_gamma((const float2*)in[i], P.N_pts, 1, P.d_gm, s);
     fp16_scales(P, true, 1, s);
   }
@@ -1696,23 +1885,33 @@ static void batch_forward_enqueue(Batch& B, const void* const* in, void* const* 
     HIP_CHECK(hipEventRecord(a, s));
   }
   for (int k = 0; k < Batch::N_SETS; ++k) fwd_contract(B.set(k), B.precision, B.n_cu, s);
+  for (int k = 0; k < Batch::N_FSETS; ++k) launch_fft_fwd(B.fsets[k], s);
   if (B.timing) {
     HIP_CHECK(hipEventRecord(b, s));
     B.timed.push_back({a, b, 0});
   }
   for (size_t i = 0; i < B.plans.size(); ++i) {
     Plan& P = *B.plans[i];
-    const LaunchSet& L = B.set(B.set_of[i]);
-    launch_fwd_reduce(P, 1, fwd_blocks(L, B.precision, L.inst[B.slot[i]]), s);
+    if (B.set_of[i] < 0) {
+      launch_fft_reduce(P, 1, s);
+    } else {
+      const LaunchSet& L = B.set(B.set_of[i]);
+      launch_fwd_reduce(P, 1, fwd_blocks(L, B.precision, L.inst[B.slot[i]]), s);
+    }
     launch_fwd_mix(P, 1, out[i], false, s);
   }
   HIP_CHECK(hipGetLastError());
 }
 
 static void batch_adjoint_enqueue(Batch& B, const void* const* in, void* const* out, hipStream_t s) {
-  OutPtrs outs[Batch::N_SETS];
+  OutPtrs outs[Batch::N_SETS], fouts[Batch::N_FSETS];
   for (size_t i = 0; i < B.plans.size(); ++i) {
     Plan& P = *B.plans[i];
+    if (B.set_of[i] < 0) {
+      launch_fft_weights(P, (const float2*)in[i], 1, s);
+      fouts[-1 - B.set_of[i]].p[B.slot[i]] = (float2*)out[i];
+      continue;
+    }
     launch_adj_unmix(P, (const float2*)in[i], 1, true, s);
     fp16_scales(P, false, 1, s);
     outs[B.set_of[i]].p[B.slot[i]] = (float2*)out[i];
@@ -1725,6 +1924,9 @@ static void batch_adjoint_enqueue(Batch& B, const void* const* in, void* const* 
     HIP_CHECK(hipEventRecord(a, s));
   }
   for (int k = 0; k < Batch::N_SETS; ++k) adj_contract(B.set(k), B.precision, outs[k], s);
+  for (int k = 0; k < Batch::N_FSETS; ++k) launch_fft_adj(B.fsets[k], fouts[k], s);
+  for (size_t i = 0; i < B.plans.size(); ++i)
+    if (B.set_of[i] < 0) launch_fft_adj_reduce(*B.plans[i], 1, (float2*)out[i], s);
   if (B.timing) {
     HIP_CHECK(hipEventRecord(b, s));
     B.timed.push_back({a, b, 1});
@@ -1891,6 +2093,28 @@ static TuneResult autotune(std::vector<Plan*>& plans, LaunchSet& L, int precisio
   return best;
 }
 
+// The fast-correlation launches have no candidates: their times only.
+static void time_fft_set(const FftSet& S, const std::vector<const Plan*>& plans, hipStream_t s, float& fwd_ms,
+                         float& adj_ms) {
+  if (S.inst.empty()) return;
+  std::vector<float2*> buf;
+  OutPtrs outs;
+  try {
+    for (size_t i = 0; i < plans.size(); ++i) {
+      buf.push_back(dalloc<float2>(plans[i]->N_pts));
+      outs.p[i] = buf[i];
+    }
+    fwd_ms += time_launches([&] { launch_fft_fwd(S, s); }, s, 3);
+    adj_ms += time_launches([&] { launch_fft_adj(S, outs, s); }, s, 3);
+    HIP_CHECK(hipStreamSynchronize(s));
+  } catch (...) {
+    hipStreamSynchronize(s);
+    for (float2* g : buf) dfree(g);
+    throw;
+  }
+  for (float2* g : buf) dfree(g);
+}
+
 template <typename F>
 static int guarded(F&& f) {
   try {
@@ -1970,6 +2194,10 @@ int born_forward_dev(born_plan_t plan, const void* gamma_c64, int32_t N_rhs, voi
     HIP_CHECK(hipSetDevice(P.device));
     hipStream_t s = (hipStream_t)stream;
     ensure_workspace(P, N_rhs);
+    if (use_fft(P)) {
+      forward_device(P, (const float2*)gamma_c64, N_rhs, u_c64, false, s, true);
+      return;
+    }
     launch_mask_gamma((const float2*)gamma_c64, P.N_pts, N_rhs, P.d_gm, s);
     forward_device(P, P.d_gm, N_rhs, u_c64, false, s);
   });
@@ -2506,6 +2734,12 @@ int born_batch_autotune(born_batch_t batch, void* stream, double* fwd_ms, double
       r.fwd_ms += rk.fwd_ms;
       r.adj_ms += rk.adj_ms;
     }
+    for (int k = 0; k < Batch::N_FSETS; ++k) {
+      std::vector<const Plan*> pk;
+      for (size_t i = 0; i < B.plans.size(); ++i)
+        if (B.set_of[i] == -1 - k) pk.push_back(B.plans[i]);
+      time_fft_set(B.fsets[k], pk, s, r.fwd_ms, r.adj_ms);
+    }
     if (fwd_ms) *fwd_ms = r.fwd_ms;
     if (adj_ms) *adj_ms = r.adj_ms;
   });
@@ -2521,6 +2755,13 @@ int born_plan_autotune(born_plan_t plan, void* stream, double* fwd_ms, double* a
     ensure_workspace(P, 1);
     hipStream_t s = (hipStream_t)stream;
     HIP_CHECK(hipDeviceSynchronize());
+    if (use_fft(P)) {
+      float f = 0.f, a = 0.f;
+      time_fft_set(P.fft.set, {&P}, s, f, a);
+      if (fwd_ms) *fwd_ms = f;
+      if (adj_ms) *adj_ms = a;
+      return;
+    }
     std::vector<Plan*> one{&P};
     const TuneResult r = autotune(one, P.ls, P.precision, P.n_cu, [&] {
       P.ls.inst.assign(1, make_inst(P));

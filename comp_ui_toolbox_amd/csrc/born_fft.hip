@@ -1,0 +1,649 @@
+// 2-D contractions by fast lateral correlation (gfx950).
+//
+// With grid point i = Np*s + phi and the lateral row H of h_ref in its Np
+// phases H_phi[m] = row[ext[Np*m + phi]], element e of the array meets point
+// s of phase phi at m = s + t, t = N_e - 1 - e.  So for one (frequency, row,
+// phase) both directions are the correlation y[t or s] = sum H[s + t] x[s or t]:
+//   forward  V[e]  = sum over rows, phases and s of H[s + t] p_inc[s] gamma[s],
+//   adjoint  Y*[s] = sum over t of H[s + t] conj(W[e]),
+//            conj(gamma_hat[s]) = sum over frequencies and waves of p_inc[s] Y*[s].
+// A correlation over S points and N_e elements with S + N_e - 1 <= L is a
+// product of discrete Fourier transforms of length L; longer rows are cut
+// into segments.  The spectra of H are kept in a table, the forward sums its
+// products over rows and phases in the frequency domain and transforms back
+// once, and the adjoint transforms the weights once per (wave, frequency).
+// Each (row, wave, frequency) then costs one transform per phase instead of
+// the N_e * S products of the direct form.  All arithmetic is FP32; the
+// spectra of H are formed in FP64 and stored in FP32.
+//
+// A transform of length L = 16 * TL runs on TL lanes of a wave with 16
+// entries each, n = j + TL * q (lane j, entry q): a DFT of 16 in registers,
+// twiddles, an exchange through the wave's own LDS, and 16 / TL DFTs of TL in
+// registers, whose outputs land in the same order.  A wave carries
+// FPW = 64 / TL transforms (lane = j * FPW + g) for FPW consecutive slots;
+// slots enumerate (row, segment, phase), phase fastest, so that with 4 points
+// per pitch and L = 256 a wave reads 64 consecutive grid points per load.
+#include "born_internal.h"
+
+#include <algorithm>
+#include <cmath>
+
+#ifndef FFT_FWD_OCC
+#define FFT_FWD_OCC 2
+#endif
+#ifndef FFT_ADJ_OCC
+#define FFT_ADJ_OCC 2
+#endif
+namespace born {
+
+template <typename R>
+struct Cx {
+  R x, y;
+};
+typedef Cx<float> cf;
+
+template <typename R>
+__device__ __forceinline__ Cx<R> cadd(Cx<R> a, Cx<R> b) { return {a.x + b.x, a.y + b.y}; }
+template <typename R>
+__device__ __forceinline__ Cx<R> csub(Cx<R> a, Cx<R> b) { return {a.x - b.x, a.y - b.y}; }
+template <typename R>
+__device__ __forceinline__ Cx<R> caddi(Cx<R> a, Cx<R> b) { return {a.x - b.y, a.y + b.x}; }   // a + i b
+template <typename R>
+__device__ __forceinline__ Cx<R> csubi(Cx<R> a, Cx<R> b) { return {a.x + b.y, a.y - b.x}; }   // a - i b
+template <typename R>
+__device__ __forceinline__ Cx<R> cmulc(Cx<R> a, R c, R s) {   // a * (c + i s)
+  return {fma(a.x, c, -(a.y * s)), fma(a.x, s, a.y * c)};
+}
+template <typename R>
+__device__ __forceinline__ void cmac(Cx<R>& acc, Cx<R> a, Cx<R> b) {
+  acc.x = fma(a.x, b.x, fma(-a.y, b.y, acc.x));
+  acc.y = fma(a.x, b.y, fma(a.y, b.x, acc.y));
+}
+
+// DFT of 4, exp(+2 pi i ab / 4), in place
+template <typename R>
+__device__ __forceinline__ void dft4(Cx<R>& a, Cx<R>& b, Cx<R>& c, Cx<R>& d) {
+  const Cx<R> s = cadd(a, c), t = csub(a, c), u = cadd(b, d), v = csub(b, d);
+  a = cadd(s, u);
+  b = caddi(t, v);
+  c = csub(s, u);
+  d = csubi(t, v);
+}
+
+constexpr double FFT_C1 = 0.92387953251128675613, FFT_S1 = 0.38268343236508977173, FFT_R2 = 0.70710678118654752440;
+
+// DFT of 16, exp(+2 pi i q k / 16), in place and in order; with HALF the
+// entries q >= 8 are taken as zero.
+template <typename R, bool HALF>
+__device__ __forceinline__ void dft16(Cx<R> (&x)[16]) {
+  const R c1 = (R)FFT_C1, s1 = (R)FFT_S1, r2 = (R)FFT_R2;
+  Cx<R> t[4][4];   // t[b][c], q = 4 a + b, k = c + 4 d
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    if (HALF) {
+      t[b][0] = cadd(x[b], x[4 + b]);
+      t[b][1] = caddi(x[b], x[4 + b]);
+      t[b][2] = csub(x[b], x[4 + b]);
+      t[b][3] = csubi(x[b], x[4 + b]);
+    } else {
+      t[b][0] = x[b];
+      t[b][1] = x[4 + b];
+      t[b][2] = x[8 + b];
+      t[b][3] = x[12 + b];
+      dft4(t[b][0], t[b][1], t[b][2], t[b][3]);
+    }
+  }
+  auto r8 = [&](Cx<R> a) -> Cx<R> { return {r2 * (a.x - a.y), r2 * (a.x + a.y)}; };     // * exp(i pi / 4)
+  auto r38 = [&](Cx<R> a) -> Cx<R> { return {-r2 * (a.x + a.y), r2 * (a.x - a.y)}; };   // * exp(3 i pi / 4)
+  t[1][1] = cmulc(t[1][1], c1, s1);
+  t[1][2] = r8(t[1][2]);
+  t[1][3] = cmulc(t[1][3], s1, c1);
+  t[2][1] = r8(t[2][1]);
+  t[2][2] = {-t[2][2].y, t[2][2].x};
+  t[2][3] = r38(t[2][3]);
+  t[3][1] = cmulc(t[3][1], s1, c1);
+  t[3][2] = r38(t[3][2]);
+  t[3][3] = cmulc(t[3][3], -c1, -s1);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    dft4(t[0][c], t[1][c], t[2][c], t[3][c]);
+    x[c] = t[0][c];
+    x[c + 4] = t[1][c];
+    x[c + 8] = t[2][c];
+    x[c + 12] = t[3][c];
+  }
+}
+
+// DFT of 8, in order
+template <typename R>
+__device__ __forceinline__ void dft8(Cx<R> (&x)[8]) {
+  const R r2 = (R)FFT_R2;
+  Cx<R> e[4] = {x[0], x[2], x[4], x[6]}, o[4] = {x[1], x[3], x[5], x[7]};
+  dft4(e[0], e[1], e[2], e[3]);
+  dft4(o[0], o[1], o[2], o[3]);
+  o[1] = {r2 * (o[1].x - o[1].y), r2 * (o[1].x + o[1].y)};
+  o[2] = {-o[2].y, o[2].x};
+  o[3] = {-r2 * (o[3].x + o[3].y), r2 * (o[3].x - o[3].y)};
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    x[c] = cadd(e[c], o[c]);
+    x[c + 4] = csub(e[c], o[c]);
+  }
+}
+
+// LDS entries of one wave: 16 rows of 64 lanes, padded by FPW entries so that
+// the reads of the exchange (rows j', lanes j * FPW + g) fall on all banks.
+template <int TL>
+struct FftShape {
+  static constexpr int FPW = 64 / TL, ROW = 64 + FPW, LDS = 16 * ROW;
+};
+
+// Transform of the FPW length-16*TL sequences of a wave, exp(+2 pi i n k / L):
+// x[q] holds entry j + TL * q on entry and on return.  tw: the lane's twiddles
+// exp(2 pi i j k / L), k = 0 .. 15; lds: the wave's own exchange buffer (the
+// LDS operations of one wave complete in order, so no barrier is needed).
+template <typename R, int TL, bool HALF>
+__device__ __forceinline__ void fft_wave(Cx<R> (&x)[16], const Cx<R> (&tw)[16], Cx<R>* lds, int lane) {
+  constexpr int FPW = FftShape<TL>::FPW, ROW = FftShape<TL>::ROW;
+  const int j = lane / FPW, g = lane % FPW;
+  dft16<R, HALF>(x);
+#pragma unroll
+  for (int k = 0; k < 16; ++k) lds[k * ROW + lane] = k == 0 ? x[0] : cmulc(x[k], tw[k].x, tw[k].y);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  if constexpr (TL == 16) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) x[i] = lds[j * ROW + i * FPW + g];
+    dft16<R, false>(x);
+  } else if constexpr (TL == 8) {
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      Cx<R> y[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) y[i] = lds[(j + 8 * m) * ROW + i * FPW + g];
+      dft8(y);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) x[m + 2 * k] = y[k];
+    }
+  } else {
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      Cx<R> y[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[i] = lds[(j + 4 * m) * ROW + i * FPW + g];
+      dft4(y[0], y[1], y[2], y[3]);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) x[m + 4 * k] = y[k];
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <int TL>
+__device__ __forceinline__ void load_twiddles(const float2* __restrict__ tw, int j, cf (&t)[16]) {
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    const float2 v = tw[j * 16 + k];
+    t[k] = {v.x, v.y};
+  }
+}
+
+// ------------------------------------------------------------------ spectra
+// H[f][slot] (FP64 transform of the FP32 row, conjugated twice for the
+// exponent's sign) and the layout its readers take: per group of FPW slots
+// [8][64 lanes][2] entries, so that a lane reads two entries at once.
+template <int TL>
+__global__ __launch_bounds__(64) void k_fft_table(const float2* __restrict__ h, const int* __restrict__ ext,
+                                                  const int* __restrict__ hrow, int H_plane, int HR, int N_ext, int Np,
+                                                  int nseg, int Sv, int n_slots, int n_ws, float2* __restrict__ H) {
+  constexpr int FPW = FftShape<TL>::FPW, L = 16 * TL;
+  __shared__ Cx<double> lds[FftShape<TL>::LDS];
+  const int lane = threadIdx.x, j = lane / FPW, g = lane % FPW;
+  const int ws = blockIdx.x, f = blockIdx.y;
+  Cx<double> tw[16], x[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    double s, c;
+    sincospi(2.0 * (double)(j * k) / L, &s, &c);
+    tw[k] = {c, s};
+  }
+  const int slot = ws * FPW + g;
+  const bool ok = slot < n_slots;
+  const int phi = slot % Np, rs = slot / Np;
+  const int seg = rs % nseg, row = rs / nseg;
+  const float2* src = h + (size_t)f * H_plane + (ok ? (size_t)hrow[row] * HR : 0);
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    const int t = Np * (seg * Sv + j + TL * q) + phi;
+    x[q] = {0.0, 0.0};
+    if (ok && t < N_ext) {
+      const float2 v = src[ext[t]];
+      x[q] = {(double)v.x, -(double)v.y};
+    }
+  }
+  fft_wave<double, TL, false>(x, tw, lds, lane);
+  float4* out = reinterpret_cast<float4*>(H + ((size_t)f * n_ws + ws) * 1024);
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+    out[q * 64 + lane] = make_float4((float)x[2 * q].x, -(float)x[2 * q].y, (float)x[2 * q + 1].x, -(float)x[2 * q + 1].y);
+}
+
+// ------------------------------------------------------------------ forward
+// Blocks in logical order: blocks are dispatched round-robin over the XCDS
+// dies, so block b takes logical block (b % XCDS) * per + b / XCDS and the
+// columns of one frequency, which read the same spectra, run on one die.
+__device__ __forceinline__ int logical_block(int per) { return (blockIdx.x % XCDS) * per + blockIdx.x / XCDS; }
+
+__device__ __forceinline__ const FftInst& fft_instance(const FftInst* inst, int n_inst, int wg, bool fwd) {
+  int i = 0;
+  while (i + 1 < n_inst && wg >= (fwd ? inst[i + 1].wg_f : inst[i + 1].wg_a)) ++i;
+  return inst[i];
+}
+
+// The masked input (occupancy, cu:466-488: a point takes part iff some
+// right-hand side has |Re| or |Im| above DBL_EPSILON) in the order the forward
+// reads it: gs[r][group of slots][NQ / 2][64 lanes][2], zero where a lane's
+// entry lies past its slot, so that the forward needs no bounds on it.
+template <int TL, int NQ>
+__global__ __launch_bounds__(256) void k_fft_gamma(const float2* __restrict__ gm, const int2* __restrict__ slot, int n_ws,
+                                                   int N_pts, int Np, int N_rhs, int mask, float2* __restrict__ gs) {
+  constexpr int FPW = FftShape<TL>::FPW;
+  const size_t idx = blockIdx.x * (size_t)256 + threadIdx.x;
+  if (idx >= (size_t)n_ws * NQ * 64) return;
+  const int lane = (int)(idx >> 1) & 63;
+  const int q = (int)((idx >> 7) % (NQ / 2)) * 2 + (int)(idx & 1);
+  const int ws = (int)((idx >> 7) / (NQ / 2));
+  const int2 sl = slot[ws * FPW + lane % FPW];
+  const int sp = lane / FPW + TL * q;
+  bool occ = sp < sl.y;
+  const int at = sl.x + (occ ? Np * sp : 0);
+  if (occ && mask) {
+    occ = false;
+    for (int r = 0; r < N_rhs; ++r) {
+      const float2 v = gm[(size_t)r * N_pts + at];
+      occ |= fabsf(v.x) > 2.220446049250313e-16f || fabsf(v.y) > 2.220446049250313e-16f;
+    }
+  }
+  for (int r = 0; r < N_rhs; ++r)
+    gs[(size_t)r * n_ws * NQ * 64 + idx] = occ ? gm[(size_t)r * N_pts + at] : make_float2(0.f, 0.f);
+}
+
+// One wave per (slot block, column, right-hand side): column = pair in
+// frequency order.  The products with the spectra of H add up in registers
+// over the wave's slots; their transform back gives the slot block's partial
+// sums of the elements.  NP: points per pitch (0: any).  A lane reads p_inc
+// past its slot's end up to the last grid point (times a zero of gs).
+template <int TL, bool HALF, int NP>
+__global__ __launch_bounds__(256, FFT_FWD_OCC) void k_fft_fwd(const FftInst* __restrict__ inst, int n_inst,
+                                                    const float2* __restrict__ twid, int n_wg, int per) {
+  constexpr int FPW = FftShape<TL>::FPW, L = 16 * TL, NQ = HALF ? 8 : 16;
+  __shared__ cf lds_all[4 * FftShape<TL>::LDS];
+  const int wg = logical_block(per);
+  if (wg >= n_wg) return;
+  const FftInst& I = fft_instance(inst, n_inst, wg, true);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int task = (wg - I.wg_f) * 4 + wave;
+  const int n_cols = I.n_cols, N_rhs = I.N_rhs;
+  if (task >= n_cols * N_rhs * I.NZB) return;
+  cf* lds = lds_all + wave * FftShape<TL>::LDS;
+  const int j = lane / FPW, g = lane % FPW;
+  const int r = task % N_rhs, cz = task / N_rhs;
+  const int c = cz % n_cols, zb = cz / n_cols;
+  const int2 pf = I.col[c];   // pair, frequency
+  const int ws0 = zb * I.ZR, ws1 = min(I.n_ws, ws0 + I.ZR);
+  BORN_GLOBAL const float2* P = I.P + (size_t)pf.x * I.N_pts;
+  BORN_GLOBAL const float4* gs = (BORN_GLOBAL const float4*)I.gs + ((size_t)r * I.n_ws + ws0) * (NQ * 32) + lane;
+  BORN_GLOBAL const float4* H = (BORN_GLOBAL const float4*)(I.H + ((size_t)pf.y * I.n_ws + ws0) * 1024) + lane;
+  BORN_GLOBAL const int2* slots = I.slot + g;
+  const int Np = NP > 0 ? NP : I.Np, nq = I.nq, last = I.N_pts - 1;
+  cf tw[16], G[16];
+  load_twiddles<TL>(twid, j, tw);
+#pragma unroll
+  for (int q = 0; q < 16; ++q) G[q] = {0.f, 0.f};
+  float2 pv[NQ];
+  float4 gv[NQ / 2];
+  auto load = [&](int base) {
+    const int at = base + Np * j;
+    if (base > last - Np * (TL * NQ)) {   // near the end of the grid
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+        if (q < nq) pv[q] = P[min(at + Np * (TL * q), last)];
+    } else {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+        if (q < nq) pv[q] = P[at + Np * (TL * q)];
+    }
+#pragma unroll
+    for (int q = 0; q < NQ / 2; ++q)
+      if (2 * q < nq) gv[q] = gs[q * 64];
+    gs += NQ * 32;
+  };
+  load(slots[ws0 * FPW].x);
+  int next = slots[min(ws0 + 1, ws1 - 1) * FPW].x;
+  for (int ws = ws0; ws < ws1; ++ws) {
+    cf x[16];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      x[q] = {0.f, 0.f};
+      if (q < nq) {
+        const float gx = q & 1 ? gv[q / 2].z : gv[q / 2].x, gy = q & 1 ? gv[q / 2].w : gv[q / 2].y;
+        x[q] = {fmaf(pv[q].x, gx, -(pv[q].y * gy)), fmaf(pv[q].x, gy, pv[q].y * gx)};
+      }
+    }
+    float4 hv[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) hv[q] = H[q * 64];
+    H += 512;
+    if (ws + 1 < ws1) {
+      load(next);
+      next = slots[min(ws + 2, ws1 - 1) * FPW].x;
+    }
+    fft_wave<float, TL, HALF>(x, tw, lds, lane);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      cmac(G[2 * q], cf{hv[q].x, hv[q].y}, x[2 * q]);
+      cmac(G[2 * q + 1], cf{hv[q].z, hv[q].w}, x[2 * q + 1]);
+    }
+  }
+  // sum over the wave's slots, transform back, store elements e = N_e - 1 - t
+#pragma unroll
+  for (int q = 0; q < 16; ++q)
+#pragma unroll
+    for (int m = 1; m < FPW; m <<= 1) {
+      G[q].x += __shfl_xor(G[q].x, m);
+      G[q].y += __shfl_xor(G[q].y, m);
+    }
+  fft_wave<float, TL, false>(G, tw, lds, lane);
+  if (g == 0) {
+    BORN_GLOBAL float2* out = I.vp + ((size_t)(zb * N_rhs + r) * n_cols + c) * I.N_e;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const int t = j + TL * q;
+      if (t < I.N_e) out[I.N_e - 1 - t] = make_float2(G[q].x * (1.f / L), G[q].y * (1.f / L));
+    }
+  }
+}
+
+// Slot-block partials -> V[pair][e][r] (FP64 sums)
+__global__ __launch_bounds__(256) void k_fft_reduce(const float2* __restrict__ vp, const int2* __restrict__ col, int n_cols,
+                                                    int NZB, int N_e, int N_rhs, double2* __restrict__ V) {
+  const size_t idx = blockIdx.x * (size_t)256 + threadIdx.x;
+  const size_t plane = (size_t)n_cols * N_e;
+  if (idx >= plane * N_rhs) return;
+  const int r = (int)(idx / plane);
+  const size_t ce = idx - (size_t)r * plane;
+  const int c = (int)(ce / N_e), e = (int)(ce - (size_t)c * N_e);
+  double sx = 0.0, sy = 0.0;
+  for (int zb = 0; zb < NZB; ++zb) {
+    const float2 v = vp[((size_t)zb * N_rhs + r) * plane + ce];
+    sx += v.x;
+    sy += v.y;
+  }
+  V[((size_t)col[c].x * N_e + e) * N_rhs + r] = make_double2(sx, sy);
+}
+
+// ------------------------------------------------------------------ adjoint
+// Un-mixing (as k_adj_unmix) and the spectra of the weights: a wave takes FPW
+// (pair, right-hand side) rows, entry t = N_e - 1 - e holds conj(W[e]) / L.
+// wt[row][8][TL lanes][2].
+template <int TL>
+__global__ __launch_bounds__(256) void k_fft_weights(const float2* __restrict__ u, const int64_t* __restrict__ pe_off,
+                                                     const int2* __restrict__ pe_ent, const double2* __restrict__ pref,
+                                                     const float2* __restrict__ twid, int N_pairs, int N_e,
+                                                     int N_rhs, int64_t N_obs, float4* __restrict__ wt) {
+  constexpr int FPW = FftShape<TL>::FPW, L = 16 * TL;
+  __shared__ cf lds_all[4 * FftShape<TL>::LDS];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int j = lane / FPW, g = lane % FPW;
+  const int row = (blockIdx.x * 4 + wave) * FPW + g;
+  const bool ok = row < N_pairs * N_rhs;
+  const int pair = ok ? row / N_rhs : 0, r = ok ? row - pair * N_rhs : 0;
+  const float2* ur = u + (int64_t)r * N_obs;
+  cf tw[16], x[16];
+  load_twiddles<TL>(twid, j, tw);
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    const int t = j + TL * q;
+    x[q] = {0.f, 0.f};
+    if (ok && t < N_e) {
+      const size_t pe = (size_t)pair * N_e + (N_e - 1 - t);
+      double sx = 0.0, sy = 0.0;
+      for (int64_t i = pe_off[pe]; i < pe_off[pe + 1]; ++i) {
+        const int2 oe = pe_ent[i];
+        const double2 c = pref[oe.y];
+        const float2 v = ur[oe.x];
+        sx += c.x * v.x + c.y * v.y;
+        sy += c.x * v.y - c.y * v.x;
+      }
+      x[q] = {(float)sx * (1.f / L), -(float)sy * (1.f / L)};
+    }
+  }
+  fft_wave<float, TL, false>(x, tw, lds_all + wave * FftShape<TL>::LDS, lane);
+  if (!ok) return;
+  float4* out = wt + (size_t)row * (L / 2) + j;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) out[q * TL] = make_float4(x[2 * q].x, x[2 * q].y, x[2 * q + 1].x, x[2 * q + 1].y);
+}
+
+// One workgroup per (slot group, right-hand side, column group); its 4 waves
+// share the group's columns and add up their sums through LDS.
+template <int TL, bool HALF>
+__global__ __launch_bounds__(256, FFT_ADJ_OCC) void k_fft_adj(const FftInst* __restrict__ inst, int n_inst, OutPtrs outs,
+                                                    const float2* __restrict__ twid, int n_wg, int per) {
+  constexpr int FPW = FftShape<TL>::FPW, NQ = HALF ? 8 : 16;
+  __shared__ cf lds_all[4 * FftShape<TL>::LDS];
+  const int wg = logical_block(per);
+  if (wg >= n_wg) return;
+  const FftInst& I = fft_instance(inst, n_inst, wg, false);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int j = lane / FPW, g = lane % FPW;
+  cf* lds = lds_all + wave * FftShape<TL>::LDS;
+  const int N_rhs = I.N_rhs, n_cols = I.n_cols, FG = I.FG;
+  int t = wg - I.wg_a;
+  const int r = t % N_rhs;
+  t /= N_rhs;
+  const int ws = t % I.n_ws, fgr = t / I.n_ws;
+  const int part = fgr * 4 + wave;   // of 4 FG contiguous column ranges
+  const int c0 = (int)((long)n_cols * part / (4 * FG)), c1 = (int)((long)n_cols * (part + 1) / (4 * FG));
+  const int2 sl = I.slot[ws * FPW + g];
+  const int Np = I.Np, nq = I.nq;
+  int at[NQ];
+  bool ok[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const int s = j + TL * q;
+    ok[q] = s < sl.y;
+    at[q] = sl.x + (ok[q] ? Np * s : 0);
+  }
+  cf tw[16], acc[NQ];
+  load_twiddles<TL>(twid, j, tw);
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) acc[q] = {0.f, 0.f};
+  float4 hv[8];
+  int f_have = -1;
+  for (int c = c0; c < c1; ++c) {
+    const int2 pf = I.col[c];
+    BORN_GLOBAL const float2* P = I.P + (size_t)pf.x * I.N_pts;
+    float2 pv[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+      if (q < nq) pv[q] = P[at[q]];
+    if (pf.y != f_have) {
+      f_have = pf.y;
+      BORN_GLOBAL const float4* H = (BORN_GLOBAL const float4*)(I.H + ((size_t)pf.y * I.n_ws + ws) * 1024) + lane;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) hv[q] = H[q * 64];
+    }
+    BORN_GLOBAL const float4* wt = (BORN_GLOBAL const float4*)I.wt + ((size_t)pf.x * N_rhs + r) * (8 * TL) + j;
+    cf x[16];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const float4 w = wt[q * TL];
+      x[2 * q] = {fmaf(hv[q].x, w.x, -(hv[q].y * w.y)), fmaf(hv[q].x, w.y, hv[q].y * w.x)};
+      x[2 * q + 1] = {fmaf(hv[q].z, w.z, -(hv[q].w * w.w)), fmaf(hv[q].z, w.w, hv[q].w * w.z)};
+    }
+    fft_wave<float, TL, false>(x, tw, lds, lane);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+      if (q < nq) cmac(acc[q], cf{pv[q].x, pv[q].y}, x[q]);
+  }
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) lds[q * 64 + lane] = acc[q];
+  __syncthreads();
+  BORN_GLOBAL float2* out = FG > 1 ? I.gp + (size_t)fgr * N_rhs * I.N_pts : (BORN_GLOBAL float2*)outs.p[&I - inst];
+  out += (size_t)r * I.N_pts;
+#pragma unroll
+  for (int q = 0; q < NQ; ++q)
+    if ((q & 3) == wave && q < nq && ok[q]) {
+      cf s = {0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < 4; ++w) s = cadd(s, lds_all[w * FftShape<TL>::LDS + q * 64 + lane]);
+      out[at[q]] = make_float2(s.x, -s.y);
+    }
+}
+
+__global__ __launch_bounds__(256) void k_fft_adj_reduce(const float2* __restrict__ gp, int FG, size_t n,
+                                                        float2* __restrict__ out) {
+  const size_t i = blockIdx.x * (size_t)256 + threadIdx.x;
+  if (i >= n) return;
+  float2 s = gp[i];
+  for (int k = 1; k < FG; ++k) {
+    const float2 v = gp[(size_t)k * n + i];
+    s.x += v.x;
+    s.y += v.y;
+  }
+  out[i] = s;
+}
+
+// ------------------------------------------------------------------ host side
+// Transform length and segments of a row of S points per phase under N_e
+// elements: the cheapest of the lengths (time grows with the entries
+// transformed; sequences at most half full skip part of the first stage).
+FftShapeChoice fft_shape(int Nx, int Np, int N_e) {
+  FftShapeChoice best;
+  const int S = (Nx + Np - 1) / Np;
+  double cost_best = 1e300;
+  for (int TL = 4; TL <= 16; TL *= 2) {
+    const int L = 16 * TL;
+    if (L < N_e) continue;
+    const int room = L - N_e + 1;
+    FftShapeChoice c;
+    c.TL = TL;
+    c.nseg = (S + room - 1) / room;
+    c.Sv = (S + c.nseg - 1) / c.nseg;
+    c.nq = (c.Sv + TL - 1) / TL;
+    const double cost = (double)c.nseg * L * (c.nq <= 8 ? 1.0 : 1.12);
+    if (cost < cost_best) {
+      cost_best = cost;
+      best = c;
+    }
+  }
+  return best;
+}
+
+void fft_twiddles(int TL, std::vector<float2>& tw) {
+  tw.resize((size_t)TL * 16);
+  for (int j = 0; j < TL; ++j)
+    for (int k = 0; k < 16; ++k) {
+      const double a = 2.0 * M_PI * j * k / (16.0 * TL);
+      tw[(size_t)j * 16 + k] = make_float2((float)std::cos(a), (float)std::sin(a));
+    }
+}
+
+void launch_fft_table(const Plan& P, hipStream_t s) {
+  const Plan::Fft& F = P.fft;
+  const dim3 grid(F.n_ws, P.N_fu);
+#define BORN_FFT_TABLE(TLv)                                                                                            \
+  hipLaunchKernelGGL(k_fft_table<TLv>, grid, dim3(64), 0, s, P.d_h, P.d_ext, P.d_hrow, P.H_plane, P.HR, P.N_ext, P.Np, \
+                     F.shape.nseg, F.shape.Sv, F.n_slots, F.n_ws, F.d_H)
+  if (F.shape.TL == 16) BORN_FFT_TABLE(16);
+  else if (F.shape.TL == 8) BORN_FFT_TABLE(8);
+  else BORN_FFT_TABLE(4);
+#undef BORN_FFT_TABLE
+}
+
+#define BORN_FFT_DISPATCH(K, ...)                                             \
+  do {                                                                        \
+    if (S.TL == 16 && S.half) hipLaunchKernelGGL((K<16, true>), __VA_ARGS__); \
+    else if (S.TL == 16) hipLaunchKernelGGL((K<16, false>), __VA_ARGS__);     \
+    else if (S.TL == 8 && S.half) hipLaunchKernelGGL((K<8, true>), __VA_ARGS__); \
+    else if (S.TL == 8) hipLaunchKernelGGL((K<8, false>), __VA_ARGS__);       \
+    else if (S.half) hipLaunchKernelGGL((K<4, true>), __VA_ARGS__);           \
+    else hipLaunchKernelGGL((K<4, false>), __VA_ARGS__);                      \
+  } while (0)
+
+void launch_fft_gamma(const Plan& P, const float2* gamma, int N_rhs, bool mask, hipStream_t s) {
+  const Plan::Fft& F = P.fft;
+  const int NQ = F.shape.nq <= 8 ? 8 : 16;
+  const dim3 grid((unsigned)(((size_t)F.n_ws * NQ * 64 + 255) / 256));
+#define BORN_FFT_G(TLv, NQv)                                                                                         \
+  hipLaunchKernelGGL((k_fft_gamma<TLv, NQv>), grid, dim3(256), 0, s, gamma, F.d_slot, F.n_ws, P.N_pts, P.Np, N_rhs, \
+                     (int)mask, F.d_gs)
+  if (F.shape.TL == 16 && NQ == 8) BORN_FFT_G(16, 8);
+  else if (F.shape.TL == 16) BORN_FFT_G(16, 16);
+  else if (F.shape.TL == 8 && NQ == 8) BORN_FFT_G(8, 8);
+  else if (F.shape.TL == 8) BORN_FFT_G(8, 16);
+  else if (NQ == 8) BORN_FFT_G(4, 8);
+  else BORN_FFT_G(4, 16);
+#undef BORN_FFT_G
+}
+
+void launch_fft_fwd(const FftSet& S, hipStream_t s) {
+  if (S.inst.empty()) return;
+  const int per = (S.n_wg_f + XCDS - 1) / XCDS;
+  int Np = S.inst[0].Np;
+  for (const FftInst& I : S.inst)
+    if (I.Np != Np) Np = 0;
+#define BORN_FFT_F(TLv, Hv, NPv)                                                                                   \
+  hipLaunchKernelGGL((k_fft_fwd<TLv, Hv, NPv>), dim3(per * XCDS), dim3(256), 0, s, S.d_inst, (int)S.inst.size(), \
+                     S.d_tw, S.n_wg_f, per)
+#define BORN_FFT_FN(TLv, Hv)                      \
+  do {                                            \
+    if (Np == 4) BORN_FFT_F(TLv, Hv, 4);          \
+    else if (Np == 2) BORN_FFT_F(TLv, Hv, 2);     \
+    else BORN_FFT_F(TLv, Hv, 0);                  \
+  } while (0)
+  if (S.TL == 16 && S.half) BORN_FFT_FN(16, true);
+  else if (S.TL == 16) BORN_FFT_FN(16, false);
+  else if (S.TL == 8 && S.half) BORN_FFT_FN(8, true);
+  else if (S.TL == 8) BORN_FFT_FN(8, false);
+  else if (S.half) BORN_FFT_FN(4, true);
+  else BORN_FFT_FN(4, false);
+#undef BORN_FFT_FN
+#undef BORN_FFT_F
+}
+
+void launch_fft_adj(const FftSet& S, const OutPtrs& outs, hipStream_t s) {
+  if (S.inst.empty()) return;
+  const int per = (S.n_wg_a + XCDS - 1) / XCDS;
+  BORN_FFT_DISPATCH(k_fft_adj, dim3(per * XCDS), dim3(256), 0, s, S.d_inst, (int)S.inst.size(), outs, S.d_tw,
+                    S.n_wg_a, per);
+}
+
+void launch_fft_reduce(const Plan& P, int N_rhs, hipStream_t s) {
+  const size_t total = (size_t)P.N_pairs * P.N_e * N_rhs;
+  hipLaunchKernelGGL(k_fft_reduce, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, P.fft.d_vp, P.fft.d_col,
+                     P.N_pairs, P.fft.NZB, P.N_e, N_rhs, P.d_V);
+}
+
+void launch_fft_weights(const Plan& P, const float2* u, int N_rhs, hipStream_t s) {
+  const int TL = P.fft.shape.TL, FPW = 64 / TL;
+  const size_t rows = (size_t)P.N_pairs * N_rhs;
+  const dim3 grid((unsigned)((rows + 4 * FPW - 1) / (4 * FPW)));
+#define BORN_FFT_W(TLv)                                                                                              \
+  hipLaunchKernelGGL(k_fft_weights<TLv>, grid, dim3(256), 0, s, u, P.d_pe_off, P.d_pe_ent, P.d_pref,                 \
+                     P.fft.d_tw, P.N_pairs, P.N_e, N_rhs, P.N_obs, (float4*)P.fft.d_wt)
+  if (TL == 16) BORN_FFT_W(16);
+  else if (TL == 8) BORN_FFT_W(8);
+  else BORN_FFT_W(4);
+#undef BORN_FFT_W
+}
+
+void launch_fft_adj_reduce(const Plan& P, int N_rhs, float2* out, hipStream_t s) {
+  if (P.fft.FG <= 1) return;
+  const size_t n = (size_t)P.N_pts * N_rhs;
+  hipLaunchKernelGGL(k_fft_adj_reduce, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, P.fft.d_gp, P.fft.FG, n, out);
+}
+
+}  // namespace born

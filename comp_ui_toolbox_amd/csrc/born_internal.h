@@ -116,6 +116,40 @@ struct LaunchSet {
   int n_wg_f = 0;                 // adjoint workgroups of the few-column kernel
 };
 
+// Fast lateral correlation of 2-D plans (born_fft.hip): transforms of length
+// 16 * TL over rows cut into nseg segments of Sv points per phase; nq: entries
+// of a lane that can hold points.
+struct FftShapeChoice {
+  int TL = 0, nseg = 1, Sv = 0, nq = 0;
+};
+
+// One operator instance of a fast-correlation launch.
+struct FftInst {
+  BORN_GLOBAL const float2* H;     // spectra [N_fu][n_ws][8][64][2]
+  BORN_GLOBAL const float2* P;     // p_inc rows
+  BORN_GLOBAL const int2* slot;    // [n_ws * 64 / TL] first point, points (0 past the last slot)
+  BORN_GLOBAL const int2* col;     // [n_cols] (pair, frequency), by frequency
+  BORN_GLOBAL const float2* gs;    // masked input [N_rhs][n_ws][8 or 16 entries / 2][64][2]
+  BORN_GLOBAL const float2* wt;    // adjoint weight spectra [N_pairs][N_rhs][8][TL][2]
+  BORN_GLOBAL float2* vp;          // forward partials [NZB][N_rhs][n_cols][N_e]
+  BORN_GLOBAL float2* gp;          // adjoint partials [FG][N_rhs][N_pts] (FG > 1)
+  int N_pts, N_e, Np, nq;
+  int n_ws, n_cols, N_rhs;
+  int NZB, ZR;                     // forward: slot blocks of ZR wave steps
+  int FG;                          // adjoint: column groups
+  int wg_f, wg_a;                  // first workgroup of the instance (forward, adjoint)
+};
+
+// Launch of instances that share the transform length and the half-full form.
+struct FftSet {
+  FftInst* d_inst = nullptr;
+  std::vector<FftInst> inst;
+  const float2* d_tw = nullptr;    // twiddles [TL][16] (owned by a plan of the set)
+  int TL = 0;
+  bool half = false;
+  int n_wg_f = 0, n_wg_a = 0;
+};
+
 // Device tables and index maps.  All device arrays are owned by the plan.
 struct Plan {
   int device = 0;
@@ -207,6 +241,23 @@ struct Plan {
   float2* d_gm = nullptr;         // masked gamma [N_rhs][N_pts]
   int items_target = 8192;        // forward work items per launch (tunable)
   LaunchSet ls;                   // structured launch of this plan alone
+  // fast lateral correlation: tables of the plan, then the per-rhs workspace
+  struct Fft {
+    bool ok = false;
+    FftShapeChoice shape;
+    int n_slots = 0, n_ws = 0;
+    float2* d_H = nullptr;
+    int2* d_slot = nullptr;
+    int2* d_col = nullptr;
+    float2* d_tw = nullptr;
+    int NZB = 1, ZR = 1, FG = 1;
+    float2* d_gs = nullptr;
+    float2* d_vp = nullptr;
+    float2* d_wt = nullptr;
+    float2* d_gp = nullptr;
+    FftSet set;                     // launch of this plan alone
+  } fft;
+  bool in_noalloc = false;          // inside an allocation-free apply (one-rhs MFMA layout)
   // FP16 split form: operand scales [5], table maxima [2] (h_ref, p_inc),
   // block partial maxima [256]
   float* d_fscale = nullptr;
@@ -332,6 +383,17 @@ void launch_energy_rx_tgc(const Plan& P, int m, int rows, float2* spill, int spi
 void launch_adj_unmix(const Plan& P, const float2* u, int N_rhs, bool chunked, hipStream_t s);
 void launch_adj_structured(const LaunchSet& L, const OutPtrs& outs, hipStream_t s);
 void launch_adj_general(const Plan& P, int N_rhs, float2* g_out, hipStream_t s);
+
+// fast lateral correlation (born_fft.hip)
+FftShapeChoice fft_shape(int Nx, int Np, int N_e);
+void fft_twiddles(int TL, std::vector<float2>& tw);
+void launch_fft_table(const Plan& P, hipStream_t s);
+void launch_fft_gamma(const Plan& P, const float2* gamma, int N_rhs, bool mask, hipStream_t s);
+void launch_fft_fwd(const FftSet& S, hipStream_t s);
+void launch_fft_adj(const FftSet& S, const OutPtrs& outs, hipStream_t s);
+void launch_fft_reduce(const Plan& P, int N_rhs, hipStream_t s);
+void launch_fft_weights(const Plan& P, const float2* u, int N_rhs, hipStream_t s);
+void launch_fft_adj_reduce(const Plan& P, int N_rhs, float2* out, hipStream_t s);
 
 struct GeomDev {
   int nd;

@@ -1,0 +1,90 @@
+"""Fast lateral correlation of 2-D plans (born_fft.hip) against the FP64
+oracle and the general gather path, at the sizes where its transforms,
+segments and slots have edges: transform lengths 64, 128 and 256 and the
+element counts beside them, one and several segments per row, rows whose
+points per phase differ, points per pitch that do not divide a wave's slots,
+slot counts that leave padding, one column, several right-hand sides.
+
+Tolerance: three FP32 transforms of at most 256 points (the spectra's
+rounding, the data, the way back) of at most 8 stages each give a relative L2
+error below 3 * 8 * 2^-24 = 1.5e-6 in the worst case and about its square
+root of 24 part of it, 3e-7, for independent roundings; 1e-6 is taken."""
+import numpy as np
+import pytest
+
+from comp_ui_toolbox_amd import OperatorBorn
+from comp_ui_toolbox_amd import configs as C
+from oracle import born_oracle as O
+from tests.test_oracle import mixed_tiny_tables
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-6
+
+
+def make(ne, nx, nz, npp, nf, waves, n_mix=0):
+    pitch = 3e-4
+    arr = C.ArraySpec((ne,), (pitch,), (2.7e-4,), (2,))
+    med = C.MediumSpec()
+    fov = C.FovSpec((nx, nz), (pitch / npp, pitch / npp), 2e-3)
+    rng = np.random.Generator(np.random.PCG64(ne * 1000 + nx))
+    ws = [C.random_wave(arr, rng, 1e-6) for _ in range(waves)]
+    mixes = [[C.MixSpec(np.arange(ne), np.where(rng.random(ne) < 0.5, -1.0, 1.0)) for _ in range(n_mix)]
+             if n_mix else C.identity_mixes(ne) for _ in ws]
+    return C.SequenceSpec("fft", arr, med, fov, np.linspace(2e6, 6e6, nf), ws, mixes)
+
+
+# elements, points x, z, points per pitch, frequencies, waves, mixes, rhs
+SIZES = [
+    (1, 5, 3, 1, 2, 1, 0, 1),          # one element, padding slots, one wave
+    (2, 9, 1, 4, 1, 1, 0, 2),          # one row
+    (17, 70, 5, 2, 3, 2, 0, 1),        # length 64
+    (48, 130, 7, 2, 2, 3, 0, 3),       # several segments or a longer transform
+    (64, 257, 3, 4, 3, 2, 0, 1),       # 65 points in phase 0, 64 in the others
+    (65, 250, 5, 4, 2, 3, 3, 2),       # one element over half of 128
+    (100, 301, 4, 2, 3, 7, 0, 1),      # more than half full
+    (127, 516, 2, 4, 2, 2, 0, 1),      # 129 points per phase: the length 256 exactly full
+    (128, 512, 2, 4, 2, 17, 0, 1),     # 128 points per phase
+    (128, 700, 3, 4, 2, 1, 0, 1),      # two segments of unequal use
+    (33, 101, 6, 3, 3, 2, 0, 2),       # phases that do not divide the slots of a wave
+    (20, 77, 3, 5, 2, 2, 2, 1),
+    (31, 40, 9, 1, 3, 2, 0, 1),        # field of view narrower than the aperture, one point per pitch
+]
+
+
+@pytest.mark.parametrize("ne,nx,nz,npp,nf,waves,n_mix,n_rhs", SIZES)
+def test_against_oracle_and_general_path(torch_cuda, ne, nx, nz, npp, nf, waves, n_mix, n_rhs):
+    import torch
+    spec = make(ne, nx, nz, npp, nf, waves, n_mix)
+    T = O.direct_tables(spec)
+    op = OperatorBorn.from_sequence(spec)
+    assert op.path == "structured"
+    rng = np.random.Generator(np.random.PCG64(7))
+    g = rng.standard_normal((n_rhs, op.N_points)) + 1j * rng.standard_normal((n_rhs, op.N_points))
+    u = rng.standard_normal((n_rhs, op.N_observations)) + 1j * rng.standard_normal((n_rhs, op.N_observations))
+    gd = torch.tensor(g.astype(np.complex64), device="cuda:0")
+    ud = torch.tensor(u.astype(np.complex64), device="cuda:0")
+    fast = [op.forward_dev(gd).cpu().numpy(), op.adjoint_dev(ud).cpu().numpy()]
+    again = [op.forward_dev(gd).cpu().numpy(), op.adjoint_dev(ud).cpu().numpy()]
+    op.force_general(True)
+    general = [op.forward_dev(gd).cpu().numpy(), op.adjoint_dev(ud).cpu().numpy()]
+    for r in range(n_rhs):
+        ref = [O.forward(T, gd[r].cpu().numpy()), O.adjoint(T, ud[r].cpu().numpy())]
+        for k in range(2):
+            assert np.array_equal(fast[k][r], again[k][r])
+            assert O.rel_l2(fast[k][r], ref[k].reshape(-1)) < TOL, ("oracle", k)
+            assert O.rel_l2(fast[k][r], general[k][r]) < 2 * TOL, ("general", k)
+
+
+def test_mixed_tables_and_zero_columns(torch_cuda):
+    """Frequency subsets, repeated frequencies and a right-hand side that is
+    zero, from an operator's own tables."""
+    _, T = mixed_tiny_tables()
+    op = OperatorBorn.from_tables(T)
+    rng = np.random.Generator(np.random.PCG64(8))
+    g = rng.standard_normal((op.N_points, 3)) + 1j * rng.standard_normal((op.N_points, 3))
+    g[:, 1] = 0
+    u = op.forward(g)
+    for r in range(3):
+        ref = O.forward(T, g[:, r]).reshape(-1)
+        assert np.all(u[:, r] == 0) if r == 1 else O.rel_l2(u[:, r], ref) < TOL
