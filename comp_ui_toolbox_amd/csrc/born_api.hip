@@ -145,6 +145,9 @@ Plan::~Plan() {
   dfree(fft.d_col);
   dfree(fft.d_tw);
   dfree(fft.set.d_inst);
+  dfree(d_ew);
+  dfree(d_erow_off);
+  dfree(d_erows);
   dfree(d_fscale);
   dfree(d_f16max);
   dfree(d_f16part);
@@ -2244,9 +2247,50 @@ int born_apply_dev_noalloc(born_plan_t plan, int32_t mode, const void* in_c64, i
   });
 }
 
+// Tables of the received energies on the structured path (on first use).
+static void ensure_energy_tables(Plan& P) {
+  if (P.e_ready) return;
+  dfree(P.d_ew);   // of a first use that failed
+  dfree(P.d_erow_off);
+  dfree(P.d_erows);
+  const int n_meas = (int)P.meas_pair_base.size(), Ney = P.nd == 3 ? P.Ney : 1;
+  P.e_single.assign(n_meas, 0);
+  P.e_multi.assign(n_meas, 0);
+  std::vector<int64_t> off;
+  for (int mk = 0; mk < P.N_mk; ++mk) {
+    (P.mk_Nact[mk] == 1 ? P.e_single : P.e_multi)[P.mk_meas[mk]] = 1;
+    if (P.mk_Nact[mk] == 1) continue;
+    if (off.empty()) off.assign((size_t)P.N_pairs + 1, 0);
+    for (int f = 0; f < P.mk_Nf[mk]; ++f) off[P.meas_pair_base[P.mk_meas[mk]] + P.fmeas[P.mk_f_off[mk] + f] + 1]++;
+  }
+  if (!off.empty()) {
+    for (int p = 0; p < P.N_pairs; ++p) off[p + 1] += off[p];
+    std::vector<int2> rows((size_t)off.back());
+    std::vector<int64_t> fill(off.begin(), off.end() - 1);
+    for (int mk = 0; mk < P.N_mk; ++mk)
+      if (P.mk_Nact[mk] != 1)
+        for (int f = 0; f < P.mk_Nf[mk]; ++f)
+          rows[fill[P.meas_pair_base[P.mk_meas[mk]] + P.fmeas[P.mk_f_off[mk] + f]]++] = make_int2(mk, f);
+    P.d_erow_off = dupload(off, P.stream);
+    P.d_erows = dupload(rows, P.stream);
+  }
+  P.d_ew = dalloc<double>((size_t)P.N_pairs * Ney * energy_pad(P.Nex));
+  launch_energy_weights(P, P.d_ew, P.stream);
+  HIP_CHECK(hipGetLastError());
+  HIP_CHECK(hipStreamSynchronize(P.stream));   // the callers' streams read it
+  P.e_ready = true;
+}
+
 static void energy_rx(Plan& P, int m, double* E_dev, hipStream_t s) {
   if (m < 0 || m >= (int)P.meas_pair_base.size())
     throw Error(BORN_ERR_INVALID_ARGUMENT, "operator_born.indices_measurement_sel must be a single index!");
+  if (use_structured(P) && energy_fast(P)) {
+    ensure_energy_tables(P);
+    if (P.e_single[m] || !P.e_multi[m]) launch_energy_single(P, m, E_dev, s);
+    if (P.e_multi[m]) launch_energy_multi(P, m, P.e_single[m], E_dev, s);
+    HIP_CHECK(hipGetLastError());
+    return;
+  }
   ensure_shift_on_device(P);
   launch_energy_rx(P, m, E_dev, s);
   HIP_CHECK(hipGetLastError());

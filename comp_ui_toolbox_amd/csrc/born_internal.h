@@ -258,6 +258,14 @@ struct Plan {
     FftSet set;                     // launch of this plan alone
   } fft;
   bool in_noalloc = false;          // inside an allocation-free apply (one-rhs MFMA layout)
+  // received energies on the structured path, built on first use: squared
+  // prefactors of the single-element mixes by (pair, y slice, element), and
+  // the observations of the other mixes by pair (none: null)
+  bool e_ready = false;
+  std::vector<char> e_single, e_multi;   // per measurement: has such mixes
+  double* d_ew = nullptr;
+  int64_t* d_erow_off = nullptr;
+  int2* d_erows = nullptr;
   // FP16 split form: operand scales [5], table maxima [2] (h_ref, p_inc),
   // block partial maxima [256]
   float* d_fscale = nullptr;
@@ -367,6 +375,12 @@ void launch_fwd_reduce(const Plan& P, int N_rhs, int nblk, hipStream_t s);
 void launch_fwd_reduce_expanded(const Plan& P, int nblk, hipStream_t s);
 void launch_expand_pg(const Plan& P, hipStream_t s);
 void launch_energy_rx(const Plan& P, int m, double* E, hipStream_t s);
+// structured plans (born_energy.hip)
+bool energy_fast(const Plan& P);
+int energy_pad(int Nex);
+void launch_energy_weights(const Plan& P, double* ew, hipStream_t s);
+void launch_energy_single(const Plan& P, int m, double* E, hipStream_t s);
+void launch_energy_multi(const Plan& P, int m, bool add, double* E, hipStream_t s);
 void launch_fp16_scales(const Plan& P, const float* x, size_t n_floats, int which, hipStream_t s);
 void launch_time_signals(const Plan& P, const float2* u, const int* q_obs, int N_rhs, int N_t, float* rf,
                          hipStream_t s);

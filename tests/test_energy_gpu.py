@@ -1,0 +1,71 @@
+"""Received energies of structured plans (born_energy.hip) against the FP64
+oracle and the map-driven kernel of the general path, over the sizes where
+the fast kernels' lanes, windows and observation groups have edges.
+
+Tolerances: both kernels take FP64 sums of at most 1e4 positive terms of the
+same FP32 tables, 1e4 * 2^-53 = 1.1e-12 apart; the tables' rounding to FP32
+(2^-24 each in h_ref and p_inc, squared) moves E by at most 4 * 2^-24 = 2.4e-7."""
+import numpy as np
+import pytest
+
+from comp_ui_toolbox_amd import OperatorBorn
+from comp_ui_toolbox_amd import configs as C
+from oracle import born_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def mixes_of(kind, ne, nf, rng):
+    if kind == "single":
+        return [C.MixSpec(np.array([e]), np.array([1.0 + 0.1 * e])) for e in range(0, ne, 2)]
+    if kind == "dense":
+        return [C.MixSpec(np.arange(ne), rng.standard_normal(ne)) for _ in range(5)]
+    # both: one element, a sub-aperture on two frequencies, all elements reversed
+    return [C.MixSpec(np.array([ne - 1]), np.array([2.0])),
+            C.MixSpec(np.arange(ne // 3, ne // 3 + 2) % ne, np.array([1.0, -1.0]), np.array([nf - 1, 0])),
+            C.MixSpec(np.arange(ne)[::-1].copy(), rng.standard_normal(ne))]
+
+
+def check(op, T, measurements, kind):
+    for m in range(measurements):
+        fast = op.energy_rx(m)
+        op.force_general(True)
+        general = op.energy_rx(m)
+        op.force_general(False)
+        ref = O.energy_rx(T, m)
+        assert np.max(np.abs(fast - general) / general) < 2e-12
+        assert np.linalg.norm(fast - ref) < 2.4e-7 * np.linalg.norm(ref)
+        if kind == "single":
+            assert np.max(np.abs(fast - ref) / ref) < 2.4e-7
+
+
+# elements, points x, z, points per pitch
+SIZES = [(3, 9, 2, 1), (17, 130, 3, 2), (64, 384, 2, 4), (65, 257, 2, 4), (128, 515, 2, 4), (24, 101, 2, 3), (8, 150, 2, 16)]
+
+
+@pytest.mark.parametrize("kind", ["single", "dense", "both"])
+@pytest.mark.parametrize("ne,nx,nz,npp", SIZES)
+def test_linear_array(torch_cuda, ne, nx, nz, npp, kind):
+    pitch, nf = 3e-4, 5
+    rng = np.random.Generator(np.random.PCG64(nx))
+    arr = C.ArraySpec((ne,), (pitch,), (2.7e-4,), (2,))
+    fov = C.FovSpec((nx, nz), (pitch / npp, pitch / npp), 2e-3)
+    waves = [C.random_wave(arr, rng, 1e-6) for _ in range(2)]
+    spec = C.SequenceSpec("e", arr, C.MediumSpec(), fov, np.linspace(2e6, 5e6, nf), waves,
+                          [mixes_of(kind, ne, nf, rng) for _ in waves])
+    op = OperatorBorn.from_sequence(spec)
+    assert op.path == "structured"
+    check(op, O.direct_tables(spec), 2, kind)
+
+
+@pytest.mark.parametrize("kind", ["single", "both"])
+def test_matrix_array(torch_cuda, kind):
+    rng = np.random.Generator(np.random.PCG64(5))
+    arr = C.ArraySpec((5, 3), (3e-4, 3e-4), (2.7e-4, 2.7e-4), (2, 2))
+    fov = C.FovSpec((19, 7, 3), (1.5e-4, 1.5e-4, 1.5e-4), 2e-3)
+    waves = [C.qsw_wave(arr, np.array([0.0, 0.0, -5e-3]), 1500.0)]
+    spec = C.SequenceSpec("e3", arr, C.MediumSpec(), fov, np.linspace(2e6, 4e6, 3), waves,
+                          [mixes_of(kind, 15, 3, rng)])
+    op = OperatorBorn.from_sequence(spec)
+    assert op.path == "structured"
+    check(op, O.direct_tables(spec), 1, kind)
