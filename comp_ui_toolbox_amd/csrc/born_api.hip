@@ -148,6 +148,10 @@ Plan::~Plan() {
   dfree(d_ew);
   dfree(d_erow_off);
   dfree(d_erows);
+  dfree(d_col_off);
+  dfree(d_col_ent);
+  dfree(d_col_multi);
+  dfree(d_pts);
   dfree(d_fscale);
   dfree(d_f16max);
   dfree(d_f16part);
@@ -248,6 +252,17 @@ static void build_index_structures(Plan& P, int N_meas, const born_measurement_d
   }
   P.N_mk = (int)P.mk_meas.size();
   P.N_obs = obs;
+  P.regular = true;
+  for (int m = 0; m < N_meas && P.regular; ++m) {
+    P.regular = P.meas_Nfm[m] == P.N_fu;
+    for (int f = 0; f < P.N_fu && P.regular; ++f) P.regular = P.pair_fg[(size_t)m * P.N_fu + f] == f;
+  }
+  for (int mk = 0; mk < P.N_mk && P.regular; ++mk) {
+    P.regular = P.mk_Nf[mk] == P.N_fu;
+    for (int f = 0; f < P.N_fu && P.regular; ++f) P.regular = P.fmeas[(size_t)mk * P.N_fu + f] == f;
+  }
+  P.col_n_single = P.col_n_multi = 0;
+  for (int mk = 0; mk < P.N_mk; ++mk) ++(P.mk_Nact[mk] == 1 ? P.col_n_single : P.col_n_multi);
 }
 
 static void upload_index_structures(Plan& P, hipStream_t s) {
@@ -2450,6 +2465,35 @@ int born_time_signals(born_plan_t plan, const double* frequencies, double delta_
   });
 }
 
+// Tables of the columns on regular structured plans (on first use): the mixes
+// of one element, by (block of COL_EB elements, group of COL_MG measurements)
+// in mix order, as (mix, element in the block | measurement in the group << 16),
+// and the other mixes.
+static void ensure_column_tables(Plan& P) {
+  if (P.col_ready) return;
+  dfree(P.d_col_off);   // of a first use that failed
+  dfree(P.d_col_ent);
+  dfree(P.d_col_multi);
+  const int N_meas = (int)P.meas_Nfm.size();
+  const int n_eb = (P.N_e + COL_EB - 1) / COL_EB, n_mg = (N_meas + COL_MG - 1) / COL_MG;
+  std::vector<int> off((size_t)n_eb * n_mg + 1, 0), multi;
+  auto cell = [&](int mk) { return (size_t)(P.act[P.mk_a_off[mk]] / COL_EB) * n_mg + P.mk_meas[mk] / COL_MG; };
+  for (int mk = 0; mk < P.N_mk; ++mk) {
+    if (P.mk_Nact[mk] == 1) off[cell(mk) + 1]++;
+    else multi.push_back(mk);
+  }
+  for (size_t i = 0; i + 1 < off.size(); ++i) off[i + 1] += off[i];
+  std::vector<int2> ent((size_t)P.col_n_single);
+  std::vector<int> fill(off.begin(), off.end() - 1);
+  for (int mk = 0; mk < P.N_mk; ++mk)
+    if (P.mk_Nact[mk] == 1)
+      ent[fill[cell(mk)]++] = make_int2(mk, P.act[P.mk_a_off[mk]] % COL_EB | (P.mk_meas[mk] % COL_MG) << 16);
+  P.d_col_off = dupload(off, P.stream);
+  P.d_col_ent = dupload(ent, P.stream);
+  P.d_col_multi = dupload(multi, P.stream);
+  P.col_ready = true;
+}
+
 // Columns of A at 1-based points; out complex FP64 column-major N_obs x n
 // (host) or complex64 n x N_obs (device); complete on return.
 static void columns(Plan& P, const double* points, int32_t n, void* out, bool host, hipStream_t s) {
@@ -2458,23 +2502,32 @@ static void columns(Plan& P, const double* points, int32_t n, void* out, bool ho
   if ((double)n * (double)P.N_obs > 2.0e11) throw Error(BORN_ERR_INVALID_ARGUMENT, "too many columns for one call");
   std::vector<int> pts(n);
   for (int j = 0; j < n; ++j) pts[j] = idx1(points[j], P.N_pts, "points");
-  ensure_shift_on_device(P);
-  int* d_pts = dupload(pts, s);
+  // force_general takes the map-driven kernel
+  const bool fast = use_structured(P) && columns_fast(P) &&
+                    (double)n * ((P.N_e + COL_EB - 1) / COL_EB) * ((P.meas_Nfm.size() + COL_MG - 1) / COL_MG) < 2e9;
+  if (fast) ensure_column_tables(P);
+  else ensure_shift_on_device(P);
+  if (P.pts_cap < n) {   // kept: calls end synchronized, so nothing reads it any more
+    dfree(P.d_pts);
+    P.pts_cap = 0;
+    P.d_pts = dalloc<int>(n);
+    P.pts_cap = n;
+  }
   void* d_out = nullptr;
   try {
     const size_t bytes = (size_t)n * P.N_obs * (host ? sizeof(double2) : sizeof(float2));
     d_out = host ? (void*)dalloc<char>(bytes) : out;
-    launch_columns(P, d_pts, n, d_out, host, s);
+    HIP_CHECK(hipMemcpyAsync(P.d_pts, pts.data(), n * sizeof(int), hipMemcpyHostToDevice, s));
+    if (fast) launch_columns_fast(P, P.d_pts, n, d_out, host, s);
+    else launch_columns(P, P.d_pts, n, d_out, host, s);
     HIP_CHECK(hipGetLastError());
     if (host) HIP_CHECK(hipMemcpyAsync(out, d_out, bytes, hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
   } catch (...) {
     hipStreamSynchronize(s);
-    dfree(d_pts);
     if (host) dfree(d_out);
     throw;
   }
-  dfree(d_pts);
   if (host) dfree(d_out);
 }
 

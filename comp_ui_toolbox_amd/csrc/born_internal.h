@@ -258,6 +258,18 @@ struct Plan {
     FftSet set;                     // launch of this plan alone
   } fft;
   bool in_noalloc = false;          // inside an allocation-free apply (one-rhs MFMA layout)
+  // every measurement and mix uses all frequencies in order: observation
+  // (mk, f) is mk * N_fu + f, pair (m, f) is m * N_fu + f
+  bool regular = false;
+  // columns of A on regular structured plans, built on first use: the mixes of
+  // one element by (element block, measurement group), the other mixes
+  bool col_ready = false;
+  int col_n_single = 0, col_n_multi = 0;   // set at plan creation
+  int* d_col_off = nullptr;
+  int2* d_col_ent = nullptr;
+  int* d_col_multi = nullptr;
+  int* d_pts = nullptr;                    // points of the last call, pts_cap of them
+  int pts_cap = 0;
   // received energies on the structured path, built on first use: squared
   // prefactors of the single-element mixes by (pair, y slice, element), and
   // the observations of the other mixes by pair (none: null)
@@ -387,6 +399,11 @@ void launch_time_signals(const Plan& P, const float2* u, const int* q_obs, int N
 void launch_fwd_mix(const Plan& P, int N_rhs, void* u, bool out_f64, hipStream_t s);
 void launch_tgc(const Plan& P, bool adjoint, bool f64, const void* in, void* out, int N_rhs, hipStream_t s);
 void launch_columns(const Plan& P, const int* pts, int n, void* u, bool out_f64, hipStream_t s);
+// regular structured plans (born_columns.hip): element block, measurement
+// group, frequency block
+constexpr int COL_EB = 16, COL_MG = 8, COL_FB = 16;
+bool columns_fast(const Plan& P);
+void launch_columns_fast(const Plan& P, const int* pts, int n, void* u, bool out_f64, hipStream_t s);
 void launch_fwd_sparse(const Plan& P, const int* pts, int n, const double2* g, int N_rhs, double2* u, hipStream_t s);
 // received energy under the plan's TGC; mixes of up to ETGC_LDS_ROWS rows keep
 // their rows in LDS, longer ones in `spill` (spill_blocks x rows x 64 float2)
