@@ -178,6 +178,8 @@ Plan::~Plan() {
   dfree(d_tgc_off);
   dfree(d_tgc_k32);
   dfree(d_tgc_k64);
+  dfree(d_tgc_spec);
+  dfree(d_tgc_tw);
   dfree(d_io_in);
   dfree(d_io_out);
   if (stream) hipStreamDestroy(stream);
@@ -2336,6 +2338,22 @@ static void energy_rx_tgc(Plan& P, int m, double* E_dev, hipStream_t s) {
   if (m < 0 || m >= (int)P.meas_pair_base.size())
     throw Error(BORN_ERR_INVALID_ARGUMENT, "operator_born.indices_measurement_sel must be a single index!");
   if (!P.tgc) throw Error(BORN_ERR_INVALID_ARGUMENT, "no TGC kernels are set on this operator");
+  if (use_structured(P) && P.tgc_TL > 0) {
+    if (!P.d_tgc_spec) {
+      dfree(P.d_tgc_tw);   // of a first use that failed
+      std::vector<float2> tw;
+      fft_twiddles(P.tgc_TL, tw);
+      P.d_tgc_tw = dupload(tw, P.stream);
+      P.d_tgc_spec = dalloc<float2>((size_t)P.N_mk * 16 * P.tgc_TL);
+      launch_tgc_spectra(P, P.tgc_TL, P.d_tgc_spec, P.stream);
+      HIP_CHECK(hipGetLastError());
+      HIP_CHECK(hipStreamSynchronize(P.stream));
+    }
+    launch_energy_tgc_fft(P, m, E_dev, s);
+    HIP_CHECK(hipGetLastError());
+    HIP_CHECK(hipStreamSynchronize(s));
+    return;
+  }
   ensure_shift_on_device(P);
   int rows = 1;
   for (int mk = 0; mk < P.N_mk; ++mk)
@@ -2555,6 +2573,9 @@ static void tgc_clear(Plan& P) {
   dfree(P.d_tgc_off);
   dfree(P.d_tgc_k32);
   dfree(P.d_tgc_k64);
+  dfree(P.d_tgc_spec);
+  dfree(P.d_tgc_tw);
+  P.tgc_TL = 0;
   P.tgc = false;
   P.n_tgc_tiles = 0;
 }
@@ -2605,6 +2626,9 @@ int born_tgc_set(born_plan_t plan, const int32_t* half_lengths, const double* ke
       throw;
     }
     P.n_tgc_tiles = (int)tiles.size();
+    int longest = 0;
+    for (int M : half) longest = std::max(longest, M);
+    P.tgc_TL = P.structured && P.regular ? energy_tgc_length(P.N_fu, longest) : 0;
     P.tgc = true;
   });
 }

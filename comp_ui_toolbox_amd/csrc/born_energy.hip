@@ -21,6 +21,7 @@
 // on those reads.  128 elements, 384 x 384 points, 129 frequencies, identity
 // mixes: 22.4 ms per measurement there, 0.35 ms here (FP64 rate: 0.06 ms; the
 // fill of the windows takes as long as the multiply-adds).
+#include "born_fft.h"
 #include "born_internal.h"
 
 #include <algorithm>
@@ -274,6 +275,150 @@ __global__ __launch_bounds__(256) void k_energy_multi(EnergyArgs A, double* __re
   }
 }
 
+// ------------------------------------------------------ energies under TGC
+// E[p] = sum over the mixes and rows i of |sum_j k[i - j] Phi[j, p]|^2, Phi[j, p]
+// = p_inc[j, p] sum_a pref[j, a] h_ref[j, shift(p, e_a)] (operator_born.m:830-848,
+// convolution.m:62-98).  On regular plans the convolution along the N
+// frequencies is a product of transforms of length L >= N + M (M the longest
+// half length), or of length L = 2 (N - 1) with the one lag pair +-(N - 1),
+// which would fall on one entry, taken separately.  A wave takes FPW
+// neighbouring points and the mixes mk0 + wave, + 4, ...: Phi in FP64,
+// rounded once, the transforms in FP32, the squares summed in FP64.
+//
+// Bound: the vector ALU, about 980 instructions per FPW points and mix in
+// place of the N (2 M + 1) products of k_energy_rx_tgc, which stays for the
+// other plans and longer mixes.  64 elements, 192 x 192 points, 65 frequencies,
+// M = 64: 8.7 ms per measurement there, 0.52 ms here; relative L2 error against
+// FP64 5.4e-8 there (the taps' rounding), 6.8e-8 here (1.1e-7 without the
+// remainders of the transforms' constants, which cost 4 %).
+
+// spec[mk][8][TL][2]: transform of the taps of mix mk (lags over L / 2 left
+// out), divided by L
+template <int TL>
+__global__ __launch_bounds__(64) void k_tgc_spectra(const double2* __restrict__ taps, const int* __restrict__ half,
+                                                    const int64_t* __restrict__ tap_off, int N_mk,
+                                                    float4* __restrict__ spec) {
+  constexpr int FPW = FftShape<TL>::FPW, L = 16 * TL;
+  __shared__ Cx<double> lds[FftShape<TL>::LDS];
+  const int lane = threadIdx.x, j = lane / FPW, g = lane % FPW;
+  const int mk = blockIdx.x * FPW + g;
+  Cx<double> tw[16], x[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    double s, c;
+    sincospi(2.0 * (double)(j * k) / L, &s, &c);
+    tw[k] = {c, s};
+  }
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    x[q] = {0.0, 0.0};
+    const int n = j + TL * q, d = n < L / 2 ? n : n - L;
+    if (mk < N_mk && n != L / 2 && d >= -half[mk] && d <= half[mk]) {
+      const double2 k = taps[tap_off[mk] + half[mk] + d];
+      x[q] = {k.x / L, k.y / L};
+    }
+  }
+  fft_wave<double, TL, false>(x, tw, lds, lane);
+  if (mk >= N_mk) return;
+  float4* out = spec + (size_t)mk * (L / 2) + j;
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+    out[q * TL] = make_float4((float)x[2 * q].x, (float)x[2 * q].y, (float)x[2 * q + 1].x, (float)x[2 * q + 1].y);
+}
+
+// NQ: entries of a lane that can hold frequencies (N <= NQ * TL)
+template <int TL, int NQ>
+__global__ __launch_bounds__(256, 2) void k_energy_tgc_fft(EnergyArgs A, const float4* __restrict__ spec,
+                                                           const double2* __restrict__ taps, const int* __restrict__ half,
+                                                           const int64_t* __restrict__ tap_off,
+                                                           const float2* __restrict__ twid, int mk0, int mk1,
+                                                           double* __restrict__ E) {
+  constexpr int FPW = FftShape<TL>::FPW, L = 16 * TL;
+  __shared__ cf lds_all[4 * FftShape<TL>::LDS];
+  __shared__ double red[4][64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int j = lane / FPW, g = lane % FPW;
+  cf* lds = lds_all + wave * FftShape<TL>::LDS;
+  const int N = A.n_pairs;
+  const int p = min((int)blockIdx.x * FPW + g, A.N_pts - 1);
+  const int row = p / A.Nx, ix = p - row * A.Nx;
+  cf tw[16];
+  load_twiddles<TL>(twid, j, tw);
+  float2 pv[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const int n = min(j + TL * q, N - 1);
+    pv[q] = A.P[(size_t)(A.pair0 + n) * A.N_pts + p];
+  }
+  const bool edge = N == L / 2 + 1;   // lags +-(N - 1) separately
+  double acc = 0.0;
+  for (int mk = mk0 + wave; mk < mk1; mk += 4) {
+    const int Na = A.mk_meta[mk * 4 + 2];
+    const int* act = A.act + A.mk_off[mk * 4 + 2];
+    const double2* pref = A.pref + A.mk_off[mk * 4 + 3];
+    double qx[NQ], qy[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) qx[q] = qy[q] = 0.0;
+    for (int a = 0; a < Na; ++a) {
+      const int e = act[a], ey = e / A.Nex, ex = e - ey * A.Nex;
+      const float2* h = A.h + (int64_t)A.hrow[ey * A.n_rows + row] * A.HR + A.ext[ix - ex * A.Np + (A.Nex - 1) * A.Np];
+      const double2* c = pref + (int64_t)a * N;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        const int n = min(j + TL * q, N - 1);
+        const float2 hv = h[(int64_t)n * A.H_plane];
+        const double2 cv = c[n];
+        qx[q] += cv.x * hv.x - cv.y * hv.y;
+        qy[q] += cv.x * hv.y + cv.y * hv.x;
+      }
+    }
+    cf x[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      x[q] = {0.f, 0.f};
+      if (q < NQ && j + TL * q < N) {
+        const int r = q < NQ ? q : 0;
+        x[q] = {(float)(qx[r] * pv[r].x - qy[r] * pv[r].y), (float)(qx[r] * pv[r].y + qy[r] * pv[r].x)};
+      }
+    }
+    // with N = L / 2 + 1, lane j = 0 holds the first (q = 0) and the last (q = 8) row
+    const cf first = x[0], last = x[8];
+    float4 kv[8];
+    const float4* ks = spec + (size_t)mk * (L / 2) + j;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) kv[q] = ks[q * TL];
+    fft_wave<float, TL, (NQ <= 8), true>(x, tw, lds, lane);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {   // conjugated, for the exponent's sign
+      const cf u = x[2 * q], v = x[2 * q + 1];
+      x[2 * q] = {fmaf(kv[q].x, u.x, -(kv[q].y * u.y)), -fmaf(kv[q].x, u.y, kv[q].y * u.x)};
+      x[2 * q + 1] = {fmaf(kv[q].z, v.x, -(kv[q].w * v.y)), -fmaf(kv[q].z, v.y, kv[q].w * v.x)};
+    }
+    fft_wave<float, TL, false, true>(x, tw, lds, lane);
+    if (NQ > 8 && edge && half[mk] == N - 1 && j == 0) {
+      const double2* k = taps + tap_off[mk];   // lags -(N - 1) .. N - 1
+      const float2 kn = make_float2((float)k[0].x, (float)k[0].y);
+      const float2 kp = make_float2((float)k[2 * (N - 1)].x, (float)k[2 * (N - 1)].y);
+      cf y0 = {x[0].x, -x[0].y}, y8 = {x[8].x, -x[8].y};
+      cmac(y0, cf{kn.x, kn.y}, last);
+      cmac(y8, cf{kp.x, kp.y}, first);
+      x[0] = y0;
+      x[8] = y8;
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+      if (j + TL * q < N) acc += (double)x[q].x * x[q].x + (double)x[q].y * x[q].y;
+  }
+  red[wave][lane] = acc;
+  __syncthreads();
+  if (wave == 0 && j == 0 && (int)blockIdx.x * FPW + g < A.N_pts) {
+    double s = 0.0;
+    for (int w = 0; w < 4; ++w)
+      for (int t = 0; t < TL; ++t) s += red[w][t * FPW + g];
+    E[p] = s;
+  }
+}
+
 // ------------------------------------------------------------------ host side
 int energy_pad(int Nex) { return (Nex + 23) / 24 * 24; }   // a multiple of 4, 6 and 8
 
@@ -376,6 +521,53 @@ void launch_energy_multi(const Plan& P, int m, bool add, double* E, hipStream_t 
   else if (P.Np == 2) BORN_EM(2);
   else BORN_EM(0);
 #undef BORN_EM
+}
+
+// Transform length (as TL = L / 16) of the energies under TGC: the smallest
+// that holds N rows and half lengths up to M; 0: none.
+int energy_tgc_length(int N, int M) {
+  for (int TL = 4; TL <= 16; TL *= 2) {
+    const int L = 16 * TL;
+    if (N + M <= L || (N == L / 2 + 1 && M == N - 1)) return TL;
+  }
+  return 0;
+}
+
+void launch_tgc_spectra(const Plan& P, int TL, float2* spec, hipStream_t s) {
+  const int FPW = 64 / TL;
+  const dim3 grid((P.N_mk + FPW - 1) / FPW);
+#define BORN_TS(TLv)                                                                                                \
+  hipLaunchKernelGGL(k_tgc_spectra<TLv>, grid, dim3(64), 0, s, P.d_tgc_k64, P.d_tgc_half, P.d_tgc_off, P.N_mk, \
+                     (float4*)spec)
+  if (TL == 16) BORN_TS(16);
+  else if (TL == 8) BORN_TS(8);
+  else BORN_TS(4);
+#undef BORN_TS
+}
+
+void launch_energy_tgc_fft(const Plan& P, int m, double* E, hipStream_t s) {
+  int mk0 = 0;
+  while (mk0 < P.N_mk && P.mk_meas[mk0] != m) ++mk0;
+  int mk1 = mk0;
+  while (mk1 < P.N_mk && P.mk_meas[mk1] == m) ++mk1;
+  const EnergyArgs A = energy_args(P, m, 4);
+  const int TL = P.tgc_TL, FPW = 64 / TL, N = P.N_fu;
+  const dim3 grid((P.N_pts + FPW - 1) / FPW);
+#define BORN_ET(TLv, NQv)                                                                                  \
+  hipLaunchKernelGGL((k_energy_tgc_fft<TLv, NQv>), grid, dim3(256), 0, s, A, (const float4*)P.d_tgc_spec, \
+                     P.d_tgc_k64, P.d_tgc_half, P.d_tgc_off, P.d_tgc_tw, mk0, mk1, E)
+#define BORN_ETN(TLv)                  \
+  do {                                 \
+    if (N <= 4 * TLv) BORN_ET(TLv, 4); \
+    else if (N <= 8 * TLv) BORN_ET(TLv, 8); \
+    else if (N <= 9 * TLv) BORN_ET(TLv, 9); \
+    else BORN_ET(TLv, 16);             \
+  } while (0)
+  if (TL == 16) BORN_ETN(16);
+  else if (TL == 8) BORN_ETN(8);
+  else BORN_ETN(4);
+#undef BORN_ETN
+#undef BORN_ET
 }
 
 }  // namespace born

@@ -313,6 +313,11 @@ struct Plan {
   int64_t* d_tgc_off = nullptr;
   float2* d_tgc_k32 = nullptr;
   double2* d_tgc_k64 = nullptr;
+  // energies under TGC by transforms of length 16 * tgc_TL (0: none), built on
+  // first use after the kernels are set: spectra of the taps, twiddles
+  int tgc_TL = 0;
+  float2* d_tgc_spec = nullptr;
+  float2* d_tgc_tw = nullptr;
   size_t io_bytes = 0;
   void* d_io_in = nullptr;        // host-path staging
   void* d_io_out = nullptr;
@@ -393,6 +398,9 @@ int energy_pad(int Nex);
 void launch_energy_weights(const Plan& P, double* ew, hipStream_t s);
 void launch_energy_single(const Plan& P, int m, double* E, hipStream_t s);
 void launch_energy_multi(const Plan& P, int m, bool add, double* E, hipStream_t s);
+int energy_tgc_length(int N, int M);
+void launch_tgc_spectra(const Plan& P, int TL, float2* spec, hipStream_t s);
+void launch_energy_tgc_fft(const Plan& P, int m, double* E, hipStream_t s);
 void launch_fp16_scales(const Plan& P, const float* x, size_t n_floats, int which, hipStream_t s);
 void launch_time_signals(const Plan& P, const float2* u, const int* q_obs, int N_rhs, int N_t, float* rf,
                          hipStream_t s);

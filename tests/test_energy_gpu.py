@@ -69,3 +69,32 @@ def test_matrix_array(torch_cuda, kind):
     op = OperatorBorn.from_sequence(spec)
     assert op.path == "structured"
     check(op, O.direct_tables(spec), 1, kind)
+
+
+@pytest.mark.parametrize("kind", ["single", "dense"])
+@pytest.mark.parametrize("nf,M", [(5, 0), (17, 3), (32, 31), (33, 32), (33, 40), (50, 14), (65, 64), (72, 56), (73, 100),
+                                  (128, 127), (129, 128), (129, 100), (200, 56)])
+def test_under_tgc(torch_cuda, nf, M, kind):
+    """Transform lengths 64, 128 and 256 for the convolution along the
+    frequencies, and the odd lengths whose longest lag is taken separately
+    (33, 65, 129).  Two FP32 transforms of at most 8 stages, 2 * 8 * 2^-24 =
+    9.5e-7 in the compensated rows, twice that in their squares, and the
+    tables' 2.4e-7: 2.2e-6."""
+    ne, npp = 6, 4
+    rng = np.random.Generator(np.random.PCG64(nf + M))
+    arr = C.ArraySpec((ne,), (3e-4,), (2.7e-4,), (2,))
+    fov = C.FovSpec((37, 3), (3e-4 / npp, 3e-4 / npp), 2e-3)
+    waves = [C.random_wave(arr, rng, 1e-6) for _ in range(2)]
+    spec = C.SequenceSpec("et", arr, C.MediumSpec(), fov, 2e6 + 3e4 * np.arange(nf), waves,
+                          [mixes_of(kind, ne, nf, rng) for _ in waves])
+    op = OperatorBorn.from_sequence(spec)
+    T = O.direct_tables(spec)
+    n_mix = len(spec.mixes[0])
+    kernels = [rng.standard_normal(2 * m + 1) + 1j * rng.standard_normal(2 * m + 1)
+               for m in ([M] * (2 * n_mix - 1) + [M // 2])]
+    op.set_tgc(kernels)
+    for m in range(2):
+        ref = O.energy_rx(T, m, kernels[m * n_mix:(m + 1) * n_mix])
+        E = op.energy_rx(m, tgc=True)
+        assert np.linalg.norm(E - ref) < 2.2e-6 * np.linalg.norm(ref)
+        assert np.array_equal(E, op.energy_rx_dev(m, tgc=True).cpu().numpy())
