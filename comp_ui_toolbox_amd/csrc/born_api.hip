@@ -178,6 +178,7 @@ Plan::~Plan() {
   dfree(d_tgc_off);
   dfree(d_tgc_k32);
   dfree(d_tgc_k64);
+  dfree(d_time_cs);
   dfree(d_tgc_spec);
   dfree(d_tgc_tw);
   dfree(d_io_in);
@@ -2457,6 +2458,26 @@ int born_time_signals(born_plan_t plan, const double* frequencies, double delta_
       throw Error(BORN_ERR_INVALID_ARGUMENT, "Number of spectral samples exceeds the maximum!");
     const size_t need = (size_t)N_rhs * P.N_mk * N_t;
     if (capacity < (int64_t)need) throw Error(BORN_ERR_INVALID_ARGUMENT, "output capacity too small");
+    const hipStream_t s = (hipStream_t)stream;
+    // regular plans with evenly spaced, increasing indices: no mix repeats one
+    bool even = P.regular;
+    const int dq = P.N_fu > 1 ? q_fg[1] - q_fg[0] : 1;
+    for (int i = 0; i + 1 < P.N_fu && even; ++i) even = dq > 0 && q_fg[i + 1] - q_fg[i] == dq;
+    if (even) {
+      if (P.time_Nt != N_t) {   // calls end synchronized, so nothing reads the old table
+        dfree(P.d_time_cs);
+        P.time_Nt = 0;
+        P.d_time_cs = dalloc<float2>(N_t);
+        launch_time_table(N_t, P.d_time_cs, s);
+        HIP_CHECK(hipGetLastError());
+        P.time_Nt = N_t;
+      }
+      launch_time_regular(P, (const float2*)u_c64, N_rhs, N_t, q_fg[0], dq, (float*)rf_f32, s);
+      HIP_CHECK(hipGetLastError());
+      HIP_CHECK(hipStreamSynchronize(s));
+      if (N_t_out) *N_t_out = N_t;
+      return;
+    }
     std::vector<int> q_obs(P.N_obs);
     for (int mk = 0; mk < P.N_mk; ++mk) {
       std::vector<int> qs(P.mk_Nf[mk]);
@@ -2468,7 +2489,6 @@ int born_time_signals(born_plan_t plan, const double* frequencies, double delta_
       if (std::adjacent_find(qs.begin(), qs.end()) != qs.end())
         throw Error(BORN_ERR_UNSUPPORTED, "signal: a mix repeats a frequency, so it has no frequency axis");
     }
-    const hipStream_t s = (hipStream_t)stream;
     int* d_q = dupload(q_obs, s);
     try {
       launch_time_signals(P, (const float2*)u_c64, d_q, N_rhs, N_t, (float*)rf_f32, s);
@@ -2595,6 +2615,9 @@ int born_tgc_set(born_plan_t plan, const int32_t* half_lengths, const double* ke
     std::vector<double2> k64;
     std::vector<int2> tiles;
     int64_t src = 0;
+    int N_max = 1;
+    for (int N : P.mk_Nf) N_max = std::max(N_max, N);
+    P.tgc_R = tgc_outputs(N_max);
     for (int mk = 0; mk < P.N_mk; ++mk) {
       const int M = half_lengths[mk];
       const int N = P.mk_Nf[mk];
@@ -2611,7 +2634,7 @@ int born_tgc_set(born_plan_t plan, const int32_t* half_lengths, const double* ke
         k64.push_back(make_double2(k[0], k[1]));
       }
       src += 2 * (int64_t)M + 1;
-      for (int i0 = 0; i0 < N; i0 += 256) tiles.push_back(make_int2(mk, i0));
+      for (int i0 = 0; i0 < N; i0 += 64 * P.tgc_R) tiles.push_back(make_int2(mk, i0));
     }
     std::vector<float2> k32(k64.size());
     for (size_t i = 0; i < k64.size(); ++i) k32[i] = make_float2((float)k64[i].x, (float)k64[i].y);

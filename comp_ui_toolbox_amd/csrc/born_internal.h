@@ -303,11 +303,15 @@ struct Plan {
   // host forward: the gather path for at most sparse_max occupied points
   // (-1: the cost rule, 0: never)
   int sparse_max = -1;
+  // phase factors of the time-domain signals of time_Nt samples, of the last call
+  int time_Nt = 0;
+  float2* d_time_cs = nullptr;
   // time gain compensation: per mix the half length M (after the cut-off
   // truncation) and the offset of its 2M + 1 taps; tiles (mix, first row) of
-  // 256 outputs
+  // 64 tgc_R outputs
   bool tgc = false;
   int n_tgc_tiles = 0;
+  int tgc_R = 4;                    // outputs per lane: tiles of 64 tgc_R rows
   int2* d_tgc_tiles = nullptr;
   int* d_tgc_half = nullptr;
   int64_t* d_tgc_off = nullptr;
@@ -404,7 +408,10 @@ void launch_energy_tgc_fft(const Plan& P, int m, double* E, hipStream_t s);
 void launch_fp16_scales(const Plan& P, const float* x, size_t n_floats, int which, hipStream_t s);
 void launch_time_signals(const Plan& P, const float2* u, const int* q_obs, int N_rhs, int N_t, float* rf,
                          hipStream_t s);
+void launch_time_table(int N_t, float2* cs, hipStream_t s);
+void launch_time_regular(const Plan& P, const float2* u, int N_rhs, int N_t, int q0, int dq, float* rf, hipStream_t s);
 void launch_fwd_mix(const Plan& P, int N_rhs, void* u, bool out_f64, hipStream_t s);
+int tgc_outputs(int N);
 void launch_tgc(const Plan& P, bool adjoint, bool f64, const void* in, void* out, int N_rhs, hipStream_t s);
 void launch_columns(const Plan& P, const int* pts, int n, void* u, bool out_f64, hipStream_t s);
 // regular structured plans (born_columns.hip): element block, measurement
