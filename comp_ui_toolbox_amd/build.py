@@ -18,7 +18,7 @@ SOURCES = [PKG / "csrc" / "born_api.hip", PKG / "csrc" / "born_kernels.hip", PKG
            PKG / "csrc" / "born_split.hip", PKG / "csrc" / "born_split3d.hip",
            PKG / "csrc" / "born_structured3d.hip", PKG / "csrc" / "born_fewcol.hip", PKG / "csrc" / "born_fft.hip",
            PKG / "csrc" / "born_energy.hip", PKG / "csrc" / "born_columns.hip",
-           PKG / "csrc" / "born_signals.hip"]
+           PKG / "csrc" / "born_signals.hip", PKG / "csrc" / "born_fft3d.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("BORN_OFFLOAD_ARCH", "gfx950")
 

@@ -440,6 +440,38 @@ static bool use_structured(const Plan& P) { return P.structured && !P.force_gene
 // apply keeps the MFMA layout.
 static bool use_fft(const Plan& P) { return use_structured(P) && P.fft.ok && !P.in_noalloc; }
 
+// Columns (pair, frequency) by frequency.
+static void upload_fft_columns(Plan& P) {
+  std::vector<int2> col(P.N_pairs);
+  for (int c = 0; c < P.N_pairs; ++c) col[c] = make_int2(P.fg_pairs[c], P.pair_fg[P.fg_pairs[c]]);
+  P.fft.d_col = dupload(col, P.stream);
+}
+
+// The same for 3-D plans whose planes fit (fft3_shape).
+static void build_fft3(Plan& P) {
+  Plan::Fft& F = P.fft;
+  F.s3 = fft3_shape(P.Nx, P.Ny, P.Np, P.Npy, P.Nex, P.Ney);
+  if (F.s3.TLX == 0) return;
+  const size_t n = (size_t)P.N_fu * P.Nz * P.Npy * P.Np * fft3_plane(F.s3);
+  size_t free_b = 0, total_b = 0;
+  HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+  if (n * sizeof(float2) + fft3_tmp(P) * sizeof(double2) + ((size_t)1 << 30) > free_b) return;
+  std::vector<float2> tw, twy;
+  fft_twiddles(F.s3.TLX, tw);
+  fft_twiddles(F.s3.TLY, twy);
+  tw.insert(tw.end(), twy.begin(), twy.end());
+  upload_fft_columns(P);
+  F.d_tw = dupload(tw, P.stream);
+  F.d_H = dalloc<float2>(n);
+  double2* tmp = dalloc<double2>(fft3_tmp(P));
+  for (int f = 0; f < P.N_fu; ++f) launch_fft3_table(P, f, tmp, P.stream);
+  const hipError_t e = hipStreamSynchronize(P.stream);
+  dfree(tmp);
+  HIP_CHECK(e);
+  HIP_CHECK(hipGetLastError());
+  F.ok = true;
+}
+
 // Tables of the fast lateral correlation, built once per plan: the slots
 // (row, segment, phase), the columns by frequency and the spectra of h_ref.
 // The spectra take about twice the space of h_ref; a plan whose spectra do
@@ -447,7 +479,11 @@ static bool use_fft(const Plan& P) { return use_structured(P) && P.fft.ok && !P.
 static void build_fft(Plan& P) {
   Plan::Fft& F = P.fft;
   F.ok = false;
-  if (P.nd != 2 || !P.structured) return;
+  if (!P.structured) return;
+  if (P.nd == 3) {
+    build_fft3(P);
+    return;
+  }
   F.shape = fft_shape(P.Nx, P.Np, P.N_e);
   if (F.shape.TL == 0) return;
   const int FPW = 64 / F.shape.TL;
@@ -467,12 +503,10 @@ static void build_fft(Plan& P) {
     const int left = first < P.Nx ? (P.Nx - first + P.Np - 1) / P.Np : 0;
     slot[s] = left > 0 ? make_int2(row * P.Nx + first, std::min(left, F.shape.Sv)) : make_int2(0, 0);
   }
-  std::vector<int2> col(P.N_pairs);
-  for (int c = 0; c < P.N_pairs; ++c) col[c] = make_int2(P.fg_pairs[c], P.pair_fg[P.fg_pairs[c]]);
   std::vector<float2> tw;
   fft_twiddles(F.shape.TL, tw);
   F.d_slot = dupload(slot, P.stream);
-  F.d_col = dupload(col, P.stream);
+  upload_fft_columns(P);
   F.d_tw = dupload(tw, P.stream);
   F.d_H = dalloc<float2>(n);
   launch_fft_table(P, P.stream);
@@ -536,8 +570,29 @@ static void finalize_fft_set(FftSet& S) {
   HIP_CHECK(hipMemcpy(S.d_inst, S.inst.data(), S.inst.size() * sizeof(FftInst), hipMemcpyHostToDevice));
 }
 
+// 3-D: forward workgroups of 4 to 32 depths, about 3072 of them; adjoint
+// workgroups of at least 8 columns, about 2048 of them.
+static void build_fft3_workspace(Plan& P, int N_rhs) {
+  Plan::Fft& F = P.fft;
+  const int64_t cols = (int64_t)P.N_pairs * N_rhs;
+  F.ZR = (int)std::max<int64_t>(4, std::min<int64_t>(32, cols * P.Nz / 3072));
+  F.ZR = std::min(F.ZR, P.Nz);
+  F.NZB = (P.Nz + F.ZR - 1) / F.ZR;
+  const int64_t wg = (int64_t)P.Nz * P.Npy * (P.Np / F.s3.px) * N_rhs;
+  F.FG = (int)std::max<int64_t>(1, std::min<int64_t>({(2048 + wg - 1) / wg, P.N_pairs / 8, 64}));
+  if (cols * F.NZB > INT32_MAX - 64 || wg * F.FG > INT32_MAX - 64)
+    throw Error(BORN_ERR_UNSUPPORTED, "too many right-hand sides for one launch");
+  F.d_vp = dalloc<float2>((size_t)F.NZB * cols * P.N_e);
+  F.d_wt = dalloc<float2>((size_t)cols * fft3_plane(F.s3));
+  if (F.FG > 1) F.d_gp = dalloc<float2>((size_t)F.FG * N_rhs * P.N_pts);
+}
+
 static void build_fft_workspace(Plan& P, int N_rhs) {
   Plan::Fft& F = P.fft;
+  if (P.nd == 3) {
+    build_fft3_workspace(P, N_rhs);
+    return;
+  }
   fft_blocking(P, N_rhs);
   F.d_gs = dalloc<float2>((size_t)N_rhs * F.n_ws * (F.shape.nq <= 8 ? 8 : 16) * 64);
   F.d_vp = dalloc<float2>((size_t)F.NZB * N_rhs * P.N_pairs * P.N_e);
@@ -1535,15 +1590,33 @@ static int fwd_blocks(const LaunchSet& L, int precision, const Inst& I) {
   return fc_path(L, precision) || precision == BORN_PRECISION_FP32 ? I.NZB : I.NZB_s * I.nseg_s;
 }
 
+// The masked input of a fast-correlation plan: in its slot order (2-D), or in
+// the plan's own buffer (3-D).
+static void fft_input(Plan& P, const float2* gm, int N_rhs, bool mask, hipStream_t s) {
+  if (P.nd == 2) launch_fft_gamma(P, gm, N_rhs, mask, s);
+  else if (mask) launch_mask_gamma(gm, P.N_pts, N_rhs, P.d_gm, s);
+  else if (gm != P.d_gm) throw Error(BORN_ERR_INVALID_ARGUMENT, "masked input outside the plan's buffer");
+}
+// Spectra of the un-mixed adjoint weights.
+static void fft_weights(Plan& P, const float2* u, int N_rhs, hipStream_t s) {
+  if (P.nd == 2) {
+    launch_fft_weights(P, u, N_rhs, s);
+    return;
+  }
+  launch_adj_unmix(P, u, N_rhs, false, s);
+  launch_fft3_weights(P, N_rhs, s);
+}
+
 // gm: the input, masked by the occupancy rule unless `mask` (fast-correlation
 // plans apply the rule as they reorder the input).
 static void forward_device(Plan& P, const float2* gm, int N_rhs, void* u, bool out_f64, hipStream_t s,
                            bool mask = false) {
   if (use_fft(P)) {
-    launch_fft_gamma(P, gm, N_rhs, mask, s);
+    fft_input(P, gm, N_rhs, mask, s);
     {
       TimedLaunch t(P, s, 0);
-      launch_fft_fwd(P.fft.set, s);
+      if (P.nd == 3) launch_fft3_fwd(P, N_rhs, s);
+      else launch_fft_fwd(P.fft.set, s);
     }
     launch_fft_reduce(P, N_rhs, s);
     launch_fwd_mix(P, N_rhs, u, out_f64, s);
@@ -1579,11 +1652,12 @@ static void forward_device(Plan& P, const float2* gm, int N_rhs, void* u, bool o
 
 static void adjoint_device(Plan& P, const float2* u, int N_rhs, float2* g, hipStream_t s) {
   if (use_fft(P)) {
-    launch_fft_weights(P, u, N_rhs, s);
+    fft_weights(P, u, N_rhs, s);
     TimedLaunch t(P, s, 1);
     OutPtrs outs;
     outs.p[0] = g;
-    launch_fft_adj(P.fft.set, outs, s);
+    if (P.nd == 3) launch_fft3_adj(P, N_rhs, g, s);
+    else launch_fft_adj(P.fft.set, outs, s);
     launch_fft_adj_reduce(P, N_rhs, g, s);
     HIP_CHECK(hipGetLastError());
     return;
@@ -1748,7 +1822,8 @@ struct Batch {
   std::vector<int> set_of;         // per plan: its launch set
   std::vector<int> slot;           // per plan: its index in its launch set
   // plans on the fast lateral correlation: a launch per transform length and
-  // half-full form (set_of = -1 - index)
+  // half-full form (set_of = -1 - index), or per plan in 3-D (set_of = SET_3D)
+  static constexpr int SET_3D = -100;
   static constexpr int N_FSETS = 6;
   FftSet fsets[N_FSETS];
   Chunk* d_chunks[N_SETS] = {};
@@ -1855,7 +1930,7 @@ static void build_batch_launch(Batch& B) {
     const Plan& P = *B.plans[i];
     if (P.fft.ok) {
       const int k = (P.fft.shape.TL == 16 ? 0 : (P.fft.shape.TL == 8 ? 2 : 4)) + (P.fft.shape.nq <= 8 ? 0 : 1);
-      B.set_of[i] = -1 - k;
+      B.set_of[i] = P.nd == 3 ? Batch::SET_3D : -1 - k;
       B.gen.push_back(P.ws_gen);
       continue;
     }
@@ -1892,7 +1967,7 @@ static void batch_forward_enqueue(Batch& B, const void* const* in, void* const* 
   for (size_t i = 0; i < B.plans.size(); ++i) {
     Plan& P = *B.plans[i];
     if (B.set_of[i] < 0) {
-      launch_fft_gamma(P, (const float2*)in[i], 1, true, s);
+      fft_input(P, (const float2*)in[i], 1, true, s);
       continue;
     }
     launch_mask_gamma((const float2*)in[i], P.N_pts, 1, P.d_gm, s);
@@ -1907,6 +1982,8 @@ static void batch_forward_enqueue(Batch& B, const void* const* in, void* const* 
   }
   for (int k = 0; k < Batch::N_SETS; ++k) fwd_contract(B.set(k), B.precision, B.n_cu, s);
   for (int k = 0; k < Batch::N_FSETS; ++k) launch_fft_fwd(B.fsets[k], s);
+  for (size_t i = 0; i < B.plans.size(); ++i)
+    if (B.set_of[i] == Batch::SET_3D) launch_fft3_fwd(*B.plans[i], 1, s);
   if (B.timing) {
     HIP_CHECK(hipEventRecord(b, s));
     B.timed.push_back({a, b, 0});
@@ -1929,8 +2006,8 @@ static void batch_adjoint_enqueue(Batch& B, const void* const* in, void* const* 
   for (size_t i = 0; i < B.plans.size(); ++i) {
     Plan& P = *B.plans[i];
     if (B.set_of[i] < 0) {
-      launch_fft_weights(P, (const float2*)in[i], 1, s);
-      fouts[-1 - B.set_of[i]].p[B.slot[i]] = (float2*)out[i];
+      fft_weights(P, (const float2*)in[i], 1, s);
+      if (B.set_of[i] != Batch::SET_3D) fouts[-1 - B.set_of[i]].p[B.slot[i]] = (float2*)out[i];
       continue;
     }
     launch_adj_unmix(P, (const float2*)in[i], 1, true, s);
@@ -1946,6 +2023,8 @@ static void batch_adjoint_enqueue(Batch& B, const void* const* in, void* const* 
   }
   for (int k = 0; k < Batch::N_SETS; ++k) adj_contract(B.set(k), B.precision, outs[k], s);
   for (int k = 0; k < Batch::N_FSETS; ++k) launch_fft_adj(B.fsets[k], fouts[k], s);
+  for (size_t i = 0; i < B.plans.size(); ++i)
+    if (B.set_of[i] == Batch::SET_3D) launch_fft3_adj(*B.plans[i], 1, (float2*)out[i], s);
   for (size_t i = 0; i < B.plans.size(); ++i)
     if (B.set_of[i] < 0) launch_fft_adj_reduce(*B.plans[i], 1, (float2*)out[i], s);
   if (B.timing) {
@@ -2134,6 +2213,20 @@ static void time_fft_set(const FftSet& S, const std::vector<const Plan*>& plans,
     throw;
   }
   for (float2* g : buf) dfree(g);
+}
+
+static void time_fft3(const Plan& P, hipStream_t s, float& fwd_ms, float& adj_ms) {
+  float2* g = dalloc<float2>(P.N_pts);
+  try {
+    fwd_ms += time_launches([&] { launch_fft3_fwd(P, 1, s); }, s, 3);
+    adj_ms += time_launches([&] { launch_fft3_adj(P, 1, g, s); }, s, 3);
+    HIP_CHECK(hipStreamSynchronize(s));
+  } catch (...) {
+    hipStreamSynchronize(s);
+    dfree(g);
+    throw;
+  }
+  dfree(g);
 }
 
 template <typename F>
@@ -2884,6 +2977,8 @@ int born_batch_autotune(born_batch_t batch, void* stream, double* fwd_ms, double
         if (B.set_of[i] == -1 - k) pk.push_back(B.plans[i]);
       time_fft_set(B.fsets[k], pk, s, r.fwd_ms, r.adj_ms);
     }
+    for (size_t i = 0; i < B.plans.size(); ++i)
+      if (B.set_of[i] == Batch::SET_3D) time_fft3(*B.plans[i], s, r.fwd_ms, r.adj_ms);
     if (fwd_ms) *fwd_ms = r.fwd_ms;
     if (adj_ms) *adj_ms = r.adj_ms;
   });
@@ -2901,7 +2996,8 @@ int born_plan_autotune(born_plan_t plan, void* stream, double* fwd_ms, double* a
     HIP_CHECK(hipDeviceSynchronize());
     if (use_fft(P)) {
       float f = 0.f, a = 0.f;
-      time_fft_set(P.fft.set, {&P}, s, f, a);
+      if (P.nd == 3) time_fft3(P, s, f, a);
+      else time_fft_set(P.fft.set, {&P}, s, f, a);
       if (fwd_ms) *fwd_ms = f;
       if (adj_ms) *adj_ms = a;
       return;

@@ -123,6 +123,28 @@ struct FftShapeChoice {
   int TL = 0, nseg = 1, Sv = 0, nq = 0;
 };
 
+// 3-D plans (born_fft3d.hip): transforms of 16 TLX x 16 TLY, px lateral
+// phases per tile, LDS bytes of a workgroup.
+constexpr int FFT3_PASSES = 2;   // rounds of row transforms per plane, at most
+struct Fft3Choice {
+  int TLX = 0, TLY = 0, Sx = 0, Sy = 0, px = 1;
+  bool half = false;               // at most half of every sequence holds points
+  size_t lds = 0;
+};
+struct Fft3Args {
+  const float2* H;                 // [N_fu][Nz][Npy][Npx][Lx Ly] in the y transforms' order
+  const float2* P;
+  const float2* gm;
+  const int2* col;
+  const float2* wt;                // [N_pairs][N_rhs][Lx Ly]
+  float2* vp;
+  float2* gp;
+  const float2* twx;
+  const float2* twy;
+  int Nx, Ny, Nz, Npx, Npy, Nex, Ney, N_e, N_pts, n_cols, N_rhs;
+  int Sy, px, ZR, FG;
+};
+
 // One operator instance of a fast-correlation launch.
 struct FftInst {
   BORN_GLOBAL const float2* H;     // spectra [N_fu][n_ws][8][64][2]
@@ -245,6 +267,7 @@ struct Plan {
   struct Fft {
     bool ok = false;
     FftShapeChoice shape;
+    Fft3Choice s3;                  // 3-D plans
     int n_slots = 0, n_ws = 0;
     float2* d_H = nullptr;
     int2* d_slot = nullptr;
@@ -430,6 +453,14 @@ void launch_adj_unmix(const Plan& P, const float2* u, int N_rhs, bool chunked, h
 void launch_adj_structured(const LaunchSet& L, const OutPtrs& outs, hipStream_t s);
 void launch_adj_general(const Plan& P, int N_rhs, float2* g_out, hipStream_t s);
 
+// fast lateral correlation in 3-D (born_fft3d.hip)
+Fft3Choice fft3_shape(int Nx, int Ny, int Npx, int Npy, int Nex, int Ney);
+size_t fft3_plane(const Fft3Choice& c);
+size_t fft3_tmp(const Plan& P);
+void launch_fft3_table(const Plan& P, int f, double2* tmp, hipStream_t s);
+void launch_fft3_fwd(const Plan& P, int N_rhs, hipStream_t s);
+void launch_fft3_weights(const Plan& P, int N_rhs, hipStream_t s);
+void launch_fft3_adj(const Plan& P, int N_rhs, float2* g, hipStream_t s);
 // fast lateral correlation (born_fft.hip)
 FftShapeChoice fft_shape(int Nx, int Np, int N_e);
 void fft_twiddles(int TL, std::vector<float2>& tw);

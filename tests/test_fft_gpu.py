@@ -88,3 +88,48 @@ def test_mixed_tables_and_zero_columns(torch_cuda):
     for r in range(3):
         ref = O.forward(T, g[:, r]).reshape(-1)
         assert np.all(u[:, r] == 0) if r == 1 else O.rel_l2(u[:, r], ref) < TOL
+
+
+# elements x, y, points x, y, z, points per pitch, frequencies, waves, rhs
+SIZES_3D = [
+    (4, 3, 19, 7, 3, 2, 2, 2, 1),      # 64 x 64, both phases of x in one tile
+    (32, 2, 66, 9, 2, 2, 2, 1, 2),     # 33 points per phase: more than half full
+    (20, 8, 70, 25, 5, 2, 1, 2, 1),
+    (32, 4, 72, 20, 2, 2, 1, 2, 3),    # 128 x 64
+    (3, 33, 10, 68, 2, 2, 2, 1, 1),    # 64 x 128
+    (34, 33, 64, 66, 1, 2, 1, 2, 1),   # 128 x 128, just over 64 on both axes
+    (5, 4, 40, 30, 9, 1, 2, 1, 2),     # one point per pitch
+    (6, 5, 50, 31, 2, 3, 2, 2, 1),     # three phases
+    (17, 2, 101, 5, 2, 4, 1, 1, 1),    # four phases, field of view wider than the aperture
+]
+
+
+@pytest.mark.parametrize("nex,ney,nx,ny,nz,npp,nf,waves,n_rhs", SIZES_3D)
+def test_volume(torch_cuda, nex, ney, nx, ny, nz, npp, nf, waves, n_rhs):
+    """Planes: two more transforms of at most 7 stages, worst case
+    3 * 14 * 2^-24 = 2.5e-6; 1.5e-6 is taken."""
+    import torch
+    pitch = 3e-4
+    arr = C.ArraySpec((nex, ney), (pitch, pitch), (2.7e-4, 2.7e-4), (2, 2))
+    fov = C.FovSpec((nx, ny, nz), (pitch / npp,) * 3, 3e-3)
+    rng = np.random.Generator(np.random.PCG64(nex * 100 + ny))
+    ws = [C.random_wave(arr, rng, 1e-6) for _ in range(waves)]
+    spec = C.SequenceSpec("fft3", arr, C.MediumSpec(), fov, np.linspace(2.5e6, 4e6, nf), ws,
+                          [C.identity_mixes(nex * ney) for _ in ws])
+    T = O.direct_tables(spec)
+    op = OperatorBorn.from_sequence(spec)
+    assert op.path == "structured"
+    g = rng.standard_normal((n_rhs, op.N_points)) + 1j * rng.standard_normal((n_rhs, op.N_points))
+    u = rng.standard_normal((n_rhs, op.N_observations)) + 1j * rng.standard_normal((n_rhs, op.N_observations))
+    gd = torch.tensor(g.astype(np.complex64), device="cuda:0")
+    ud = torch.tensor(u.astype(np.complex64), device="cuda:0")
+    fast = [op.forward_dev(gd).cpu().numpy(), op.adjoint_dev(ud).cpu().numpy()]
+    assert np.array_equal(fast[0], op.forward_dev(gd).cpu().numpy())
+    assert np.array_equal(fast[1], op.adjoint_dev(ud).cpu().numpy())
+    op.force_general(True)
+    general = [op.forward_dev(gd).cpu().numpy(), op.adjoint_dev(ud).cpu().numpy()]
+    for r in range(n_rhs):
+        ref = [O.forward(T, gd[r].cpu().numpy()), O.adjoint(T, ud[r].cpu().numpy())]
+        for k in range(2):
+            assert O.rel_l2(fast[k][r], ref[k].reshape(-1)) < 1.5e-6, ("oracle", k)
+            assert O.rel_l2(fast[k][r], general[k][r]) < 3e-6, ("general", k)
