@@ -486,6 +486,7 @@ static void build_fft(Plan& P) {
   }
   F.shape = fft_shape(P.Nx, P.Np, P.N_e);
   if (F.shape.TL == 0) return;
+  if (((int64_t)P.N_pts + 256ll * P.Np) * 8 > INT32_MAX) return;   // the forward addresses a row of p_inc by 32-bit byte offsets
   const int FPW = 64 / F.shape.TL;
   const int64_t n_slots = (int64_t)P.n_rows * F.shape.nseg * P.Np;
   if (n_slots > INT32_MAX - 64) return;
@@ -543,7 +544,6 @@ static FftInst make_fft_inst(const Plan& P, int N_rhs) {
   I.N_pts = P.N_pts;
   I.N_e = P.N_e;
   I.Np = P.Np;
-  I.nq = F.shape.nq;
   I.n_ws = F.n_ws;
   I.n_cols = P.N_pairs;
   I.N_rhs = N_rhs;
@@ -594,14 +594,14 @@ static void build_fft_workspace(Plan& P, int N_rhs) {
     return;
   }
   fft_blocking(P, N_rhs);
-  F.d_gs = dalloc<float2>((size_t)N_rhs * F.n_ws * (F.shape.nq <= 8 ? 8 : 16) * 64);
+  F.d_gs = dalloc<float2>((size_t)N_rhs * F.n_ws * F.shape.nz * 64);
   F.d_vp = dalloc<float2>((size_t)F.NZB * N_rhs * P.N_pairs * P.N_e);
   F.d_wt = dalloc<float2>((size_t)P.N_pairs * N_rhs * 16 * F.shape.TL);
   if (F.FG > 1) F.d_gp = dalloc<float2>((size_t)F.FG * N_rhs * P.N_pts);
   F.set.inst.assign(1, make_fft_inst(P, N_rhs));
   F.set.d_tw = F.d_tw;
   F.set.TL = F.shape.TL;
-  F.set.half = F.shape.nq <= 8;
+  F.set.nz = F.shape.nz;
   finalize_fft_set(F.set);
 }
 
@@ -1822,9 +1822,12 @@ struct Batch {
   std::vector<int> set_of;         // per plan: its launch set
   std::vector<int> slot;           // per plan: its index in its launch set
   // plans on the fast lateral correlation: a launch per transform length and
-  // half-full form (set_of = -1 - index), or per plan in 3-D (set_of = SET_3D)
+  // entries per lane (set_of = -1 - index), or per plan in 3-D (set_of = SET_3D)
   static constexpr int SET_3D = -100;
-  static constexpr int N_FSETS = 6;
+  static constexpr int N_FSETS = 18;
+  static int fft_set(const FftShapeChoice& c) {
+    return (c.TL == 16 ? 0 : (c.TL == 8 ? 6 : 12)) + (c.nz == 16 ? 5 : c.nz / 2 - 2);
+  }
   FftSet fsets[N_FSETS];
   Chunk* d_chunks[N_SETS] = {};
   int* d_chunk_pairs[N_SETS] = {};
@@ -1929,8 +1932,7 @@ static void build_batch_launch(Batch& B) {
   for (size_t i = 0; i < B.plans.size(); ++i) {
     const Plan& P = *B.plans[i];
     if (P.fft.ok) {
-      const int k = (P.fft.shape.TL == 16 ? 0 : (P.fft.shape.TL == 8 ? 2 : 4)) + (P.fft.shape.nq <= 8 ? 0 : 1);
-      B.set_of[i] = P.nd == 3 ? Batch::SET_3D : -1 - k;
+      B.set_of[i] = P.nd == 3 ? Batch::SET_3D : -1 - Batch::fft_set(P.fft.shape);
       B.gen.push_back(P.ws_gen);
       continue;
     }
@@ -1956,7 +1958,7 @@ static void build_batch_launch(Batch& B) {
       S.inst.push_back(make_fft_inst(P, 1));
       S.d_tw = P.fft.d_tw;
       S.TL = P.fft.shape.TL;
-      S.half = P.fft.shape.nq <= 8;
+      S.nz = P.fft.shape.nz;
     }
     if (!S.inst.empty()) finalize_fft_set(S);
   }

@@ -57,19 +57,27 @@ __device__ __forceinline__ R fft_r2(R a) {
 
 constexpr double FFT_C1 = 0.92387953251128675613, FFT_S1 = 0.38268343236508977173;
 
-// DFT of 16, exp(+2 pi i q k / 16), in place and in order; with HALF the
-// entries q >= 8 are taken as zero.
-template <typename R, bool HALF, bool ACC = false>
+// DFT of 16, exp(+2 pi i q k / 16), in place and in order; the entries
+// q >= NZ are taken as zero.
+template <typename R, int NZ, bool ACC = false>
 __device__ __forceinline__ void dft16(Cx<R> (&x)[16]) {
   const R c1 = (R)FFT_C1, s1 = (R)FFT_S1;
   Cx<R> t[4][4];   // t[b][c], q = 4 a + b, k = c + 4 d
 #pragma unroll
   for (int b = 0; b < 4; ++b) {
-    if (HALF) {
+    if (4 + b >= NZ) {   // one entry
+      t[b][0] = t[b][1] = t[b][2] = t[b][3] = x[b];
+    } else if (8 + b >= NZ) {   // two
       t[b][0] = cadd(x[b], x[4 + b]);
       t[b][1] = caddi(x[b], x[4 + b]);
       t[b][2] = csub(x[b], x[4 + b]);
       t[b][3] = csubi(x[b], x[4 + b]);
+    } else if (12 + b >= NZ) {   // three
+      const Cx<R> s = cadd(x[b], x[8 + b]), d = csub(x[b], x[8 + b]);
+      t[b][0] = cadd(s, x[4 + b]);
+      t[b][1] = caddi(d, x[4 + b]);
+      t[b][2] = csub(s, x[4 + b]);
+      t[b][3] = csubi(d, x[4 + b]);
     } else {
       t[b][0] = x[b];
       t[b][1] = x[4 + b];
@@ -133,22 +141,32 @@ struct FftShape {
 };
 
 // Transform of the FPW length-16*TL sequences of a wave, exp(+2 pi i n k / L):
-// x[q] holds entry j + TL * q on entry and on return.  tw: the lane's twiddles
-// exp(2 pi i j k / L), k = 0 .. 15; lds: the wave's own exchange buffer (the
-// LDS operations of one wave complete in order, so no barrier is needed).
-template <typename R, int TL, bool HALF, bool ACC = false>
-__device__ __forceinline__ void fft_wave(Cx<R> (&x)[16], const Cx<R> (&tw)[16], Cx<R>* lds, int lane) {
+// x[q] holds entry j + TL * q on entry and on return, entries q >= NZ are
+// taken as zero.  tw(k): the lane's twiddle exp(2 pi i j k / L); lds: the
+// wave's own exchange buffer (the LDS operations of one wave complete in
+// order, so no barrier is needed).
+// mid: called between the exchange's writes and its reads (loads that the
+// second half should cover).
+template <typename R, int TL, int NZ, bool ACC, typename Tw, typename Mid>
+__device__ __forceinline__ void fft_wave_t(Cx<R> (&x)[16], Tw&& tw, Cx<R>* lds, int lane, Mid&& mid) {
   constexpr int FPW = FftShape<TL>::FPW, ROW = FftShape<TL>::ROW;
   const int j = lane / FPW, g = lane % FPW;
-  dft16<R, HALF, ACC>(x);
+  dft16<R, NZ, ACC>(x);
 #pragma unroll
-  for (int k = 0; k < 16; ++k) lds[k * ROW + lane] = k == 0 ? x[0] : cmulc(x[k], tw[k].x, tw[k].y);
+  for (int k = 0; k < 16; ++k) {
+    if (k > 0) {
+      const Cx<R> w = tw(k);
+      x[k] = cmulc(x[k], w.x, w.y);
+    }
+    lds[k * ROW + lane] = x[k];
+  }
+  mid();
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
   if constexpr (TL == 16) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) x[i] = lds[j * ROW + i * FPW + g];
-    dft16<R, false, ACC>(x);
+    dft16<R, 16, ACC>(x);
   } else if constexpr (TL == 8) {
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
@@ -172,6 +190,38 @@ __device__ __forceinline__ void fft_wave(Cx<R> (&x)[16], const Cx<R> (&tw)[16], 
   }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
+}
+
+// Twiddles in registers
+template <typename R, int TL, bool HALF, bool ACC = false>
+__device__ __forceinline__ void fft_wave(Cx<R> (&x)[16], const Cx<R> (&tw)[16], Cx<R>* lds, int lane) {
+  fft_wave_t<R, TL, HALF ? 8 : 16, ACC>(x, [&](int k) { return tw[k]; }, lds, lane, [] {});
+}
+
+// Twiddles in LDS, [16][TL]: 30 registers fewer, a third wave per SIMD where
+// these were what kept it out.
+template <int TL, int NZ, typename Mid>
+__device__ __forceinline__ void fft_wave_l(cf (&x)[16], const cf* twl, cf* lds, int lane, Mid&& mid) {
+  const cf* mine = twl + lane / FftShape<TL>::FPW;
+  cf tw[16];
+#pragma unroll
+  for (int k = 1; k < 16; ++k) tw[k] = mine[k * TL];
+  __builtin_amdgcn_sched_barrier(0);   // in flight during the first DFT
+  fft_wave_t<float, TL, NZ, false>(x, [&](int k) { return tw[k]; }, lds, lane, mid);
+}
+template <int TL, int NZ>
+__device__ __forceinline__ void fft_wave_l(cf (&x)[16], const cf* twl, cf* lds, int lane) {
+  fft_wave_l<TL, NZ>(x, twl, lds, lane, [] {});
+}
+
+// All threads of the workgroup.
+template <int TL>
+__device__ __forceinline__ void load_twiddles_lds(const float2* __restrict__ tw, cf* twl) {
+  for (int i = threadIdx.x; i < 16 * TL; i += blockDim.x) {
+    const float2 v = tw[(i % TL) * 16 + i / TL];
+    twl[i] = {v.x, v.y};
+  }
+  __syncthreads();
 }
 
 template <int TL>

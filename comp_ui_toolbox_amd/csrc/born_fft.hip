@@ -21,24 +21,22 @@
 // fastest, so that with 4 points per pitch and L = 256 a wave reads 64
 // consecutive grid points per load.
 //
-// Bound: the vector ALU (about 480 instructions per step of 1024 entries, 86 %
-// of the adjoint's cycles) close to the stream of the p_inc table (7.1 GB per
-// direction at 128 elements, 512 x 512 points, 257 frequencies, 11 waves).
-// Measured there per call: forward 1.90 ms, adjoint 1.60 ms, against 7.2 and
-// 6.8 ms of the direct products on FP32 MFMA and 2.4 and 2.6 ms in split
-// BF16; relative L2 error against FP64 3.1e-7 (3.3e-7 and 6.3e-6 there).
+// Bound: the stream of the p_inc table (7.1 GB per direction at 128 elements,
+// 512 x 512 points, 257 frequencies, 11 waves) close to the vector ALU.
+// Measured there per call: forward kernel 1.75 ms, adjoint kernel 1.37 ms (5.2
+// TB/s, what the memory gives), against 7.2 and 6.8 ms of the direct products
+// on FP32 MFMA and 2.4 and 2.6 ms in split BF16; relative L2 error against
+// FP64 3.1e-7 (3.3e-7 and 6.3e-6 there).  Entries of a lane come in counts of
+// 4 to 16 (fft_entries), twiddles from LDS: with 8 or 16 entries, branches on
+// the slot's length and twiddles in registers the two took 1.79 and 1.54 ms,
+// and 264 and 232 instead of 223 and 202 us at 100 elements, 301 x 411 points,
+// 2 points per pitch, 7 waves.
 #include "born_fft.h"
 #include "born_internal.h"
 
 #include <algorithm>
 #include <cmath>
 
-#ifndef FFT_FWD_OCC
-#define FFT_FWD_OCC 2
-#endif
-#ifndef FFT_ADJ_OCC
-#define FFT_ADJ_OCC 2
-#endif
 namespace born {
 
 // ------------------------------------------------------------------ spectra
@@ -95,17 +93,18 @@ __device__ __forceinline__ const FftInst& fft_instance(const FftInst* inst, int 
 
 // The masked input (occupancy, cu:466-488: a point takes part iff some
 // right-hand side has |Re| or |Im| above DBL_EPSILON) in the order the forward
-// reads it: gs[r][group of slots][NQ / 2][64 lanes][2], zero where a lane's
+// reads it: gs[r][group of slots][NZ / 2][64 lanes][2], zero where a lane's
 // entry lies past its slot, so that the forward needs no bounds on it.
-template <int TL, int NQ>
+template <int TL>
 __global__ __launch_bounds__(256) void k_fft_gamma(const float2* __restrict__ gm, const int2* __restrict__ slot, int n_ws,
-                                                   int N_pts, int Np, int N_rhs, int mask, float2* __restrict__ gs) {
+                                                   int NZ, int N_pts, int Np, int N_rhs, int mask,
+                                                   float2* __restrict__ gs) {
   constexpr int FPW = FftShape<TL>::FPW;
   const size_t idx = blockIdx.x * (size_t)256 + threadIdx.x;
-  if (idx >= (size_t)n_ws * NQ * 64) return;
+  if (idx >= (size_t)n_ws * NZ * 64) return;
   const int lane = (int)(idx >> 1) & 63;
-  const int q = (int)((idx >> 7) % (NQ / 2)) * 2 + (int)(idx & 1);
-  const int ws = (int)((idx >> 7) / (NQ / 2));
+  const size_t wq = idx >> 7;
+  const int ws = (int)(wq / (NZ / 2)), q = (int)(wq - (size_t)ws * (NZ / 2)) * 2 + (int)(idx & 1);
   const int2 sl = slot[ws * FPW + lane % FPW];
   const int sp = lane / FPW + TL * q;
   bool occ = sp < sl.y;
@@ -118,19 +117,30 @@ __global__ __launch_bounds__(256) void k_fft_gamma(const float2* __restrict__ gm
     }
   }
   for (int r = 0; r < N_rhs; ++r)
-    gs[(size_t)r * n_ws * NQ * 64 + idx] = occ ? gm[(size_t)r * N_pts + at] : make_float2(0.f, 0.f);
+    gs[(size_t)r * n_ws * NZ * 64 + idx] = occ ? gm[(size_t)r * N_pts + at] : make_float2(0.f, 0.f);
 }
 
 // One wave per (slot block, column, right-hand side): column = pair in
 // frequency order.  The products with the spectra of H add up in registers
 // over the wave's slots; their transform back gives the slot block's partial
-// sums of the elements.  NP: points per pitch (0: any).  A lane reads p_inc
-// past its slot's end up to the last grid point (times a zero of gs).
-template <int TL, bool HALF, int NP>
-__global__ __launch_bounds__(256, FFT_FWD_OCC) void k_fft_fwd(const FftInst* __restrict__ inst, int n_inst,
+// sums of the elements.  NZ: entries of a lane that can hold points, NP:
+// points per pitch (0: any).  Lanes read NZ entries of p_inc whether or not
+// their slot holds as many (the others meet a zero of gs), with no branch on
+// the slot's length: a branch around a load makes the compiler wait for the
+// whole batch in front of the transform.  p_inc and the input of the next
+// step are in flight during a step, the spectra of a step during the second
+// half of its transform.
+// Compute alone (p_inc not read) takes 1.22-1.31 ms of the 1.75 ms at the
+// size above, the stream of p_inc alone 1.3 ms; measured and no faster: p_inc
+// two steps ahead (1.77), two columns per wave (1.79), four waves of a block
+// on one column's rows (1.94-2.26), three waves per SIMD with spills.
+template <int TL, int NZ, int NP>
+__global__ __launch_bounds__(256, 2) void k_fft_fwd(const FftInst* __restrict__ inst, int n_inst,
                                                     const float2* __restrict__ twid, int n_wg, int per) {
-  constexpr int FPW = FftShape<TL>::FPW, L = 16 * TL, NQ = HALF ? 8 : 16;
+  constexpr int FPW = FftShape<TL>::FPW, L = 16 * TL;
   __shared__ cf lds_all[4 * FftShape<TL>::LDS];
+  __shared__ cf twl[16 * TL];
+  load_twiddles_lds<TL>(twid, twl);
   const int wg = logical_block(per);
   if (wg >= n_wg) return;
   const FftInst& I = fft_instance(inst, n_inst, wg, true);
@@ -144,54 +154,48 @@ __global__ __launch_bounds__(256, FFT_FWD_OCC) void k_fft_fwd(const FftInst* __r
   const int c = cz % n_cols, zb = cz / n_cols;
   const int2 pf = I.col[c];   // pair, frequency
   const int ws0 = zb * I.ZR, ws1 = min(I.n_ws, ws0 + I.ZR);
+  const int Np = NP > 0 ? NP : I.Np;
   BORN_GLOBAL const float2* P = I.P + (size_t)pf.x * I.N_pts;
-  BORN_GLOBAL const float4* gs = (BORN_GLOBAL const float4*)I.gs + ((size_t)r * I.n_ws + ws0) * (NQ * 32) + lane;
+  BORN_GLOBAL const float4* gs = (BORN_GLOBAL const float4*)I.gs + ((size_t)r * I.n_ws + ws0) * (NZ * 32) + lane;
   BORN_GLOBAL const float4* H = (BORN_GLOBAL const float4*)(I.H + ((size_t)pf.y * I.n_ws + ws0) * 1024) + lane;
   BORN_GLOBAL const int2* slots = I.slot + g;
-  const int Np = NP > 0 ? NP : I.Np, nq = I.nq, last = I.N_pts - 1;
-  cf tw[16], G[16];
-  load_twiddles<TL>(twid, j, tw);
+  cf G[16];
 #pragma unroll
   for (int q = 0; q < 16; ++q) G[q] = {0.f, 0.f};
-  float2 pv[NQ];
-  float4 gv[NQ / 2];
-  auto load = [&](int base) {
-    const int at = base + Np * j;
-    if (base > last - Np * (TL * NQ)) {   // near the end of the grid
+  // p_inc of the pair through a buffer descriptor: reads past the grid give 0
+  const auto pr = __builtin_amdgcn_make_buffer_rsrc((void*)P, 0, (int)((unsigned)I.N_pts * 8u), 0x27000);
+  float2 pv[NZ];
+  float4 gv[NZ / 2];
+  auto load = [&](int ws, int base) {
+    const int off = (base + Np * j) * 8;
 #pragma unroll
-      for (int q = 0; q < NQ; ++q)
-        if (q < nq) pv[q] = P[min(at + Np * (TL * q), last)];
-    } else {
-#pragma unroll
-      for (int q = 0; q < NQ; ++q)
-        if (q < nq) pv[q] = P[at + Np * (TL * q)];
+    for (int q = 0; q < NZ; ++q) {
+      const auto v = __builtin_amdgcn_raw_buffer_load_b64(pr, off + Np * TL * 8 * q, 0, 0);
+      pv[q] = make_float2(__uint_as_float(v[0]), __uint_as_float(v[1]));
     }
 #pragma unroll
-    for (int q = 0; q < NQ / 2; ++q)
-      if (2 * q < nq) gv[q] = gs[q * 64];
-    gs += NQ * 32;
+    for (int q = 0; q < NZ / 2; ++q) gv[q] = gs[(size_t)(ws - ws0) * (NZ * 32) + q * 64];
   };
-  load(slots[ws0 * FPW].x);
+  load(ws0, slots[ws0 * FPW].x);
   int next = slots[min(ws0 + 1, ws1 - 1) * FPW].x;
   for (int ws = ws0; ws < ws1; ++ws) {
     cf x[16];
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      x[q] = {0.f, 0.f};
-      if (q < nq) {
-        const float gx = q & 1 ? gv[q / 2].z : gv[q / 2].x, gy = q & 1 ? gv[q / 2].w : gv[q / 2].y;
-        x[q] = {fmaf(pv[q].x, gx, -(pv[q].y * gy)), fmaf(pv[q].x, gy, pv[q].y * gx)};
-      }
+    for (int q = 0; q < NZ; ++q) {
+      const float gx = q & 1 ? gv[q / 2].z : gv[q / 2].x, gy = q & 1 ? gv[q / 2].w : gv[q / 2].y;
+      x[q] = {fmaf(pv[q].x, gx, -(pv[q].y * gy)), fmaf(pv[q].x, gy, pv[q].y * gx)};
     }
+    load(min(ws + 1, ws1 - 1), next);   // (the last step reads its own entries again)
+    next = slots[min(ws + 2, ws1 - 1) * FPW].x;
+    __builtin_amdgcn_sched_barrier(0);
     float4 hv[8];
+    fft_wave_l<TL, NZ>(x, twl, lds, lane, [&] {
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int q = 0; q < 8; ++q) hv[q] = H[q * 64];
+      for (int q = 0; q < 8; ++q) hv[q] = H[q * 64];
+      __builtin_amdgcn_sched_barrier(0);
+    });
     H += 512;
-    if (ws + 1 < ws1) {
-      load(next);
-      next = slots[min(ws + 2, ws1 - 1) * FPW].x;
-    }
-    fft_wave<float, TL, HALF>(x, tw, lds, lane);
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
       cmac(G[2 * q], cf{hv[q].x, hv[q].y}, x[2 * q]);
@@ -206,7 +210,7 @@ __global__ __launch_bounds__(256, FFT_FWD_OCC) void k_fft_fwd(const FftInst* __r
       G[q].x += __shfl_xor(G[q].x, m);
       G[q].y += __shfl_xor(G[q].y, m);
     }
-  fft_wave<float, TL, false>(G, tw, lds, lane);
+  fft_wave_l<TL, 16>(G, twl, lds, lane);
   if (g == 0) {
     BORN_GLOBAL float2* out = I.vp + ((size_t)(zb * N_rhs + r) * n_cols + c) * I.N_e;
 #pragma unroll
@@ -280,11 +284,13 @@ __global__ __launch_bounds__(256) void k_fft_weights(const float2* __restrict__ 
 
 // One workgroup per (slot group, right-hand side, column group); its 4 waves
 // share the group's columns and add up their sums through LDS.
-template <int TL, bool HALF>
-__global__ __launch_bounds__(256, FFT_ADJ_OCC) void k_fft_adj(const FftInst* __restrict__ inst, int n_inst, OutPtrs outs,
+template <int TL, int NZ>
+__global__ __launch_bounds__(256, 2) void k_fft_adj(const FftInst* __restrict__ inst, int n_inst, OutPtrs outs,
                                                     const float2* __restrict__ twid, int n_wg, int per) {
-  constexpr int FPW = FftShape<TL>::FPW, NQ = HALF ? 8 : 16;
+  constexpr int FPW = FftShape<TL>::FPW;
   __shared__ cf lds_all[4 * FftShape<TL>::LDS];
+  __shared__ cf twl[16 * TL];
+  load_twiddles_lds<TL>(twid, twl);
   const int wg = logical_block(per);
   if (wg >= n_wg) return;
   const FftInst& I = fft_instance(inst, n_inst, wg, false);
@@ -299,28 +305,23 @@ __global__ __launch_bounds__(256, FFT_ADJ_OCC) void k_fft_adj(const FftInst* __r
   const int part = fgr * 4 + wave;   // of 4 FG contiguous column ranges
   const int c0 = (int)((long)n_cols * part / (4 * FG)), c1 = (int)((long)n_cols * (part + 1) / (4 * FG));
   const int2 sl = I.slot[ws * FPW + g];
-  const int Np = I.Np, nq = I.nq;
-  int at[NQ];
-  bool ok[NQ];
+  const int Np = I.Np;
+  int at[NZ];
+  bool ok[NZ];
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) {
+  for (int q = 0; q < NZ; ++q) {
     const int s = j + TL * q;
     ok[q] = s < sl.y;
     at[q] = sl.x + (ok[q] ? Np * s : 0);
   }
-  cf tw[16], acc[NQ];
-  load_twiddles<TL>(twid, j, tw);
+  cf acc[NZ];
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) acc[q] = {0.f, 0.f};
+  for (int q = 0; q < NZ; ++q) acc[q] = {0.f, 0.f};
   float4 hv[8];
   int f_have = -1;
   for (int c = c0; c < c1; ++c) {
     const int2 pf = I.col[c];
     BORN_GLOBAL const float2* P = I.P + (size_t)pf.x * I.N_pts;
-    float2 pv[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
-      if (q < nq) pv[q] = P[at[q]];
     if (pf.y != f_have) {
       f_have = pf.y;
       BORN_GLOBAL const float4* H = (BORN_GLOBAL const float4*)(I.H + ((size_t)pf.y * I.n_ws + ws) * 1024) + lane;
@@ -328,26 +329,32 @@ __global__ __launch_bounds__(256, FFT_ADJ_OCC) void k_fft_adj(const FftInst* __r
       for (int q = 0; q < 8; ++q) hv[q] = H[q * 64];
     }
     BORN_GLOBAL const float4* wt = (BORN_GLOBAL const float4*)I.wt + ((size_t)pf.x * N_rhs + r) * (8 * TL) + j;
+    float4 wv[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) wv[q] = wt[q * TL];
+    __builtin_amdgcn_sched_barrier(0);   // all loads in flight before the first is waited for,
+    float2 pv[NZ];                       // p_inc last: it stays in flight during the transform
+#pragma unroll
+    for (int q = 0; q < NZ; ++q) pv[q] = P[at[q]];
+    __builtin_amdgcn_sched_barrier(0);
     cf x[16];
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-      const float4 w = wt[q * TL];
-      x[2 * q] = {fmaf(hv[q].x, w.x, -(hv[q].y * w.y)), fmaf(hv[q].x, w.y, hv[q].y * w.x)};
-      x[2 * q + 1] = {fmaf(hv[q].z, w.z, -(hv[q].w * w.w)), fmaf(hv[q].z, w.w, hv[q].w * w.z)};
+      x[2 * q] = {fmaf(hv[q].x, wv[q].x, -(hv[q].y * wv[q].y)), fmaf(hv[q].x, wv[q].y, hv[q].y * wv[q].x)};
+      x[2 * q + 1] = {fmaf(hv[q].z, wv[q].z, -(hv[q].w * wv[q].w)), fmaf(hv[q].z, wv[q].w, hv[q].w * wv[q].z)};
     }
-    fft_wave<float, TL, false>(x, tw, lds, lane);
+    fft_wave_l<TL, 16>(x, twl, lds, lane);
 #pragma unroll
-    for (int q = 0; q < NQ; ++q)
-      if (q < nq) cmac(acc[q], cf{pv[q].x, pv[q].y}, x[q]);
+    for (int q = 0; q < NZ; ++q) cmac(acc[q], cf{pv[q].x, pv[q].y}, x[q]);
   }
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) lds[q * 64 + lane] = acc[q];
+  for (int q = 0; q < NZ; ++q) lds[q * 64 + lane] = acc[q];
   __syncthreads();
   BORN_GLOBAL float2* out = FG > 1 ? I.gp + (size_t)fgr * N_rhs * I.N_pts : (BORN_GLOBAL float2*)outs.p[&I - inst];
   out += (size_t)r * I.N_pts;
 #pragma unroll
-  for (int q = 0; q < NQ; ++q)
-    if ((q & 3) == wave && q < nq && ok[q]) {
+  for (int q = 0; q < NZ; ++q)
+    if ((q & 3) == wave && ok[q]) {
       cf s = {0.f, 0.f};
 #pragma unroll
       for (int w = 0; w < 4; ++w) s = cadd(s, lds_all[w * FftShape<TL>::LDS + q * 64 + lane]);
@@ -369,6 +376,9 @@ __global__ __launch_bounds__(256) void k_fft_adj_reduce(const float2* __restrict
 }
 
 // ------------------------------------------------------------------ host side
+// Entries of a lane that the kernels take, at least n: 4, 6, 8, 10, 12 or 16.
+static int fft_entries(int n) { return n <= 4 ? 4 : n <= 12 ? (n + 1) / 2 * 2 : 16; }
+
 // Transform length and segments of a row of S points per phase under N_e
 // elements: the cheapest of the lengths (time grows with the entries
 // transformed; sequences at most half full skip part of the first stage).
@@ -384,8 +394,8 @@ FftShapeChoice fft_shape(int Nx, int Np, int N_e) {
     c.TL = TL;
     c.nseg = (S + room - 1) / room;
     c.Sv = (S + c.nseg - 1) / c.nseg;
-    c.nq = (c.Sv + TL - 1) / TL;
-    const double cost = (double)c.nseg * L * (c.nq <= 8 ? 1.0 : 1.12);
+    c.nz = fft_entries((c.Sv + TL - 1) / TL);
+    const double cost = (double)c.nseg * L * (c.nz <= 8 ? 1.0 : 1.12);
     if (cost < cost_best) {
       cost_best = cost;
       best = c;
@@ -415,29 +425,33 @@ void launch_fft_table(const Plan& P, hipStream_t s) {
 #undef BORN_FFT_TABLE
 }
 
-#define BORN_FFT_DISPATCH(K, ...)                                             \
-  do {                                                                        \
-    if (S.TL == 16 && S.half) hipLaunchKernelGGL((K<16, true>), __VA_ARGS__); \
-    else if (S.TL == 16) hipLaunchKernelGGL((K<16, false>), __VA_ARGS__);     \
-    else if (S.TL == 8 && S.half) hipLaunchKernelGGL((K<8, true>), __VA_ARGS__); \
-    else if (S.TL == 8) hipLaunchKernelGGL((K<8, false>), __VA_ARGS__);       \
-    else if (S.half) hipLaunchKernelGGL((K<4, true>), __VA_ARGS__);           \
-    else hipLaunchKernelGGL((K<4, false>), __VA_ARGS__);                      \
+#define BORN_FFT_NZ(F, TLv)         \
+  do {                              \
+    switch (S.nz) {                 \
+      case 4: F(TLv, 4); break;     \
+      case 6: F(TLv, 6); break;     \
+      case 8: F(TLv, 8); break;     \
+      case 10: F(TLv, 10); break;   \
+      case 12: F(TLv, 12); break;   \
+      default: F(TLv, 16); break;   \
+    }                               \
+  } while (0)
+#define BORN_FFT_DISPATCH(F)               \
+  do {                                     \
+    if (S.TL == 16) BORN_FFT_NZ(F, 16);    \
+    else if (S.TL == 8) BORN_FFT_NZ(F, 8); \
+    else BORN_FFT_NZ(F, 4);                \
   } while (0)
 
 void launch_fft_gamma(const Plan& P, const float2* gamma, int N_rhs, bool mask, hipStream_t s) {
   const Plan::Fft& F = P.fft;
-  const int NQ = F.shape.nq <= 8 ? 8 : 16;
-  const dim3 grid((unsigned)(((size_t)F.n_ws * NQ * 64 + 255) / 256));
-#define BORN_FFT_G(TLv, NQv)                                                                                         \
-  hipLaunchKernelGGL((k_fft_gamma<TLv, NQv>), grid, dim3(256), 0, s, gamma, F.d_slot, F.n_ws, P.N_pts, P.Np, N_rhs, \
-                     (int)mask, F.d_gs)
-  if (F.shape.TL == 16 && NQ == 8) BORN_FFT_G(16, 8);
-  else if (F.shape.TL == 16) BORN_FFT_G(16, 16);
-  else if (F.shape.TL == 8 && NQ == 8) BORN_FFT_G(8, 8);
-  else if (F.shape.TL == 8) BORN_FFT_G(8, 16);
-  else if (NQ == 8) BORN_FFT_G(4, 8);
-  else BORN_FFT_G(4, 16);
+  const dim3 grid((unsigned)(((size_t)F.n_ws * F.shape.nz * 64 + 255) / 256));
+#define BORN_FFT_G(TLv)                                                                                               \
+  hipLaunchKernelGGL(k_fft_gamma<TLv>, grid, dim3(256), 0, s, gamma, F.d_slot, F.n_ws, F.shape.nz, P.N_pts, P.Np, \
+                     N_rhs, (int)mask, F.d_gs)
+  if (F.shape.TL == 16) BORN_FFT_G(16);
+  else if (F.shape.TL == 8) BORN_FFT_G(8);
+  else BORN_FFT_G(4);
 #undef BORN_FFT_G
 }
 
@@ -447,21 +461,16 @@ void launch_fft_fwd(const FftSet& S, hipStream_t s) {
   int Np = S.inst[0].Np;
   for (const FftInst& I : S.inst)
     if (I.Np != Np) Np = 0;
-#define BORN_FFT_F(TLv, Hv, NPv)                                                                                   \
-  hipLaunchKernelGGL((k_fft_fwd<TLv, Hv, NPv>), dim3(per * XCDS), dim3(256), 0, s, S.d_inst, (int)S.inst.size(), \
+#define BORN_FFT_F(TLv, NZv, NPv)                                                                                   \
+  hipLaunchKernelGGL((k_fft_fwd<TLv, NZv, NPv>), dim3(per * XCDS), dim3(256), 0, s, S.d_inst, (int)S.inst.size(), \
                      S.d_tw, S.n_wg_f, per)
-#define BORN_FFT_FN(TLv, Hv)                      \
-  do {                                            \
-    if (Np == 4) BORN_FFT_F(TLv, Hv, 4);          \
-    else if (Np == 2) BORN_FFT_F(TLv, Hv, 2);     \
-    else BORN_FFT_F(TLv, Hv, 0);                  \
+#define BORN_FFT_FN(TLv, NZv)                  \
+  do {                                         \
+    if (Np == 4) BORN_FFT_F(TLv, NZv, 4);      \
+    else if (Np == 2) BORN_FFT_F(TLv, NZv, 2); \
+    else BORN_FFT_F(TLv, NZv, 0);              \
   } while (0)
-  if (S.TL == 16 && S.half) BORN_FFT_FN(16, true);
-  else if (S.TL == 16) BORN_FFT_FN(16, false);
-  else if (S.TL == 8 && S.half) BORN_FFT_FN(8, true);
-  else if (S.TL == 8) BORN_FFT_FN(8, false);
-  else if (S.half) BORN_FFT_FN(4, true);
-  else BORN_FFT_FN(4, false);
+  BORN_FFT_DISPATCH(BORN_FFT_FN);
 #undef BORN_FFT_FN
 #undef BORN_FFT_F
 }
@@ -469,8 +478,11 @@ void launch_fft_fwd(const FftSet& S, hipStream_t s) {
 void launch_fft_adj(const FftSet& S, const OutPtrs& outs, hipStream_t s) {
   if (S.inst.empty()) return;
   const int per = (S.n_wg_a + XCDS - 1) / XCDS;
-  BORN_FFT_DISPATCH(k_fft_adj, dim3(per * XCDS), dim3(256), 0, s, S.d_inst, (int)S.inst.size(), outs, S.d_tw,
-                    S.n_wg_a, per);
+#define BORN_FFT_A(TLv, NZv)                                                                                          \
+  hipLaunchKernelGGL((k_fft_adj<TLv, NZv>), dim3(per * XCDS), dim3(256), 0, s, S.d_inst, (int)S.inst.size(), outs, \
+                     S.d_tw, S.n_wg_a, per)
+  BORN_FFT_DISPATCH(BORN_FFT_A);
+#undef BORN_FFT_A
 }
 
 void launch_fft_reduce(const Plan& P, int N_rhs, hipStream_t s) {

@@ -117,10 +117,10 @@ struct LaunchSet {
 };
 
 // Fast lateral correlation of 2-D plans (born_fft.hip): transforms of length
-// 16 * TL over rows cut into nseg segments of Sv points per phase; nq: entries
-// of a lane that can hold points.
+// 16 * TL over rows cut into nseg segments of Sv points per phase; nz: entries
+// of a lane that the kernels take (those that can hold points, rounded up).
 struct FftShapeChoice {
-  int TL = 0, nseg = 1, Sv = 0, nq = 0;
+  int TL = 0, nseg = 1, Sv = 0, nz = 0;
 };
 
 // 3-D plans (born_fft3d.hip): transforms of 16 TLX x 16 TLY, px lateral
@@ -151,24 +151,23 @@ struct FftInst {
   BORN_GLOBAL const float2* P;     // p_inc rows
   BORN_GLOBAL const int2* slot;    // [n_ws * 64 / TL] first point, points (0 past the last slot)
   BORN_GLOBAL const int2* col;     // [n_cols] (pair, frequency), by frequency
-  BORN_GLOBAL const float2* gs;    // masked input [N_rhs][n_ws][8 or 16 entries / 2][64][2]
+  BORN_GLOBAL const float2* gs;    // masked input [N_rhs][n_ws][nz / 2][64][2]
   BORN_GLOBAL const float2* wt;    // adjoint weight spectra [N_pairs][N_rhs][8][TL][2]
   BORN_GLOBAL float2* vp;          // forward partials [NZB][N_rhs][n_cols][N_e]
   BORN_GLOBAL float2* gp;          // adjoint partials [FG][N_rhs][N_pts] (FG > 1)
-  int N_pts, N_e, Np, nq;
+  int N_pts, N_e, Np;
   int n_ws, n_cols, N_rhs;
   int NZB, ZR;                     // forward: slot blocks of ZR wave steps
   int FG;                          // adjoint: column groups
   int wg_f, wg_a;                  // first workgroup of the instance (forward, adjoint)
 };
 
-// Launch of instances that share the transform length and the half-full form.
+// Launch of instances that share the transform length and the entries per lane.
 struct FftSet {
   FftInst* d_inst = nullptr;
   std::vector<FftInst> inst;
   const float2* d_tw = nullptr;    // twiddles [TL][16] (owned by a plan of the set)
-  int TL = 0;
-  bool half = false;
+  int TL = 0, nz = 0;
   int n_wg_f = 0, n_wg_a = 0;
 };
 

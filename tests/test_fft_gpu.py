@@ -49,6 +49,11 @@ SIZES = [
     (33, 101, 6, 3, 3, 2, 0, 2),       # phases that do not divide the slots of a wave
     (20, 77, 3, 5, 2, 2, 2, 1),
     (31, 40, 9, 1, 3, 2, 0, 1),        # field of view narrower than the aperture, one point per pitch
+    # the remaining counts of entries per lane (4 to 16) of each length
+    (27, 30, 3, 1, 2, 2, 0, 1), (13, 134, 3, 1, 2, 2, 0, 2), (6, 214, 2, 2, 2, 2, 0, 1),       # 64: 8, 12, 16
+    (91, 36, 3, 3, 2, 2, 0, 1), (70, 90, 3, 1, 2, 2, 0, 2), (32, 176, 2, 1, 2, 2, 0, 1),       # 128: 4, 6, 12
+    (17, 402, 2, 2, 2, 2, 0, 1),                                                              # 128: 16
+    (98, 63, 3, 1, 2, 2, 0, 2), (61, 353, 2, 2, 2, 2, 0, 1), (33, 209, 3, 1, 2, 2, 0, 1),      # 256: 4, 12, 16
 ]
 
 
