@@ -475,11 +475,25 @@ static void build_fft3(Plan& P) {
 // Tables of the fast lateral correlation, built once per plan: the slots
 // (row, segment, phase), the columns by frequency and the spectra of h_ref.
 // The spectra take about twice the space of h_ref; a plan whose spectra do
-// not fit in the free memory with 1 GiB to spare stays on the MFMA kernels.
+// not fit in the free memory with 1 GiB to spare stays on the MFMA kernels,
+// and so does one whose rows of h_ref are too uneven (k_fft_range).
 static void build_fft(Plan& P) {
   Plan::Fft& F = P.fft;
   F.ok = false;
-  if (!P.structured) return;
+  if (!P.structured || P.N_fu > 65535 || (int64_t)P.Nz * P.N_fu > INT32_MAX) return;   // (grids of the tables' kernels)
+  {
+    int bad = 0;
+    int* d_bad = dupload(std::vector<int>(1, 0), P.stream);
+    launch_fft_range(P, d_bad, P.stream);
+    const hipError_t e = hipGetLastError();
+    const hipError_t e2 = hipMemcpyAsync(&bad, d_bad, sizeof(int), hipMemcpyDeviceToHost, P.stream);
+    const hipError_t e3 = hipStreamSynchronize(P.stream);
+    dfree(d_bad);
+    HIP_CHECK(e);
+    HIP_CHECK(e2);
+    HIP_CHECK(e3);
+    if (bad) return;
+  }
   if (P.nd == 3) {
     build_fft3(P);
     return;

@@ -79,6 +79,66 @@ __global__ __launch_bounds__(64) void k_fft_table(const float2* __restrict__ h, 
     out[q * 64 + lane] = make_float4((float)x[2 * q].x, -(float)x[2 * q].y, (float)x[2 * q + 1].x, -(float)x[2 * q + 1].y);
 }
 
+// Whether the lateral rows (2-D) or planes (3-D) of h_ref may be transformed.
+// A transform spreads the rounding of a row's norm over all its entries, where
+// the direct products keep that of an entry to itself.  A field's row has its
+// norm in a main lobe of many entries.  One that has it in a single entry (a
+// grid point next to an element) would lose the others: bad is set for a row
+// whose largest entry is not finite, or holds more than a quarter of the row's
+// energy and exceeds the geometric mean of the nonzero entries 16 times (rows
+// of few entries reach the first by themselves).  In volumes the entry in
+// front of an element has 1/8 of its plane's energy at half a grid spacing and
+// 1/4 at a third of one; in 2-D it stays below.  One block per (row or plane, frequency).
+__global__ __launch_bounds__(256) void k_fft_range(const float2* __restrict__ h, const int* __restrict__ ext,
+                                                   const int* __restrict__ exty, int N_ext, int ny, int H_plane, int HR,
+                                                   int HY, int Nz, int* __restrict__ bad) {
+  __shared__ float red[3][256];
+  const int tid = threadIdx.x;
+  const float2* src = h + (size_t)(blockIdx.x / Nz) * H_plane + (size_t)(blockIdx.x % Nz) * HY * HR;
+  const int n = N_ext * ny;
+  auto entry = [&](int i) { return src[(exty ? (size_t)exty[i / N_ext] * HR : 0) + ext[i % N_ext]]; };
+  float top = 0.f;
+  bool fine = true;
+  for (int i = tid; i < n; i += 256) {
+    const float2 v = entry(i);
+    fine = fine && fabsf(v.x) < 1e30f && fabsf(v.y) < 1e30f;   // (false for NaN)
+    top = fmaxf(top, fmaxf(fabsf(v.x), fabsf(v.y)));
+  }
+  red[0][tid] = fine ? top : 2e30f;
+  __syncthreads();
+  for (int k = 128; k > 0; k >>= 1) {
+    if (tid < k) red[0][tid] = fmaxf(red[0][tid], red[0][tid + k]);
+    __syncthreads();
+  }
+  top = red[0][0];
+  __syncthreads();
+  float peak = 0.f, energy = 0.f, logs = 0.f, count = 0.f;
+  if (top > 0.f && top < 1e30f)
+    for (int i = tid; i < n; i += 256) {
+      const float2 v = entry(i);
+      const float x = v.x / top, y = v.y / top, m = x * x + y * y;
+      peak = fmaxf(peak, m);
+      energy += m;
+      if (m > 0.f) {
+        logs += log2f(m);
+        count += 1.f;
+      }
+    }
+  red[0][tid] = energy;
+  red[1][tid] = logs;
+  red[2][tid] = count;
+  __syncthreads();
+  for (int k = 128; k > 0; k >>= 1) {
+    if (tid < k)
+      for (int a = 0; a < 3; ++a) red[a][tid] += red[a][tid + k];
+    __syncthreads();
+  }
+  energy = red[0][0];
+  const float mean = red[1][0] / fmaxf(red[2][0], 1.f);
+  const bool uneven = peak > 0.25f * energy && log2f(peak) - mean > 8.f;   // (of squares)
+  if (uneven || top >= 1e30f) atomicOr(bad, 1);
+}
+
 // ------------------------------------------------------------------ forward
 // Blocks in logical order: blocks are dispatched round-robin over the XCDS
 // dies, so block b takes logical block (b % XCDS) * per + b / XCDS and the
@@ -442,6 +502,13 @@ void launch_fft_table(const Plan& P, hipStream_t s) {
     else if (S.TL == 8) BORN_FFT_NZ(F, 8); \
     else BORN_FFT_NZ(F, 4);                \
   } while (0)
+
+void launch_fft_range(const Plan& P, int* bad, hipStream_t s) {
+  const bool y = P.nd == 3;
+  hipLaunchKernelGGL(k_fft_range, dim3((unsigned)P.Nz * (unsigned)P.N_fu), dim3(256), 0, s, P.d_h, P.d_ext,
+                     y ? P.d_exty : nullptr, P.N_ext, y ? P.Ny + (P.Ney - 1) * P.Npy : 1, P.H_plane, P.HR, P.HY, P.Nz,
+                     bad);
+}
 
 void launch_fft_gamma(const Plan& P, const float2* gamma, int N_rhs, bool mask, hipStream_t s) {
   const Plan::Fft& F = P.fft;

@@ -138,3 +138,43 @@ def test_volume(torch_cuda, nex, ney, nx, ny, nz, npp, nf, waves, n_rhs):
         for k in range(2):
             assert O.rel_l2(fast[k][r], ref[k].reshape(-1)) < 1.5e-6, ("oracle", k)
             assert O.rel_l2(fast[k][r], general[k][r]) < 3e-6, ("general", k)
+
+
+@pytest.mark.parametrize("three", [False, True])
+@pytest.mark.parametrize("entry", [1e7, np.inf])
+def test_uneven_tables_keep_the_direct_products(torch_cuda, three, entry):
+    """One entry of h_ref far above the others (a grid point next to an
+    element): what the other entries give has to keep its accuracy, which a
+    transform over the row would lose to the rounding of the large one."""
+    spec = make(33, 101, 6, 3, 3, 2)
+    if three:
+        arr = C.ArraySpec((4, 3), (3e-4, 3e-4), (2.7e-4, 2.7e-4), (2, 2))
+        waves = [C.random_wave(arr, np.random.Generator(np.random.PCG64(w)), 1e-6) for w in range(2)]
+        spec = C.SequenceSpec("fft3", arr, C.MediumSpec(), C.FovSpec((19, 7, 3), (1.5e-4,) * 3, 3e-3),
+                              np.linspace(2.5e6, 4e6, 2), waves, [C.identity_mixes(12) for _ in waves])
+    T = O.build_tables(spec)
+    at = T.N_points // 3
+    touched = np.any(np.asarray(T.shift).reshape(T.N_points, -1) - 1 == at, axis=1)
+    assert touched.any() and not touched.all()
+    clean = T.h_ref.copy()
+    T.h_ref[1, at] = entry
+    op = OperatorBorn.from_tables(T)
+    assert op.path == "structured"
+    rng = np.random.Generator(np.random.PCG64(9))
+    u = rng.standard_normal(op.N_observations) + 1j * rng.standard_normal(op.N_observations)
+    g = rng.standard_normal(op.N_points) + 1j * rng.standard_normal(op.N_points)
+    g[touched] = 0
+    op.force_general(True)
+    general = op.adjoint(u)
+    op.force_general(False)
+    back = op.adjoint(u)
+    T.h_ref = clean
+    ref = O.adjoint(T, u).reshape(-1)
+    assert O.rel_l2(general[~touched], ref[~touched]) < TOL
+    if np.isfinite(entry):
+        assert O.rel_l2(back[~touched], ref[~touched]) < TOL
+        assert O.rel_l2(op.forward(g), O.forward(T, g).reshape(-1)) < TOL
+    else:   # the points whose rows of the table hold no such entry
+        plane = T.N_points // spec.fov.N_points_axis[-1]
+        rest = np.arange(T.N_points) // plane != at // plane
+        assert O.rel_l2(back[rest], ref[rest]) < TOL
