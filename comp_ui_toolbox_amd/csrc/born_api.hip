@@ -529,18 +529,26 @@ static void build_fft(Plan& P) {
   F.ok = true;
 }
 
-// Work split of a plan's fast-correlation launches: forward waves of at least
-// 4 steps (a wave's final transform costs about two) and at most 64, about
-// 24576 of them; adjoint workgroups of 4 waves with at least 8 columns each,
-// about 12288 waves.
+// Work split of a plan's fast-correlation launches (the chip holds 3072 waves
+// of either kernel).  Forward: a wave's final transform costs about two steps,
+// so waves take 8 steps, fewer while that leaves less than half of the chip's
+// waves (3 at least; launch and first loads cost as much), and from 24576
+// waves on as many as keep that number, 64 at most.  Call at 128 elements,
+// 300 x 300 points, 65 frequencies, 2 waves: 62 us with 4 steps, 56 with 8; at
+// 256 x 256, 33 frequencies, one wave: 28 with 5, 30 with 4 and 8.
+// Adjoint: 3072 workgroups of 4 waves with at least 8 columns each, or 256 of
+// at least 2 columns (32 elements, 128 x 128 points, 65 frequencies: 25 us with
+// 32 workgroups, 17 with 128).
 static void fft_blocking(Plan& P, int N_rhs) {
   Plan::Fft& F = P.fft;
-  const int64_t cols = (int64_t)P.N_pairs * N_rhs;
-  F.ZR = (int)std::max<int64_t>(4, std::min<int64_t>(64, cols * F.n_ws / 24576));
+  const int64_t steps = (int64_t)P.N_pairs * N_rhs * F.n_ws;
+  F.ZR = (int)std::min<int64_t>(64, std::max<int64_t>(std::max<int64_t>(3, std::min<int64_t>(8, steps / 1536)), steps / 24576));
   F.ZR = std::min(F.ZR, F.n_ws);
   F.NZB = (F.n_ws + F.ZR - 1) / F.ZR;
   const int64_t wg = (int64_t)F.n_ws * N_rhs;
-  F.FG = (int)std::max<int64_t>(1, std::min<int64_t>({(3072 + wg - 1) / wg, P.N_pairs / 32, 64}));
+  const int64_t many = std::min<int64_t>((3072 + wg - 1) / wg, P.N_pairs / 32);
+  const int64_t few = std::min<int64_t>((256 + wg - 1) / wg, P.N_pairs / 8);
+  F.FG = (int)std::max<int64_t>(1, std::min<int64_t>(64, std::max(many, few)));
 }
 
 static FftInst make_fft_inst(const Plan& P, int N_rhs) {

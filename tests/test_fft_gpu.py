@@ -140,6 +140,15 @@ def test_volume(torch_cuda, nex, ney, nx, ny, nz, npp, nf, waves, n_rhs):
             assert O.rel_l2(fast[k][r], general[k][r]) < 3e-6, ("general", k)
 
 
+@pytest.mark.parametrize("ne,nx,nz,npp,nf,waves,n_mix,n_rhs", [
+    (8, 16, 400, 2, 2, 1, 0, 1),       # 24 slot blocks of a few values: eight threads per value
+    (9, 15, 200, 4, 3, 2, 5, 3),       # the same, several mixes and right-hand sides
+    (24, 40, 34, 1, 17, 3, 3, 1),      # columns in several groups per slot group
+])
+def test_split_of_small_plans(torch_cuda, ne, nx, nz, npp, nf, waves, n_mix, n_rhs):
+    test_against_oracle_and_general_path(torch_cuda, ne, nx, nz, npp, nf, waves, n_mix, n_rhs)
+
+
 @pytest.mark.parametrize("three", [False, True])
 @pytest.mark.parametrize("entry", [1e7, np.inf])
 def test_uneven_tables_keep_the_direct_products(torch_cuda, three, entry):
