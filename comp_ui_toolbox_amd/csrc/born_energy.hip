@@ -19,8 +19,7 @@
 // The map-driven kernel (k_energy_rx, one thread per point, one map read and
 // one gather per element) stays for plans off the structured path: it waits
 // on those reads.  128 elements, 384 x 384 points, 129 frequencies, identity
-// mixes: 22.4 ms per measurement there, 0.35 ms here (FP64 rate: 0.06 ms; the
-// fill of the windows takes as long as the multiply-adds).
+// mixes: 22.4 ms per measurement there, 0.18 ms here (FP64 rate: 0.06 ms).
 #include "born_fft.h"
 #include "born_internal.h"
 
@@ -98,17 +97,51 @@ __device__ __forceinline__ void e_fill(const EnergyArgs& A, const float2* __rest
   }
 }
 
-template <int R, int NP>
-__global__ __launch_bounds__(1024) void k_energy_single(EnergyArgs A, double* __restrict__ E) {
+// Entry N of the 16 that each row of 16 lanes holds, in all lanes.
+template <int N>
+__device__ __forceinline__ double e_bcast(double w) {
+  return __builtin_amdgcn_update_dpp(w, w, 0x150 + N, 0xf, 0xf, true);
+}
+
+// S[k] += w[D .. D1 - 1] of the chunk times entries k + D .. of x (block 0 at
+// x0, the next at x1).
+template <int R, int D, int D1>
+__device__ __forceinline__ void e_mac(double (&S)[R], double w, const double (&x0)[R], const double (&x1)[R]) {
+  if constexpr (D < D1) {
+    const double wv = e_bcast<D>(w);
+#pragma unroll
+    for (int k = 0; k < R; ++k) S[k] = fma(wv, k + D % R < R ? x0[(k + D) % R] : x1[(k + D) % R], S[k]);
+    e_mac<R, D + 1, D1>(S, w, x0, x1);
+  }
+}
+
+// The elements' weights are taken 2 R at a time: lane l holds number l % 16 of
+// the chunk, and each is broadcast within the rows of 16 lanes (through the
+// scalar cache, which they miss, a step of R elements took 750 cycles for 36
+// multiply-adds).  MI > 0: a lane's MI entries of the window and its weights are
+// loaded for the next pair during the multiply-adds of this one (positions in
+// the row and in LDS are the same for all pairs); MI = 0, for more than 16
+// entries: in between.
+// 128 elements, 384 x 384 points, 129 frequencies: 354 us with scalar weights
+// and windows filled in between, 268 with the windows loaded ahead, 182 with
+// both (the FP64 multiply-adds alone: 62).  What is left: 384 workgroups on 256
+// compute units (1.33), one broadcast and the window's LDS reads per R
+// multiply-adds.  Positions packed in one register (three waves per SIMD
+// instead of two) cost 14 % for the unpacking.
+template <int R, int MI>
+__global__ __launch_bounds__(512) void k_energy_single(EnergyArgs A, double* __restrict__ E) {
   extern __shared__ double e_lds[];
-  const int Np = NP > 0 ? NP : A.Np;
+  const int Np = A.Np;
   const int W = blockDim.x >> 6, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int row = blockIdx.x / A.nseg, seg = blockIdx.x - row * A.nseg;
   const int jl = lane / Np, phi = lane - jl * Np;
   const bool on = jl < A.LPW;
   const int s0 = seg * A.LPW * R;
-  double* win = e_lds + (size_t)wave * Np * A.WLp;
+  const int n_win = Np * A.WLp, n_w = A.nb * R;   // window, weights, then an entry for what lies past both
+  const int per_wave = n_win + n_w + 1;
+  double* win = e_lds + (size_t)wave * per_wave;
   const double* mine = win + phi * A.WLp + (on ? jl : 0) * (R + 1);
+  const double* wl = win + n_win + min(lane & 15, 2 * R - 1);
   const int c0 = (int)((long)A.n_pairs * wave / W), c1 = (int)((long)A.n_pairs * (wave + 1) / W);
   int at[R];
   double acc[R];
@@ -118,10 +151,49 @@ __global__ __launch_bounds__(1024) void k_energy_single(EnergyArgs A, double* __
     at[k] = row * A.Nx + min(i, A.Nx - 1);
     acc[k] = 0.0;
   }
+  constexpr int M = MI > 0 ? MI : 1;
+  unsigned from[M];   // byte in the row; past its end where the window has no entry: reads 0
+  int to[M];          // entry of the window
+  float2 hv[M];
+  double wv[3];
+  if constexpr (MI > 0) {
+    const int n = Np * (A.LPW + A.nb) * R, t0 = Np * s0;
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const int idx = lane + 64 * i, x = idx / Np;
+      const unsigned at_x = 8u * (unsigned)A.ext[min(t0 + idx, A.N_ext - 1)];
+      from[i] = idx < n && t0 + idx < A.N_ext ? at_x : 0x7ffffff0u;
+      to[i] = idx < n ? (idx - x * Np) * A.WLp + x + x / R : per_wave - 1;
+    }
+  }
+  auto row_of = [&](int fg, int ey) {
+    return A.h + (size_t)fg * A.H_plane + (size_t)A.hrow[ey * A.n_rows + row] * A.HR;
+  };
+  auto load_w = [&](int c, int ey) {
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)(A.ew + ((size_t)(A.pair0 + c) * A.Ney + ey) * A.NeP), 0, A.NeP * 8, 0x27000);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {   // (at most 144)
+      const auto v = __builtin_amdgcn_raw_buffer_load_b64(rs, 8 * (lane + 64 * i), 0, 0);
+      wv[i] = __hiloint2double((int)v[1], (int)v[0]);
+    }
+  };
+  auto load = [&](int c, int fg, int ey) {
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)row_of(fg, ey), 0, A.HR * 8, 0x27000);
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const auto v = __builtin_amdgcn_raw_buffer_load_b64(rs, from[i], 0, 0);
+      hv[i] = make_float2(__uint_as_float(v[0]), __uint_as_float(v[1]));
+    }
+    load_w(c, ey);
+  };
+  int fg = 0;   // frequency of the pair, a pair ahead (MI > 0) of the loads that it is for
+  if (c0 < c1) {
+    fg = A.pair_fg[A.pair0 + c0];
+    if constexpr (MI > 0) load(c0, fg, 0);
+  }
   for (int c = c0; c < c1; ++c) {
-    const int pair = A.pair0 + c;
-    const float2* P = A.P + (size_t)pair * A.N_pts;
-    const float2* h = A.h + (size_t)A.pair_fg[pair] * A.H_plane;
+    const int fg_next = A.pair_fg[A.pair0 + min(c + 1, c1 - 1)];
+    const float2* P = A.P + (size_t)(A.pair0 + c) * A.N_pts;
     float2 pv[R];
 #pragma unroll
     for (int k = 0; k < R; ++k) pv[k] = P[at[k]];
@@ -130,28 +202,42 @@ __global__ __launch_bounds__(1024) void k_energy_single(EnergyArgs A, double* __
     for (int k = 0; k < R; ++k) S[k] = 0.0;
     for (int ey = 0; ey < A.Ney; ++ey) {
       e_fence();
-      e_fill<R, NP>(A, h + (size_t)A.hrow[ey * A.n_rows + row] * A.HR, s0, lane, win,
-                    [](float2 v) { return (double)v.x * v.x + (double)v.y * v.y; });
+      auto square = [](float2 v) { return (double)v.x * v.x + (double)v.y * v.y; };
+      if constexpr (MI > 0) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i) win[to[i]] = square(hv[i]);
+      } else {
+        load_w(c, ey);
+        e_fill<R, 0>(A, row_of(fg, ey), s0, lane, win, square);
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i) win[n_win + min(lane + 64 * i, n_w)] = wv[i];
+      if constexpr (MI > 0) {
+        __builtin_amdgcn_sched_barrier(0);
+        const bool last = ey + 1 == A.Ney;
+        load(last ? min(c + 1, c1 - 1) : c, last ? fg_next : fg, last ? 0 : ey + 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       e_fence();
-      const double* w = A.ew + ((size_t)pair * A.Ney + ey) * A.NeP;
       double a[R], b[R];
 #pragma unroll
       for (int i = 0; i < R; ++i) a[i] = mine[i];
-      for (int t = 0; t < A.nb; ++t) {
+      const double* x = mine + R + 1;
+      for (int t = 0; t < A.nb; t += 2) {
+        const double w = wl[t * R];
 #pragma unroll
-        for (int i = 0; i < R; ++i) b[i] = mine[(t + 1) * (R + 1) + i];
+        for (int i = 0; i < R; ++i) b[i] = x[i];
+        x += R + 1;
+        e_mac<R, 0, R>(S, w, a, b);
 #pragma unroll
-        for (int d = 0; d < R; ++d) {
-          const double wv = w[t * R + d];
-#pragma unroll
-          for (int k = 0; k < R; ++k) S[k] = fma(wv, k + d < R ? a[k + d] : b[k + d - R], S[k]);
-        }
-#pragma unroll
-        for (int i = 0; i < R; ++i) a[i] = b[i];
+        for (int i = 0; i < R; ++i) a[i] = x[i];
+        x += R + 1;
+        e_mac<R, R, 2 * R>(S, w, b, a);
       }
     }
 #pragma unroll
     for (int k = 0; k < R; ++k) acc[k] = fma((double)pv[k].x * pv[k].x + (double)pv[k].y * pv[k].y, S[k], acc[k]);
+    fg = fg_next;
   }
   e_fence();
 #pragma unroll
@@ -162,7 +248,7 @@ __global__ __launch_bounds__(1024) void k_energy_single(EnergyArgs A, double* __
     const int i = Np * (s0 + jl * R + k) + phi;
     if (k % W == wave && on && i < A.Nx) {
       double s = 0.0;
-      for (int v = 0; v < W; ++v) s += e_lds[(size_t)v * Np * A.WLp + k * 64 + lane];
+      for (int v = 0; v < W; ++v) s += e_lds[(size_t)v * per_wave + k * 64 + lane];
       E[(size_t)row * A.Nx + i] = s;
     }
   }
@@ -478,18 +564,23 @@ static int energy_waves(int wgs, size_t lds_per_wave, int most) {
 
 template <int R>
 static void energy_single(const Plan& P, int m, double* E, hipStream_t s) {
-  const EnergyArgs A = energy_args(P, m, R);
+  EnergyArgs A = energy_args(P, m, R);
+  A.nb += A.nb & 1;
+  A.WLp = e_window(A.LPW, A.nb, R);
   const int wgs = A.n_rows * A.nseg;
-  const size_t per_wave = (size_t)A.Np * A.WLp * sizeof(double);
-  const int W = energy_waves(wgs, per_wave, 16);
+  const size_t per_wave = ((size_t)A.Np * A.WLp + A.nb * R + 1) * sizeof(double);
+  int W = wgs < 384 ? 8 : 4;   // 384 rows of 384 points: 183 us with 4, 190 with 8; 256 of 256 points: 42 and 36
+  while (W > 1 && W * per_wave > 150 * 1024) W /= 2;
   const size_t lds = W * per_wave;
-#define BORN_ES(NPv)                                                                                                   \
+  const int mi = (A.Np * (A.LPW + A.nb) * R + 63) / 64;
+#define BORN_ES(MIv)                                                                                                   \
   do {                                                                                                                 \
-    hipFuncSetAttribute((const void*)k_energy_single<R, NPv>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
-    hipLaunchKernelGGL((k_energy_single<R, NPv>), dim3(wgs), dim3(64 * W), lds, s, A, E);                             \
+    hipFuncSetAttribute((const void*)k_energy_single<R, MIv>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
+    hipLaunchKernelGGL((k_energy_single<R, MIv>), dim3(wgs), dim3(64 * W), lds, s, A, E);                             \
   } while (0)
-  if (P.Np == 4) BORN_ES(4);
-  else if (P.Np == 2) BORN_ES(2);
+  if (R < 8 && mi <= 8) BORN_ES((R < 8 ? 8 : 12));   // (8 points per lane have more)
+  else if (mi <= 12) BORN_ES(12);
+  else if (mi <= 16) BORN_ES(16);
   else BORN_ES(0);
 #undef BORN_ES
 }

@@ -40,7 +40,9 @@ def check(op, T, measurements, kind):
 
 
 # elements, points x, z, points per pitch
-SIZES = [(3, 9, 2, 1), (17, 130, 3, 2), (64, 384, 2, 4), (65, 257, 2, 4), (128, 515, 2, 4), (24, 101, 2, 3), (8, 150, 2, 16)]
+SIZES = [(3, 9, 2, 1), (17, 130, 3, 2), (64, 384, 2, 4), (65, 257, 2, 4), (128, 515, 2, 4), (24, 101, 2, 3), (8, 150, 2, 16),
+         # the remaining counts of points and window entries per lane, and a window filled in between
+         (20, 512, 2, 4), (128, 512, 2, 4), (9, 380, 2, 4), (128, 240, 2, 5), (64, 150, 2, 16)]
 
 
 @pytest.mark.parametrize("kind", ["single", "dense", "both"])
