@@ -2460,9 +2460,9 @@ static void energy_rx_tgc(Plan& P, int m, double* E_dev, hipStream_t s) {
     if (!P.d_tgc_spec) {
       dfree(P.d_tgc_tw);   // of a first use that failed
       std::vector<float2> tw;
-      fft_twiddles(P.tgc_TL, tw);
+      fft_twiddles(P.tgc_TL, tw, true);
       P.d_tgc_tw = dupload(tw, P.stream);
-      P.d_tgc_spec = dalloc<float2>((size_t)P.N_mk * 16 * P.tgc_TL);
+      P.d_tgc_spec = dalloc<float2>((size_t)P.N_mk * 32 * P.tgc_TL);
       launch_tgc_spectra(P, P.tgc_TL, P.d_tgc_spec, P.stream);
       HIP_CHECK(hipGetLastError());
       HIP_CHECK(hipStreamSynchronize(P.stream));

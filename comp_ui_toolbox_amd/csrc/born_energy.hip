@@ -374,12 +374,13 @@ __global__ __launch_bounds__(256) void k_energy_multi(EnergyArgs A, double* __re
 // Bound: the vector ALU, about 980 instructions per FPW points and mix in
 // place of the N (2 M + 1) products of k_energy_rx_tgc, which stays for the
 // other plans and longer mixes.  64 elements, 192 x 192 points, 65 frequencies,
-// M = 64: 8.7 ms per measurement there, 0.52 ms here; relative L2 error against
-// FP64 5.4e-8 there (the taps' rounding), 6.8e-8 here (1.1e-7 without the
-// remainders of the transforms' constants, which cost 4 %).
+// M = 64: 8.7 ms per measurement there, 0.54 ms here; relative L2 error against
+// FP64 5.4e-8 there (the taps' rounding), 4.0e-8 here (1.1e-7 without the
+// remainders of the transforms' constants and spectra, 4 % each, and twiddles of
+// magnitude 1).
 
-// spec[mk][8][TL][2]: transform of the taps of mix mk (lags over L / 2 left
-// out), divided by L
+// spec[mk][2][8][TL][2]: transform of the taps of mix mk (lags over L / 2 left
+// out), divided by L, and what its rounding to FP32 leaves
 template <int TL>
 __global__ __launch_bounds__(64) void k_tgc_spectra(const double2* __restrict__ taps, const int* __restrict__ half,
                                                     const int64_t* __restrict__ tap_off, int N_mk,
@@ -406,10 +407,14 @@ __global__ __launch_bounds__(64) void k_tgc_spectra(const double2* __restrict__ 
   }
   fft_wave<double, TL, false>(x, tw, lds, lane);
   if (mk >= N_mk) return;
-  float4* out = spec + (size_t)mk * (L / 2) + j;
+  float4* out = spec + (size_t)mk * L + j;
 #pragma unroll
-  for (int q = 0; q < 8; ++q)
-    out[q * TL] = make_float4((float)x[2 * q].x, (float)x[2 * q].y, (float)x[2 * q + 1].x, (float)x[2 * q + 1].y);
+  for (int q = 0; q < 8; ++q) {
+    const float4 k = make_float4((float)x[2 * q].x, (float)x[2 * q].y, (float)x[2 * q + 1].x, (float)x[2 * q + 1].y);
+    out[q * TL] = k;
+    out[L / 2 + q * TL] = make_float4((float)(x[2 * q].x - k.x), (float)(x[2 * q].y - k.y), (float)(x[2 * q + 1].x - k.z),
+                                      (float)(x[2 * q + 1].y - k.w));
+  }
 }
 
 // NQ: entries of a lane that can hold frequencies (N <= NQ * TL)
@@ -469,16 +474,21 @@ __global__ __launch_bounds__(256, 2) void k_energy_tgc_fft(EnergyArgs A, const f
     }
     // with N = L / 2 + 1, lane j = 0 holds the first (q = 0) and the last (q = 8) row
     const cf first = x[0], last = x[8];
-    float4 kv[8];
-    const float4* ks = spec + (size_t)mk * (L / 2) + j;
+    float4 kv[8], kl[8];
+    const float4* ks = spec + (size_t)mk * L + j;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) kv[q] = ks[q * TL];
+    for (int q = 0; q < 8; ++q) {
+      kv[q] = ks[q * TL];
+      kl[q] = ks[L / 2 + q * TL];
+    }
     fft_wave<float, TL, (NQ <= 8), true>(x, tw, lds, lane);
 #pragma unroll
     for (int q = 0; q < 8; ++q) {   // conjugated, for the exponent's sign
       const cf u = x[2 * q], v = x[2 * q + 1];
-      x[2 * q] = {fmaf(kv[q].x, u.x, -(kv[q].y * u.y)), -fmaf(kv[q].x, u.y, kv[q].y * u.x)};
-      x[2 * q + 1] = {fmaf(kv[q].z, v.x, -(kv[q].w * v.y)), -fmaf(kv[q].z, v.y, kv[q].w * v.x)};
+      x[2 * q] = {fmaf(kv[q].x, u.x, fmaf(kl[q].x, u.x, -fmaf(kv[q].y, u.y, kl[q].y * u.y))),
+                  -fmaf(kv[q].x, u.y, fmaf(kl[q].x, u.y, fmaf(kv[q].y, u.x, kl[q].y * u.x)))};
+      x[2 * q + 1] = {fmaf(kv[q].z, v.x, fmaf(kl[q].z, v.x, -fmaf(kv[q].w, v.y, kl[q].w * v.y))),
+                      -fmaf(kv[q].z, v.y, fmaf(kl[q].z, v.y, fmaf(kv[q].w, v.x, kl[q].w * v.x)))};
     }
     fft_wave<float, TL, false, true>(x, tw, lds, lane);
     if (NQ > 8 && edge && half[mk] == N - 1 && j == 0) {

@@ -462,7 +462,7 @@ void launch_fft3_weights(const Plan& P, int N_rhs, hipStream_t s);
 void launch_fft3_adj(const Plan& P, int N_rhs, float2* g, hipStream_t s);
 // fast lateral correlation (born_fft.hip)
 FftShapeChoice fft_shape(int Nx, int Np, int N_e);
-void fft_twiddles(int TL, std::vector<float2>& tw);
+void fft_twiddles(int TL, std::vector<float2>& tw, bool unit = false);
 void launch_fft_range(const Plan& P, int* bad, hipStream_t s);
 void launch_fft_table(const Plan& P, hipStream_t s);
 void launch_fft_gamma(const Plan& P, const float2* gamma, int N_rhs, bool mask, hipStream_t s);
