@@ -347,6 +347,8 @@ struct Plan {
   size_t io_bytes = 0;
   void* d_io_in = nullptr;        // host-path staging
   void* d_io_out = nullptr;
+  void* h_stage = nullptr;         // pinned staging of the host calls
+  size_t h_stage_bytes = 0;
   hipStream_t stream = nullptr;   // host-path stream
 
   // Allocation-free apply (born_apply_dev_noalloc): a one-rhs chunk layout

@@ -372,18 +372,23 @@ class OperatorBorn:
                                                     for k in kernels]))
         check(L.born_tgc_set(self._plan, half, dptr(taps.view(np.float64))))
 
-    def _tgc_host(self, u, mode: int) -> np.ndarray:
-        uu = np.asarray(u)
-        squeeze = uu.ndim == 1
-        u2 = uu[:, None] if squeeze else uu
-        if u2.shape[0] != self.N_observations:
+    def _host(self, call, x, rows_in: int, rows_out: int) -> np.ndarray:
+        """One host FP64 call, call(in, N_rhs, out), on x (rows_in,) or
+        (rows_in, N_rhs)."""
+        xx = np.asarray(x)
+        squeeze = xx.ndim == 1
+        x2 = xx[:, None] if squeeze else xx
+        if x2.shape[0] != rows_in:
             raise BornError(7, "combined_quick_gpu:NoValidDoubleMatrix",
-                            f"input must be a double matrix with {self.N_observations} rows!")
-        uin = _c128_colmajor(u2)
-        out = np.empty((u2.shape[1], self.N_observations), dtype=np.complex128)
-        check(_lib.lib().born_tgc_apply(self._plan, int(mode), dptr(uin), u2.shape[1], dptr(out.view(np.float64))))
-        res = out.T
-        return res[:, 0].copy() if squeeze else np.ascontiguousarray(res)
+                            f"input must be a double matrix with {rows_in} rows!")
+        xin = _c128_colmajor(x2)
+        out = np.empty((x2.shape[1], rows_out), dtype=np.complex128)
+        check(call(dptr(xin), x2.shape[1], dptr(out.view(np.float64))))
+        return out[0] if squeeze else np.ascontiguousarray(out.T)
+
+    def _tgc_host(self, u, mode: int) -> np.ndarray:
+        return self._host(lambda i, n, o: _lib.lib().born_tgc_apply(self._plan, int(mode), i, n, o),
+                          u, self.N_observations, self.N_observations)
 
     def tgc_forward(self, u) -> np.ndarray:
         """TGC of u (N_obs,) or (N_obs, N_rhs), FP64 (forward_transform)."""
@@ -411,33 +416,13 @@ class OperatorBorn:
     def forward(self, gamma) -> np.ndarray:
         """u_M = A gamma with MEX semantics (occupancy rule, zero output when
         nothing is occupied).  gamma: (N_pts,) or (N_pts, N_rhs)."""
-        g = np.asarray(gamma)
-        squeeze = g.ndim == 1
-        g2 = g[:, None] if squeeze else g
-        if g2.shape[0] != self.N_points:
-            raise BornError(7, "combined_quick_gpu:NoValidDoubleMatrix",
-                            f"input must be a double matrix with {self.N_points} rows!")
-        nrhs = g2.shape[1]
-        gin = _c128_colmajor(g2)
-        out = np.empty((nrhs, self.N_observations), dtype=np.complex128)
-        check(_lib.lib().born_forward(self._plan, dptr(gin), nrhs, dptr(out.view(np.float64))))
-        res = out.T
-        return res[:, 0].copy() if squeeze else np.ascontiguousarray(res)
+        return self._host(lambda i, n, o: _lib.lib().born_forward(self._plan, i, n, o),
+                          gamma, self.N_points, self.N_observations)
 
     def adjoint(self, u) -> np.ndarray:
         """gamma_hat = A^H u_M over all N_pts points."""
-        uu = np.asarray(u)
-        squeeze = uu.ndim == 1
-        u2 = uu[:, None] if squeeze else uu
-        if u2.shape[0] != self.N_observations:
-            raise BornError(7, "combined_quick_gpu:NoValidDoubleMatrix",
-                            f"input must be a double matrix with {self.N_observations} rows!")
-        nrhs = u2.shape[1]
-        uin = _c128_colmajor(u2)
-        out = np.empty((nrhs, self.N_points), dtype=np.complex128)
-        check(_lib.lib().born_adjoint(self._plan, dptr(uin), nrhs, dptr(out.view(np.float64))))
-        res = out.T
-        return res[:, 0].copy() if squeeze else np.ascontiguousarray(res)
+        return self._host(lambda i, n, o: _lib.lib().born_adjoint(self._plan, i, n, o),
+                          u, self.N_observations, self.N_points)
 
     def __matmul__(self, gamma):
         return self.forward(gamma)
@@ -492,6 +477,13 @@ class OperatorBorn:
                             f"expected a contiguous complex64 device tensor with last dimension {rows}")
 
     # ---------------------------------------------------------- solver contract
+    def _apply_tgc(self, x, mode: int) -> np.ndarray:
+        """tgc_forward(forward(x)) (mode 1) or adjoint(tgc_adjoint(x)) (mode 2)
+        in one call."""
+        sizes = (self.N_points, self.N_observations)
+        return self._host(lambda i, n, o: _lib.lib().born_apply_tgc(self._plan, mode, i, n, o),
+                          x, *(sizes if mode == 1 else sizes[::-1]))
+
     def op_A(self, x, mode: int, tgc: bool = False, dictionary=None):
         """operator.combined_scalar: mode 0 size, 1 forward, 2 adjoint
         (operator.m:1019-1072).  tgc=True applies the kernels of set_tgc
@@ -505,10 +497,9 @@ class OperatorBorn:
             return list(self.size)
         if mode == 1:
             g = dictionary.adjoint_transform(x) if dictionary is not None else x
-            u = self.forward(g)
-            return self.tgc_forward(u) if tgc else u
+            return self._apply_tgc(g, 1) if tgc else self.forward(g)
         if mode == 2:
-            g = self.adjoint(self.tgc_adjoint(x) if tgc else x)
+            g = self._apply_tgc(x, 2) if tgc else self.adjoint(x)
             return dictionary.forward_transform(g) if dictionary is not None else g
         raise BornError(6, "combined_scalar:InvalidMode", "mode must be 0, 1 or 2")
 

@@ -255,9 +255,13 @@ int born_columns_dev(born_plan_t plan, const double* points, int32_t n, void* ou
  * interleaved complex (in == out allowed), computed in FP64, synchronous.
  * born_tgc_apply_dev: complex64 device N_rhs x N_obs, in and out must not
  * overlap, enqueued on `stream`.  mode 1 = forward, any other value adjoint.
+ * born_apply_tgc: op_A with its TGC in one call, born_forward and
+ * born_tgc_apply (mode 1) or born_tgc_apply and born_adjoint (other values),
+ * with the values of the two calls; in and out as theirs.
  * No counterpart in the MEX (a MATLAB-side linear transform). */
 int born_tgc_set(born_plan_t plan, const int32_t* half_lengths, const double* kernels_c128);
 int born_tgc_apply(born_plan_t plan, int32_t mode, const double* in, int32_t N_rhs, double* out);
+int born_apply_tgc(born_plan_t plan, int32_t mode, const double* in, int32_t N_rhs, double* out);
 int born_tgc_apply_dev(born_plan_t plan, int32_t mode, const void* in_c64, void* out_c64, int32_t N_rhs,
                        void* stream);
 

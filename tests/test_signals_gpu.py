@@ -7,8 +7,9 @@ entry); the phase factors of the signals add 3 * 2^-24 per product."""
 import numpy as np
 import pytest
 
-from comp_ui_toolbox_amd import OperatorBorn
+from comp_ui_toolbox_amd import BornError, OperatorBorn
 from comp_ui_toolbox_amd import configs as C
+from tests.test_oracle import mixed_tiny_tables
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +70,30 @@ def test_time_signals_regular(torch_cuda, nf, q0, dq, more, n_rhs):
     ref = np.fft.irfft(spec, n=n_t) * n_t
     size = 2.0 * np.abs(x).sum(axis=2, keepdims=True)
     assert np.all(np.abs(rf.cpu().numpy() - ref) <= (2 * nf + 12) * 2.0 ** -24 * size)
+
+
+@pytest.mark.parametrize("sparse", [0, 5])
+@pytest.mark.parametrize("n_rhs", [0, 1, 3])
+def test_operator_with_time_gain_in_one_call(torch_cuda, n_rhs, sparse):
+    """op_A with time gain gives the values of the two calls bit for bit:
+    dense and few occupied points, one vector and matrices, nothing occupied,
+    and calls that grow and reuse the staging."""
+    _, T = mixed_tiny_tables(distinct=True)
+    op = OperatorBorn.from_tables(T)
+    with pytest.raises(BornError):
+        op.op_A(np.ones(op.N_points), 1, tgc=True)
+    rng = np.random.Generator(np.random.PCG64(3))
+    op.set_tgc([rng.standard_normal(5) + 1j * rng.standard_normal(5) for _ in op.meta["mix_n_obs"]])
+    op.set_sparse_forward(sparse)
+    shape = lambda n: (n,) if n_rhs == 0 else (n, n_rhs)
+    x = rng.standard_normal(shape(op.N_points)) + 1j * rng.standard_normal(shape(op.N_points))
+    few = np.zeros_like(x)
+    few[2:4] = x[2:4]
+    y = rng.standard_normal(shape(op.N_observations)) + 1j * rng.standard_normal(shape(op.N_observations))
+    for g in (few, x, np.zeros_like(x), few):
+        u = op.op_A(g, 1, tgc=True)
+        assert u.shape == shape(op.N_observations)
+        assert np.array_equal(u, op.tgc_forward(op.forward(g)))
+        assert np.any(u) == np.any(g)
+    back = op.op_A(y, 2, tgc=True)
+    assert np.array_equal(back, op.adjoint(op.tgc_adjoint(y)))
