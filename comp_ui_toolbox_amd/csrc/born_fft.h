@@ -10,8 +10,10 @@
 
 namespace born {
 
+// Aligned as a whole: for the LDS that a launch sizes the compiler has no other
+// word that an entry may be read and written in one access.
 template <typename R>
-struct Cx {
+struct alignas(2 * sizeof(R)) Cx {
   R x, y;
 };
 typedef Cx<float> cf;

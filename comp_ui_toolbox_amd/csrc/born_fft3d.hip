@@ -18,10 +18,14 @@
 //
 // Bound: the vector ALU, per plane of 64 x 64 points at 2 points per pitch
 // 384 transforms of 64 points (about 7400 wave instructions) in place of
-// 32 x 32 x 64 x 64 complex multiply-adds.  32 x 32 elements, 64^3 points, 33
-// frequencies, 3 waves, 4 right-hand sides: forward 0.73 ms, adjoint 0.66 ms
-// against 5.6 and 7.0 ms of the split BF16 products (128 x 128 x 192 points,
-// 65 frequencies, 5 waves: 43 and 30 ms against 138 and 158 ms).
+// 32 x 32 x 64 x 64 complex multiply-adds, at 60 % of its rate with two waves
+// per SIMD (registers and LDS) and two barriers per tile.  32 x 32 elements,
+// 64^3 points, 33 frequencies, 3 waves, 4 right-hand sides: forward 0.67 ms,
+// adjoint 0.58 ms against 5.6 and 7.0 ms of the split BF16 products (128 x 128 x
+// 192 points, 65 frequencies, 5 waves, one: 8.4 and 8.1 ms).  What the loads
+// ahead, the twiddles in LDS and 64-bit LDS accesses gave: 0.72 and 0.62 ms
+// before, 242 -> 180 and 231 -> 180 us at 20 x 8 elements, 33 x 70 x 60 points,
+// 20 frequencies, 3 waves, and 12.9 -> 8.4 ms for the forward of the large one.
 #include "born_fft.h"
 #include "born_internal.h"
 
@@ -114,12 +118,19 @@ __global__ __launch_bounds__(64) void k_fft3_table_y(const double2* __restrict__
 __device__ __forceinline__ int fft3_block(int per) { return (blockIdx.x % XCDS) * per + blockIdx.x / XCDS; }
 
 // ------------------------------------------------------------------ forward
-// One workgroup per (depth block, column, right-hand side).
+// One workgroup per (depth block, column, right-hand side).  p_inc and the
+// input of the next tile's rows are loaded during the last column transforms of
+// this one (behind the spectra of these, which return first).
 template <int TLX, int TLY, bool HALF>
 __global__ __launch_bounds__((64 * Fft3Shape<TLX, TLY>::W), 2) void k_fft3_fwd(Fft3Args A, int n_wg, int per) {
   using S = Fft3Shape<TLX, TLY>;
   constexpr int NQ = HALF ? 8 : 16;
-  extern __shared__ cf f3_lds[];
+  constexpr bool AHEAD = HALF && S::NBP == 1;   // (the others have no registers left for it)
+  extern __shared__ cf f3_lds[];   // exchange buffers, plane, twiddles
+  cf* twlx = f3_lds + A.tw_at;
+  cf* twly = twlx + 16 * TLX;
+  load_twiddles_lds<TLX>(A.twx, twlx);
+  load_twiddles_lds<TLY>(A.twy, twly);
   const int wg = fft3_block(per);
   if (wg >= n_wg) return;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -132,42 +143,57 @@ __global__ __launch_bounds__((64 * Fft3Shape<TLX, TLY>::W), 2) void k_fft3_fwd(F
   const int z0 = zb * A.ZR, z1 = min(A.Nz, z0 + A.ZR);
   const float2* P = A.P + (size_t)pf.x * A.N_pts;
   const float2* gm = A.gm + (size_t)r * A.N_pts;
-  cf twx[16], twy[16], G[S::NBP][16];
-  load_twiddles<TLX>(A.twx, jx, twx);
-  if constexpr (TLX != TLY) load_twiddles<TLY>(A.twy, jy, twy);
+  cf G[S::NBP][16];
 #pragma unroll
   for (int b = 0; b < S::NBP; ++b)
 #pragma unroll
     for (int q = 0; q < 16; ++q) G[b][q] = {0.f, 0.f};
-  const int n_tx = A.Npx / A.px, n_slot = A.px * A.Sy;
+  const int n_tx = A.Npx / A.px, n_slot = A.px * A.Sy, n_tile = A.Npy * n_tx;
+  // the rows of slots s0 .. of a tile: whether the lane has one, its first x,
+  // and its entries' values (those past the grid read entry 0 of the row)
+  struct Row {
+    bool ok;
+    int phx;
+  };
+  auto row_of = [&](int tile, int s0) {
+    const int phy = tile / n_tx, slot = s0 + gx, sy = slot / A.px;
+    return Row{slot < n_slot && A.Npy * sy + phy < A.Ny, (tile - phy * n_tx) * A.px + slot - sy * A.px};
+  };
+  float2 pv[NQ], gv[NQ];
+  auto load = [&](int z, int tile, int s0) {
+    const Row R = row_of(tile, s0);
+    const int phy = tile / n_tx, sy = (s0 + gx) / A.px;
+    const int base = (z * A.Ny + (R.ok ? A.Npy * sy + phy : 0)) * A.Nx;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const int ix = A.Npx * (jx + TLX * q) + R.phx;
+      const int at = base + (ix < A.Nx ? ix : 0);
+      pv[q] = P[at];
+      gv[q] = gm[at];
+    }
+  };
+  const int first = wave * S::FPWX;
+  if (AHEAD && z0 < z1 && first < n_slot) load(z0, 0, first);
   for (int z = z0; z < z1; ++z) {
     const float4* Hz = reinterpret_cast<const float4*>(A.H) +
                        ((size_t)pf.y * A.Nz + z) * A.Npy * A.Npx * (S::LX * S::LY / 2) + lane;
-    for (int tile = 0; tile < A.Npy * n_tx; ++tile) {
+    for (int tile = 0; tile < n_tile; ++tile) {
       const int phy = tile / n_tx, phx0 = (tile - phy * n_tx) * A.px;
-      const int Syp = (A.Ny - phy + A.Npy - 1) / A.Npy;   // rows of this phase
-      for (int s0 = wave * S::FPWX; s0 < n_slot; s0 += S::W * S::FPWX) {
-        const int slot = s0 + gx;
-        const int sy = slot / A.px, phx = phx0 + slot - sy * A.px;
-        const bool row_ok = slot < n_slot && sy < Syp;
-        const int base = (z * A.Ny + (row_ok ? A.Npy * sy + phy : 0)) * A.Nx;
+      for (int s0 = first; s0 < n_slot; s0 += S::W * S::FPWX) {
+        if (!AHEAD || s0 != first) load(z, tile, s0);
+        const Row R = row_of(tile, s0);
         cf x[16];
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
-          const int ix = A.Npx * (jx + TLX * q) + phx;
-          const bool ok = row_ok && ix < A.Nx;
-          const int at = base + (ok ? ix : 0);
-          const float2 pv = P[at];
-          float2 gv = gm[at];
-          if (!ok) gv = make_float2(0.f, 0.f);
-          x[q] = {fmaf(pv.x, gv.x, -(pv.y * gv.y)), fmaf(pv.x, gv.y, pv.y * gv.x)};
+          const bool ok = R.ok && A.Npx * (jx + TLX * q) + R.phx < A.Nx;
+          const float2 g = ok ? gv[q] : make_float2(0.f, 0.f);
+          x[q] = {fmaf(pv[q].x, g.x, -(pv[q].y * g.y)), fmaf(pv[q].x, g.y, pv[q].y * g.x)};
         }
+        fft_wave_l<TLX, NQ>(x, twlx, lds, lane);
+        if (s0 + gx < n_slot) {
+          cf* row = plane + (s0 + gx) * S::ROW + jx;
 #pragma unroll
-        for (int q = NQ; q < 16; ++q) x[q] = {0.f, 0.f};
-        fft_wave<float, TLX, HALF>(x, twx, lds, lane);
-        if (slot < n_slot) {
-#pragma unroll
-          for (int q = 0; q < 16; ++q) plane[slot * S::ROW + jx + TLX * q] = x[q];
+          for (int q = 0; q < 16; ++q) row[TLX * q] = x[q];
         }
       }
       __syncthreads();
@@ -178,16 +204,21 @@ __global__ __launch_bounds__((64 * Fft3Shape<TLX, TLY>::W), 2) void k_fft3_fwd(F
           float4 hv[8];
 #pragma unroll
           for (int q = 0; q < 8; ++q) hv[q] = Hp[((b * S::W + wave) * 8 + q) * 64];
+          __builtin_amdgcn_sched_barrier(0);
+          if (AHEAD && ph == A.px - 1 && first < n_slot) {
+            const bool last = tile + 1 == n_tile;
+            load(last ? min(z + 1, z1 - 1) : z, last ? 0 : tile + 1, first);   // (the last tile loads one again)
+          }
+          __builtin_amdgcn_sched_barrier(0);
           const int kx = (b * S::W + wave) * S::FPWY + gy;
           cf x[16];
 #pragma unroll
-          for (int q = 0; q < 16; ++q) {
+          for (int q = 0; q < NQ; ++q) {
             x[q] = {0.f, 0.f};
             const int sy = jy + TLY * q;
-            if (q < NQ && sy < A.Sy) x[q] = plane[(sy * A.px + ph) * S::ROW + kx];
+            if (sy < A.Sy) x[q] = plane[(sy * A.px + ph) * S::ROW + kx];
           }
-          if constexpr (TLX == TLY) fft_wave<float, TLY, HALF>(x, twx, lds, lane);
-          else fft_wave<float, TLY, HALF>(x, twy, lds, lane);
+          fft_wave_l<TLY, NQ>(x, twly, lds, lane);
 #pragma unroll
           for (int q = 0; q < 8; ++q) {
             cmac(G[b][2 * q], cf{hv[q].x, hv[q].y}, x[2 * q]);
@@ -201,8 +232,7 @@ __global__ __launch_bounds__((64 * Fft3Shape<TLX, TLY>::W), 2) void k_fft3_fwd(F
   // transform back: rows t_y < N_ey, then entries t_x < N_ex
 #pragma unroll
   for (int b = 0; b < S::NBP; ++b) {
-    if constexpr (TLX == TLY) fft_wave<float, TLY, false>(G[b], twx, lds, lane);
-    else fft_wave<float, TLY, false>(G[b], twy, lds, lane);
+    fft_wave_l<TLY, 16>(G[b], twly, lds, lane);
     const int kx = (b * S::W + wave) * S::FPWY + gy;
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
@@ -221,7 +251,7 @@ __global__ __launch_bounds__((64 * Fft3Shape<TLX, TLY>::W), 2) void k_fft3_fwd(F
       x[q] = {0.f, 0.f};
       if (ty < A.Ney) x[q] = plane[ty * S::ROW + jx + TLX * q];
     }
-    fft_wave<float, TLX, false>(x, twx, lds, lane);
+    fft_wave_l<TLX, 16>(x, twlx, lds, lane);
     if (ty < A.Ney) {
 #pragma unroll
       for (int q = 0; q < 16; ++q) {
@@ -293,7 +323,12 @@ __global__ __launch_bounds__((64 * Fft3Shape<TLX, TLY>::W), 2) void k_fft3_adj(F
                                                                             int n_wg, int per) {
   using S = Fft3Shape<TLX, TLY>;
   constexpr int NQ = HALF ? 8 : 16;
-  extern __shared__ cf f3_lds[];
+  constexpr bool AHEAD = HALF && S::NBP == 1;   // (the others have no registers left for it)
+  extern __shared__ cf f3_lds[];   // exchange buffers, plane, twiddles
+  cf* twlx = f3_lds + A.tw_at;
+  cf* twly = twlx + 16 * TLX;
+  load_twiddles_lds<TLX>(A.twx, twlx);
+  load_twiddles_lds<TLY>(A.twy, twly);
   int t = fft3_block(per);
   if (t >= n_wg) return;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -309,33 +344,59 @@ __global__ __launch_bounds__((64 * Fft3Shape<TLX, TLY>::W), 2) void k_fft3_adj(F
   const int c0 = (int)((long)A.n_cols * fgr / A.FG), c1 = (int)((long)A.n_cols * (fgr + 1) / A.FG);
   const int phy = tile / n_tx, phx0 = (tile - phy * n_tx) * A.px;
   const int Syp = (A.Ny - phy + A.Npy - 1) / A.Npy;
-  cf twx[16], twy[16], acc[FFT3_PASSES][NQ];
-  load_twiddles<TLX>(A.twx, jx, twx);
-  if constexpr (TLX != TLY) load_twiddles<TLY>(A.twy, jy, twy);
+  cf acc[FFT3_PASSES][NQ];
 #pragma unroll
   for (int a = 0; a < FFT3_PASSES; ++a)
 #pragma unroll
     for (int q = 0; q < NQ; ++q) acc[a][q] = {0.f, 0.f};
-  for (int c = c0; c < c1; ++c) {
-    const int2 pf = A.col[c];
-    const float4* Hz = reinterpret_cast<const float4*>(A.H) +
-                       (((size_t)pf.y * A.Nz + z) * A.Npy + phy) * A.Npx * (S::LX * S::LY / 2) + lane;
+  // Spectra of H and of the weights, [b][8]: with one pass per phase (AHEAD) those
+  // of the next phase or column are loaded during this one's transforms.
+  float4 hv[8], wv[8];
+  auto load_h = [&](int2 pf, int ph, int b) {
+    const float4* Hp = reinterpret_cast<const float4*>(A.H) + lane +
+                       ((((size_t)pf.y * A.Nz + z) * A.Npy + phy) * A.Npx + phx0 + ph) * (S::LX * S::LY / 2);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) hv[q] = Hp[((b * S::W + wave) * 8 + q) * 64];
+  };
+  auto load_w = [&](int2 pf, int b) {
     const float4* Wp = reinterpret_cast<const float4*>(A.wt) + ((size_t)pf.x * A.N_rhs + r) * (S::LX * S::LY / 2) + lane;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) wv[q] = Wp[((b * S::W + wave) * 8 + q) * 64];
+  };
+  int2 pf_next = A.col[min(c0, A.n_cols - 1)];
+  if (AHEAD && c0 < c1) {
+    load_h(pf_next, 0, 0);
+    load_w(pf_next, 0);
+  }
+  for (int c = c0; c < c1; ++c) {
+    const int2 pf = pf_next;
+    pf_next = A.col[min(c + 1, c1 - 1)];
     for (int ph = 0; ph < A.px; ++ph) {
-      const float4* Hp = Hz + (size_t)(phx0 + ph) * (S::LX * S::LY / 2);
 #pragma unroll
       for (int b = 0; b < S::NBP; ++b) {
         const int kx = (b * S::W + wave) * S::FPWY + gy;
+        if (!AHEAD) {
+          load_h(pf, ph, b);
+          load_w(pf, b);
+        }
         cf x[16];
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-          const int at = ((b * S::W + wave) * 8 + q) * 64;
-          const float4 h = Hp[at], w = Wp[at];
+          const float4 h = hv[q], w = wv[q];
           x[2 * q] = {fmaf(h.x, w.x, -(h.y * w.y)), fmaf(h.x, w.y, h.y * w.x)};
           x[2 * q + 1] = {fmaf(h.z, w.z, -(h.w * w.w)), fmaf(h.z, w.w, h.w * w.z)};
         }
-        if constexpr (TLX == TLY) fft_wave<float, TLY, false>(x, twx, lds, lane);
-        else fft_wave<float, TLY, false>(x, twy, lds, lane);
+        if (AHEAD) {
+          __builtin_amdgcn_sched_barrier(0);
+          if (ph + 1 < A.px) {
+            load_h(pf, ph + 1, 0);
+          } else {   // (the last column's again)
+            load_h(pf_next, 0, 0);
+            load_w(pf_next, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        fft_wave_l<TLY, 16>(x, twly, lds, lane);
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
           const int sy = jy + TLY * q;
@@ -362,7 +423,7 @@ __global__ __launch_bounds__((64 * Fft3Shape<TLX, TLY>::W), 2) void k_fft3_adj(F
         const cf* src = plane + (slot < n_slot ? slot : 0) * S::ROW + jx;
 #pragma unroll
         for (int q = 0; q < 16; ++q) x[q] = src[TLX * q];
-        fft_wave<float, TLX, false>(x, twx, lds, lane);
+        fft_wave_l<TLX, 16>(x, twlx, lds, lane);
 #pragma unroll
         for (int q = 0; q < NQ; ++q) cmac(acc[a][q], cf{pv[q].x, pv[q].y}, x[q]);
       }
@@ -395,7 +456,7 @@ __global__ __launch_bounds__((64 * Fft3Shape<TLX, TLY>::W), 2) void k_fft3_adj(F
   } while (0)
 
 // Lengths, phases per tile and LDS of a plan; TLX = 0 where the planes do not
-// fit (a workgroup's plane and exchange buffers within 150 KB, FFT3_PASSES
+// fit (a workgroup's plane and exchange buffers within 152 KB, FFT3_PASSES
 // rounds of row transforms): those plans keep the direct kernels.
 Fft3Choice fft3_shape(int Nx, int Ny, int Npx, int Npy, int Nex, int Ney) {
   Fft3Choice c;
@@ -409,11 +470,12 @@ Fft3Choice fft3_shape(int Nx, int Ny, int Npx, int Npy, int Nex, int Ney) {
   c.half = c.Sx <= 8 * TLX && c.Sy <= 8 * TLY;
   for (int px = Npx; px >= 1; --px) {
     if (Npx % px != 0) continue;
-    const size_t lds = ((size_t)W * ex + (size_t)std::max(px * c.Sy, Ney) * (16 * TLX + 1)) * sizeof(float2);
+    c.tw_at = W * ex + std::max(px * c.Sy, Ney) * (16 * TLX + 1);
+    const size_t lds = ((size_t)c.tw_at + 16 * (TLX + TLY)) * sizeof(float2);
     // several phases at once only while they fill no more than one round of
     // row transforms (and two workgroups share a compute unit)
     if (px > 1 && (px * c.Sy > slots || lds > 80 * 1024)) continue;
-    if (px * c.Sy > FFT3_PASSES * slots || lds > 150 * 1024) continue;
+    if (px * c.Sy > FFT3_PASSES * slots || lds > 152 * 1024) continue;
     c.TLX = TLX;
     c.TLY = TLY;
     c.px = px;
@@ -448,6 +510,7 @@ static Fft3Args fft3_args(const Plan& P, int N_rhs) {
   A.N_rhs = N_rhs;
   A.Sy = F.s3.Sy;
   A.px = F.s3.px;
+  A.tw_at = F.s3.tw_at;
   A.ZR = F.ZR;
   A.FG = F.FG;
   return A;

@@ -127,7 +127,7 @@ struct FftShapeChoice {
 // phases per tile, LDS bytes of a workgroup.
 constexpr int FFT3_PASSES = 2;   // rounds of row transforms per plane, at most
 struct Fft3Choice {
-  int TLX = 0, TLY = 0, Sx = 0, Sy = 0, px = 1;
+  int TLX = 0, TLY = 0, Sx = 0, Sy = 0, px = 1, tw_at = 0;
   bool half = false;               // at most half of every sequence holds points
   size_t lds = 0;
 };
@@ -142,7 +142,7 @@ struct Fft3Args {
   const float2* twx;
   const float2* twy;
   int Nx, Ny, Nz, Npx, Npy, Nex, Ney, N_e, N_pts, n_cols, N_rhs;
-  int Sy, px, ZR, FG;
+  int Sy, px, ZR, FG, tw_at;       // tw_at: the twiddles' place in LDS
 };
 
 // One operator instance of a fast-correlation launch.
