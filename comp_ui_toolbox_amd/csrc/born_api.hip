@@ -325,6 +325,7 @@ static void upload_index_structures(Plan& P, hipStream_t s) {
   }
   P.d_pe_off = dupload(peoff, s);
   P.d_pe_ent = dupload(ent, s);
+  P.n_pe_ent = peoff.back();
 }
 
 // The lateral Toeplitz structure of setup_grid_symmetric.shift_lateral

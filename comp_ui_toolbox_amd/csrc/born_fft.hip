@@ -35,6 +35,7 @@
 #include "born_internal.h"
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 
 namespace born {
@@ -316,10 +317,14 @@ __global__ __launch_bounds__(256) void k_fft_reduce(const float2* __restrict__ v
 }
 
 // ------------------------------------------------------------------ adjoint
+struct alignas(8) Ent4 {
+  int2 e[4];
+};
+
 // Un-mixing (as k_adj_unmix) and the spectra of the weights: a wave takes FPW
 // (pair, right-hand side) rows, entry t = N_e - 1 - e holds conj(W[e]) / L.
 // wt[row][8][TL lanes][2].
-template <int TL>
+template <int TL, bool LONG>
 __global__ __launch_bounds__(256) void k_fft_weights(const float2* __restrict__ u, const int64_t* __restrict__ pe_off,
                                                      const int2* __restrict__ pe_ent, const double2* __restrict__ pref,
                                                      const float2* __restrict__ twid, int N_pairs, int N_e,
@@ -332,52 +337,83 @@ __global__ __launch_bounds__(256) void k_fft_weights(const float2* __restrict__ 
   const bool ok = row < N_pairs * N_rhs;
   const int pair = ok ? row / N_rhs : 0, r = ok ? row - pair * N_rhs : 0;
   const float2* ur = u + (int64_t)r * N_obs;
-  // 8 elements at a time: the offsets of their lists, then list entry by list
-  // entry the loads of all 8 together (past the end of a list its first entry
-  // again); element by element the dependent loads took 10.6 us for one wave of
-  // 64 elements and 33 frequencies, now 8.2
+  // QB elements at a time: the offsets of their lists, then the loads of all of
+  // them together (past the end of a list its first entry again; element by
+  // element they took 10.6 us for one wave of 64 elements and 33 frequencies, now
+  // 8.2).  LONG: 4 entries of each list at a time while all have 4 left: the lanes
+  // read as many lists, a line of the L2 each, and one entry of 8 bytes per line
+  // is what bounds it (32 waves x 16 mixes of 128 elements, 257 frequencies: 426
+  // us by single entries, 215 by four; with lists of one entry 8 elements at a
+  // time are 1 us faster).
+  constexpr int QB = LONG ? 4 : 8;
   cf tw[16], x[16];
   load_twiddles<TL>(twid, j, tw);
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    int64_t first[8];
-    int n[8], most = 0;
-    double sx[8], sy[8];
+  for (int h = 0; h < 16 / QB; ++h) {
+    int64_t first[QB];
+    int n[QB], most = 0, least = INT_MAX;
+    double sx[QB], sy[QB];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int t = j + TL * (8 * h + q);
+    for (int q = 0; q < QB; ++q) {
+      const int t = j + TL * (QB * h + q);
       const bool have = ok && t < N_e;
       const size_t pe = (size_t)pair * N_e + (have ? N_e - 1 - t : 0);
       first[q] = pe_off[pe];
-      n[q] = have ? (int)(pe_off[pe + 1] - first[q]) : 0;
+      n[q] = have ? (int)(pe_off[pe + 1] - first[q]) : -1;
       sx[q] = sy[q] = 0.0;
     }
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      if (n[q] == 0) first[q] = 0;
+    for (int q = 0; q < QB; ++q) {
+      if (n[q] <= 0) first[q] = 0;
       most = max(most, n[q]);
+      if (n[q] >= 0) least = min(least, n[q]);
     }
-    for (int i = 0; i < most; ++i) {
-      int2 oe[8];
-      double2 c[8];
-      float2 v[8];
+    int i = 0;
+    if constexpr (LONG)
+      for (; most > 0 && i + 4 <= least; i += 4) {
+        Ent4 oe[QB];
+        double2 c[QB][4];
+        float2 v[QB][4];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) oe[q] = pe_ent[first[q] + (i < n[q] ? i : 0)];
+        for (int q = 0; q < QB; ++q) oe[q] = *reinterpret_cast<const Ent4*>(pe_ent + first[q] + (n[q] > 0 ? i : 0));
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
+        for (int q = 0; q < QB; ++q)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            c[q][k] = pref[oe[q].e[k].y];
+            v[q][k] = ur[oe[q].e[k].x];
+          }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < QB; ++q)
+          if (n[q] > 0)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              sx[q] += c[q][k].x * v[q][k].x + c[q][k].y * v[q][k].y;
+              sy[q] += c[q][k].x * v[q][k].y - c[q][k].y * v[q][k].x;
+            }
+      }
+    for (; i < most; ++i) {
+      int2 oe[QB];
+      double2 c[QB];
+      float2 v[QB];
+#pragma unroll
+      for (int q = 0; q < QB; ++q) oe[q] = pe_ent[first[q] + (i < n[q] ? i : 0)];
+#pragma unroll
+      for (int q = 0; q < QB; ++q) {
         c[q] = pref[oe[q].y];
         v[q] = ur[oe[q].x];
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int q = 0; q < 8; ++q)
+      for (int q = 0; q < QB; ++q)
         if (i < n[q]) {
           sx[q] += c[q].x * v[q].x + c[q].y * v[q].y;
           sy[q] += c[q].x * v[q].y - c[q].y * v[q].x;
         }
     }
 #pragma unroll
-    for (int q = 0; q < 8; ++q) x[8 * h + q] = {(float)sx[q] * (1.f / L), -(float)sy[q] * (1.f / L)};
+    for (int q = 0; q < QB; ++q) x[QB * h + q] = {(float)sx[q] * (1.f / L), -(float)sy[q] * (1.f / L)};
   }
   fft_wave<float, TL, false>(x, tw, lds_all + wave * FftShape<TL>::LDS, lane);
   if (!ok) return;
@@ -632,12 +668,18 @@ void launch_fft_weights(const Plan& P, const float2* u, int N_rhs, hipStream_t s
   const int TL = P.fft.shape.TL, FPW = 64 / TL;
   const size_t rows = (size_t)P.N_pairs * N_rhs;
   const dim3 grid((unsigned)((rows + 4 * FPW - 1) / (4 * FPW)));
-#define BORN_FFT_W(TLv)                                                                                              \
-  hipLaunchKernelGGL(k_fft_weights<TLv>, grid, dim3(256), 0, s, u, P.d_pe_off, P.d_pe_ent, P.d_pref,                 \
+#define BORN_FFT_WL(TLv, LONGv)                                                                                      \
+  hipLaunchKernelGGL((k_fft_weights<TLv, LONGv>), grid, dim3(256), 0, s, u, P.d_pe_off, P.d_pe_ent, P.d_pref,        \
                      P.fft.d_tw, P.N_pairs, P.N_e, N_rhs, P.N_obs, (float4*)P.fft.d_wt)
+#define BORN_FFT_W(TLv)                                                          \
+  do {                                                                           \
+    if (P.n_pe_ent >= 4 * (int64_t)P.N_pairs * P.N_e) BORN_FFT_WL(TLv, true);    \
+    else BORN_FFT_WL(TLv, false);                                                \
+  } while (0)
   if (TL == 16) BORN_FFT_W(16);
   else if (TL == 8) BORN_FFT_W(8);
   else BORN_FFT_W(4);
+#undef BORN_FFT_WL
 #undef BORN_FFT_W
 }
 

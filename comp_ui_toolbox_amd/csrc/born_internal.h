@@ -237,6 +237,7 @@ struct Plan {
   // adjoint un-mixing gather lists: for each pair, the (mk, f) that read it
   int64_t* d_pe_off = nullptr;    // [N_pairs * N_e + 1]: un-mixing entries of (pair, element)
   int2* d_pe_ent = nullptr;       // (observation, prefactor index)
+  int64_t n_pe_ent = 0;
   std::vector<int> h_shift;       // host copy of the 0-based shift map [N_e][N_pts]
 
   // per-N_rhs workspace

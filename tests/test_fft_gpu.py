@@ -81,6 +81,20 @@ def test_against_oracle_and_general_path(torch_cuda, ne, nx, nz, npp, nf, waves,
             assert O.rel_l2(fast[k][r], general[k][r]) < 2 * TOL, ("general", k)
 
 
+def test_lists_of_unequal_length(torch_cuda):
+    """Un-mixing lists of 0 to 11 entries side by side, 5 on average."""
+    spec = make(20, 60, 3, 2, 3, 2, 5)
+    rng = np.random.Generator(np.random.PCG64(4))
+    for k, mixes in enumerate(spec.mixes):
+        for n in (3, 7, 12, 20, 20, 20):
+            e = rng.permutation(np.arange(1, 20))[:min(n, 19)]   # element 0 in the dense mixes only
+            mixes.append(C.MixSpec(e, rng.standard_normal(len(e)), np.array([k, 2])))
+    T = O.direct_tables(spec)
+    op = OperatorBorn.from_sequence(spec)
+    u = rng.standard_normal(op.N_observations) + 1j * rng.standard_normal(op.N_observations)
+    assert O.rel_l2(op.adjoint(u), O.adjoint(T, u).reshape(-1)) < TOL
+
+
 def test_mixed_tables_and_zero_columns(torch_cuda):
     """Frequency subsets, repeated frequencies and a right-hand side that is
     zero, from an operator's own tables."""
@@ -144,6 +158,7 @@ def test_volume(torch_cuda, nex, ney, nx, ny, nz, npp, nf, waves, n_rhs):
     (8, 16, 400, 2, 2, 1, 0, 1),       # 24 slot blocks of a few values: eight threads per value
     (9, 15, 200, 4, 3, 2, 5, 3),       # the same, several mixes and right-hand sides
     (24, 40, 34, 1, 17, 3, 3, 1),      # columns in several groups per slot group
+    (33, 60, 3, 2, 2, 2, 4, 2), (70, 40, 2, 1, 3, 1, 5, 1), (128, 60, 2, 1, 2, 1, 11, 2),      # lists of 4, 5 and 11
 ])
 def test_split_of_small_plans(torch_cuda, ne, nx, nz, npp, nf, waves, n_mix, n_rhs):
     test_against_oracle_and_general_path(torch_cuda, ne, nx, nz, npp, nf, waves, n_mix, n_rhs)
