@@ -51,7 +51,12 @@ enum born_status {
     BORN_ERR_OUT_OF_MEMORY = 12          /* born:OutOfMemory */
 };
 
-/* Numeric form of the grid contraction. */
+/* Numeric form of the grid contraction on the matrix cores.  Plans with the
+ * lateral structure apply the operator by fast correlation in FP32 whatever
+ * form is asked for (faster than the split forms and more accurate); the form
+ * decides for those that cannot: spectra of h_ref that do not fit in memory,
+ * rows of h_ref with one entry far above the others, planes over 128 points
+ * and elements per phase in 3-D, and born_apply_dev_noalloc. */
 enum born_precision {
     BORN_PRECISION_FP32 = 0,     /* plain FP32 operands, FP32 MFMA products      */
     BORN_PRECISION_SPLIT_BF16 = 1,/* hi+lo BF16 operands, FP32 accumulation       */
@@ -170,7 +175,8 @@ int born_adjoint_dev(born_plan_t plan, const void* u_c64, int32_t N_rhs, void* g
 /* The operator pair applied without allocating: mode 1 is the forward of
  * born_forward_dev, any other value the adjoint of born_adjoint_dev (the
  * MEX's mode rule, cu:404-409), same buffers and layouts, computed by the
- * same kernels.  No counterpart in the reference: it is for callers that
+ * matrix kernels in the plan's precision (the fast correlation needs the
+ * workspace).  No counterpart in the reference: it is for callers that
  * cannot allocate device memory -- code under HIP graph capture, serving
  * loops, harnesses that forbid it.  It calls no hipMalloc or hipFree:
  * instead of the plan's per-rhs workspace it uses a one-rhs layout built at
@@ -183,7 +189,7 @@ int born_adjoint_dev(born_plan_t plan, const void* u_c64, int32_t N_rhs, void* g
  * the array holds, gets BORN_ERR_UNSUPPORTED with the sizes in
  * born_last_error().  Event timing (born_plan_set_timing) does not cover
  * these calls.  Results agree with born_forward_dev / born_adjoint_dev within
- * FP32 rounding (the forward's partial sums may be blocked differently). */
+ * the rounding of the precision (they are computed by other kernels there). */
 #define BORN_NOALLOC_SCRATCH_BYTES (64ull << 20)
 int born_apply_dev_noalloc(born_plan_t plan, int32_t mode, const void* in_c64, int32_t N_rhs, void* out_c64,
                            void* stream);
@@ -327,7 +333,8 @@ int born_batch_set_graph(born_batch_t batch, int32_t on);
 /* Autotuner: times the candidate work-item counts and persistent grid sizes
  * of the forward contraction and the segment widths of the adjoint on the
  * batch's own instances and keeps the fastest, for each MFMA launch set of
- * the batch; returns their times (ms, summed over the sets). */
+ * the batch; returns their times (ms, summed over the sets).  Plans on the
+ * fast correlation have nothing to choose: their launches are timed. */
 int born_batch_autotune(born_batch_t batch, void* stream, double* fwd_ms, double* adj_ms);
 int born_plan_autotune(born_plan_t plan, void* stream, double* fwd_ms, double* adj_ms);
 /* Event timing of the batched contraction launches (as born_plan_set_timing). */
