@@ -326,6 +326,8 @@ static void upload_index_structures(Plan& P, hipStream_t s) {
   P.d_pe_off = dupload(peoff, s);
   P.d_pe_ent = dupload(ent, s);
   P.n_pe_ent = peoff.back();
+  P.single_mixes = true;
+  for (int mk = 0; mk < P.N_mk; ++mk) P.single_mixes = P.single_mixes && P.mk_Nact[mk] == 1;
 }
 
 // The lateral Toeplitz structure of setup_grid_symmetric.shift_lateral
@@ -1667,8 +1669,7 @@ static void forward_device(Plan& P, const float2* gm, int N_rhs, void* u, bool o
       if (P.nd == 3) launch_fft3_fwd(P, N_rhs, s);
       else launch_fft_fwd(P.fft.set, s);
     }
-    launch_fft_reduce(P, N_rhs, s);
-    launch_fwd_mix(P, N_rhs, u, out_f64, s);
+    launch_fft_reduce(P, N_rhs, u, out_f64, s);
     HIP_CHECK(hipGetLastError());
     return;
   }
@@ -2071,12 +2072,12 @@ static void batch_forward_enqueue(Batch& B, const void* const* in, void* const* 
   for (size_t i = 0; i < B.plans.size(); ++i) {
     Plan& P = *B.plans[i];
     if (B.set_of[i] < 0) {
-      launch_fft_reduce(P, 1, s);
+      launch_fft_reduce(P, 1, out[i], false, s);
     } else {
       const LaunchSet& L = B.set(B.set_of[i]);
       launch_fwd_reduce(P, 1, fwd_blocks(L, B.precision, L.inst[B.slot[i]]), s);
+      launch_fwd_mix(P, 1, out[i], false, s);
     }
-    launch_fwd_mix(P, 1, out[i], false, s);
   }
   HIP_CHECK(hipGetLastError());
 }

@@ -282,10 +282,16 @@ __global__ __launch_bounds__(256, 2) void k_fft_fwd(const FftInst* __restrict__ 
   }
 }
 
-// Slot-block partials -> V[pair][e][r] (FP64 sums), NS threads per value.
-template <int NS>
+// Slot-block partials -> V[pair][e][r] (FP64 sums), NS threads per value.  MIX:
+// plans whose mixes have one active element each: every observation is one
+// value times its prefactor, written here (OutT) in place of V and a mixing
+// kernel behind it (64 elements, 256 x 256 points, 65 frequencies, one wave:
+// 3.9 and 4.1 us for the two kernels, 4.5 here).
+template <int NS, bool MIX, typename OutT>
 __global__ __launch_bounds__(256) void k_fft_reduce(const float2* __restrict__ vp, const int2* __restrict__ col, int n_cols,
-                                                    int NZB, int N_e, int N_rhs, double2* __restrict__ V) {
+                                                    int NZB, int N_e, int N_rhs, double2* __restrict__ V,
+                                                    const int64_t* __restrict__ pe_off, const int2* __restrict__ pe_ent,
+                                                    const double2* __restrict__ pref, int64_t N_obs, OutT* __restrict__ u) {
   constexpr int NV = 256 / NS;
   __shared__ double2 part[NS][NV];
   const int k = threadIdx.x % NV, slice = threadIdx.x / NV;
@@ -313,7 +319,20 @@ __global__ __launch_bounds__(256) void k_fft_reduce(const float2* __restrict__ v
   const int r = (int)(idx / plane);
   const size_t ce = idx - (size_t)r * plane;
   const int c = (int)(ce / N_e), e = (int)(ce - (size_t)c * N_e);
-  V[((size_t)col[c].x * N_e + e) * N_rhs + r] = make_double2(sx, sy);
+  const size_t pe = (size_t)col[c].x * N_e + e;
+  if constexpr (MIX) {
+    const int64_t i1 = pe_off[pe + 1];
+    for (int64_t i = pe_off[pe]; i < i1; ++i) {
+      const int2 oe = pe_ent[i];
+      const double2 w = pref[oe.y];
+      OutT o;
+      o.x = w.x * sx - w.y * sy;
+      o.y = w.x * sy + w.y * sx;
+      u[r * N_obs + oe.x] = o;
+    }
+  } else {
+    V[pe * N_rhs + r] = make_double2(sx, sy);
+  }
 }
 
 // ------------------------------------------------------------------ adjoint
@@ -654,14 +673,24 @@ void launch_fft_adj(const FftSet& S, const OutPtrs& outs, hipStream_t s) {
 // holds and more than 16 blocks to add (one thread takes them one after the
 // other: 10 us for 32 blocks of 1400 values, 28 us for 64 of 10^4, with 8
 // threads 4 and 6), else 1 (10^6 values of 8 blocks: 19 us, with 8 threads 31).
-void launch_fft_reduce(const Plan& P, int N_rhs, hipStream_t s) {
+void launch_fft_reduce(const Plan& P, int N_rhs, void* u, bool out_f64, hipStream_t s) {
   const size_t total = (size_t)P.N_pairs * P.N_e * N_rhs;
-  if (total < ((size_t)1 << 19) && P.fft.NZB > 16)
-    hipLaunchKernelGGL(k_fft_reduce<8>, dim3((unsigned)((total + 31) / 32)), dim3(256), 0, s, P.fft.d_vp, P.fft.d_col,
-                       P.N_pairs, P.fft.NZB, P.N_e, N_rhs, P.d_V);
-  else
-    hipLaunchKernelGGL(k_fft_reduce<1>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, P.fft.d_vp, P.fft.d_col,
-                       P.N_pairs, P.fft.NZB, P.N_e, N_rhs, P.d_V);
+  const bool many = total < ((size_t)1 << 19) && P.fft.NZB > 16;
+  const dim3 grid((unsigned)(many ? (total + 31) / 32 : (total + 255) / 256));
+#define BORN_FFT_R(NSv, MIXv, T)                                                                                        \
+  hipLaunchKernelGGL((k_fft_reduce<NSv, MIXv, T>), grid, dim3(256), 0, s, P.fft.d_vp, P.fft.d_col, P.N_pairs, P.fft.NZB, \
+                     P.N_e, N_rhs, P.d_V, P.d_pe_off, P.d_pe_ent, P.d_pref, P.N_obs, (T*)u)
+#define BORN_FFT_RM(NSv)                                  \
+  do {                                                    \
+    if (!P.single_mixes) BORN_FFT_R(NSv, false, float2);  \
+    else if (out_f64) BORN_FFT_R(NSv, true, double2);     \
+    else BORN_FFT_R(NSv, true, float2);                   \
+  } while (0)
+  if (many) BORN_FFT_RM(8);
+  else BORN_FFT_RM(1);
+#undef BORN_FFT_RM
+#undef BORN_FFT_R
+  if (!P.single_mixes) launch_fwd_mix(P, N_rhs, u, out_f64, s);
 }
 
 void launch_fft_weights(const Plan& P, const float2* u, int N_rhs, hipStream_t s) {

@@ -238,6 +238,7 @@ struct Plan {
   int64_t* d_pe_off = nullptr;    // [N_pairs * N_e + 1]: un-mixing entries of (pair, element)
   int2* d_pe_ent = nullptr;       // (observation, prefactor index)
   int64_t n_pe_ent = 0;
+  bool single_mixes = false;      // every mix has one active element
   std::vector<int> h_shift;       // host copy of the 0-based shift map [N_e][N_pts]
 
   // per-N_rhs workspace
@@ -471,7 +472,7 @@ void launch_fft_table(const Plan& P, hipStream_t s);
 void launch_fft_gamma(const Plan& P, const float2* gamma, int N_rhs, bool mask, hipStream_t s);
 void launch_fft_fwd(const FftSet& S, hipStream_t s);
 void launch_fft_adj(const FftSet& S, const OutPtrs& outs, hipStream_t s);
-void launch_fft_reduce(const Plan& P, int N_rhs, hipStream_t s);
+void launch_fft_reduce(const Plan& P, int N_rhs, void* u, bool out_f64, hipStream_t s);   // and the mixing
 void launch_fft_weights(const Plan& P, const float2* u, int N_rhs, hipStream_t s);
 void launch_fft_adj_reduce(const Plan& P, int N_rhs, float2* out, hipStream_t s);
 
