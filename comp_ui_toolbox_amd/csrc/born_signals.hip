@@ -187,10 +187,13 @@ __global__ __launch_bounds__(256) void k_time_table(int N_t, float2* __restrict_
 // Regular plans (row = signal of a right-hand side, rows of N_f coefficients
 // one after the other) with q = q0 + dq f.  A wave takes 64 samples of RB rows:
 // the phase factor of 8 frequencies is one table entry times the kept factors
-// of 1 .. 7 steps, and serves RB rows, whose coefficients are uniform.  Bound:
-// the vector ALU, 2 RB + 5 instructions per frequency in place of a sincos and
-// a 64-bit remainder per product (5632 rows of 640 samples from 257
-// frequencies: 1150 us there, 90 us here).
+// of 1 .. 7 steps, and serves RB rows, whose coefficients are uniform.  With C
+// the sum of the cosine and S that of the sine products, sample n is C - S and
+// sample N_t - n is C + S: half of the samples are summed, and the one at N_t / 2
+// by a sum of alternating signs.  Bound: the vector ALU, 2 RB + 5 instructions
+// per frequency and two samples in place of a sincos and a 64-bit remainder per
+// product (5632 rows of 640 samples from 257 frequencies: 1150 us there, 88 us
+// here sample by sample, 63 in pairs).
 template <int RB>
 __global__ __launch_bounds__(256) void k_time_regular(const float2* __restrict__ u, const float2* __restrict__ cs,
                                                       int64_t rows, int Nf, int N_t, int q0, int dq, int n_nb,
@@ -199,8 +202,8 @@ __global__ __launch_bounds__(256) void k_time_regular(const float2* __restrict__
   const int64_t task = (int64_t)blockIdx.x * 4 + wave;
   const int64_t row0 = task / n_nb * RB;
   if (row0 >= rows) return;
-  const int n = (int)(task % n_nb) * 64 + lane;
-  const int nn = min(n, N_t - 1);
+  const int n = (int)(task % n_nb) * 64 + lane, n_half = (N_t + 1) / 2;   // samples 0 .. n_half - 1
+  const int nn = min(n, n_half - 1);
   const int rb = (int)(rows - row0 < RB ? rows - row0 : RB);
   const float2* x[RB];
 #pragma unroll
@@ -218,17 +221,17 @@ __global__ __launch_bounds__(256) void k_time_regular(const float2* __restrict__
     }
   }
   const int step8 = (int)((int64_t)dq * 8 * nn % N_t);
-  float acc[RB];
+  float C[RB], S[RB];
 #pragma unroll
-  for (int r = 0; r < RB; ++r) acc[r] = 0.f;
+  for (int r = 0; r < RB; ++r) C[r] = S[r] = 0.f;
   int f = 0;
   for (; f + 8 <= Nf; f += 8) {
     const float2 w = cs[at];
     at += step8;
     if (at >= N_t) at -= N_t;
-    float sum[RB];   // of 8 frequencies: shorter chains round less
+    float sc[RB], ss[RB];   // of 8 frequencies: shorter chains round less
 #pragma unroll
-    for (int r = 0; r < RB; ++r) sum[r] = 0.f;
+    for (int r = 0; r < RB; ++r) sc[r] = ss[r] = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const float c = i ? fmaf(w.x, pw[i].x, -(w.y * pw[i].y)) : w.x;
@@ -236,11 +239,15 @@ __global__ __launch_bounds__(256) void k_time_regular(const float2* __restrict__
 #pragma unroll
       for (int r = 0; r < RB; ++r) {
         const float2 v = x[r][f + i];
-        sum[r] = fmaf(v.x, c, fmaf(-v.y, s, sum[r]));
+        sc[r] = fmaf(v.x, c, sc[r]);
+        ss[r] = fmaf(v.y, s, ss[r]);
       }
     }
 #pragma unroll
-    for (int r = 0; r < RB; ++r) acc[r] += sum[r];
+    for (int r = 0; r < RB; ++r) {
+      C[r] += sc[r];
+      S[r] += ss[r];
+    }
   }
   for (; f < Nf; ++f) {
     const float2 w = cs[at];
@@ -249,17 +256,35 @@ __global__ __launch_bounds__(256) void k_time_regular(const float2* __restrict__
 #pragma unroll
     for (int r = 0; r < RB; ++r) {
       const float2 v = x[r][f];
-      acc[r] = fmaf(v.x, w.x, fmaf(-v.y, w.y, acc[r]));
+      C[r] = fmaf(v.x, w.x, C[r]);
+      S[r] = fmaf(v.y, w.y, S[r]);
     }
   }
   // the zero and Nyquist indices count once: take half of them back
   const int fz = q0 == 0 ? 0 : -1, fn = 2 * (q0 + dq * (Nf - 1)) == N_t ? Nf - 1 : -1;
 #pragma unroll
   for (int r = 0; r < RB; ++r) {
-    float a = acc[r];
-    if (fz >= 0) a -= 0.5f * x[r][0].x;
-    if (fn >= 0) a -= 0.5f * (nn & 1 ? -x[r][fn].x : x[r][fn].x);
-    if (r < rb && n < N_t) rf[(row0 + r) * N_t + n] = 2.f * a;
+    float c = C[r];
+    if (fz >= 0) c -= 0.5f * x[r][0].x;
+    if (fn >= 0) c -= 0.5f * (nn & 1 ? -x[r][fn].x : x[r][fn].x);
+    if (r < rb && n < n_half) {
+      float* out = rf + (row0 + r) * N_t;
+      out[n] = 2.f * (c - S[r]);
+      if (n > 0) out[N_t - n] = 2.f * (c + S[r]);
+    }
+  }
+  if ((N_t & 1) || n >= 64) return;
+  // sample N_t / 2, by the wave of samples 0 .. 63
+#pragma unroll
+  for (int r = 0; r < RB; ++r) {
+    float c = 0.f;
+    for (int k = lane; k < Nf; k += 64) {
+      const float v = (k == fz || k == fn ? 0.5f : 1.f) * x[r][k].x;
+      c += (q0 + dq * k) & 1 ? -v : v;
+    }
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) c += __shfl_xor(c, m);
+    if (lane == 0 && r < rb) rf[(row0 + r) * N_t + N_t / 2] = 2.f * c;
   }
 }
 
@@ -270,7 +295,7 @@ void launch_time_table(int N_t, float2* cs, hipStream_t s) {
 void launch_time_regular(const Plan& P, const float2* u, int N_rhs, int N_t, int q0, int dq, float* rf, hipStream_t s) {
   constexpr int RB = 8;
   const int64_t rows = (int64_t)P.N_mk * N_rhs;
-  const int n_nb = (N_t + 63) / 64;
+  const int n_nb = ((N_t + 1) / 2 + 63) / 64;
   const int64_t tasks = (rows + RB - 1) / RB * n_nb;
   hipLaunchKernelGGL(k_time_regular<RB>, dim3((unsigned)((tasks + 3) / 4)), dim3(256), 0, s, u, P.d_time_cs, rows,
                      P.N_fu, N_t, q0, dq, n_nb, rf);

@@ -97,3 +97,22 @@ def test_operator_with_time_gain_in_one_call(torch_cuda, n_rhs, sparse):
         assert np.any(u) == np.any(g)
     back = op.op_A(y, 2, tgc=True)
     assert np.array_equal(back, op.adjoint(op.tgc_adjoint(y)))
+
+
+@pytest.mark.parametrize("n_t", [21, 126, 127, 128, 129, 130, 257])
+def test_time_signals_sample_counts(torch_cuda, n_t):
+    """Even and odd numbers of samples around whole wave blocks of sample pairs;
+    the bound of test_time_signals_regular."""
+    import torch
+    nf, q = 10, np.arange(10)
+    op = operator(nf)
+    rng = np.random.Generator(np.random.PCG64(n_t))
+    u = (rng.standard_normal((1, op.N_observations)) + 1j * rng.standard_normal((1, op.N_observations))).astype(np.complex64)
+    rf, got = op.time_signals(torch.tensor(u, device="cuda:0"), 1e4 * q, delta_f=1e4, delta_t=1.0 / (1e4 * n_t))
+    assert got == n_t
+    x = u.reshape(1, 6, nf).astype(np.complex128)
+    spec = np.zeros((1, 6, n_t // 2 + 1), dtype=np.complex128)
+    spec[..., q] = x
+    ref = np.fft.irfft(spec, n=n_t) * n_t
+    size = 2.0 * np.abs(x).sum(axis=2, keepdims=True)
+    assert np.all(np.abs(rf.cpu().numpy().reshape(ref.shape) - ref) <= (2 * nf + 12) * 2.0 ** -24 * size)
