@@ -193,7 +193,7 @@ __global__ __launch_bounds__(256) void k_time_table(int N_t, float2* __restrict_
 // by a sum of alternating signs.  Bound: the vector ALU, 2 RB + 5 instructions
 // per frequency and two samples in place of a sincos and a 64-bit remainder per
 // product (5632 rows of 640 samples from 257 frequencies: 1150 us there, 88 us
-// here sample by sample, 63 in pairs).
+// here sample by sample, 56 in pairs).
 template <int RB>
 __global__ __launch_bounds__(256) void k_time_regular(const float2* __restrict__ u, const float2* __restrict__ cs,
                                                       int64_t rows, int Nf, int N_t, int q0, int dq, int n_nb,
@@ -293,7 +293,7 @@ void launch_time_table(int N_t, float2* cs, hipStream_t s) {
 }
 
 void launch_time_regular(const Plan& P, const float2* u, int N_rhs, int N_t, int q0, int dq, float* rf, hipStream_t s) {
-  constexpr int RB = 8;
+  constexpr int RB = 4;   // 8: 6 us slower at 5632 rows; 12 and 16: the uniform coefficients no longer fit, 190 and 230 us
   const int64_t rows = (int64_t)P.N_mk * N_rhs;
   const int n_nb = ((N_t + 1) / 2 + 63) / 64;
   const int64_t tasks = (rows + RB - 1) / RB * n_nb;
