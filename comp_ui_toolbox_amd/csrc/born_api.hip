@@ -496,6 +496,7 @@ static void build_fft(Plan& P) {
     HIP_CHECK(e);
     HIP_CHECK(e2);
     HIP_CHECK(e3);
+    P.h_uneven = bad != 0;
     if (bad) return;
   }
   if (P.nd == 3) {

@@ -100,3 +100,21 @@ def test_under_tgc(torch_cuda, nf, M, kind):
         E = op.energy_rx(m, tgc=True)
         assert np.linalg.norm(E - ref) < 2.2e-6 * np.linalg.norm(ref)
         assert np.array_equal(E, op.energy_rx_dev(m, tgc=True).cpu().numpy())
+
+
+@pytest.mark.parametrize("kind", ["single", "dense"])
+def test_entry_that_is_not_finite(torch_cuda, kind):
+    """A table entry that is not finite stays with the points that see it."""
+    rng = np.random.Generator(np.random.PCG64(2))
+    arr = C.ArraySpec((17,), (3e-4,), (2.7e-4,), (2,))
+    waves = [C.random_wave(arr, rng, 1e-6)]
+    spec = C.SequenceSpec("e", arr, C.MediumSpec(), C.FovSpec((130, 3), (1.5e-4, 1.5e-4), 2e-3), np.linspace(2e6, 5e6, 3),
+                          waves, [mixes_of(kind, 17, 3, rng)])
+    T = O.build_tables(spec)
+    at = T.N_points // 3 + 20
+    seen = np.any(np.asarray(T.shift) - 1 == at, axis=1)
+    ref = O.energy_rx(T, 0)
+    T.h_ref[1, at] = np.inf
+    op = OperatorBorn.from_tables(T)
+    assert op.path == "structured" and seen.any() and not seen.all()
+    assert np.linalg.norm((op.energy_rx(0) - ref)[~seen]) < 2.4e-7 * np.linalg.norm(ref[~seen])
