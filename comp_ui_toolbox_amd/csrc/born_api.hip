@@ -2721,8 +2721,7 @@ static void columns(Plan& P, const double* points, int32_t n, void* out, bool ho
   std::vector<int> pts(n);
   for (int j = 0; j < n; ++j) pts[j] = idx1(points[j], P.N_pts, "points");
   // force_general takes the map-driven kernel
-  const bool fast = use_structured(P) && columns_fast(P) &&
-                    (double)n * ((P.N_e + COL_EB - 1) / COL_EB) * ((P.meas_Nfm.size() + COL_MG - 1) / COL_MG) < 2e9;
+  const bool fast = use_structured(P) && columns_fast(P);
   if (fast) ensure_column_tables(P);
   else ensure_shift_on_device(P);
   if (P.pts_cap < n) {   // kept: calls end synchronized, so nothing reads it any more

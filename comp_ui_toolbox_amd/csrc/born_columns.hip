@@ -196,6 +196,13 @@ bool columns_fast(const Plan& P) {
          (P.col_n_multi == 0 || multi_points(P.N_e) > 0);
 }
 
+// Points that one launch takes, in groups of JB with `blocks` workgroups of
+// `threads` each: a launch holds less than 2^32 threads.
+static int launch_points(int64_t blocks, int threads, int JB) {
+  const int64_t groups = std::max<int64_t>(1, ((int64_t)0xffffffff / threads - XCDS) / blocks);
+  return (int)std::min<int64_t>(groups, INT32_MAX / JB) * JB;
+}
+
 template <typename OutT>
 static void launch_fast(const Plan& P, const int* pts, int n, OutT* u, hipStream_t s) {
   ColArgs A;
@@ -213,35 +220,44 @@ static void launch_fast(const Plan& P, const int* pts, int n, OutT* u, hipStream
   A.N_pts = P.N_pts;
   A.H_plane = P.H_plane;
   A.N_obs = P.N_obs;
-  A.pts = pts;
-  A.n = n;
   if (P.col_n_single > 0) {
     const int N_meas = (int)P.meas_Nfm.size();
     const int n_eb = (P.N_e + COL_EB - 1) / COL_EB, n_mg = (N_meas + COL_MG - 1) / COL_MG;
     const size_t lds = single_lds(P.N_fu);
     hipFuncSetAttribute((const void*)k_columns_single<OutT>, hipFuncAttributeMaxDynamicSharedMemorySize, 152 * 1024);
     // few points: the measurement groups of a block go to several workgroups
-    const int n_part = std::max(1, std::min(n_mg, 1024 / std::max(1, n * n_eb)));
-    hipLaunchKernelGGL(k_columns_single<OutT>, dim3((unsigned)(((size_t)n * n_eb * n_part + XCDS - 1) / XCDS * XCDS)), dim3(COL_NT), lds, s, A,
-                       P.d_col_off, P.d_col_ent, P.d_mk_off, P.d_pref, n_eb, n_mg, n_part, N_meas, u);
+    const int n_part = std::max(1, (int)std::min<int64_t>(n_mg, 1024 / ((int64_t)n * n_eb)));
+    const int at_once = launch_points((int64_t)n_eb * n_part, COL_NT, 1);
+    for (int64_t j0 = 0; j0 < n; j0 += at_once) {
+      A.pts = pts + j0;
+      A.n = (int)std::min<int64_t>(at_once, n - j0);
+      hipLaunchKernelGGL(k_columns_single<OutT>, dim3((unsigned)(((size_t)A.n * n_eb * n_part + XCDS - 1) / XCDS * XCDS)),
+                         dim3(COL_NT), lds, s, A, P.d_col_off, P.d_col_ent, P.d_mk_off, P.d_pref, n_eb, n_mg, n_part,
+                         N_meas, u + j0 * P.N_obs);
+    }
   }
   if (P.col_n_multi > 0) {
     const int JB = multi_points(P.N_e);
     const int n_fb = (P.N_fu + COL_FB - 1) / COL_FB, n_jb = (n + JB - 1) / JB;
     // parts: enough workgroups for the chip, at least 16 mixes each
-    const int n_part = std::max(1, std::min((P.col_n_multi + 15) / 16, 1024 / std::max(1, n_fb * n_jb)));
+    const int n_part = std::max(1, (int)std::min<int64_t>((P.col_n_multi + 15) / 16, 1024 / std::max<int64_t>(1, (int64_t)n_fb * n_jb)));
     const size_t lds = (size_t)JB * P.N_e * (COL_FB + 1) * sizeof(float2);
-    const dim3 grid((unsigned)((size_t)n_jb * n_fb * n_part));
+    const int at_once = launch_points((int64_t)n_fb * n_part, 256, JB);
 #define BORN_COL_M(JBv)                                                                                               \
   do {                                                                                                                \
     hipFuncSetAttribute((const void*)k_columns_multi<OutT, JBv>, hipFuncAttributeMaxDynamicSharedMemorySize,          \
                         160 * 1024);                                                                                  \
     hipLaunchKernelGGL((k_columns_multi<OutT, JBv>), grid, dim3(256), lds, s, A, P.d_col_multi, P.col_n_multi,       \
-                       P.d_mk_meta, P.d_mk_off, P.d_act, P.d_pref, n_part, u);                                        \
+                       P.d_mk_meta, P.d_mk_off, P.d_act, P.d_pref, n_part, u + j0 * P.N_obs);               \
   } while (0)
-    if (JB == 4) BORN_COL_M(4);
-    else if (JB == 2) BORN_COL_M(2);
-    else BORN_COL_M(1);
+    for (int64_t j0 = 0; j0 < n; j0 += at_once) {
+      A.pts = pts + j0;
+      A.n = (int)std::min<int64_t>(at_once, n - j0);
+      const dim3 grid((unsigned)((size_t)((A.n + JB - 1) / JB) * n_fb * n_part));
+      if (JB == 4) BORN_COL_M(4);
+      else if (JB == 2) BORN_COL_M(2);
+      else BORN_COL_M(1);
+    }
 #undef BORN_COL_M
   }
 }

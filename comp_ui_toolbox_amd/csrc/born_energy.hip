@@ -422,7 +422,7 @@ template <int TL, int NQ>
 __global__ __launch_bounds__(256, 2) void k_energy_tgc_fft(EnergyArgs A, const float4* __restrict__ spec,
                                                            const double2* __restrict__ taps, const int* __restrict__ half,
                                                            const int64_t* __restrict__ tap_off,
-                                                           const float2* __restrict__ twid, int mk0, int mk1,
+                                                           const float2* __restrict__ twid, int mk0, int mk1, int b0,
                                                            double* __restrict__ E) {
   constexpr int FPW = FftShape<TL>::FPW, L = 16 * TL;
   __shared__ cf lds_all[4 * FftShape<TL>::LDS];
@@ -431,7 +431,7 @@ __global__ __launch_bounds__(256, 2) void k_energy_tgc_fft(EnergyArgs A, const f
   const int j = lane / FPW, g = lane % FPW;
   cf* lds = lds_all + wave * FftShape<TL>::LDS;
   const int N = A.n_pairs;
-  const int p = min((int)blockIdx.x * FPW + g, A.N_pts - 1);
+  const int p0 = (b0 + (int)blockIdx.x) * FPW + g, p = min(p0, A.N_pts - 1);
   const int row = p / A.Nx, ix = p - row * A.Nx;
   cf tw[16];
   load_twiddles<TL>(twid, j, tw);
@@ -507,7 +507,7 @@ __global__ __launch_bounds__(256, 2) void k_energy_tgc_fft(EnergyArgs A, const f
   }
   red[wave][lane] = acc;
   __syncthreads();
-  if (wave == 0 && j == 0 && (int)blockIdx.x * FPW + g < A.N_pts) {
+  if (wave == 0 && j == 0 && p0 < A.N_pts) {
     double s = 0.0;
     for (int w = 0; w < 4; ++w)
       for (int t = 0; t < TL; ++t) s += red[w][t * FPW + g];
@@ -655,10 +655,10 @@ void launch_energy_tgc_fft(const Plan& P, int m, double* E, hipStream_t s) {
   while (mk1 < P.N_mk && P.mk_meas[mk1] == m) ++mk1;
   const EnergyArgs A = energy_args(P, m, 4);
   const int TL = P.tgc_TL, FPW = 64 / TL, N = P.N_fu;
-  const dim3 grid((P.N_pts + FPW - 1) / FPW);
+  const int blocks = (int)(((int64_t)P.N_pts + FPW - 1) / FPW), at_once = (1 << 24) - 1;   // (a launch holds less than 2^32 threads)
 #define BORN_ET(TLv, NQv)                                                                                  \
   hipLaunchKernelGGL((k_energy_tgc_fft<TLv, NQv>), grid, dim3(256), 0, s, A, (const float4*)P.d_tgc_spec, \
-                     P.d_tgc_k64, P.d_tgc_half, P.d_tgc_off, P.d_tgc_tw, mk0, mk1, E)
+                     P.d_tgc_k64, P.d_tgc_half, P.d_tgc_off, P.d_tgc_tw, mk0, mk1, b0, E)
 #define BORN_ETN(TLv)                  \
   do {                                 \
     if (N <= 4 * TLv) BORN_ET(TLv, 4); \
@@ -666,9 +666,12 @@ void launch_energy_tgc_fft(const Plan& P, int m, double* E, hipStream_t s) {
     else if (N <= 9 * TLv) BORN_ET(TLv, 9); \
     else BORN_ET(TLv, 16);             \
   } while (0)
-  if (TL == 16) BORN_ETN(16);
-  else if (TL == 8) BORN_ETN(8);
-  else BORN_ETN(4);
+  for (int b0 = 0; b0 < blocks; b0 += at_once) {
+    const dim3 grid(std::min(at_once, blocks - b0));
+    if (TL == 16) BORN_ETN(16);
+    else if (TL == 8) BORN_ETN(8);
+    else BORN_ETN(4);
+  }
 #undef BORN_ETN
 #undef BORN_ET
 }

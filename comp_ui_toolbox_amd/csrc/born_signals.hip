@@ -197,9 +197,9 @@ __global__ __launch_bounds__(256) void k_time_table(int N_t, float2* __restrict_
 template <int RB>
 __global__ __launch_bounds__(256) void k_time_regular(const float2* __restrict__ u, const float2* __restrict__ cs,
                                                       int64_t rows, int Nf, int N_t, int q0, int dq, int n_nb,
-                                                      float* __restrict__ rf) {
+                                                      int64_t task0, float* __restrict__ rf) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int64_t task = (int64_t)blockIdx.x * 4 + wave;
+  const int64_t task = task0 + (int64_t)blockIdx.x * 4 + wave;
   const int64_t row0 = task / n_nb * RB;
   if (row0 >= rows) return;
   const int n = (int)(task % n_nb) * 64 + lane, n_half = (N_t + 1) / 2;   // samples 0 .. n_half - 1
@@ -296,9 +296,10 @@ void launch_time_regular(const Plan& P, const float2* u, int N_rhs, int N_t, int
   constexpr int RB = 4;   // 8: 6 us slower at 5632 rows; 12 and 16: the uniform coefficients no longer fit, 190 and 230 us
   const int64_t rows = (int64_t)P.N_mk * N_rhs;
   const int n_nb = ((N_t + 1) / 2 + 63) / 64;
-  const int64_t tasks = (rows + RB - 1) / RB * n_nb;
-  hipLaunchKernelGGL(k_time_regular<RB>, dim3((unsigned)((tasks + 3) / 4)), dim3(256), 0, s, u, P.d_time_cs, rows,
-                     P.N_fu, N_t, q0, dq, n_nb, rf);
+  const int64_t tasks = (rows + RB - 1) / RB * n_nb, at_once = 4 * ((1ll << 24) - 1);   // (a launch holds less than 2^32 threads)
+  for (int64_t t0 = 0; t0 < tasks; t0 += at_once)
+    hipLaunchKernelGGL(k_time_regular<RB>, dim3((unsigned)((std::min(at_once, tasks - t0) + 3) / 4)), dim3(256), 0, s, u,
+                       P.d_time_cs, rows, P.N_fu, N_t, q0, dq, n_nb, t0, rf);
 }
 
 }  // namespace born
