@@ -534,6 +534,17 @@ static void build_fft(Plan& P) {
   F.ok = true;
 }
 
+// Column groups of the adjoint: `fill` for the chip, and as many as keep a
+// group within `most` columns, partial images within 16 GiB.  A group's columns
+// are added one after the other in FP32, whose rounding grows with the root of
+// their number; the groups are added in FP64.  8224 columns of 128 elements,
+// 512 x 512 points: relative L2 error against FP64 4.9e-7 with 343 columns per
+// wave, 2.8e-7 with 86, same time (9.04 ms the pair).
+static int adj_groups(const Plan& P, int N_rhs, int64_t fill, int64_t most) {
+  const int64_t g = std::max<int64_t>({1, fill, (P.N_pairs + most - 1) / most});
+  return (int)std::min<int64_t>(g, std::max<int64_t>(1, (1ll << 31) / ((int64_t)N_rhs * P.N_pts)));
+}
+
 // Work split of a plan's fast-correlation launches (the chip holds 3072 waves
 // of either kernel).  Forward: a wave's final transform costs about two steps,
 // so waves take 8 steps, fewer while that leaves less than half of the chip's
@@ -543,7 +554,8 @@ static void build_fft(Plan& P) {
 // 256 x 256, 33 frequencies, one wave: 28 with 5, 30 with 4 and 8.
 // Adjoint: 3072 workgroups of 4 waves with at least 8 columns each, or 256 of
 // at least 2 columns (32 elements, 128 x 128 points, 65 frequencies: 25 us with
-// 32 workgroups, 17 with 128).
+// 32 workgroups, 17 with 128), and for the rounding of the FP32 sums at most 64
+// columns per wave (adj_groups).
 static void fft_blocking(Plan& P, int N_rhs) {
   Plan::Fft& F = P.fft;
   const int64_t steps = (int64_t)P.N_pairs * N_rhs * F.n_ws;
@@ -557,7 +569,7 @@ static void fft_blocking(Plan& P, int N_rhs) {
   const int64_t wg = (int64_t)F.n_ws * N_rhs;
   const int64_t many = std::min<int64_t>((3072 + wg - 1) / wg, P.N_pairs / 32);
   const int64_t few = std::min<int64_t>((256 + wg - 1) / wg, P.N_pairs / 8);
-  F.FG = (int)std::max<int64_t>(1, std::min<int64_t>(64, std::max(many, few)));
+  F.FG = adj_groups(P, N_rhs, std::min<int64_t>(64, std::max(many, few)), 256);
 }
 
 static FftInst make_fft_inst(const Plan& P, int N_rhs) {
@@ -611,7 +623,7 @@ static void build_fft3_workspace(Plan& P, int N_rhs) {
   F.ZR = std::min(F.ZR, P.Nz);
   F.NZB = (P.Nz + F.ZR - 1) / F.ZR;
   const int64_t wg = (int64_t)P.Nz * P.Npy * (P.Np / F.s3.px) * N_rhs;
-  F.FG = (int)std::max<int64_t>(1, std::min<int64_t>({(2048 + wg - 1) / wg, P.N_pairs / 8, 64}));
+  F.FG = adj_groups(P, N_rhs, std::min<int64_t>({(2048 + wg - 1) / wg, P.N_pairs / 8, 64}), 64);
   if (cols * F.NZB > INT32_MAX - 64 || wg * F.FG > INT32_MAX - 64)
     throw Error(BORN_ERR_UNSUPPORTED, "too many right-hand sides for one launch");
   F.d_vp = dalloc<float2>((size_t)F.NZB * cols * P.N_e);

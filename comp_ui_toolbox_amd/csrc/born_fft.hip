@@ -525,14 +525,14 @@ __global__ __launch_bounds__(256) void k_fft_adj_reduce(const float2* __restrict
                                                         float2* __restrict__ out) {
   const size_t i = blockIdx.x * (size_t)256 + threadIdx.x;
   if (i >= n) return;
-  float2 s = gp[i];
+  double x = 0.0, y = 0.0;
 #pragma unroll 8
-  for (int k = 1; k < FG; ++k) {
+  for (int k = 0; k < FG; ++k) {
     const float2 v = gp[(size_t)k * n + i];
-    s.x += v.x;
-    s.y += v.y;
+    x += v.x;
+    y += v.y;
   }
-  out[i] = s;
+  out[i] = make_float2((float)x, (float)y);
 }
 
 // ------------------------------------------------------------------ host side
