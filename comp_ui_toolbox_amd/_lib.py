@@ -32,7 +32,7 @@ EXPORTED = (
     "born_batch_create", "born_batch_destroy", "born_batch_forward_dev", "born_batch_adjoint_dev",
     "born_batch_set_graph", "born_batch_autotune", "born_plan_autotune", "born_batch_set_timing",
     "born_batch_get_timing", "born_tgc_set", "born_tgc_apply", "born_tgc_apply_dev",
-    "born_apply_tgc",
+    "born_apply_tgc", "born_plan_set_correlation", "born_plan_kernels",
     "born_energy_rx_tgc", "born_energy_rx_tgc_dev", "born_debug_fail_allocation",
     "born_debug_live_allocations", "born_columns", "born_columns_dev",
     "born_plan_set_sparse_forward", "born_apply_dev_noalloc",
@@ -122,6 +122,8 @@ def lib() -> C.CDLL:
     L.born_energy_rx_dev.argtypes = [vp, C.c_int32, vp, vp]
     L.born_time_signals.argtypes = [vp, pd, C.c_double, C.c_double, vp, C.c_int32, vp, C.c_int64,
                                     C.POINTER(C.c_int32), vp]
+    L.born_plan_set_correlation.argtypes = [vp, C.c_int32]
+    L.born_plan_kernels.argtypes = [vp, C.POINTER(C.c_int32)]
     L.born_tgc_set.argtypes = [vp, C.POINTER(C.c_int32), pd]
     L.born_tgc_apply.argtypes = [vp, C.c_int32, pd, C.c_int32, pd]
     L.born_apply_tgc.argtypes = [vp, C.c_int32, pd, C.c_int32, pd]

@@ -442,7 +442,8 @@ static bool use_structured(const Plan& P) { return P.structured && !P.force_gene
 // 2-D structured plans apply both directions by fast lateral correlation in
 // every numeric form (the split forms gain accuracy); the allocation-free
 // apply keeps the MFMA layout.
-static bool use_fft(const Plan& P) { return use_structured(P) && P.fft.ok && !P.in_noalloc; }
+static bool fft_on(const Plan& P) { return P.fft.ok && !P.fft.off; }
+static bool use_fft(const Plan& P) { return use_structured(P) && fft_on(P) && !P.in_noalloc; }
 
 // Columns (pair, frequency) by frequency.
 static void upload_fft_columns(Plan& P) {
@@ -1017,7 +1018,7 @@ static void build_workspace(Plan& P, int N_rhs);
 // could not get its workspace holds none.
 static void ensure_workspace(Plan& P, int N_rhs) {
   const bool split = P.precision != BORN_PRECISION_FP32;
-  if (P.ws_rhs == N_rhs && (N_rhs == 1 || P.fft.ok || P.ws_split == split)) return;
+  if (P.ws_rhs == N_rhs && (N_rhs == 1 || fft_on(P) || P.ws_split == split)) return;
   free_workspace(P);
   P.ws_split = split;
   try {
@@ -1031,7 +1032,7 @@ static void ensure_workspace(Plan& P, int N_rhs) {
 static void build_workspace(Plan& P, int N_rhs) {
   P.chunks.clear();
   P.col_pair.clear();
-  if (P.fft.ok) {   // V, W and the masked input also serve the general path
+  if (fft_on(P)) {   // V, W and the masked input also serve the general path
     P.d_V = dalloc<double2>((size_t)P.N_pairs * P.N_e * N_rhs);
     P.d_W = dalloc<float2>((size_t)P.N_pairs * P.N_e * N_rhs);
     P.d_gm = dalloc<float2>((size_t)N_rhs * P.N_pts);
@@ -2028,7 +2029,7 @@ static void build_batch_launch(Batch& B) {
   B.slot.assign(B.plans.size(), 0);
   for (size_t i = 0; i < B.plans.size(); ++i) {
     const Plan& P = *B.plans[i];
-    if (P.fft.ok) {
+    if (fft_on(P)) {
       B.set_of[i] = P.nd == 3 ? Batch::SET_3D : -1 - Batch::fft_set(P.fft.shape);
       B.gen.push_back(P.ws_gen);
       continue;
@@ -2957,6 +2958,30 @@ int born_plan_force_general(born_plan_t plan, int32_t on) {
     P.force_general = on != 0;
     if (P.force_general) ensure_shift_on_device(P);
     HIP_CHECK(hipStreamSynchronize(P.stream));
+  });
+}
+
+int born_plan_set_correlation(born_plan_t plan, int32_t on) {
+  return guarded([&] {
+    if (!plan) throw Error(BORN_ERR_INVALID_ARGUMENT, "plan is NULL");
+    Plan& P = *reinterpret_cast<Plan*>(plan);
+    HIP_CHECK(hipSetDevice(P.device));
+    if (P.fft.off == (on == 0)) return;
+    HIP_CHECK(hipDeviceSynchronize());
+    free_workspace(P);   // the next call builds that of the other kernels
+    P.fft.off = on == 0;
+  });
+}
+
+int born_plan_kernels(born_plan_t plan, int32_t* kernels) {
+  return guarded([&] {
+    if (!plan || !kernels) throw Error(BORN_ERR_INVALID_ARGUMENT, "plan and output are required");
+    Plan& P = *reinterpret_cast<Plan*>(plan);
+    const bool st = use_structured(P);
+    kernels[0] = !st ? BORN_KERNELS_GATHER : use_fft(P) ? BORN_KERNELS_FAST : BORN_KERNELS_DIRECT;
+    kernels[1] = st && energy_fast(P) ? BORN_KERNELS_FAST : BORN_KERNELS_GATHER;
+    kernels[2] = st && P.tgc_TL > 0 ? BORN_KERNELS_FAST : BORN_KERNELS_GATHER;
+    kernels[3] = st && columns_fast(P) ? BORN_KERNELS_FAST : BORN_KERNELS_GATHER;
   });
 }
 

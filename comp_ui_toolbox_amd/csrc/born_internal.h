@@ -268,6 +268,7 @@ struct Plan {
   // fast lateral correlation: tables of the plan, then the per-rhs workspace
   struct Fft {
     bool ok = false;
+    bool off = false;               // switched off by the caller
     FftShapeChoice shape;
     Fft3Choice s3;                  // 3-D plans
     int n_slots = 0, n_ws = 0;

@@ -207,6 +207,19 @@ class OperatorBorn:
     def force_general(self, on: bool = True):
         check(_lib.lib().born_plan_force_general(self._plan, int(on)))
 
+    def set_correlation(self, on: bool = True):
+        """Forward and adjoint by fast correlation where the plan can (default),
+        or by the direct products of its numeric form."""
+        check(_lib.lib().born_plan_set_correlation(self._plan, int(on)))
+
+    @property
+    def kernels(self) -> dict:
+        """Which kernels the plan's calls take: 'gather', 'direct' or 'fast' for
+        'pair', 'energy', 'energy_tgc' and 'columns'."""
+        k = (C.c_int32 * 4)()
+        check(_lib.lib().born_plan_kernels(self._plan, k))
+        return {n: ("gather", "direct", "fast")[v] for n, v in zip(("pair", "energy", "energy_tgc", "columns"), k)}
+
     def set_timing(self, on: bool = True):
         """Record HIP events around every contraction launch (on its stream)."""
         check(_lib.lib().born_plan_set_timing(self._plan, int(on)))

@@ -300,6 +300,24 @@ int born_plan_path(born_plan_t plan);
 /* Force the general gather path (for cross-checking the structured one). */
 int born_plan_force_general(born_plan_t plan, int32_t on);
 
+/* Whether forward and adjoint of a structured plan may go by fast correlation
+ * (on, the default) or keep to the matrix and vector kernels of the plan's
+ * numeric form (0).  A transform carries the rounding of a whole row of h_ref,
+ * the direct products only that of each entry: a program whose results hang
+ * on outputs far below the others of their row (one active element, a point
+ * outside every element's cone) switches it off.  The next call builds the
+ * workspace of the other kernels. */
+int born_plan_set_correlation(born_plan_t plan, int32_t on);
+
+/* Which kernels a plan's calls take: kernels[0] forward and adjoint, [1]
+ * received energies, [2] those under time gain, [3] columns. */
+enum born_kernels {
+    BORN_KERNELS_GATHER = 0,     /* by the shift map, any plan                      */
+    BORN_KERNELS_DIRECT = 1,     /* products on the lateral structure (born_precision) */
+    BORN_KERNELS_FAST = 2        /* fast correlation; staged lateral rows           */
+};
+int born_plan_kernels(born_plan_t plan, int32_t* kernels);
+
 /* Kernel timing with HIP events recorded on the launch stream around the
  * grid-contraction kernels (no counterpart in the reference; used by the
  * benchmark).  While enabled, every forward/adjoint apply records one event

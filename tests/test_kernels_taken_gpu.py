@@ -1,0 +1,65 @@
+"""Which kernels the plans of the fast kernels' tests take: a rule that sent
+them elsewhere would leave those tests comparing one kernel with itself."""
+import numpy as np
+import pytest
+
+from comp_ui_toolbox_amd import OperatorBorn
+from comp_ui_toolbox_amd import configs as C
+from oracle import born_oracle as O
+from tests import test_columns_gpu, test_energy_gpu, test_fft_gpu
+from tests.test_oracle import mixed_tiny_tables
+
+pytestmark = pytest.mark.gpu
+
+
+def spec_3d(nex, ney, nx, ny, nz, npp, nf, waves):
+    arr = C.ArraySpec((nex, ney), (3e-4,) * 2, (2.7e-4,) * 2, (2, 2))
+    rng = np.random.Generator(np.random.PCG64(1))
+    ws = [C.random_wave(arr, rng, 1e-6) for _ in range(waves)]
+    return C.SequenceSpec("k", arr, C.MediumSpec(), C.FovSpec((nx, ny, nz), (3e-4 / npp,) * 3, 3e-3),
+                          np.linspace(2.5e6, 4e6, nf), ws, [C.identity_mixes(nex * ney) for _ in ws])
+
+
+def test_forward_and_adjoint(torch_cuda):
+    specs = [test_fft_gpu.make(*s[:-1]) for s in test_fft_gpu.SIZES]
+    specs += [spec_3d(*s[:-1]) for s in test_fft_gpu.SIZES_3D]
+    for spec in specs:
+        op = OperatorBorn.from_sequence(spec)
+        assert op.kernels["pair"] == "fast", spec
+        op.forward_dev(torch_cuda.zeros(op.N_points, dtype=torch_cuda.complex64, device="cuda:0"))
+        assert op.kernels["pair"] == "fast", spec
+        op.force_general(True)
+        assert set(op.kernels.values()) == {"gather"}
+        op.close()
+
+
+@pytest.mark.parametrize("three", [False, True])
+@pytest.mark.parametrize("entry", [1e7, np.inf])
+def test_uneven_tables(torch_cuda, three, entry):
+    T = O.build_tables(spec_3d(4, 3, 19, 7, 3, 2, 2, 2) if three else test_fft_gpu.make(33, 101, 6, 3, 3, 2))
+    assert OperatorBorn.from_tables(T).kernels["pair"] == "fast"
+    T.h_ref[1, T.N_points // 3] = entry
+    assert OperatorBorn.from_tables(T).kernels["pair"] == "direct"
+
+
+@pytest.mark.parametrize("kind", ["single", "dense", "both"])
+def test_energies(torch_cuda, kind):
+    for ne, nx, nz, npp in test_energy_gpu.SIZES:
+        rng = np.random.Generator(np.random.PCG64(1))
+        spec = test_fft_gpu.make(ne, nx, nz, npp, 5, 2)
+        spec.mixes = [test_energy_gpu.mixes_of(kind, ne, 5, rng) for _ in spec.waves]
+        op = OperatorBorn.from_sequence(spec)
+        assert op.kernels["energy"] == "fast"
+        assert op.kernels["energy_tgc"] == "gather"
+        if kind != "both":      # (a mix on two of the frequencies)
+            op.set_tgc([np.ones(2 * (k % 4) + 1) for k in range(op.meta["n_mix_signals"])])
+            assert op.kernels["energy_tgc"] == "fast"
+
+
+def test_columns(torch_cuda):
+    for ne, nx, nz, npp, nf, waves in [(3, 9, 2, 1, 1, 1), (16, 70, 3, 2, 17, 9), (33, 150, 4, 4, 16, 8), (40, 61, 5, 3, 35, 2)]:
+        for kind in ("single", "multi", "both"):
+            op = OperatorBorn.from_sequence(test_columns_gpu.build(ne, nx, nz, npp, nf, waves, kind))
+            assert op.kernels["columns"] == "fast"
+    _, T = mixed_tiny_tables()      # mixes on subsets of the frequencies
+    assert OperatorBorn.from_tables(T).kernels["columns"] == "gather"
