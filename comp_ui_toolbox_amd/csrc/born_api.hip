@@ -97,6 +97,8 @@ static float2* alloc_p_table(const Plan& P) {
   return d;
 }
 
+static void free_fft_tables(Plan& P);
+
 static void free_workspace(Plan& P) {
   dfree(P.d_chunks);
   dfree(P.d_col_pair);
@@ -119,6 +121,7 @@ static void free_workspace(Plan& P) {
   dfree(P.fft.d_vp);
   dfree(P.fft.d_wt);
   dfree(P.fft.d_gp);
+  P.fft.ok = false;
   P.fwd_expand = false;
   P.fwd_table_expanded = false;
   P.fchunks.clear();
@@ -140,10 +143,7 @@ Plan::~Plan() {
   dfree(na.ls.d_inst);
   dfree(ls.d_inst);
   dfree(ls_fwd.d_inst);
-  dfree(fft.d_H);
-  dfree(fft.d_slot);
-  dfree(fft.d_col);
-  dfree(fft.d_tw);
+  free_fft_tables(*this);
   dfree(fft.set.d_inst);
   dfree(d_ew);
   dfree(d_erow_off);
@@ -442,8 +442,8 @@ static bool use_structured(const Plan& P) { return P.structured && !P.force_gene
 // 2-D structured plans apply both directions by fast lateral correlation in
 // every numeric form (the split forms gain accuracy); the allocation-free
 // apply keeps the MFMA layout.
-static bool fft_on(const Plan& P) { return P.fft.ok && !P.fft.off; }
-static bool use_fft(const Plan& P) { return use_structured(P) && fft_on(P) && !P.in_noalloc; }
+// (P.fft.ok: as of the workspace.)
+static bool use_fft(const Plan& P) { return use_structured(P) && P.fft.ok && !P.in_noalloc; }
 
 // Columns (pair, frequency) by frequency.
 static void upload_fft_columns(Plan& P) {
@@ -452,87 +452,115 @@ static void upload_fft_columns(Plan& P) {
   P.fft.d_col = dupload(col, P.stream);
 }
 
-// The same for 3-D plans whose planes fit (fft3_shape).
-static void build_fft3(Plan& P) {
+// Rows of h_ref that cannot be transformed (k_fft_range), once per plan.
+static void check_rows(Plan& P) {
+  if (P.h_checked) return;
+  int bad = 0;
+  int* d_bad = dupload(std::vector<int>(1, 0), P.stream);
+  launch_fft_range(P, d_bad, P.stream);
+  const hipError_t e = hipGetLastError();
+  const hipError_t e2 = hipMemcpyAsync(&bad, d_bad, sizeof(int), hipMemcpyDeviceToHost, P.stream);
+  const hipError_t e3 = hipStreamSynchronize(P.stream);
+  dfree(d_bad);
+  HIP_CHECK(e);
+  HIP_CHECK(e2);
+  HIP_CHECK(e3);
+  P.h_uneven = bad != 0;
+  P.h_checked = true;
+}
+
+static void free_fft_tables(Plan& P) {
+  dfree(P.fft.d_H);
+  dfree(P.fft.d_slot);
+  dfree(P.fft.d_col);
+  dfree(P.fft.d_tw);
+}
+
+// Whether the plan's workspace is to be that of the fast lateral correlation:
+// a transform that holds its rows or planes, rows of h_ref that can be
+// transformed, and spectra that are there or fit in the free memory with 1 GiB
+// to spare (they take about twice the space of h_ref); the others keep the
+// direct products.
+static bool fft_wanted(Plan& P) {
   Plan::Fft& F = P.fft;
-  F.s3 = fft3_shape(P.Nx, P.Ny, P.Np, P.Npy, P.Nex, P.Ney);
-  if (F.s3.TLX == 0) return;
-  const size_t n = (size_t)P.N_fu * P.Nz * P.Npy * P.Np * fft3_plane(F.s3);
+  if (!P.structured || F.off) return false;
+  if (F.d_H) return true;
+  if (P.N_fu > 65535) return false;   // (grids of the tables' kernels)
+  size_t n = 0;
+  if (P.nd == 3) {
+    F.s3 = fft3_shape(P.Nx, P.Ny, P.Np, P.Npy, P.Nex, P.Ney);
+    if (F.s3.TLX == 0) return false;
+    n = (size_t)P.N_fu * P.Nz * P.Npy * P.Np * fft3_plane(F.s3) * sizeof(float2) + fft3_tmp(P) * sizeof(double2);
+  } else {
+    F.shape = fft_shape(P.Nx, P.Np, P.N_e);
+    if (F.shape.TL == 0) return false;
+    if (((int64_t)P.N_pts + 256ll * P.Np) * 8 > INT32_MAX) return false;   // the forward addresses a row of p_inc by 32-bit byte offsets
+    const int FPW = 64 / F.shape.TL;
+    const int64_t n_slots = (int64_t)P.n_rows * F.shape.nseg * P.Np;
+    if (n_slots > INT32_MAX - 64) return false;
+    F.n_slots = (int)n_slots;
+    F.n_ws = (F.n_slots + FPW - 1) / FPW;
+    n = (size_t)P.N_fu * F.n_ws * 1024 * sizeof(float2);
+  }
+  check_rows(P);
+  if (P.h_uneven) return false;
   size_t free_b = 0, total_b = 0;
   HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
-  if (n * sizeof(float2) + fft3_tmp(P) * sizeof(double2) + ((size_t)1 << 30) > free_b) return;
+  return n + ((size_t)1 << 30) <= free_b;
+}
+
+static void build_fft3_tables(Plan& P) {
+  Plan::Fft& F = P.fft;
   std::vector<float2> tw, twy;
   fft_twiddles(F.s3.TLX, tw);
   fft_twiddles(F.s3.TLY, twy);
   tw.insert(tw.end(), twy.begin(), twy.end());
   upload_fft_columns(P);
   F.d_tw = dupload(tw, P.stream);
-  F.d_H = dalloc<float2>(n);
+  F.d_H = dalloc<float2>((size_t)P.N_fu * P.Nz * P.Npy * P.Np * fft3_plane(F.s3));
   double2* tmp = dalloc<double2>(fft3_tmp(P));
   for (int f = 0; f < P.N_fu; ++f) launch_fft3_table(P, f, tmp, P.stream);
   const hipError_t e = hipStreamSynchronize(P.stream);
   dfree(tmp);
   HIP_CHECK(e);
   HIP_CHECK(hipGetLastError());
-  F.ok = true;
 }
 
-// Tables of the fast lateral correlation, built once per plan: the slots
-// (row, segment, phase), the columns by frequency and the spectra of h_ref.
-// The spectra take about twice the space of h_ref; a plan whose spectra do
-// not fit in the free memory with 1 GiB to spare stays on the MFMA kernels,
-// and so does one whose rows of h_ref are too uneven (k_fft_range).
-static void build_fft(Plan& P) {
+// Tables of the fast lateral correlation, built with a plan's first workspace
+// (a plan that only serves energies, columns or signals has no use for them):
+// the slots (row, segment, phase), the columns by frequency and the spectra of
+// h_ref.
+static void build_fft_tables(Plan& P) {
   Plan::Fft& F = P.fft;
-  F.ok = false;
-  if (!P.structured || P.N_fu > 65535 || (int64_t)P.Nz * P.N_fu > INT32_MAX) return;   // (grids of the tables' kernels)
-  {
-    int bad = 0;
-    int* d_bad = dupload(std::vector<int>(1, 0), P.stream);
-    launch_fft_range(P, d_bad, P.stream);
-    const hipError_t e = hipGetLastError();
-    const hipError_t e2 = hipMemcpyAsync(&bad, d_bad, sizeof(int), hipMemcpyDeviceToHost, P.stream);
-    const hipError_t e3 = hipStreamSynchronize(P.stream);
-    dfree(d_bad);
-    HIP_CHECK(e);
-    HIP_CHECK(e2);
-    HIP_CHECK(e3);
-    P.h_uneven = bad != 0;
-    if (bad) return;
+  if (F.d_H) return;
+  try {
+    if (P.nd == 3) {
+      build_fft3_tables(P);
+      return;
+    }
+    const int FPW = 64 / F.shape.TL;
+    std::vector<int2> slot((size_t)F.n_ws * FPW, make_int2(0, 0));
+    for (int s = 0; s < F.n_slots; ++s) {
+      const int phi = s % P.Np, rs = s / P.Np;
+      const int seg = rs % F.shape.nseg, row = rs / F.shape.nseg;
+      const int first = P.Np * seg * F.shape.Sv + phi;
+      const int left = first < P.Nx ? (P.Nx - first + P.Np - 1) / P.Np : 0;
+      slot[s] = left > 0 ? make_int2(row * P.Nx + first, std::min(left, F.shape.Sv)) : make_int2(0, 0);
+    }
+    std::vector<float2> tw;
+    fft_twiddles(F.shape.TL, tw);
+    F.d_slot = dupload(slot, P.stream);
+    upload_fft_columns(P);
+    F.d_tw = dupload(tw, P.stream);
+    F.d_H = dalloc<float2>((size_t)P.N_fu * F.n_ws * 1024);
+    launch_fft_table(P, P.stream);
+    HIP_CHECK(hipGetLastError());
+    HIP_CHECK(hipStreamSynchronize(P.stream));   // the callers' streams read them
+  } catch (...) {
+    hipStreamSynchronize(P.stream);
+    free_fft_tables(P);
+    throw;
   }
-  if (P.nd == 3) {
-    build_fft3(P);
-    return;
-  }
-  F.shape = fft_shape(P.Nx, P.Np, P.N_e);
-  if (F.shape.TL == 0) return;
-  if (((int64_t)P.N_pts + 256ll * P.Np) * 8 > INT32_MAX) return;   // the forward addresses a row of p_inc by 32-bit byte offsets
-  const int FPW = 64 / F.shape.TL;
-  const int64_t n_slots = (int64_t)P.n_rows * F.shape.nseg * P.Np;
-  if (n_slots > INT32_MAX - 64) return;
-  F.n_slots = (int)n_slots;
-  F.n_ws = (F.n_slots + FPW - 1) / FPW;
-  const size_t n = (size_t)P.N_fu * F.n_ws * 1024;
-  size_t free_b = 0, total_b = 0;
-  HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
-  if (n * sizeof(float2) + ((size_t)1 << 30) > free_b) return;
-  std::vector<int2> slot((size_t)F.n_ws * FPW, make_int2(0, 0));
-  for (int s = 0; s < F.n_slots; ++s) {
-    const int phi = s % P.Np, rs = s / P.Np;
-    const int seg = rs % F.shape.nseg, row = rs / F.shape.nseg;
-    const int first = P.Np * seg * F.shape.Sv + phi;
-    const int left = first < P.Nx ? (P.Nx - first + P.Np - 1) / P.Np : 0;
-    slot[s] = left > 0 ? make_int2(row * P.Nx + first, std::min(left, F.shape.Sv)) : make_int2(0, 0);
-  }
-  std::vector<float2> tw;
-  fft_twiddles(F.shape.TL, tw);
-  F.d_slot = dupload(slot, P.stream);
-  upload_fft_columns(P);
-  F.d_tw = dupload(tw, P.stream);
-  F.d_H = dalloc<float2>(n);
-  launch_fft_table(P, P.stream);
-  HIP_CHECK(hipGetLastError());
-  F.ok = true;
 }
 
 // Column groups of the adjoint: `fill` for the chip, and as many as keep a
@@ -1018,7 +1046,7 @@ static void build_workspace(Plan& P, int N_rhs);
 // could not get its workspace holds none.
 static void ensure_workspace(Plan& P, int N_rhs) {
   const bool split = P.precision != BORN_PRECISION_FP32;
-  if (P.ws_rhs == N_rhs && (N_rhs == 1 || fft_on(P) || P.ws_split == split)) return;
+  if (P.ws_rhs == N_rhs && (N_rhs == 1 || P.fft.ok || P.ws_split == split)) return;
   free_workspace(P);
   P.ws_split = split;
   try {
@@ -1032,12 +1060,14 @@ static void ensure_workspace(Plan& P, int N_rhs) {
 static void build_workspace(Plan& P, int N_rhs) {
   P.chunks.clear();
   P.col_pair.clear();
-  if (fft_on(P)) {   // V, W and the masked input also serve the general path
+  if (fft_wanted(P)) {   // V, W and the masked input also serve the general path
     P.d_V = dalloc<double2>((size_t)P.N_pairs * P.N_e * N_rhs);
     P.d_W = dalloc<float2>((size_t)P.N_pairs * P.N_e * N_rhs);
     P.d_gm = dalloc<float2>((size_t)N_rhs * P.N_pts);
+    build_fft_tables(P);
     build_fft_workspace(P, N_rhs);
     HIP_CHECK(hipDeviceSynchronize());
+    P.fft.ok = true;
     P.ws_rhs = N_rhs;
     ++P.ws_gen;
     return;
@@ -1346,7 +1376,6 @@ static void finish_plan(Plan& P, bool structure_known = false) {
   set_max_lds_split(160 * 1024);
   set_max_lds_split3(160 * 1024);
   set_max_lds_fc(160 * 1024);
-  build_fft(P);
   build_noalloc_layout(P);
   HIP_CHECK(hipStreamSynchronize(P.stream));
 }
@@ -2029,7 +2058,7 @@ static void build_batch_launch(Batch& B) {
   B.slot.assign(B.plans.size(), 0);
   for (size_t i = 0; i < B.plans.size(); ++i) {
     const Plan& P = *B.plans[i];
-    if (fft_on(P)) {
+    if (P.fft.ok) {
       B.set_of[i] = P.nd == 3 ? Batch::SET_3D : -1 - Batch::fft_set(P.fft.shape);
       B.gen.push_back(P.ws_gen);
       continue;
@@ -2495,6 +2524,7 @@ static void ensure_energy_tables(Plan& P) {
 static void energy_rx(Plan& P, int m, double* E_dev, hipStream_t s) {
   if (m < 0 || m >= (int)P.meas_pair_base.size())
     throw Error(BORN_ERR_INVALID_ARGUMENT, "operator_born.indices_measurement_sel must be a single index!");
+  if (use_structured(P)) check_rows(P);
   if (use_structured(P) && energy_fast(P)) {
     ensure_energy_tables(P);
     if (P.e_single[m] || !P.e_multi[m]) launch_energy_single(P, m, E_dev, s);
@@ -2969,6 +2999,7 @@ int born_plan_set_correlation(born_plan_t plan, int32_t on) {
     if (P.fft.off == (on == 0)) return;
     HIP_CHECK(hipDeviceSynchronize());
     free_workspace(P);   // the next call builds that of the other kernels
+    free_fft_tables(P);
     P.fft.off = on == 0;
   });
 }
@@ -2977,8 +3008,11 @@ int born_plan_kernels(born_plan_t plan, int32_t* kernels) {
   return guarded([&] {
     if (!plan || !kernels) throw Error(BORN_ERR_INVALID_ARGUMENT, "plan and output are required");
     Plan& P = *reinterpret_cast<Plan*>(plan);
+    HIP_CHECK(hipSetDevice(P.device));
     const bool st = use_structured(P);
-    kernels[0] = !st ? BORN_KERNELS_GATHER : use_fft(P) ? BORN_KERNELS_FAST : BORN_KERNELS_DIRECT;
+    if (st) check_rows(P);
+    const bool fast = P.ws_rhs > 0 ? P.fft.ok : fft_wanted(P);   // without a workspace: as the next would be
+    kernels[0] = !st ? BORN_KERNELS_GATHER : fast ? BORN_KERNELS_FAST : BORN_KERNELS_DIRECT;
     kernels[1] = st && energy_fast(P) ? BORN_KERNELS_FAST : BORN_KERNELS_GATHER;
     kernels[2] = st && P.tgc_TL > 0 ? BORN_KERNELS_FAST : BORN_KERNELS_GATHER;
     kernels[3] = st && columns_fast(P) ? BORN_KERNELS_FAST : BORN_KERNELS_GATHER;

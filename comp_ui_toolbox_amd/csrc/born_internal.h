@@ -239,7 +239,8 @@ struct Plan {
   int2* d_pe_ent = nullptr;       // (observation, prefactor index)
   int64_t n_pe_ent = 0;
   bool single_mixes = false;      // every mix has one active element
-  bool h_uneven = false;          // a row of h_ref that is not finite or lies in one entry (k_fft_range)
+  bool h_checked = false;
+  bool h_uneven = false;          // a row of h_ref that is not finite or lies in one entry (k_fft_range, check_rows)
   std::vector<int> h_shift;       // host copy of the 0-based shift map [N_e][N_pts]
 
   // per-N_rhs workspace
@@ -265,9 +266,10 @@ struct Plan {
   float2* d_gm = nullptr;         // masked gamma [N_rhs][N_pts]
   int items_target = 8192;        // forward work items per launch (tunable)
   LaunchSet ls;                   // structured launch of this plan alone
-  // fast lateral correlation: tables of the plan, then the per-rhs workspace
+  // fast lateral correlation: tables, built with the first workspace (d_H null: not yet),
+  // then the per-rhs workspace
   struct Fft {
-    bool ok = false;
+    bool ok = false;                // the workspace is that of the fast correlation
     bool off = false;               // switched off by the caller
     FftShapeChoice shape;
     Fft3Choice s3;                  // 3-D plans

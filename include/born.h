@@ -310,7 +310,8 @@ int born_plan_force_general(born_plan_t plan, int32_t on);
 int born_plan_set_correlation(born_plan_t plan, int32_t on);
 
 /* Which kernels a plan's calls take: kernels[0] forward and adjoint, [1]
- * received energies, [2] those under time gain, [3] columns. */
+ * received energies, [2] those under time gain, [3] columns.  [0] is that of
+ * the workspace of the last call, or what the first call would get. */
 enum born_kernels {
     BORN_KERNELS_GATHER = 0,     /* by the shift map, any plan                      */
     BORN_KERNELS_DIRECT = 1,     /* products on the lateral structure (born_precision) */
