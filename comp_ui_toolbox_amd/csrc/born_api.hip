@@ -99,6 +99,14 @@ static float2* alloc_p_table(const Plan& P) {
 
 static void free_fft_tables(Plan& P);
 
+static void free_fft_workspace(Plan& P) {
+  dfree(P.fft.d_gs);
+  dfree(P.fft.d_vp);
+  dfree(P.fft.d_wt);
+  dfree(P.fft.d_gp);
+  P.fft.ok = false;
+}
+
 static void free_workspace(Plan& P) {
   dfree(P.d_chunks);
   dfree(P.d_col_pair);
@@ -117,11 +125,7 @@ static void free_workspace(Plan& P) {
   dfree(P.d_pexp);
   dfree(P.d_ones);
   dfree(P.d_fvpart);
-  dfree(P.fft.d_gs);
-  dfree(P.fft.d_vp);
-  dfree(P.fft.d_wt);
-  dfree(P.fft.d_gp);
-  P.fft.ok = false;
+  free_fft_workspace(P);
   P.fwd_expand = false;
   P.fwd_table_expanded = false;
   P.fchunks.clear();
@@ -633,7 +637,7 @@ static void finalize_fft_set(FftSet& S) {
     f += ((int64_t)I.n_cols * I.N_rhs * I.NZB + 3) / 4;
     I.wg_a = (int)a;
     a += (int64_t)I.n_ws * I.N_rhs * I.FG;
-    if (f > INT32_MAX - 64 || a > INT32_MAX - 64)
+    if (std::max(f, a) > (1 << 24) - 1 - XCDS)   // (2^32 threads)
       throw Error(BORN_ERR_UNSUPPORTED, "too many right-hand sides for one launch");
   }
   S.n_wg_f = (int)f;
@@ -653,7 +657,7 @@ static void build_fft3_workspace(Plan& P, int N_rhs) {
   F.NZB = (P.Nz + F.ZR - 1) / F.ZR;
   const int64_t wg = (int64_t)P.Nz * P.Npy * (P.Np / F.s3.px) * N_rhs;
   F.FG = adj_groups(P, N_rhs, std::min<int64_t>({(2048 + wg - 1) / wg, P.N_pairs / 8, 64}), 64);
-  if (cols * F.NZB > INT32_MAX - 64 || wg * F.FG > INT32_MAX - 64)
+  if (std::max(cols * F.NZB, wg * F.FG) > (1 << 23) - 1 - XCDS)   // (2^32 threads, up to 512 each)
     throw Error(BORN_ERR_UNSUPPORTED, "too many right-hand sides for one launch");
   F.d_vp = dalloc<float2>((size_t)F.NZB * cols * P.N_e);
   F.d_wt = dalloc<float2>((size_t)cols * fft3_plane(F.s3));
@@ -1040,32 +1044,58 @@ static void setup_column_rhs_adjoint(Plan& P, int N_rhs) {
 }
 
 // Chunks of <= NC (pair, rhs) columns per frequency, rhs-major.
-static void build_workspace(Plan& P, int N_rhs);
+static void build_workspace(Plan& P, int N_rhs, bool fft);
+static bool no_room(const Error& e) { return e.status == BORN_ERR_OUT_OF_MEMORY || e.status == BORN_ERR_UNSUPPORTED; }
 
 // A failure while building frees the partial workspace, so a plan that
-// could not get its workspace holds none.
+// could not get its workspace holds none.  Where the memory that the spectra
+// hold is what is missing, the workspace of the direct products takes its place.
 static void ensure_workspace(Plan& P, int N_rhs) {
   const bool split = P.precision != BORN_PRECISION_FP32;
   if (P.ws_rhs == N_rhs && (N_rhs == 1 || P.fft.ok || P.ws_split == split)) return;
   free_workspace(P);
   P.ws_split = split;
   try {
-    build_workspace(P, N_rhs);
+    build_workspace(P, N_rhs, fft_wanted(P));
+  } catch (const Error& e) {
+    free_workspace(P);
+    if (!P.fft.d_H || !no_room(e)) throw;
+    free_fft_tables(P);
+    try {
+      build_workspace(P, N_rhs, false);
+    } catch (...) {
+      free_workspace(P);
+      throw;
+    }
   } catch (...) {
     free_workspace(P);
     throw;
   }
 }
 
-static void build_workspace(Plan& P, int N_rhs) {
-  P.chunks.clear();
-  P.col_pair.clear();
-  if (fft_wanted(P)) {   // V, W and the masked input also serve the general path
-    P.d_V = dalloc<double2>((size_t)P.N_pairs * P.N_e * N_rhs);
-    P.d_W = dalloc<float2>((size_t)P.N_pairs * P.N_e * N_rhs);
-    P.d_gm = dalloc<float2>((size_t)N_rhs * P.N_pts);
+// The workspace of the fast correlation; false where there is no room for it
+// (memory, or a launch's limits) and nothing of it is left.
+static bool try_fft_workspace(Plan& P, int N_rhs) {
+  try {
     build_fft_tables(P);
     build_fft_workspace(P, N_rhs);
+    return true;
+  } catch (const Error& e) {
+    if (!no_room(e)) throw;
+  }
+  free_fft_workspace(P);
+  free_fft_tables(P);
+  return false;
+}
+
+static void build_workspace(Plan& P, int N_rhs, bool fft) {
+  P.chunks.clear();
+  P.col_pair.clear();
+  // V, W and the masked input, of all paths
+  P.d_V = dalloc<double2>((size_t)P.N_pairs * P.N_e * N_rhs);
+  P.d_W = dalloc<float2>((size_t)P.N_pairs * P.N_e * N_rhs);
+  P.d_gm = dalloc<float2>((size_t)N_rhs * P.N_pts);
+  if (fft && try_fft_workspace(P, N_rhs)) {
     HIP_CHECK(hipDeviceSynchronize());
     P.fft.ok = true;
     P.ws_rhs = N_rhs;
@@ -1102,14 +1132,11 @@ static void build_workspace(Plan& P, int N_rhs) {
   P.d_pr_chunk = dupload(pr_chunk, P.stream);
   P.d_pr_pos = dupload(pr_pos, P.stream);
   if (P.structured) P.d_vpart = dalloc<float2>((size_t)n_chunks * P.vblk * P.Ne_pad * NC);
-  P.d_V = dalloc<double2>((size_t)P.N_pairs * P.N_e * N_rhs);
-  P.d_W = dalloc<float2>((size_t)P.N_pairs * P.N_e * N_rhs);
   if (P.structured) {
     const size_t n = (size_t)n_chunks * (P.nd == 3 ? P.Ney : 1) * P.Ne_pad * NC;
     P.d_Wc = dalloc<float2>(n);
     HIP_CHECK(hipMemset(P.d_Wc, 0, n * sizeof(float2)));  // padding columns/elements stay zero
   }
-  P.d_gm = dalloc<float2>((size_t)N_rhs * P.N_pts);
   // partial sums of the few-column adjoint (plans with at most 4 pairs per frequency)
   int ppf = 0;
   for (int fg = 0; fg < P.N_fu; ++fg) ppf = std::max(ppf, P.fg_pair_off[fg + 1] - P.fg_pair_off[fg]);
