@@ -42,8 +42,10 @@ namespace born {
 
 // ------------------------------------------------------------------ spectra
 // H[f][slot] (FP64 transform of the FP32 row, conjugated twice for the
-// exponent's sign) and the layout its readers take: per group of FPW slots
-// [8][64 lanes][2] entries, so that a lane reads two entries at once.
+// exponent's sign, divided by L: the inverse transforms of both directions need
+// no other factor, and products and sums keep the range of the direct form's)
+// and the layout its readers take: per group of FPW slots [8][64 lanes][2]
+// entries, so that a lane reads two entries at once.
 template <int TL>
 __global__ __launch_bounds__(64) void k_fft_table(const float2* __restrict__ h, const int* __restrict__ ext,
                                                   const int* __restrict__ hrow, int H_plane, int HR, int N_ext, int Np,
@@ -70,7 +72,7 @@ __global__ __launch_bounds__(64) void k_fft_table(const float2* __restrict__ h, 
     x[q] = {0.0, 0.0};
     if (ok && t < N_ext) {
       const float2 v = src[ext[t]];
-      x[q] = {(double)v.x, -(double)v.y};
+      x[q] = {(double)v.x / L, -(double)v.y / L};
     }
   }
   fft_wave<double, TL, false>(x, tw, lds, lane);
@@ -198,7 +200,7 @@ __global__ __launch_bounds__(256) void k_fft_gamma(const float2* __restrict__ gm
 template <int TL, int NZ, int NP>
 __global__ __launch_bounds__(256, 2) void k_fft_fwd(const FftInst* __restrict__ inst, int n_inst,
                                                     const float2* __restrict__ twid, int n_wg, int per) {
-  constexpr int FPW = FftShape<TL>::FPW, L = 16 * TL;
+  constexpr int FPW = FftShape<TL>::FPW;
   __shared__ cf lds_all[4 * FftShape<TL>::LDS];
   __shared__ cf twl[16 * TL];
   load_twiddles_lds<TL>(twid, twl);
@@ -277,7 +279,7 @@ __global__ __launch_bounds__(256, 2) void k_fft_fwd(const FftInst* __restrict__ 
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
       const int t = j + TL * q;
-      if (t < I.N_e) out[I.N_e - 1 - t] = make_float2(G[q].x * (1.f / L), G[q].y * (1.f / L));
+      if (t < I.N_e) out[I.N_e - 1 - t] = make_float2(G[q].x, G[q].y);
     }
   }
 }
@@ -341,7 +343,7 @@ struct alignas(8) Ent4 {
 };
 
 // Un-mixing (as k_adj_unmix) and the spectra of the weights: a wave takes FPW
-// (pair, right-hand side) rows, entry t = N_e - 1 - e holds conj(W[e]) / L.
+// (pair, right-hand side) rows, entry t = N_e - 1 - e holds conj(W[e]).
 // wt[row][8][TL lanes][2].
 template <int TL, bool LONG>
 __global__ __launch_bounds__(256) void k_fft_weights(const float2* __restrict__ u, const int64_t* __restrict__ pe_off,
@@ -432,7 +434,7 @@ __global__ __launch_bounds__(256) void k_fft_weights(const float2* __restrict__ 
         }
     }
 #pragma unroll
-    for (int q = 0; q < QB; ++q) x[QB * h + q] = {(float)sx[q] * (1.f / L), -(float)sy[q] * (1.f / L)};
+    for (int q = 0; q < QB; ++q) x[QB * h + q] = {(float)sx[q], -(float)sy[q]};
   }
   fft_wave<float, TL, false>(x, tw, lds_all + wave * FftShape<TL>::LDS, lane);
   if (!ok) return;

@@ -44,8 +44,8 @@ struct Fft3Shape {
 };
 
 // ------------------------------------------------------------------ spectra
-// x transforms (FP64) of the rows m_y of every phase, one frequency:
-// tmp[z][phi_y][phi_x][m_y][k_x].
+// x transforms (FP64) of the rows m_y of every phase, divided by Lx Ly, one
+// frequency: tmp[z][phi_y][phi_x][m_y][k_x].
 template <int TLX>
 __global__ __launch_bounds__(64) void k_fft3_table_x(const float2* __restrict__ h, const int* __restrict__ ext,
                                                      const int* __restrict__ exty, int HR, int HY, int N_ext, int N_exty,
@@ -71,13 +71,14 @@ __global__ __launch_bounds__(64) void k_fft3_table_x(const float2* __restrict__ 
   const int ty = Npy * my + phy;
   const bool have = on && ty < N_exty;
   const float2* src = h + (have ? ((int64_t)exty[ty] + HY * z) * HR : 0);
+  const double scale = 1.0 / ((double)L * Ly);
 #pragma unroll
   for (int q = 0; q < 16; ++q) {
     const int tx = Npx * (j + TLX * q) + phx;
     x[q] = {0.0, 0.0};
     if (have && tx < N_ext) {
       const float2 v = src[ext[tx]];
-      x[q] = {(double)v.x, -(double)v.y};   // conjugated twice for the exponent's sign
+      x[q] = {v.x * scale, -v.y * scale};   // conjugated twice for the exponent's sign
     }
   }
   fft_wave<double, TLX, false>(x, tw, lds, lane);
@@ -241,7 +242,6 @@ __global__ __launch_bounds__((64 * Fft3Shape<TLX, TLY>::W), 2) void k_fft3_fwd(F
     }
   }
   __syncthreads();
-  const float scale = 1.f / (S::LX * S::LY);
   float2* out = A.vp + ((size_t)(zb * A.N_rhs + r) * A.n_cols + c) * A.N_e;
   for (int s0 = wave * S::FPWX; s0 < A.Ney; s0 += S::W * S::FPWX) {
     const int ty = s0 + gx;
@@ -256,7 +256,7 @@ __global__ __launch_bounds__((64 * Fft3Shape<TLX, TLY>::W), 2) void k_fft3_fwd(F
 #pragma unroll
       for (int q = 0; q < 16; ++q) {
         const int tx = jx + TLX * q;
-        if (tx < A.Nex) out[(A.Ney - 1 - ty) * A.Nex + A.Nex - 1 - tx] = make_float2(x[q].x * scale, x[q].y * scale);
+        if (tx < A.Nex) out[(A.Ney - 1 - ty) * A.Nex + A.Nex - 1 - tx] = make_float2(x[q].x, x[q].y);
       }
     }
   }
@@ -264,7 +264,7 @@ __global__ __launch_bounds__((64 * Fft3Shape<TLX, TLY>::W), 2) void k_fft3_fwd(F
 
 // ------------------------------------------------------------------ adjoint
 // Spectra of the un-mixed weights (d_W) of one (pair, right-hand side) per
-// workgroup: conj(W) / (Lx Ly) at t, wt[row][k_x / FPWY][8][64 lanes][2].
+// workgroup: conj(W) at t, wt[row][k_x / FPWY][8][64 lanes][2].
 template <int TLX, int TLY>
 __global__ __launch_bounds__((64 * Fft3Shape<TLX, TLY>::W)) void k_fft3_weights(Fft3Args A, const float2* __restrict__ Wt,
                                                                              float2* __restrict__ wt) {
@@ -279,7 +279,6 @@ __global__ __launch_bounds__((64 * Fft3Shape<TLX, TLY>::W)) void k_fft3_weights(
   const float2* src = Wt + pair * A.N_e * A.N_rhs + r;
   cf tw[16];
   load_twiddles<TLX>(A.twx, jx, tw);
-  const float scale = 1.f / (S::LX * S::LY);
   for (int s0 = wave * S::FPWX; s0 < A.Ney; s0 += S::W * S::FPWX) {
     const int ty = s0 + gx;
     cf x[16];
@@ -289,7 +288,7 @@ __global__ __launch_bounds__((64 * Fft3Shape<TLX, TLY>::W)) void k_fft3_weights(
       x[q] = {0.f, 0.f};
       if (ty < A.Ney && tx < A.Nex) {
         const float2 v = src[(size_t)((A.Ney - 1 - ty) * A.Nex + A.Nex - 1 - tx) * A.N_rhs];
-        x[q] = {v.x * scale, -v.y * scale};
+        x[q] = {v.x, -v.y};
       }
     }
     fft_wave<float, TLX, false>(x, tw, lds, lane);

@@ -38,3 +38,32 @@ def test_adjoint_of_many_columns(torch_cuda, three):
         e = O.rel_l2(g[r].cpu().numpy(), ref)
         print(f"three={three} rhs {r}: {e:.2e}", flush=True)
         assert e < (4.5e-7 if three else 4.2e-7)
+
+
+@pytest.mark.parametrize("three", [False, True])
+def test_small_weights(torch_cuda, three):
+    """Weights just above FP32's smallest normal number, tables that bring the
+    products back: the result is that of larger weights times their ratio.  A
+    factor 1 / L on the weights made them subnormal, 2^-19 (2^-15 in planes)
+    off; their own rounding there is 2^-150 of 2^-122."""
+    import torch
+    if three:
+        arr = C.ArraySpec((4, 3), (3e-4, 3e-4), (2.7e-4, 2.7e-4), (1, 1))
+        fov = C.FovSpec((19, 7, 3), (1.5e-4,) * 3, 3e-3)
+    else:
+        arr = C.ArraySpec((100,), (3e-4,), (2.7e-4,), (2,))
+        fov = C.FovSpec((301, 4), (1.5e-4,) * 2, 2e-3)
+    rng = np.random.Generator(np.random.PCG64(5))
+    ws = [C.random_wave(arr, rng, 1e-6) for _ in range(2)]
+    spec = C.SequenceSpec("w", arr, C.MediumSpec(), fov, np.linspace(2e6, 4e6, 3), ws,
+                          [C.identity_mixes(arr.N_elements) for _ in ws])
+    T = O.build_tables(spec)
+    T.h_ref = T.h_ref * 2.0 ** 80
+    for m in T.meas:
+        for x in m.mixes:
+            x.prefactors = np.ones_like(x.prefactors)
+    op = OperatorBorn.from_tables(T)
+    assert op.kernels["pair"] == "fast"
+    u = torch.view_as_complex(torch.tensor(rng.integers(1, 9, (op.N_observations, 2)).astype(np.float32), device="cuda:0"))
+    large, small = op.adjoint_dev(u), op.adjoint_dev(u * 2.0 ** -122)
+    assert float((small.to(torch.complex128) * 2.0 ** 122 - large).norm() / large.norm()) < 2.0 ** -24
