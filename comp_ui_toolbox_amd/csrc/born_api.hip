@@ -456,21 +456,17 @@ static void upload_fft_columns(Plan& P) {
   P.fft.d_col = dupload(col, P.stream);
 }
 
-// Rows of h_ref that cannot be transformed (k_fft_range), once per plan.
+// Rows of h_ref that are not finite or may not be transformed (k_fft_range).
 static void check_rows(Plan& P) {
-  if (P.h_checked) return;
-  int bad = 0;
-  int* d_bad = dupload(std::vector<int>(1, 0), P.stream);
-  launch_fft_range(P, d_bad, P.stream);
-  const hipError_t e = hipGetLastError();
-  const hipError_t e2 = hipMemcpyAsync(&bad, d_bad, sizeof(int), hipMemcpyDeviceToHost, P.stream);
-  const hipError_t e3 = hipStreamSynchronize(P.stream);
-  dfree(d_bad);
-  HIP_CHECK(e);
-  HIP_CHECK(e2);
-  HIP_CHECK(e3);
-  P.h_uneven = bad != 0;
-  P.h_checked = true;
+  if (!P.structured) return;
+  int* flag = reinterpret_cast<int*>(P.d_f16part), bad = 0;   // (scratch of the operand scales)
+  HIP_CHECK(hipMemcpyAsync(flag, &bad, sizeof(int), hipMemcpyHostToDevice, P.stream));
+  launch_fft_range(P, flag, P.stream);
+  HIP_CHECK(hipGetLastError());
+  HIP_CHECK(hipMemcpyAsync(&bad, flag, sizeof(int), hipMemcpyDeviceToHost, P.stream));
+  HIP_CHECK(hipStreamSynchronize(P.stream));
+  P.h_odd = bad & 1;
+  P.h_uneven = bad & 2;
 }
 
 static void free_fft_tables(Plan& P) {
@@ -506,7 +502,6 @@ static bool fft_wanted(Plan& P) {
     F.n_ws = (F.n_slots + FPW - 1) / FPW;
     n = (size_t)P.N_fu * F.n_ws * 1024 * sizeof(float2);
   }
-  check_rows(P);
   if (P.h_uneven) return false;
   size_t free_b = 0, total_b = 0;
   HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
@@ -1403,6 +1398,7 @@ static void finish_plan(Plan& P, bool structure_known = false) {
   set_max_lds_split(160 * 1024);
   set_max_lds_split3(160 * 1024);
   set_max_lds_fc(160 * 1024);
+  check_rows(P);
   build_noalloc_layout(P);
   HIP_CHECK(hipStreamSynchronize(P.stream));
 }
@@ -2551,7 +2547,6 @@ static void ensure_energy_tables(Plan& P) {
 static void energy_rx(Plan& P, int m, double* E_dev, hipStream_t s) {
   if (m < 0 || m >= (int)P.meas_pair_base.size())
     throw Error(BORN_ERR_INVALID_ARGUMENT, "operator_born.indices_measurement_sel must be a single index!");
-  if (use_structured(P)) check_rows(P);
   if (use_structured(P) && energy_fast(P)) {
     ensure_energy_tables(P);
     if (P.e_single[m] || !P.e_multi[m]) launch_energy_single(P, m, E_dev, s);
@@ -3037,7 +3032,6 @@ int born_plan_kernels(born_plan_t plan, int32_t* kernels) {
     Plan& P = *reinterpret_cast<Plan*>(plan);
     HIP_CHECK(hipSetDevice(P.device));
     const bool st = use_structured(P);
-    if (st) check_rows(P);
     const bool fast = P.ws_rhs > 0 ? P.fft.ok : fft_wanted(P);   // without a workspace: as the next would be
     kernels[0] = !st ? BORN_KERNELS_GATHER : fast ? BORN_KERNELS_FAST : BORN_KERNELS_DIRECT;
     kernels[1] = st && energy_fast(P) ? BORN_KERNELS_FAST : BORN_KERNELS_GATHER;

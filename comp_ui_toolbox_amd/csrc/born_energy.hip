@@ -564,7 +564,7 @@ static EnergyArgs energy_args(const Plan& P, int m, int R) {
 // per pitch, and a window of 4 points per lane within one wave's share of LDS.
 // Their windows meet padding weights of 0 past the elements, which a table
 // entry that is not finite would carry to points that do not see it.
-bool energy_fast(const Plan& P) { return P.structured && P.Np <= 64 && !P.h_uneven; }
+bool energy_fast(const Plan& P) { return P.structured && P.Np <= 64 && !P.h_odd; }
 
 // Waves per workgroup: 4, up to 16 while the launch has fewer than 4096 waves.
 static int energy_waves(int wgs, size_t lds_per_wave, int most) {

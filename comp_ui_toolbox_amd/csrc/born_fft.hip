@@ -83,63 +83,100 @@ __global__ __launch_bounds__(64) void k_fft_table(const float2* __restrict__ h, 
 }
 
 // Whether the lateral rows (2-D) or planes (3-D) of h_ref may be transformed.
-// A transform spreads the rounding of a row's norm over all its entries, where
-// the direct products keep that of an entry to itself.  A field's row has its
-// norm in a main lobe of many entries.  One that has it in a single entry (a
-// grid point next to an element) would lose the others: bad is set for a row
-// whose largest entry is not finite, or holds more than a quarter of the row's
-// energy and exceeds the geometric mean of the nonzero entries 16 times (rows
-// of few entries reach the first by themselves).  In volumes the entry in
-// front of an element has 1/8 of its plane's energy at half a grid spacing and
-// 1/4 at a third of one; in 2-D it stays below.  One block per (row or plane, frequency).
+// A transform spreads the rounding of the whole sequence over all its outputs,
+// where the direct products keep that of an entry to itself.  A field's row has
+// its norm in a main lobe of many entries.  One that has it in one (a grid
+// point next to an element, entries of another scale) would lose the others.
+// *bad gets bit 0 for a row with an entry that is not finite, and bit 1 for one
+//   - whose largest entry holds more than a quarter of the row's energy and
+//     exceeds the geometric mean of the nonzero entries 16 times (rows of few
+//     entries reach the first by themselves): in volumes the entry in front of
+//     an element has 1/8 of its plane's energy at half a grid spacing and 1/4 at
+//     a third of one, in 2-D it stays below;
+//   - one of whose phases, the sequences that are transformed, has more than
+//     1/16 of its energy in one entry and more than half of the nonzero ones, 8 at
+//     least, 2^32 times below that (a lobe of a few entries in every phase, which
+//     holds less of the row).  Sharper rules meet ordinary fields: a receive filter
+//     leaves rows of three or four entries close to the array, and where its edge
+//     falls on grazing angles (half a wavelength per pitch) all beyond 11 times the
+//     depth is 2^32 times below the lobe, which has 1/32 in one entry at 2 mm and
+//     1/16 at 1 mm;
+//   - whose entries all lie below 2^-100 (spectra divided by the length would
+//     become subnormal).
 __global__ __launch_bounds__(256) void k_fft_range(const float2* __restrict__ h, const int* __restrict__ ext,
                                                    const int* __restrict__ exty, int N_ext, int ny, int H_plane, int HR,
-                                                   int HY, int Nz, int* __restrict__ bad) {
-  __shared__ float red[3][256];
-  const int tid = threadIdx.x;
-  const float2* src = h + (size_t)(blockIdx.x / Nz) * H_plane + (size_t)(blockIdx.x % Nz) * HY * HR;
-  const int n = N_ext * ny;
-  auto entry = [&](int i) { return src[(exty ? (size_t)exty[i / N_ext] * HR : 0) + ext[i % N_ext]]; };
-  float top = 0.f;
-  bool fine = true;
-  for (int i = tid; i < n; i += 256) {
-    const float2 v = entry(i);
-    fine = fine && fabsf(v.x) < 1e30f && fabsf(v.y) < 1e30f;   // (false for NaN)
-    top = fmaxf(top, fmaxf(fabsf(v.x), fabsf(v.y)));
-  }
-  red[0][tid] = fine ? top : 2e30f;
-  __syncthreads();
-  for (int k = 128; k > 0; k >>= 1) {
-    if (tid < k) red[0][tid] = fmaxf(red[0][tid], red[0][tid + k]);
+                                                   int HY, int Nz, int Npx, int Npy, int64_t n_rows,
+                                                   int* __restrict__ bad) {
+  __shared__ float red[3][4];
+  const int tid = threadIdx.x, wave = tid >> 6;
+  auto reduce = [&](float& a, float& b, float& c, bool largest) {   // over the block, in all threads
     __syncthreads();
-  }
-  top = red[0][0];
-  __syncthreads();
-  float peak = 0.f, energy = 0.f, logs = 0.f, count = 0.f;
-  if (top > 0.f && top < 1e30f)
-    for (int i = tid; i < n; i += 256) {
-      const float2 v = entry(i);
-      const float x = v.x / top, y = v.y / top, m = x * x + y * y;
-      peak = fmaxf(peak, m);
-      energy += m;
-      if (m > 0.f) {
-        logs += log2f(m);
-        count += 1.f;
-      }
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) {
+      a = largest ? fmaxf(a, __shfl_xor(a, m)) : a + __shfl_xor(a, m);
+      b += __shfl_xor(b, m);
+      c += __shfl_xor(c, m);
     }
-  red[0][tid] = energy;
-  red[1][tid] = logs;
-  red[2][tid] = count;
-  __syncthreads();
-  for (int k = 128; k > 0; k >>= 1) {
-    if (tid < k)
-      for (int a = 0; a < 3; ++a) red[a][tid] += red[a][tid + k];
+    if ((tid & 63) == 0) {
+      red[0][wave] = a;
+      red[1][wave] = b;
+      red[2][wave] = c;
+    }
     __syncthreads();
+    a = largest ? fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3])) : red[0][0] + red[0][1] + red[0][2] + red[0][3];
+    b = red[1][0] + red[1][1] + red[1][2] + red[1][3];
+    c = red[2][0] + red[2][1] + red[2][2] + red[2][3];
+  };
+  for (int64_t row = blockIdx.x; row < n_rows; row += gridDim.x) {
+    const float2* src = h + (size_t)(row / Nz) * H_plane + (size_t)(row % Nz) * HY * HR;
+    auto entry = [&](int ty, int tx) { return src[(exty ? (size_t)exty[ty] * HR : 0) + ext[tx]]; };
+    float top = 0.f, odd = 0.f, none = 0.f;
+    for (int i = tid; i < N_ext * ny; i += 256) {
+      const float2 v = entry(i / N_ext, i % N_ext);
+      if (!(fabsf(v.x) < 1e30f && fabsf(v.y) < 1e30f)) odd = 1.f;   // (NaN among them)
+      else top = fmaxf(top, fmaxf(fabsf(v.x), fabsf(v.y)));
+    }
+    reduce(top, odd, none, true);
+    if (odd > 0.f) {
+      if (tid == 0) atomicOr(bad, 3);
+      continue;
+    }
+    if (top == 0.f) continue;
+    bool uneven = top < 0x1p-100f;
+    float peak = 0.f, energy = 0.f, logs = 0.f, count = 0.f;
+    for (int ph = 0; ph < Npx * Npy; ++ph) {
+      const int px = ph % Npx, py = ph / Npx, nx = (N_ext - px + Npx - 1) / Npx, m = nx * ((ny - py + Npy - 1) / Npy);
+      float e = 0.f, l = 0.f, n = 0.f, first = 0.f;
+      for (int i = tid; i < m; i += 256) {
+        const float2 v = entry(py + Npy * (i / nx), px + Npx * (i % nx));
+        const float x = v.x / top, y = v.y / top, q = x * x + y * y;
+        first = fmaxf(first, q);
+        e += q;
+        if (q > 0.f) {
+          l += log2f(q);
+          n += 1.f;
+        }
+      }
+      reduce(e, l, n, false);
+      reduce(first, none, none, true);
+      peak = fmaxf(peak, first);
+      if (16.f * first > e) {
+        float low = 0.f;
+        for (int i = tid; i < m; i += 256) {
+          const float2 v = entry(py + Npy * (i / nx), px + Npx * (i % nx));
+          const float x = v.x / top, y = v.y / top, q = x * x + y * y;
+          if (q > 0.f && q * 0x1p32f < first) low += 1.f;
+        }
+        reduce(low, none, none, false);
+        if (low >= 8.f && 2.f * low > n) uneven = true;
+      }
+      energy += e;
+      logs += l;
+      count += n;
+    }
+    if (peak > 0.25f * energy && log2f(peak) - logs / count > 8.f) uneven = true;   // (of squares)
+    if (uneven && tid == 0) atomicOr(bad, 2);
   }
-  energy = red[0][0];
-  const float mean = red[1][0] / fmaxf(red[2][0], 1.f);
-  const bool uneven = peak > 0.25f * energy && log2f(peak) - mean > 8.f;   // (of squares)
-  if (uneven || top >= 1e30f) atomicOr(bad, 1);
 }
 
 // ------------------------------------------------------------------ forward
@@ -624,9 +661,10 @@ void launch_fft_table(const Plan& P, hipStream_t s) {
 
 void launch_fft_range(const Plan& P, int* bad, hipStream_t s) {
   const bool y = P.nd == 3;
-  hipLaunchKernelGGL(k_fft_range, dim3((unsigned)P.Nz * (unsigned)P.N_fu), dim3(256), 0, s, P.d_h, P.d_ext,
+  const int64_t rows = (int64_t)P.Nz * P.N_fu;
+  hipLaunchKernelGGL(k_fft_range, dim3((unsigned)std::min<int64_t>(rows, 1 << 20)), dim3(256), 0, s, P.d_h, P.d_ext,
                      y ? P.d_exty : nullptr, P.N_ext, y ? P.Ny + (P.Ney - 1) * P.Npy : 1, P.H_plane, P.HR, P.HY, P.Nz,
-                     bad);
+                     P.Np, y ? P.Npy : 1, rows, bad);
 }
 
 void launch_fft_gamma(const Plan& P, const float2* gamma, int N_rhs, bool mask, hipStream_t s) {

@@ -239,8 +239,8 @@ struct Plan {
   int2* d_pe_ent = nullptr;       // (observation, prefactor index)
   int64_t n_pe_ent = 0;
   bool single_mixes = false;      // every mix has one active element
-  bool h_checked = false;
-  bool h_uneven = false;          // a row of h_ref that is not finite or lies in one entry (k_fft_range, check_rows)
+  bool h_odd = false;             // structured plans: an entry of h_ref that is not finite,
+  bool h_uneven = false;          // a row of it that may not be transformed (k_fft_range)
   std::vector<int> h_shift;       // host copy of the 0-based shift map [N_e][N_pts]
 
   // per-N_rhs workspace

@@ -67,3 +67,42 @@ def test_small_weights(torch_cuda, three):
     u = torch.view_as_complex(torch.tensor(rng.integers(1, 9, (op.N_observations, 2)).astype(np.float32), device="cuda:0"))
     large, small = op.adjoint_dev(u), op.adjoint_dev(u * 2.0 ** -122)
     assert float((small.to(torch.complex128) * 2.0 ** 122 - large).norm() / large.norm()) < 2.0 ** -24
+
+
+@pytest.mark.parametrize("three", [False, True])
+@pytest.mark.parametrize("width", [1, 5])
+def test_lobes_of_another_scale(torch_cuda, three, width):
+    """Adjacent entries of h_ref 10^7 times the others, less than a quarter of
+    the row's energy each: the plan keeps the direct products, whose FP32 error
+    (5e-7) the points and images without these entries keep; its energies,
+    sums in FP64, keep the fast kernels (2e-12 of the general ones, as for
+    tables without such entries)."""
+    if three:
+        arr = C.ArraySpec((4, 3), (3e-4, 3e-4), (2.7e-4, 2.7e-4), (2, 2))
+        fov = C.FovSpec((19, 7, 3) if width == 1 else (40, 21, 2), (1.5e-4,) * 3, 3e-3)
+    else:
+        arr = C.ArraySpec((33,), (3e-4,), (2.7e-4,), (2,))
+        fov = C.FovSpec((101, 6), (1e-4,) * 2, 2e-3)
+    rng = np.random.Generator(np.random.PCG64(9))
+    ws = [C.random_wave(arr, rng, 1e-6) for _ in range(2)]
+    spec = C.SequenceSpec("lobe", arr, C.MediumSpec(), fov, np.linspace(2e6, 6e6, 3), ws,
+                          [C.identity_mixes(arr.N_elements) for _ in ws])
+    T = O.build_tables(spec)
+    nx = fov.N_points_axis[0]
+    at = T.N_points // 2 // nx * nx + nx // 2 + np.arange(width)
+    touched = np.any(np.isin(np.asarray(T.shift).reshape(T.N_points, -1) - 1, at), axis=1)
+    assert touched.any() and not touched.all()
+    clean = T.h_ref.copy()
+    T.h_ref[1, at] = 1e7
+    op = OperatorBorn.from_tables(T)
+    assert op.kernels == {"pair": "direct", "energy": "fast", "energy_tgc": "gather", "columns": "fast"}
+    u = rng.standard_normal(op.N_observations) + 1j * rng.standard_normal(op.N_observations)
+    g = rng.standard_normal(op.N_points) + 1j * rng.standard_normal(op.N_points)
+    g[touched] = 0
+    back, forth, energy = op.adjoint(u), op.forward(g), op.energy_rx(1)
+    op.force_general(True)
+    general = op.energy_rx(1)
+    assert np.max(np.abs(energy - general) / general) < 2e-12
+    T.h_ref = clean
+    assert O.rel_l2(back[~touched], O.adjoint(T, u).reshape(-1)[~touched]) < 1e-6
+    assert O.rel_l2(forth, O.forward(T, g).reshape(-1)) < 1e-6

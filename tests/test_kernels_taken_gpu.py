@@ -42,6 +42,17 @@ def test_uneven_tables(torch_cuda, three, entry):
     assert OperatorBorn.from_tables(T).kernels["pair"] == "direct"
 
 
+def test_ordinary_rows(torch_cuda):
+    """Fields with most of a row far below its lobe: 60 times as wide as the
+    array at half a wavelength per pitch, where the receive filter's edge falls
+    on grazing angles, and a quarter of a pitch deep."""
+    arr = C.ArraySpec((8,), (3.048e-4,), (2.7e-4,), (4,))
+    wave = [C.qpw_wave(arr, 0.0, 1500.0)]
+    for n, npp, z0, f in (((505, 20), 1, 2e-3, np.linspace(2e6, 6e6, 28)), ((130, 40), 2, 3.81e-5, np.linspace(4e6, 10e6, 9))):
+        spec = C.SequenceSpec("o", arr, C.MediumSpec(), C.FovSpec(n, (3.048e-4 / npp,) * 2, z0), f, wave, [C.identity_mixes(8)])
+        assert OperatorBorn.from_sequence(spec).kernels["pair"] == "fast"
+
+
 @pytest.mark.parametrize("kind", ["single", "dense", "both"])
 def test_energies(torch_cuda, kind):
     for ne, nx, nz, npp in test_energy_gpu.SIZES:
