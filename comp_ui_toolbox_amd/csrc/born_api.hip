@@ -456,6 +456,8 @@ static void upload_fft_columns(Plan& P) {
   P.fft.d_col = dupload(col, P.stream);
 }
 
+static bool no_room(const Error& e) { return e.status == BORN_ERR_OUT_OF_MEMORY || e.status == BORN_ERR_UNSUPPORTED; }
+
 // Rows of h_ref that are not finite or may not be transformed (k_fft_range).
 static void check_rows(Plan& P) {
   if (!P.structured) return;
@@ -525,10 +527,12 @@ static void build_fft3_tables(Plan& P) {
   HIP_CHECK(hipGetLastError());
 }
 
-// Tables of the fast lateral correlation, built with a plan's first workspace
-// (a plan that only serves energies, columns or signals has no use for them):
-// the slots (row, segment, phase), the columns by frequency and the spectra of
-// h_ref.
+// Tables of the fast lateral correlation: the slots (row, segment, phase), the
+// columns by frequency and the spectra of h_ref.  Built at creation, where they
+// cost no time (in flight during other host work: 162.9 ms with and without
+// them at 128 elements, 512 x 512 points, 257 frequencies, 11 waves; the first
+// apply would take 5.0 instead of 3.7 ms), and again with a workspace after
+// they were given up.
 static void build_fft_tables(Plan& P) {
   Plan::Fft& F = P.fft;
   if (F.d_H) return;
@@ -553,8 +557,7 @@ static void build_fft_tables(Plan& P) {
     F.d_tw = dupload(tw, P.stream);
     F.d_H = dalloc<float2>((size_t)P.N_fu * F.n_ws * 1024);
     launch_fft_table(P, P.stream);
-    HIP_CHECK(hipGetLastError());
-    HIP_CHECK(hipStreamSynchronize(P.stream));   // the callers' streams read them
+    HIP_CHECK(hipGetLastError());   // (creation and ensure_workspace wait before any other stream reads them)
   } catch (...) {
     hipStreamSynchronize(P.stream);
     free_fft_tables(P);
@@ -1039,25 +1042,33 @@ static void setup_column_rhs_adjoint(Plan& P, int N_rhs) {
 }
 
 // Chunks of <= NC (pair, rhs) columns per frequency, rhs-major.
-static void build_workspace(Plan& P, int N_rhs, bool fft);
-static bool no_room(const Error& e) { return e.status == BORN_ERR_OUT_OF_MEMORY || e.status == BORN_ERR_UNSUPPORTED; }
+static void build_workspace(Plan& P, int N_rhs);
+
+// V, W and the masked input, of all kernels
+static size_t common_bytes(const Plan& P, int N_rhs) {
+  return (size_t)N_rhs * ((size_t)P.N_pairs * P.N_e * (sizeof(double2) + sizeof(float2)) + P.N_pts * sizeof(float2));
+}
 
 // A failure while building frees the partial workspace, so a plan that
 // could not get its workspace holds none.  Where the memory that the spectra
-// hold is what is missing, the workspace of the direct products takes its place.
+// hold is what is missing, the workspace of the direct products takes the place
+// of the fast correlation's.
 static void ensure_workspace(Plan& P, int N_rhs) {
   const bool split = P.precision != BORN_PRECISION_FP32;
   if (P.ws_rhs == N_rhs && (N_rhs == 1 || P.fft.ok || P.ws_split == split)) return;
   free_workspace(P);
   P.ws_split = split;
   try {
-    build_workspace(P, N_rhs, fft_wanted(P));
+    build_workspace(P, N_rhs);
   } catch (const Error& e) {
     free_workspace(P);
-    if (!P.fft.d_H || !no_room(e)) throw;
+    size_t free_b = 0, total_b = 0;
+    if (!P.fft.d_H || e.status != BORN_ERR_OUT_OF_MEMORY || hipMemGetInfo(&free_b, &total_b) != hipSuccess ||
+        free_b >= common_bytes(P, N_rhs))
+      throw;
     free_fft_tables(P);
     try {
-      build_workspace(P, N_rhs, false);
+      build_workspace(P, N_rhs);
     } catch (...) {
       free_workspace(P);
       throw;
@@ -1083,14 +1094,13 @@ static bool try_fft_workspace(Plan& P, int N_rhs) {
   return false;
 }
 
-static void build_workspace(Plan& P, int N_rhs, bool fft) {
+static void build_workspace(Plan& P, int N_rhs) {
   P.chunks.clear();
   P.col_pair.clear();
-  // V, W and the masked input, of all paths
   P.d_V = dalloc<double2>((size_t)P.N_pairs * P.N_e * N_rhs);
   P.d_W = dalloc<float2>((size_t)P.N_pairs * P.N_e * N_rhs);
   P.d_gm = dalloc<float2>((size_t)N_rhs * P.N_pts);
-  if (fft && try_fft_workspace(P, N_rhs)) {
+  if (fft_wanted(P) && try_fft_workspace(P, N_rhs)) {
     HIP_CHECK(hipDeviceSynchronize());
     P.fft.ok = true;
     P.ws_rhs = N_rhs;
@@ -1399,6 +1409,11 @@ static void finish_plan(Plan& P, bool structure_known = false) {
   set_max_lds_split3(160 * 1024);
   set_max_lds_fc(160 * 1024);
   check_rows(P);
+  try {   // (in flight during the layout below)
+    if (fft_wanted(P)) build_fft_tables(P);
+  } catch (const Error& e) {
+    if (!no_room(e)) throw;   // the first workspace tries again
+  }
   build_noalloc_layout(P);
   HIP_CHECK(hipStreamSynchronize(P.stream));
 }

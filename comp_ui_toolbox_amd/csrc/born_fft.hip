@@ -129,10 +129,14 @@ __global__ __launch_bounds__(256) void k_fft_range(const float2* __restrict__ h,
   };
   for (int64_t row = blockIdx.x; row < n_rows; row += gridDim.x) {
     const float2* src = h + (size_t)(row / Nz) * H_plane + (size_t)(row % Nz) * HY * HR;
-    auto entry = [&](int ty, int tx) { return src[(exty ? (size_t)exty[ty] * HR : 0) + ext[tx]]; };
+    auto entry = [&](int i, int n, int px, int py, int sx, int sy) {   // the i-th of a phase with n along x
+      if (!exty) return src[ext[px + sx * i]];
+      const int ty = i / n;
+      return src[(size_t)exty[py + sy * ty] * HR + ext[px + sx * (i - ty * n)]];
+    };
     float top = 0.f, odd = 0.f, none = 0.f;
     for (int i = tid; i < N_ext * ny; i += 256) {
-      const float2 v = entry(i / N_ext, i % N_ext);
+      const float2 v = entry(i, N_ext, 0, 0, 1, 1);
       if (!(fabsf(v.x) < 1e30f && fabsf(v.y) < 1e30f)) odd = 1.f;   // (NaN among them)
       else top = fmaxf(top, fmaxf(fabsf(v.x), fabsf(v.y)));
     }
@@ -142,14 +146,19 @@ __global__ __launch_bounds__(256) void k_fft_range(const float2* __restrict__ h,
       continue;
     }
     if (top == 0.f) continue;
-    bool uneven = top < 0x1p-100f;
+    if (top < 0x1p-100f) {
+      if (tid == 0) atomicOr(bad, 2);
+      continue;
+    }
+    bool uneven = false;
     float peak = 0.f, energy = 0.f, logs = 0.f, count = 0.f;
+    const float scale = 1.f / top;
     for (int ph = 0; ph < Npx * Npy; ++ph) {
       const int px = ph % Npx, py = ph / Npx, nx = (N_ext - px + Npx - 1) / Npx, m = nx * ((ny - py + Npy - 1) / Npy);
       float e = 0.f, l = 0.f, n = 0.f, first = 0.f;
       for (int i = tid; i < m; i += 256) {
-        const float2 v = entry(py + Npy * (i / nx), px + Npx * (i % nx));
-        const float x = v.x / top, y = v.y / top, q = x * x + y * y;
+        const float2 v = entry(i, nx, px, py, Npx, Npy);
+        const float x = v.x * scale, y = v.y * scale, q = x * x + y * y;
         first = fmaxf(first, q);
         e += q;
         if (q > 0.f) {
@@ -163,8 +172,8 @@ __global__ __launch_bounds__(256) void k_fft_range(const float2* __restrict__ h,
       if (16.f * first > e) {
         float low = 0.f;
         for (int i = tid; i < m; i += 256) {
-          const float2 v = entry(py + Npy * (i / nx), px + Npx * (i % nx));
-          const float x = v.x / top, y = v.y / top, q = x * x + y * y;
+          const float2 v = entry(i, nx, px, py, Npx, Npy);
+          const float x = v.x * scale, y = v.y * scale, q = x * x + y * y;
           if (q > 0.f && q * 0x1p32f < first) low += 1.f;
         }
         reduce(low, none, none, false);

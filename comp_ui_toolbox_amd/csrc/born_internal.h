@@ -266,8 +266,7 @@ struct Plan {
   float2* d_gm = nullptr;         // masked gamma [N_rhs][N_pts]
   int items_target = 8192;        // forward work items per launch (tunable)
   LaunchSet ls;                   // structured launch of this plan alone
-  // fast lateral correlation: tables, built with the first workspace (d_H null: not yet),
-  // then the per-rhs workspace
+  // fast lateral correlation: tables of the plan (d_H null: none), then the per-rhs workspace
   struct Fft {
     bool ok = false;                // the workspace is that of the fast correlation
     bool off = false;               // switched off by the caller

@@ -305,8 +305,9 @@ int born_plan_force_general(born_plan_t plan, int32_t on);
  * numeric form (0).  A transform carries the rounding of a whole row of h_ref,
  * the direct products only that of each entry: a program whose results hang
  * on outputs far below the others of their row (one active element, a point
- * outside every element's cone) switches it off.  The next call builds the
- * workspace of the other kernels. */
+ * outside every element's cone) switches it off, and so may one that has no
+ * use for forward and adjoint: the spectra of h_ref, about twice its size, are
+ * given back.  The next call builds the workspace of the other kernels. */
 int born_plan_set_correlation(born_plan_t plan, int32_t on);
 
 /* Which kernels a plan's calls take: kernels[0] forward and adjoint, [1]

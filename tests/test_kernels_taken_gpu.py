@@ -76,19 +76,22 @@ def test_columns(torch_cuda):
     assert OperatorBorn.from_tables(T).kernels["columns"] == "gather"
 
 
-def test_spectra_come_with_the_first_apply(torch_cuda):
-    """Energies, columns and signals hold the tables alone: 33.5 MiB of h_ref
-    and of p_inc here, 65 MiB of spectra."""
+def test_spectra_are_given_back(torch_cuda):
+    """Energies, columns and signals need the tables alone, 33.5 MiB of h_ref
+    and of p_inc here; switching the fast correlation off gives its 65 MiB of
+    spectra back and leaves their kernels."""
     spec = C.config0()
     base = torch_cuda.cuda.mem_get_info()[0]
     op = OperatorBorn.from_sequence(spec)
     tables = 2 * 8 * len(spec.frequencies) * op.N_points
     spectra = 8 * len(spec.frequencies) * op.N_points * 2     # rows of 64 + 63 points in transforms of 128
-    op.energy_rx(0)
+    assert base - torch_cuda.cuda.mem_get_info()[0] >= tables + spectra
+    op.set_correlation(False)
+    energy = op.energy_rx(0)
     op.columns([0, op.N_points - 1])
     op.time_signals(torch_cuda.zeros(op.N_observations, dtype=torch_cuda.complex64, device="cuda:0"), spec.frequencies)
-    assert op.kernels["pair"] == "fast"
-    used = base - torch_cuda.cuda.mem_get_info()[0]
-    assert tables <= used < tables + spectra // 2
+    assert op.kernels == {"pair": "direct", "energy": "fast", "energy_tgc": "gather", "columns": "fast"}
+    assert tables <= base - torch_cuda.cuda.mem_get_info()[0] < tables + spectra // 2
+    op.set_correlation(True)
     op.forward_dev(torch_cuda.zeros(op.N_points, dtype=torch_cuda.complex64, device="cuda:0"))
-    assert base - torch_cuda.cuda.mem_get_info()[0] >= used + spectra
+    assert op.kernels["pair"] == "fast" and np.array_equal(energy, op.energy_rx(0))

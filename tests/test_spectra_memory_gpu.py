@@ -3,7 +3,7 @@ over, with the results, bit by bit, of a plan on which the fast correlation is
 switched off.  The failures are forced on the host, before hipMalloc."""
 import pytest
 
-from comp_ui_toolbox_amd import OperatorBatch, OperatorBorn, _lib
+from comp_ui_toolbox_amd import BornError, OperatorBatch, OperatorBorn, _lib
 from tests.test_fft_gpu import make
 from tests.test_kernels_taken_gpu import spec_3d
 
@@ -58,12 +58,43 @@ def expected(create, n_rhs):
     return out
 
 
+def test_creation(create):
+    """An allocation that fails at creation either is an error that leaves
+    nothing behind or one of the spectra, which the first workspace builds."""
+    one = expected(create, 1)
+    base = live()
+    whole = create()
+    held = live() - base
+    whole.close()
+    errors = fallbacks = 0
+    for k in range(200):
+        fail_at(k)
+        try:
+            op = create()
+        except BornError as e:
+            assert e.identifier == "born:OutOfMemory" and live() == base
+            errors += 1
+            continue
+        finally:
+            fail_at(-1)
+        if live() - base == held:
+            break
+        fallbacks += 1
+        assert same(results(op, 1), one["fast"][0]) and op.kernels["pair"] == "fast"
+        op.close()
+        assert live() == base
+    assert k < 199 and errors >= 10 and fallbacks >= 3
+    op.close()
+
+
 @pytest.mark.parametrize("n_rhs", [1, 3])
 def test_first_workspace(create, n_rhs):
     ref, after = expected(create, n_rhs), expected(create, n_rhs + 1)
     base = live()
     for k in range(COMMON, 40):
         op = create()
+        op.set_correlation(False)
+        op.set_correlation(True)      # the spectra come with the workspace
         before = live()
         assert same(results(op, n_rhs, k), ref[op.kernels["pair"]][0])
         if op.kernels["pair"] == "fast":
@@ -78,15 +109,21 @@ def test_first_workspace(create, n_rhs):
 
 
 def test_later_workspace(create):
-    """With the spectra there, a failure anywhere makes room by giving them up."""
+    """With the spectra there, a failure of the fast correlation's own buffers
+    gives them up; one of the common buffers, with memory to spare, is an error."""
     one, two = expected(create, 1), expected(create, 2)
     base = live()
     for k in range(40):
         op = create()
         assert same(results(op, 1), one["fast"][0])
-        assert same(results(op, 2, k), two[op.kernels["pair"]][0])
-        if op.kernels["pair"] == "fast":
+        if k < COMMON:
+            with pytest.raises(BornError, match="born:OutOfMemory"):
+                results(op, 2, k)
+            fail_at(-1)
+        assert same(results(op, 2, -1 if k < COMMON else k), two[op.kernels["pair"]][0])
+        if k >= COMMON and op.kernels["pair"] == "fast":
             break
+        assert op.kernels["pair"] == ("fast" if k < COMMON else "direct")
         op.close()
         assert live() == base
     assert k > COMMON
@@ -98,7 +135,7 @@ def test_batch(create):
     import torch
     one = expected(create, 1)
     a, b = create(), create()
-    results(b, 1, COMMON + 2)
+    results(b, 1, COMMON)
     B = OperatorBatch([a, b])
     assert [a.kernels["pair"], b.kernels["pair"]] == ["fast", "direct"]
     g = torch.ones(a.N_points, dtype=torch.complex64, device="cuda:0")
