@@ -682,10 +682,14 @@ static void build_fft_workspace(Plan& P, int N_rhs) {
 
 static void materialize_shift(Plan& P);
 
-static void ensure_shift_on_device(Plan& P) {
+static void upload_shift(Plan& P) {   // under P.shared
   if (P.d_shift) return;
   if (P.h_shift.empty()) materialize_shift(P);
   P.d_shift = dupload(P.h_shift, P.stream);
+}
+static void ensure_shift_on_device(Plan& P) {
+  std::lock_guard<std::mutex> lock(P.shared);
+  upload_shift(P);
 }
 
 // Forward blocking: about items_target work items per launch, (chunk,
@@ -2527,6 +2531,7 @@ int born_apply_dev_noalloc(born_plan_t plan, int32_t mode, const void* in_c64, i
 
 // Tables of the received energies on the structured path (on first use).
 static void ensure_energy_tables(Plan& P) {
+  std::lock_guard<std::mutex> lock(P.shared);
   if (P.e_ready) return;
   dfree(P.d_ew);   // of a first use that failed
   dfree(P.d_erow_off);
@@ -2595,21 +2600,28 @@ int born_energy_rx(born_plan_t plan, int32_t measurement, double* energy) {
 
 // Energy under the plan's TGC; synchronous on s (a spill buffer for long
 // mixes lives for the launch only).
+// Spectra of the time gain kernels (on first use).
+static void ensure_tgc_spectra(Plan& P) {
+  std::lock_guard<std::mutex> lock(P.shared);
+  if (P.tgc_ready) return;
+  dfree(P.d_tgc_tw);   // of a first use that failed
+  dfree(P.d_tgc_spec);
+  std::vector<float2> tw;
+  fft_twiddles(P.tgc_TL, tw, true);
+  P.d_tgc_tw = dupload(tw, P.stream);
+  P.d_tgc_spec = dalloc<float2>((size_t)P.N_mk * 32 * P.tgc_TL);
+  launch_tgc_spectra(P, P.tgc_TL, P.d_tgc_spec, P.stream);
+  HIP_CHECK(hipGetLastError());
+  HIP_CHECK(hipStreamSynchronize(P.stream));
+  P.tgc_ready = true;
+}
+
 static void energy_rx_tgc(Plan& P, int m, double* E_dev, hipStream_t s) {
   if (m < 0 || m >= (int)P.meas_pair_base.size())
     throw Error(BORN_ERR_INVALID_ARGUMENT, "operator_born.indices_measurement_sel must be a single index!");
   if (!P.tgc) throw Error(BORN_ERR_INVALID_ARGUMENT, "no TGC kernels are set on this operator");
   if (use_structured(P) && P.tgc_TL > 0) {
-    if (!P.d_tgc_spec) {
-      dfree(P.d_tgc_tw);   // of a first use that failed
-      std::vector<float2> tw;
-      fft_twiddles(P.tgc_TL, tw, true);
-      P.d_tgc_tw = dupload(tw, P.stream);
-      P.d_tgc_spec = dalloc<float2>((size_t)P.N_mk * 32 * P.tgc_TL);
-      launch_tgc_spectra(P, P.tgc_TL, P.d_tgc_spec, P.stream);
-      HIP_CHECK(hipGetLastError());
-      HIP_CHECK(hipStreamSynchronize(P.stream));
-    }
+    ensure_tgc_spectra(P);
     launch_energy_tgc_fft(P, m, E_dev, s);
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipStreamSynchronize(s));
@@ -2724,7 +2736,8 @@ int born_time_signals(born_plan_t plan, const double* frequencies, double delta_
     const int dq = P.N_fu > 1 ? q_fg[1] - q_fg[0] : 1;
     for (int i = 0; i + 1 < P.N_fu && even; ++i) even = dq > 0 && q_fg[i + 1] - q_fg[i] == dq;
     if (even) {
-      if (P.time_Nt != N_t) {   // calls end synchronized, so nothing reads the old table
+      std::lock_guard<std::mutex> lock(P.shared);
+      if (P.time_Nt != N_t) {   // calls hold the lock until they are synchronized, so nothing reads the old table
         dfree(P.d_time_cs);
         P.time_Nt = 0;
         P.d_time_cs = dalloc<float2>(N_t);
@@ -2800,11 +2813,12 @@ static void columns(Plan& P, const double* points, int32_t n, void* out, bool ho
   if ((double)n * (double)P.N_obs > 2.0e11) throw Error(BORN_ERR_INVALID_ARGUMENT, "too many columns for one call");
   std::vector<int> pts(n);
   for (int j = 0; j < n; ++j) pts[j] = idx1(points[j], P.N_pts, "points");
+  std::lock_guard<std::mutex> lock(P.shared);   // the plan's point list, until the call is done with it
   // force_general takes the map-driven kernel
   const bool fast = use_structured(P) && columns_fast(P);
   if (fast) ensure_column_tables(P);
-  else ensure_shift_on_device(P);
-  if (P.pts_cap < n) {   // kept: calls end synchronized, so nothing reads it any more
+  else upload_shift(P);
+  if (P.pts_cap < n) {   // kept: calls hold the lock until they are synchronized, so nothing reads it any more
     dfree(P.d_pts);
     P.pts_cap = 0;
     P.d_pts = dalloc<int>(n);
@@ -2854,6 +2868,7 @@ static void tgc_clear(Plan& P) {
   dfree(P.d_tgc_k64);
   dfree(P.d_tgc_spec);
   dfree(P.d_tgc_tw);
+  P.tgc_ready = false;
   P.tgc_TL = 0;
   P.tgc = false;
   P.n_tgc_tiles = 0;

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <cstdint>
 #include <string>
+#include <mutex>
 #include <vector>
 
 namespace born {
@@ -174,6 +175,9 @@ struct FftSet {
 // Device tables and index maps.  All device arrays are owned by the plan.
 struct Plan {
   int device = 0;
+  // of the tables built on first use and the buffers that columns and time
+  // signals keep: these calls and the energies may come from several threads
+  std::mutex shared;
   int n_cu = 256;           // compute units of the device (persistent grids)
   int precision = 0;
   bool force_general = false;
@@ -347,6 +351,7 @@ struct Plan {
   // energies under TGC by transforms of length 16 * tgc_TL (0: none), built on
   // first use after the kernels are set: spectra of the taps, twiddles
   int tgc_TL = 0;
+  bool tgc_ready = false;
   float2* d_tgc_spec = nullptr;
   float2* d_tgc_tw = nullptr;
   size_t io_bytes = 0;

@@ -21,7 +21,9 @@
  *   - observations are ordered measurement-major, then mix, then frequency
  *     (cu:773, :978);
  *   - a plan is not re-entrant: calls on one plan must not overlap.  Use one
- *     plan per stream.
+ *     plan per stream.  (Columns, time signals and received energies share
+ *     nothing but tables built on first use and buffers that a lock guards;
+ *     these may come from several threads.)
  */
 #ifndef BORN_H
 #define BORN_H
