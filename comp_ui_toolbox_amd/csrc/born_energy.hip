@@ -566,14 +566,6 @@ static EnergyArgs energy_args(const Plan& P, int m, int R) {
 // entry that is not finite would carry to points that do not see it.
 bool energy_fast(const Plan& P) { return P.structured && P.Np <= 64 && !P.h_odd; }
 
-// Waves per workgroup: 4, up to 16 while the launch has fewer than 4096 waves.
-static int energy_waves(int wgs, size_t lds_per_wave, int most) {
-  int W = 4;
-  while (W < most && wgs * W < 4096 && 2 * W * lds_per_wave <= 150 * 1024) W *= 2;
-  while (W > 1 && W * lds_per_wave > 150 * 1024) W /= 2;
-  return W;
-}
-
 template <int R>
 static void energy_single(const Plan& P, int m, double* E, hipStream_t s) {
   EnergyArgs A = energy_args(P, m, R);
@@ -613,7 +605,8 @@ void launch_energy_multi(const Plan& P, int m, bool add, double* E, hipStream_t 
   A.add = add;
   const int wgs = A.n_rows * A.nseg;
   const size_t per_wave = ((size_t)A.Np * A.WLp + (size_t)A.nb * R * KB * 2) * sizeof(double);
-  const int W = energy_waves(wgs, per_wave, 4);
+  int W = 4;   // (the kernel's launch bound; fewer where LDS does not hold them)
+  while (W > 1 && W * per_wave > 150 * 1024) W /= 2;
   const size_t lds = W * per_wave;
 #define BORN_EM(NPv)                                                                                                      \
   do {                                                                                                                    \
