@@ -2558,6 +2558,7 @@ static void ensure_energy_tables(Plan& P) {
     P.d_erows = dupload(rows, P.stream);
   }
   P.d_ew = dalloc<double>((size_t)P.N_pairs * Ney * energy_pad(P.Nex));
+  P.e_waves = energy_single_waves(P);
   launch_energy_weights(P, P.d_ew, P.stream);
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipStreamSynchronize(P.stream));   // the callers' streams read it

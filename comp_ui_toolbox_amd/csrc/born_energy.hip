@@ -24,6 +24,7 @@
 #include "born_internal.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace born {
 
@@ -566,37 +567,66 @@ static EnergyArgs energy_args(const Plan& P, int m, int R) {
 // entry that is not finite would carry to points that do not see it.
 bool energy_fast(const Plan& P) { return P.structured && P.Np <= 64 && !P.h_odd; }
 
-template <int R>
-static void energy_single(const Plan& P, int m, double* E, hipStream_t s) {
+// f(R, MI) of the single-element kernel that a plan takes.  R = 4, 6 or 8 points
+// per lane: the fewest points computed past the row's end, then the largest (one
+// LDS read per R multiply-adds).
+template <int R, typename F>
+static void with_single_entries(const EnergyArgs& A, F&& f) {
+  const int mi = (A.Np * (A.LPW + A.nb) * R + 63) / 64;
+  using I = std::integral_constant<int, R>;
+  if (R < 8 && mi <= 8) f(I(), std::integral_constant<int, (R < 8 ? 8 : 12)>());   // (8 points per lane have more)
+  else if (mi <= 12) f(I(), std::integral_constant<int, 12>());
+  else if (mi <= 16) f(I(), std::integral_constant<int, 16>());
+  else f(I(), std::integral_constant<int, 0>());
+}
+static EnergyArgs single_args(const Plan& P, int m, int R) {
   EnergyArgs A = energy_args(P, m, R);
   A.nb += A.nb & 1;
   A.WLp = e_window(A.LPW, A.nb, R);
-  const int wgs = A.n_rows * A.nseg;
-  const size_t per_wave = ((size_t)A.Np * A.WLp + A.nb * R + 1) * sizeof(double);
-  int W = wgs < 384 ? 8 : 4;   // 384 rows of 384 points: 183 us with 4, 190 with 8; 256 of 256 points: 42 and 36
-  while (W > 1 && W * per_wave > 150 * 1024) W /= 2;
-  const size_t lds = W * per_wave;
-  const int mi = (A.Np * (A.LPW + A.nb) * R + 63) / 64;
-#define BORN_ES(MIv)                                                                                                   \
-  do {                                                                                                                 \
-    hipFuncSetAttribute((const void*)k_energy_single<R, MIv>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
-    hipLaunchKernelGGL((k_energy_single<R, MIv>), dim3(wgs), dim3(64 * W), lds, s, A, E);                             \
-  } while (0)
-  if (R < 8 && mi <= 8) BORN_ES((R < 8 ? 8 : 12));   // (8 points per lane have more)
-  else if (mi <= 12) BORN_ES(12);
-  else if (mi <= 16) BORN_ES(16);
-  else BORN_ES(0);
-#undef BORN_ES
+  return A;
 }
-
-// R = 4, 6 or 8 points per lane: the fewest points computed past the row's
-// end, then the largest (one LDS read per R multiply-adds).
-void launch_energy_single(const Plan& P, int m, double* E, hipStream_t s) {
+static size_t single_lds(const EnergyArgs& A, int R) { return ((size_t)A.Np * A.WLp + A.nb * R + 1) * sizeof(double); }
+template <typename F>
+static void with_single_kernel(const Plan& P, int m, F&& f) {
   const int LPW = 64 / P.Np, S = (P.Nx + P.Np - 1) / P.Np;
   auto pad = [&](int R) { return (S + LPW * R - 1) / (LPW * R) * LPW * R; };
-  if (pad(8) <= pad(6) && pad(8) <= pad(4)) energy_single<8>(P, m, E, s);
-  else if (pad(6) <= pad(4)) energy_single<6>(P, m, E, s);
-  else energy_single<4>(P, m, E, s);
+  auto run = [&](auto R) {
+    const EnergyArgs A = single_args(P, m, R());
+    with_single_entries<R()>(A, [&](auto, auto MI) { f(A, R, MI); });
+  };
+  if (pad(8) <= pad(6) && pad(8) <= pad(4)) run(std::integral_constant<int, 8>());
+  else if (pad(6) <= pad(4)) run(std::integral_constant<int, 6>());
+  else run(std::integral_constant<int, 4>());
+}
+
+// Waves per workgroup of the single-element kernel: 8 while the compute units
+// hold all workgroups at once (one each, two of the smallest kernels), else 4,
+// of which two share a compute unit.  One measurement of 128 elements, rows of
+// 384 points, 65 frequencies: 256 rows 61 us with 4 waves and 53 with 8, 272 rows
+// 89 and 96, 384 rows 90 and 100; rows of 250 points (4 points per lane), 64
+// elements, 300 rows: 43 and 38.
+int energy_single_waves(const Plan& P) {
+  int W = 4;
+  with_single_kernel(P, 0, [&](const EnergyArgs& A, auto R, auto MI) {
+    const size_t per_wave = single_lds(A, R());
+    const void* fn = (const void*)k_energy_single<R(), MI()>;
+    int at_once = 0;
+    if (8 * per_wave <= 150 * 1024 &&
+        hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess &&
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&at_once, fn, 512, 8 * per_wave) == hipSuccess &&
+        (int64_t)A.n_rows * A.nseg <= (int64_t)at_once * P.n_cu)
+      W = 8;
+    while (W > 1 && W * per_wave > 150 * 1024) W /= 2;
+  });
+  return W;
+}
+
+void launch_energy_single(const Plan& P, int m, double* E, hipStream_t s) {
+  with_single_kernel(P, m, [&](const EnergyArgs& A, auto R, auto MI) {
+    hipFuncSetAttribute((const void*)k_energy_single<R(), MI()>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    hipLaunchKernelGGL((k_energy_single<R(), MI()>), dim3(A.n_rows * A.nseg), dim3(64 * P.e_waves),
+                       P.e_waves * single_lds(A, R()), s, A, E);
+  });
 }
 
 void launch_energy_multi(const Plan& P, int m, bool add, double* E, hipStream_t s) {

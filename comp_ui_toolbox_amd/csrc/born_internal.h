@@ -305,6 +305,7 @@ struct Plan {
   // prefactors of the single-element mixes by (pair, y slice, element), and
   // the observations of the other mixes by pair (none: null)
   bool e_ready = false;
+  int e_waves = 4;                       // of a workgroup of k_energy_single
   std::vector<char> e_single, e_multi;   // per measurement: has such mixes
   double* d_ew = nullptr;
   int64_t* d_erow_off = nullptr;
@@ -434,6 +435,7 @@ void launch_energy_rx(const Plan& P, int m, double* E, hipStream_t s);
 bool energy_fast(const Plan& P);
 int energy_pad(int Nex);
 void launch_energy_weights(const Plan& P, double* ew, hipStream_t s);
+int energy_single_waves(const Plan& P);
 void launch_energy_single(const Plan& P, int m, double* E, hipStream_t s);
 void launch_energy_multi(const Plan& P, int m, bool add, double* E, hipStream_t s);
 int energy_tgc_length(int N, int M);
