@@ -1348,10 +1348,13 @@ static void ensure_io(Plan& P, size_t in_bytes, size_t out_bytes) {
 }
 
 // Pinned staging of the host calls, kept with the plan; nullptr past 256 MiB or
-// where there is none (the callers then stage through pageable memory).
+// where there is none (the callers then stage through pageable memory).  Given
+// back to what the calls need after 16 that need less than an eighth of it.
 static void* host_staging(Plan& P, size_t bytes) {
   if (bytes > ((size_t)256 << 20)) return nullptr;
-  if (P.h_stage_bytes >= bytes) return P.h_stage;
+  P.h_stage_idle = 8 * bytes < P.h_stage_bytes ? P.h_stage_idle + 1 : 0;
+  if (P.h_stage_bytes >= bytes && P.h_stage_idle < 16) return P.h_stage;
+  P.h_stage_idle = 0;
   if (P.h_stage) hipHostFree(P.h_stage);
   P.h_stage = nullptr;
   P.h_stage_bytes = 0;

@@ -360,6 +360,7 @@ struct Plan {
   void* d_io_out = nullptr;
   void* h_stage = nullptr;         // pinned staging of the host calls
   size_t h_stage_bytes = 0;
+  int h_stage_idle = 0;            // calls in a row that needed a fraction of it
   hipStream_t stream = nullptr;   // host-path stream
 
   // Allocation-free apply (born_apply_dev_noalloc): a one-rhs chunk layout

@@ -161,7 +161,8 @@ int born_plan_set_precision(born_plan_t plan, int32_t precision);
  * forward occupancy rule (cu:466-488), zero output when nothing is occupied
  * (cu:496); with few occupied points the gather path of
  * born_plan_set_sparse_forward.  gamma: complex N_points x N_rhs; u:
- * complex N_obs x N_rhs. */
+ * complex N_obs x N_rhs.  The host calls stage through pinned memory that the
+ * plan keeps, up to 256 MiB of what its recent calls needed. */
 int born_forward(born_plan_t plan, const double* gamma, int32_t N_rhs, double* u);
 
 /* combined_quick_gpu( op, 2, u ): host FP64 in/out; all N_points rows
