@@ -260,13 +260,15 @@ __global__ __launch_bounds__(256) void k_time_regular(const float2* __restrict__
       S[r] = fmaf(v.y, w.y, S[r]);
     }
   }
-  // the zero and Nyquist indices count once: take half of them back
+  // the zero and Nyquist indices count once: take half of them back (an infinite
+  // one stays what it is)
+  auto half = [](float v) { return fabsf(v) <= 3.402823466e+38f ? 0.5f * v : 0.f; };
   const int fz = q0 == 0 ? 0 : -1, fn = 2 * (q0 + dq * (Nf - 1)) == N_t ? Nf - 1 : -1;
 #pragma unroll
   for (int r = 0; r < RB; ++r) {
     float c = C[r];
-    if (fz >= 0) c -= 0.5f * x[r][0].x;
-    if (fn >= 0) c -= 0.5f * (nn & 1 ? -x[r][fn].x : x[r][fn].x);
+    if (fz >= 0) c -= half(x[r][0].x);
+    if (fn >= 0) c -= half(nn & 1 ? -x[r][fn].x : x[r][fn].x);
     if (r < rb && n < n_half) {
       float* out = rf + (row0 + r) * N_t;
       out[n] = 2.f * (c - S[r]);
