@@ -510,12 +510,21 @@ static bool fft_wanted(Plan& P) {
   return n + ((size_t)1 << 30) <= free_b;
 }
 
+static void append_floats(std::vector<float2>& v, const std::vector<float>& f) {   // an even number
+  for (size_t i = 0; i + 1 < f.size(); i += 2) v.push_back(make_float2(f[i], f[i + 1]));
+}
+
 static void build_fft3_tables(Plan& P) {
   Plan::Fft& F = P.fft;
   std::vector<float2> tw, twy;
+  std::vector<float> delta, delta_y;
   fft_twiddles(F.s3.TLX, tw);
   fft_twiddles(F.s3.TLY, twy);
+  fft_gains(F.s3.TLX, tw, F.s3.Sx, P.Nex, delta);
+  fft_gains(F.s3.TLY, twy, F.s3.Sy, P.Ney, delta_y);
   tw.insert(tw.end(), twy.begin(), twy.end());
+  delta.insert(delta.end(), delta_y.begin(), delta_y.end());
+  append_floats(tw, delta);
   upload_fft_columns(P);
   F.d_tw = dupload(tw, P.stream);
   F.d_H = dalloc<float2>((size_t)P.N_fu * P.Nz * P.Npy * P.Np * fft3_plane(F.s3));
@@ -551,7 +560,10 @@ static void build_fft_tables(Plan& P) {
       slot[s] = left > 0 ? make_int2(row * P.Nx + first, std::min(left, F.shape.Sv)) : make_int2(0, 0);
     }
     std::vector<float2> tw;
+    std::vector<float> delta;
     fft_twiddles(F.shape.TL, tw);
+    fft_gains(F.shape.TL, tw, F.shape.Sv, P.N_e, delta);
+    append_floats(tw, delta);
     F.d_slot = dupload(slot, P.stream);
     upload_fft_columns(P);
     F.d_tw = dupload(tw, P.stream);

@@ -49,7 +49,8 @@ struct Fft3Shape {
 template <int TLX>
 __global__ __launch_bounds__(64) void k_fft3_table_x(const float2* __restrict__ h, const int* __restrict__ ext,
                                                      const int* __restrict__ exty, int HR, int HY, int N_ext, int N_exty,
-                                                     int Npx, int Npy, int Ly, int64_t n_rows, double2* __restrict__ tmp) {
+                                                     int Npx, int Npy, int Ly, int64_t n_rows,
+                                                     const float* __restrict__ delta, double2* __restrict__ tmp) {
   constexpr int FPW = FftShape<TLX>::FPW, L = 16 * TLX;
   __shared__ Cx<double> lds[FftShape<TLX>::LDS];
   const int lane = threadIdx.x, j = lane / FPW, g = lane % FPW;
@@ -84,13 +85,16 @@ __global__ __launch_bounds__(64) void k_fft3_table_x(const float2* __restrict__ 
   fft_wave<double, TLX, false>(x, tw, lds, lane);
   if (!on) return;
 #pragma unroll
-  for (int q = 0; q < 16; ++q) tmp[row * L + j + TLX * q] = make_double2(x[q].x, x[q].y);
+  for (int q = 0; q < 16; ++q) {
+    const double d = 1.0 + delta[j + TLX * q];
+    tmp[row * L + j + TLX * q] = make_double2(x[q].x * d, x[q].y * d);
+  }
 }
 
 // y transforms (FP64): H[(z, phi_y, phi_x)][k_x / FPWY][8][64 lanes][2]
 template <int TLY>
 __global__ __launch_bounds__(64) void k_fft3_table_y(const double2* __restrict__ tmp, int Lx, int64_t n_cols,
-                                                     float2* __restrict__ H) {
+                                                     const float* __restrict__ delta, float2* __restrict__ H) {
   constexpr int FPW = FftShape<TLY>::FPW, L = 16 * TLY;
   __shared__ Cx<double> lds[FftShape<TLY>::LDS];
   const int lane = threadIdx.x, j = lane / FPW, g = lane % FPW;
@@ -110,6 +114,11 @@ __global__ __launch_bounds__(64) void k_fft3_table_y(const double2* __restrict__
     x[q] = {v.x, v.y};
   }
   fft_wave<double, TLY, false>(x, tw, lds, lane);
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    const double d = 1.0 + delta[j + TLY * q];
+    x[q] = {x[q].x * d, x[q].y * d};
+  }
   float4* out = reinterpret_cast<float4*>(H) + (col / FPW) * 512 + lane;
 #pragma unroll
   for (int q = 0; q < 8; ++q)
@@ -525,11 +534,13 @@ void launch_fft3_table(const Plan& P, int f, double2* tmp, hipStream_t s) {
   const float2* h = P.d_h + (size_t)f * P.H_plane;
   float2* H = P.fft.d_H + (size_t)f * planes * Lx * Ly;
   const int fx = 64 / c.TLX, fy = 64 / c.TLY;
+  const float* delta = reinterpret_cast<const float*>(P.fft.d_tw + Lx + Ly);   // behind the twiddles of both axes
 #define BORN_T3X(T)                                                                                                    \
   hipLaunchKernelGGL(k_fft3_table_x<T>, dim3((unsigned)(planes * Ly / fx)), dim3(64), 0, s, h, P.d_ext, P.d_exty, P.HR, \
-                     P.HY, P.N_ext, (int)P.exty.size(), P.Np, P.Npy, Ly, planes* Ly, tmp)
+                     P.HY, P.N_ext, (int)P.exty.size(), P.Np, P.Npy, Ly, planes* Ly, delta, tmp)
 #define BORN_T3Y(T) \
-  hipLaunchKernelGGL(k_fft3_table_y<T>, dim3((unsigned)(planes * Lx / fy)), dim3(64), 0, s, tmp, Lx, planes* Lx, H)
+  hipLaunchKernelGGL(k_fft3_table_y<T>, dim3((unsigned)(planes * Lx / fy)), dim3(64), 0, s, tmp, Lx, planes* Lx,   \
+                     delta + Lx, H)
   if (c.TLX == 4) BORN_T3X(4);
   else BORN_T3X(8);
   if (c.TLY == 4) BORN_T3Y(4);

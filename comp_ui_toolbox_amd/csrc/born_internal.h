@@ -280,7 +280,7 @@ struct Plan {
     float2* d_H = nullptr;
     int2* d_slot = nullptr;
     int2* d_col = nullptr;
-    float2* d_tw = nullptr;
+    float2* d_tw = nullptr;         // twiddles of the axes, then what fft_gains gives for them (floats)
     int NZB = 1, ZR = 1, FG = 1;
     float2* d_gs = nullptr;
     float2* d_vp = nullptr;
@@ -478,6 +478,7 @@ void launch_fft3_adj(const Plan& P, int N_rhs, float2* g, hipStream_t s);
 // fast lateral correlation (born_fft.hip)
 FftShapeChoice fft_shape(int Nx, int Np, int N_e);
 void fft_twiddles(int TL, std::vector<float2>& tw, bool unit = false);
+void fft_gains(int TL, const std::vector<float2>& tw, int S, int N_e, std::vector<float>& delta);
 void launch_fft_range(const Plan& P, int* bad, hipStream_t s);
 void launch_fft_table(const Plan& P, hipStream_t s);
 void launch_fft_gamma(const Plan& P, const float2* gamma, int N_rhs, bool mask, hipStream_t s);

@@ -106,3 +106,33 @@ def test_lobes_of_another_scale(torch_cuda, three, width):
     T.h_ref = clean
     assert O.rel_l2(back[~touched], O.adjoint(T, u).reshape(-1)[~touched]) < 1e-6
     assert O.rel_l2(forth, O.forward(T, g).reshape(-1)) < 1e-6
+
+
+@pytest.mark.parametrize("ne,n,npp", [((20,), (40, 30), 1), ((64,), (200, 20), 4), ((128,), (400, 12), 4), ((16, 8), (24, 20, 8), 2),
+                                      ((33, 4), (66, 12, 4), 2)])
+def test_energy_of_the_outputs(torch_cuda, ne, n, npp):
+    """Sums of squares of the outputs, as a data misfit takes them.  Their
+    roundings (1.3e-7 each) average out: over the 540 outputs of the smallest
+    case, a hundred of them of weight, to 2e-8, over eight inputs to 7e-9.  The
+    transforms' constants, rounded to FP32 and the same for all outputs, took
+    0.8 to 1.5e-7 off before the spectra made up for it.  Half a unit in the last
+    place, 2^-25 = 3.0e-8, lies between."""
+    import torch
+    d = len(ne)
+    arr = C.ArraySpec(ne, (3e-4,) * d, (2.7e-4,) * d, (1,) * d)
+    rng = np.random.Generator(np.random.PCG64(8))
+    ws = [C.random_wave(arr, rng, 1e-6) for _ in range(3)]
+    spec = C.SequenceSpec("m", arr, C.MediumSpec(), C.FovSpec(n, (3e-4 / npp,) * len(n), 3e-3), np.linspace(2e6, 5e6, 9), ws,
+                          [C.identity_mixes(arr.N_elements) for _ in ws])
+    op = OperatorBorn.from_sequence(spec)
+    assert op.kernels["pair"] == "fast"
+    T = O.direct_tables(spec)
+    g = torch.view_as_complex(torch.tensor(rng.standard_normal((8, op.N_points, 2)).astype(np.float32), device="cuda:0"))
+    u = torch.view_as_complex(torch.tensor(rng.standard_normal((8, op.N_observations, 2)).astype(np.float32), device="cuda:0"))
+    for run, exact, x in ((op.forward_dev, O.forward, g), (op.adjoint_dev, O.adjoint, u)):
+        e = 0.0
+        for r in range(8):
+            y, ref = run(x[r]).cpu().numpy().astype(np.complex128), exact(T, x[r].cpu().numpy().astype(np.complex128))
+            e += (np.linalg.norm(y) ** 2 / np.linalg.norm(ref) ** 2 - 1.0) / 8
+        print(f"{ne} {n}: {e:.2e}", flush=True)
+        assert abs(e) < 2.0 ** -25
