@@ -9,11 +9,12 @@ are resident in HBM.  Prints one JSON line (see the keys below).
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--precision split_bf16]
                     [--no-compare] [--no-cpu]
 
-`value` is pairs/s of the selected form (split BF16 by default); the plain
-FP32 form is timed beside it on the same plan and input, and the ratio and
-the relative L2 difference between the two forms' outputs are reported (on
-the fast lateral correlation every form runs the same FP32 kernels).
-`err_vs_fp64` gives each form's relative L2 and max-abs error against the
+`value` is pairs/s of the selected form (split BF16 by default).  Plans on the
+fast lateral correlation run its FP32 kernels whatever form is selected, and
+`dtype` says so.  The direct products in plain FP32 (fast correlation switched
+off) are timed beside it on the same plan and input as "fp32_direct", and the
+ratio and the relative L2 difference between the outputs are reported.
+`err_vs_fp64` gives the relative L2 and max-abs error of both against the
 FP64 oracle on a dense input at 3 of the frequencies (outside the timed
 region).  `cpu_baseline` times the oracle's C FP64 loop nest (Phi
 materialized, as the reference's CPU path) on a sample of the config-1 pair,
@@ -35,6 +36,15 @@ sys.path.insert(0, str(ROOT))
 
 METRIC = "fwd+adj operator pairs/s vs plain FP32 at ≤1e-4 rel L2 err vs FP64 oracle"
 PRECISIONS = ("fp32", "split_bf16", "split_fp16")
+DIRECT = "fp32_direct"
+
+
+def select(op, form):
+    """Sets the form that later calls take (a precision, or DIRECT: the direct
+    products in plain FP32); returns the type that its kernels compute in."""
+    op.set_correlation(form != DIRECT)
+    op.set_precision("fp32" if form == DIRECT else form)
+    return "fp32" if form == DIRECT or op.kernels["pair"] == "fast" else form
 
 
 def algorithmic_flops(spec, n_rhs: int) -> float:
@@ -140,7 +150,7 @@ def host_entry_rate(op, form, x0, pairs: int = 3):
     """Pairs/s through the host-buffer entry points (born_forward /
     born_adjoint: FP64 host arrays, conversions and PCIe transfers
     included), timed after the device legs, outside their timed region."""
-    op.set_precision(form)
+    select(op, form)
     xh = np.asarray(x0, dtype=np.complex128).reshape(-1, 1)
     op.adjoint(op.forward(xh))   # warm-up
     t0 = time.perf_counter()
@@ -152,7 +162,7 @@ def host_entry_rate(op, form, x0, pairs: int = 3):
 
 
 def err_vs_fp64(op, spec, forms, f_sel=(0, 128, 256)):
-    """The checker: error of each numeric form against the FP64 oracle on a
+    """The checker: error of each form against the FP64 oracle on a
     dense input over the whole FOV, at 3 of the frequencies (first, middle,
     last) -- the forward of the speckle phantom at those frequencies'
     observations and the adjoint of random u supported on them -- through
@@ -175,7 +185,7 @@ def err_vs_fp64(op, spec, forms, f_sel=(0, 128, 256)):
     out = {"sample": f"dense speckle phantom over all {spec.fov.N_points} points; frequencies {list(f_sel)} "
                      f"({len(rows)} observations); FP64 oracle in {t_oracle:.1f} s"}
     for form in forms:
-        op.set_precision(form)
+        select(op, form)
         u = op.forward_dev(x).cpu().numpy()[rows]
         gh = op.adjoint_dev(uu).cpu().numpy()
         out[form] = {"forward": O.rel_l2(u, u_ref), "adjoint": O.rel_l2(gh, g_ref),
@@ -188,7 +198,7 @@ def err_vs_fp64(op, spec, forms, f_sel=(0, 128, 256)):
 def config0_full(threads: int, steps: int):
     """Config 0 in full (64 elements, 256x256 FOV, 65 bins, one wave, 30
     occupied points): the C FP64 loop nest, Phi materialized and fused, and
-    the device pair in both forms, all on the same input."""
+    the device pair by fast correlation and by direct products, all on the same input."""
     import torch
     from comp_ui_toolbox_amd import OperatorBorn
     from comp_ui_toolbox_amd import configs as C
@@ -202,7 +212,7 @@ def config0_full(threads: int, steps: int):
     u = torch.empty((1, op.N_observations), dtype=torch.complex64, device="cuda")
     g = torch.empty((1, op.N_points), dtype=torch.complex64, device="cuda")
     gpu = {}
-    for form in ("split_bf16", "fp32"):
+    for form in ("fp32", DIRECT):
         el, _ = time_form(op, form, x, u, g, steps, 3)
         gpu[form] = steps / el
     op.close()
@@ -224,12 +234,12 @@ def spec_gamma(spec):
     return _GAMMA[spec.name]
 
 
-def time_form(op, precision, x, u, g, steps, warmup):
-    """Warm up, then time `steps` forward+adjoint pairs of one numeric form.
+def time_form(op, form, x, u, g, steps, warmup):
+    """Warm up, then time `steps` forward+adjoint pairs of one form.
     x (N_rhs, N_pts), u (N_rhs, N_obs), g (N_rhs, N_pts).  Returns wall
     seconds and the per-launch kernel milliseconds."""
     import torch
-    op.set_precision(precision)
+    select(op, form)
     for _ in range(warmup):
         op.forward_dev(x, out=u)
         op.adjoint_dev(u, out=g)
@@ -246,9 +256,18 @@ def time_form(op, precision, x, u, g, steps, warmup):
     op.set_timing(False)
     timing = op.get_timing()
     kern = {name: timing[name][0] / max(timing[name][1], 1) for name in ("forward", "adjoint")}
-    print(f"[bench] {precision}: {steps} pairs in {elapsed * 1e3:.1f} ms, kernels "
+    print(f"[bench] {form}: {steps} pairs in {elapsed * 1e3:.1f} ms, kernels "
           f"fwd {kern['forward']:.3f} ms adj {kern['adjoint']:.3f} ms", file=sys.stderr, flush=True)
     return elapsed, kern
+
+
+def roofline_direct(F, kern):
+    """The dominant kernel of the direct products in plain FP32 against the
+    FP32 rate, which the matrix cores and the vector ALUs share."""
+    dom = max(kern, key=kern.get)
+    achieved = F / (kern[dom] * 1e-3) / 1e12
+    return {"bound": "flops", "kernel": f"{dom} contraction ({DIRECT})", "achieved": achieved, "peak": 157.3,
+            "unit": "TFLOP/s", "frac": achieved / 157.3}
 
 
 def roofline(F, B, kern, precision, config):
@@ -379,7 +398,7 @@ def bench_batched(args):
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": prec,
+        "dtype": "fp32" if all(op.kernels["pair"] == "fast" for op in ops) else prec,
         "data": "synthetic (config-3 instances, 30-point phantoms; tables built on the device)",
         "config": {
             "workload": "config3: 24 instances, FOV side {128,256,384,512} at pitch/4, 33-257 f, 1-11 waves, "
@@ -407,7 +426,7 @@ def main():
     ap.add_argument("--precision", default="split_bf16", choices=list(PRECISIONS),
                     help="the form whose pairs/s is reported as value")
     ap.add_argument("--no-compare", action="store_true",
-                    help="do not time the plain FP32 form beside the selected one")
+                    help="do not time the direct products in plain FP32 beside the selected form")
     ap.add_argument("--config", default="config1")
     ap.add_argument("--autotune", action="store_true",
                     help="run the library's autotuner for each form before timing it (its candidate "
@@ -456,15 +475,14 @@ def main():
     g = torch.empty((n_rhs, op.N_points), dtype=torch.complex64, device="cuda")
 
     forms = [args.precision]
-    if not args.no_compare and args.precision != "fp32":
-        forms.append("fp32")
-    res, outs = {}, {}
-    tuned = {}
+    if not args.no_compare:
+        forms.append(DIRECT)
+    res, outs, dtypes = {}, {}, {}
     for form in forms:
+        dtypes[form] = select(op, form)
         if args.autotune:
-            op.set_precision(form)
-            tuned[form] = op.autotune()
-            print(f"[bench] {form}: autotuned contraction fwd {tuned[form][0]:.3f} ms adj {tuned[form][1]:.3f} ms",
+            tuned = op.autotune()
+            print(f"[bench] {form}: autotuned contraction fwd {tuned[0]:.3f} ms adj {tuned[1]:.3f} ms",
                   file=sys.stderr, flush=True)
         res[form] = time_form(op, form, x, u, g, args.steps, args.warmup)
         # one pair from the same input, kept for the cross-form comparison
@@ -478,6 +496,8 @@ def main():
     F = algorithmic_flops(spec, n_rhs)
     B = algorithmic_bytes(spec, n_rhs)
     elapsed, kern = res[args.precision]
+    select(op, args.precision)
+    kernels = op.kernels["pair"]
     pairs_per_s = args.steps / elapsed
     result = {
         "metric": METRIC,
@@ -490,13 +510,14 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "fp32" if args.precision == "fp32" else args.precision,
+        "dtype": dtypes[args.precision],
         "data": f"synthetic ({args.config} speckle phantom; tables built on the device from the {args.config} geometry)",
         "config": {
             "workload": f"{args.config}: {spec.array.N_elements} el, {spec.fov.N_points_axis[0]}x"
                         f"{spec.fov.N_points_axis[-1]} FOV, {len(spec.frequencies)} f, "
                         f"{spec.N_measurements} waves, {spec.N_observations()} obs, {n_rhs} rhs",
             "precision": args.precision,
+            "kernels": kernels,
             "path": op.path,
             "autotuned": bool(args.autotune),
             "table_build_s": round(t_tables, 3),
@@ -504,18 +525,18 @@ def main():
             "flops_per_pass": F,
             "bytes_per_pass": B,
         },
-        "roofline": roofline(F, B, kern, args.precision, args.config),
+        "roofline": roofline(F, B, kern, dtypes[args.precision], args.config),
     }
-    if "fp32" in res and args.precision != "fp32":
-        e32, k32 = res["fp32"]
+    if DIRECT in res:
+        e32, k32 = res[DIRECT]
         result["config"]["fp32_pairs_per_s"] = args.steps / e32
         result["config"]["fp32_kernel_ms"] = {k: round(v, 4) for k, v in k32.items()}
         result["config"]["ratio_vs_fp32"] = e32 / elapsed
         result["config"]["rel_l2_vs_fp32"] = {
-            "forward": rel_l2(outs[args.precision][0], outs["fp32"][0]),
-            "adjoint": rel_l2(outs[args.precision][1], outs["fp32"][1]),
+            "forward": rel_l2(outs[args.precision][0], outs[DIRECT][0]),
+            "adjoint": rel_l2(outs[args.precision][1], outs[DIRECT][1]),
         }
-        result["roofline_fp32"] = roofline(F, B, k32, "fp32", args.config)
+        result["roofline_fp32"] = roofline_direct(F, k32)
     if n_rhs == 1:
         try:
             result["config"]["host_entry"] = host_entry_rate(op, args.precision, x0)
