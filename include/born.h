@@ -55,8 +55,9 @@ enum born_status {
 
 /* Numeric form of the grid contraction on the matrix cores.  Plans with the
  * lateral structure apply the operator by fast correlation in FP32 whatever
- * form is asked for (faster than the split forms and more accurate); the form
- * decides for those that cannot: spectra of h_ref that do not fit in memory,
+ * form is asked for (faster than the split forms and more accurate; its error
+ * is relative to the norm of all outputs of a row of the grid or of a channel
+ * set, see born_plan_set_correlation); the form decides for those that cannot: spectra of h_ref that do not fit in memory,
  * rows of h_ref with one entry far above the others, planes over 128 points
  * and elements per phase in 3-D, and born_apply_dev_noalloc. */
 enum born_precision {
@@ -305,11 +306,13 @@ int born_plan_force_general(born_plan_t plan, int32_t on);
 
 /* Whether forward and adjoint of a structured plan may go by fast correlation
  * (on, the default) or keep to the matrix and vector kernels of the plan's
- * numeric form (0).  A transform carries the rounding of a whole row of h_ref,
- * the direct products only that of each entry: a program whose results hang
- * on outputs far below the others of their row (one active element, a point
- * outside every element's cone) switches it off, and so may one that has no
- * use for forward and adjoint: the spectra of h_ref, about twice its size, are
+ * numeric form (0).  A transform carries the rounding of a whole row, about
+ * 1e-7 of the root mean square of its outputs, to each of them; the direct
+ * products keep an output's rounding to itself, and outputs whose products are
+ * all 0 exactly 0.  A program whose results hang on outputs far below the
+ * others (channels that do not see a scatterer 100 dB above the rest, one
+ * active element) switches it off, and so may one that has no use for forward
+ * and adjoint: the spectra of h_ref, about twice its size, are
  * given back.  The next call builds the workspace of the other kernels. */
 int born_plan_set_correlation(born_plan_t plan, int32_t on);
 

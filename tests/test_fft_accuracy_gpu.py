@@ -136,3 +136,41 @@ def test_energy_of_the_outputs(torch_cuda, ne, n, npp):
             e += (np.linalg.norm(y) ** 2 / np.linalg.norm(ref) ** 2 - 1.0) / 8
         print(f"{ne} {n}: {e:.2e}", flush=True)
         assert abs(e) < 2.0 ** -25
+
+
+def test_localized_inputs(torch_cuda):
+    """One strong point in front of weak ones, one strong channel beside weak
+    ones, and a receive filter that hides the strong one from most outputs: the
+    fast correlation carries the strong one's rounding everywhere, 2^-24 times
+    the root mean square of all outputs by some units (3e-7 taken for transforms
+    of these lengths, 1e-6 here), the direct products keep that of an output to
+    itself (their 1e-5 for the outputs that do not see it).  Programs that need
+    the latter switch the fast correlation off."""
+    import torch
+    ne, nx, nz, npp, nf = 64, 256, 48, 4, 5
+    arr = C.ArraySpec((ne,), (3e-4,), (2.7e-4,), (2,))
+    rng = np.random.Generator(np.random.PCG64(12))
+    waves = [C.qpw_wave(arr, 0.0, 1500.0)]
+    spec = C.SequenceSpec("s", arr, C.MediumSpec(), C.FovSpec((nx, nz), (3e-4 / npp,) * 2, 2e-3), np.linspace(4e6, 8e6, nf),
+                          waves, [C.identity_mixes(ne) for _ in waves])
+    T = O.direct_tables(spec)
+    op = OperatorBorn.from_sequence(spec)
+    strong = 1e5
+    g = np.zeros(op.N_points)
+    g[nx * (nz - 8):] = rng.standard_normal(8 * nx)
+    g[3 * nx + nx // 2] = strong
+    u = rng.standard_normal((ne, nf)) + 1j * rng.standard_normal((ne, nf))
+    u[ne // 2] *= strong
+    alone_g, alone_u = np.zeros_like(g), np.zeros_like(u)
+    alone_g[3 * nx + nx // 2], alone_u[ne // 2] = strong, u[ne // 2]
+    for run, exact, x, alone in ((op.forward_dev, O.forward, g, alone_g), (op.adjoint_dev, O.adjoint, u.reshape(-1), alone_u.reshape(-1))):
+        ref, of_strong = exact(T, x).reshape(-1), exact(T, alone).reshape(-1)
+        hidden = np.abs(of_strong) < 1e-12 * np.abs(of_strong).max()      # outputs that do not see it
+        assert 0.2 < hidden.mean() < 0.98 and np.linalg.norm(ref[hidden]) > 0
+        xd = torch.tensor(x.astype(np.complex64), device="cuda:0")
+        for on, tol in ((True, 1e-6 * np.sqrt(np.mean(np.abs(ref) ** 2))),
+                        (False, 1e-5 * np.sqrt(np.mean(np.abs(ref[hidden]) ** 2)))):
+            op.set_correlation(on)
+            err = np.sqrt(np.mean(np.abs(run(xd).cpu().numpy() - ref)[hidden] ** 2))
+            print(f"{run.__name__} correlation={on}: {err:.2e} of {tol:.2e}", flush=True)
+            assert err < tol
