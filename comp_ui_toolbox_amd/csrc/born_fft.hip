@@ -113,25 +113,28 @@ __global__ __launch_bounds__(256) void k_fft_range(const float2* __restrict__ h,
                                                    const int* __restrict__ exty, int N_ext, int ny, int H_plane, int HR,
                                                    int HY, int Nz, int Npx, int Npy, int64_t n_rows,
                                                    int* __restrict__ bad) {
-  __shared__ float red[3][4];
+  __shared__ float red[4][4];
   const int tid = threadIdx.x, wave = tid >> 6;
-  auto reduce = [&](float& a, float& b, float& c, bool largest) {   // over the block, in all threads
+  auto reduce = [&](float& most, float& a, float& b, float& c) {   // a maximum and three sums over the block, in all threads
     __syncthreads();
 #pragma unroll
     for (int m = 1; m < 64; m <<= 1) {
-      a = largest ? fmaxf(a, __shfl_xor(a, m)) : a + __shfl_xor(a, m);
+      most = fmaxf(most, __shfl_xor(most, m));
+      a += __shfl_xor(a, m);
       b += __shfl_xor(b, m);
       c += __shfl_xor(c, m);
     }
     if ((tid & 63) == 0) {
-      red[0][wave] = a;
-      red[1][wave] = b;
-      red[2][wave] = c;
+      red[0][wave] = most;
+      red[1][wave] = a;
+      red[2][wave] = b;
+      red[3][wave] = c;
     }
     __syncthreads();
-    a = largest ? fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3])) : red[0][0] + red[0][1] + red[0][2] + red[0][3];
-    b = red[1][0] + red[1][1] + red[1][2] + red[1][3];
-    c = red[2][0] + red[2][1] + red[2][2] + red[2][3];
+    most = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
+    a = red[1][0] + red[1][1] + red[1][2] + red[1][3];
+    b = red[2][0] + red[2][1] + red[2][2] + red[2][3];
+    c = red[3][0] + red[3][1] + red[3][2] + red[3][3];
   };
   for (int64_t row = blockIdx.x; row < n_rows; row += gridDim.x) {
     const float2* src = h + (size_t)(row / Nz) * H_plane + (size_t)(row % Nz) * HY * HR;
@@ -140,13 +143,13 @@ __global__ __launch_bounds__(256) void k_fft_range(const float2* __restrict__ h,
       const int ty = i / n;
       return src[(size_t)exty[py + sy * ty] * HR + ext[px + sx * (i - ty * n)]];
     };
-    float top = 0.f, odd = 0.f, none = 0.f;
+    float top = 0.f, odd = 0.f, n1 = 0.f, n2 = 0.f;   // (n1, n2: not used)
     for (int i = tid; i < N_ext * ny; i += 256) {
       const float2 v = entry(i, N_ext, 0, 0, 1, 1);
       if (!(fabsf(v.x) < 1e30f && fabsf(v.y) < 1e30f)) odd = 1.f;   // (NaN among them)
       else top = fmaxf(top, fmaxf(fabsf(v.x), fabsf(v.y)));
     }
-    reduce(top, odd, none, true);
+    reduce(top, odd, n1, n2);
     if (odd > 0.f) {
       if (tid == 0) atomicOr(bad, 3);
       continue;
@@ -172,8 +175,7 @@ __global__ __launch_bounds__(256) void k_fft_range(const float2* __restrict__ h,
           n += 1.f;
         }
       }
-      reduce(e, l, n, false);
-      reduce(first, none, none, true);
+      reduce(first, e, l, n);
       peak = fmaxf(peak, first);
       if (16.f * first > e) {
         float low = 0.f;
@@ -182,7 +184,7 @@ __global__ __launch_bounds__(256) void k_fft_range(const float2* __restrict__ h,
           const float x = v.x * scale, y = v.y * scale, q = x * x + y * y;
           if (q > 0.f && q * 0x1p32f < first) low += 1.f;
         }
-        reduce(low, none, none, false);
+        reduce(n1, low, n1, n2);
         if (low >= 8.f && 2.f * low > n) uneven = true;
       }
       energy += e;
