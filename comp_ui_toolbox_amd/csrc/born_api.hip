@@ -582,7 +582,9 @@ static void build_fft_tables(Plan& P) {
 // are added one after the other in FP32, whose rounding grows with the root of
 // their number; the groups are added in FP64.  8224 columns of 128 elements,
 // 512 x 512 points: relative L2 error against FP64 4.9e-7 with 343 columns per
-// wave, 2.8e-7 with 86, same time (9.04 ms the pair).
+// wave, 3.0e-7 with 121, both at 9.20 ms the pair, 2.3e-7 with 62 at 9.25
+// (direct products 3.75e-7); 1280 columns, 8 right-hand sides: 2.8e-7 with 107
+// where the direct products have 2.3e-7.
 static int adj_groups(const Plan& P, int N_rhs, int64_t fill, int64_t most) {
   const int64_t g = std::max<int64_t>({1, fill, (P.N_pairs + most - 1) / most});
   return (int)std::min<int64_t>(g, std::max<int64_t>(1, (1ll << 31) / ((int64_t)N_rhs * P.N_pts)));
