@@ -584,7 +584,10 @@ static void build_fft_tables(Plan& P) {
 // 512 x 512 points: relative L2 error against FP64 4.9e-7 with 343 columns per
 // wave, 3.0e-7 with 121, both at 9.20 ms the pair, 2.3e-7 with 62 at 9.25
 // (direct products 3.75e-7); 1280 columns, 8 right-hand sides: 2.8e-7 with 107
-// where the direct products have 2.3e-7.
+// where the direct products have 2.3e-7.  Volumes: 384 columns per workgroup (32 x
+// 32 elements, 64^3 points, 325 columns in one group 4.8e-7, in two 3.4e-7, direct
+// products 7.3e-7; 128 x 128 x 192 points, 4 right-hand sides: 28.8 ms in one group,
+// 29.4 in two).
 static int adj_groups(const Plan& P, int N_rhs, int64_t fill, int64_t most) {
   const int64_t g = std::max<int64_t>({1, fill, (P.N_pairs + most - 1) / most});
   return (int)std::min<int64_t>(g, std::max<int64_t>(1, (1ll << 31) / ((int64_t)N_rhs * P.N_pts)));
@@ -668,7 +671,7 @@ static void build_fft3_workspace(Plan& P, int N_rhs) {
   F.ZR = std::min(F.ZR, P.Nz);
   F.NZB = (P.Nz + F.ZR - 1) / F.ZR;
   const int64_t wg = (int64_t)P.Nz * P.Npy * (P.Np / F.s3.px) * N_rhs;
-  F.FG = adj_groups(P, N_rhs, std::min<int64_t>({(2048 + wg - 1) / wg, P.N_pairs / 8, 64}), 64);
+  F.FG = adj_groups(P, N_rhs, std::min<int64_t>({(2048 + wg - 1) / wg, P.N_pairs / 8, 64}), 384);
   if (std::max(cols * F.NZB, wg * F.FG) > (1 << 23) - 1 - XCDS)   // (2^32 threads, up to 512 each)
     throw Error(BORN_ERR_UNSUPPORTED, "too many right-hand sides for one launch");
   F.d_vp = dalloc<float2>((size_t)F.NZB * cols * P.N_e);
