@@ -46,7 +46,7 @@ __device__ __forceinline__ OutT col_value(double qx, double qy, float2 p) {
 // N_f outputs, the rows of neighbouring elements adjacent.  Bound: the writes
 // of the output and, per output, one prefactor from the L2; scattered points
 // also wait on one page of the tables per (pair, point).  256 random points
-// at 361,856 observations: 2.39 ms map-driven, 0.37 ms here (0.25 ms with all
+// at 361,856 observations: 2.39 ms map-driven, 0.33 ms here (0.25 ms with all
 // points alike; writing the output alone takes 0.12 ms).
 template <typename OutT>
 __global__ __launch_bounds__(COL_NT) void k_columns_single(ColArgs A, const int* __restrict__ ent_off,

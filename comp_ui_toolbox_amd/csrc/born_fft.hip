@@ -23,10 +23,10 @@
 //
 // Bound: the stream of the p_inc table (7.1 GB per direction at 128 elements,
 // 512 x 512 points, 257 frequencies, 11 waves) close to the vector ALU.
-// Measured there per call: forward kernel 1.75 ms, adjoint kernel 1.37 ms (5.2
+// Measured there per call: forward kernel 1.77 ms, adjoint kernel 1.39 ms (5.2
 // TB/s, what the memory gives), against 7.2 and 6.8 ms of the direct products
-// on FP32 MFMA and 2.4 and 2.6 ms in split BF16; relative L2 error against
-// FP64 3.1e-7 (3.3e-7 and 6.3e-6 there).  Entries of a lane come in counts of
+// on FP32 MFMA and 2.4 and 2.6 ms in split BF16; relative L2 error of
+// the pair against FP64 2.3e-7 (3.3e-7 and 6.3e-6 there).  Entries of a lane come in counts of
 // 4 to 16 (fft_entries), twiddles from LDS: with 8 or 16 entries, branches on
 // the slot's length and twiddles in registers the two took 1.79 and 1.54 ms,
 // and 264 and 232 instead of 223 and 202 us at 100 elements, 301 x 411 points,
@@ -42,10 +42,11 @@ namespace born {
 
 // ------------------------------------------------------------------ spectra
 // H[f][slot] (FP64 transform of the FP32 row, conjugated twice for the
-// exponent's sign, divided by L and by the transforms' mean gain (fft_gains): the inverse transforms of both directions need
-// no other factor, and products and sums keep the range of the direct form's)
-// and the layout its readers take: per group of FPW slots [8][64 lanes][2]
-// entries, so that a lane reads two entries at once.
+// exponent's sign, divided by L and by the transforms' mean gain (fft_gains):
+// the inverse transforms of both directions need no other factor, and products
+// and sums keep the range of the direct form's).  Layout, that of its readers:
+// per group of FPW slots [8][64 lanes][2] entries, so that a lane reads two
+// entries at once.
 template <int TL>
 __global__ __launch_bounds__(64) void k_fft_table(const float2* __restrict__ h, const int* __restrict__ ext,
                                                   const int* __restrict__ hrow, int H_plane, int HR, int N_ext, int Np,

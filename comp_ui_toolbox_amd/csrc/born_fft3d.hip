@@ -18,7 +18,7 @@
 //
 // Bound: the vector ALU, per plane of 64 x 64 points at 2 points per pitch
 // 384 transforms of 64 points (about 7400 wave instructions) in place of
-// 32 x 32 x 64 x 64 complex multiply-adds, at 60 % of its rate with two waves
+// 32 x 32 x 64 x 64 complex multiply-adds, at 60-65 % of its rate with two waves
 // per SIMD (registers and LDS) and two barriers per tile.  32 x 32 elements,
 // 64^3 points, 33 frequencies, 3 waves, 4 right-hand sides: forward 0.67 ms,
 // adjoint 0.58 ms against 5.6 and 7.0 ms of the split BF16 products (128 x 128 x

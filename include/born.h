@@ -57,9 +57,10 @@ enum born_status {
  * lateral structure apply the operator by fast correlation in FP32 whatever
  * form is asked for (faster than the split forms and more accurate; its error
  * is relative to the norm of all outputs of a row of the grid or of a channel
- * set, see born_plan_set_correlation); the form decides for those that cannot: spectra of h_ref that do not fit in memory,
- * rows of h_ref with one entry far above the others, planes over 128 points
- * and elements per phase in 3-D, and born_apply_dev_noalloc. */
+ * set, see born_plan_set_correlation).  The form decides for those that
+ * cannot: spectra of h_ref that do not fit in memory, rows of h_ref with one
+ * entry far above the others, planes over 128 points and elements per phase in
+ * 3-D, and born_apply_dev_noalloc. */
 enum born_precision {
     BORN_PRECISION_FP32 = 0,     /* plain FP32 operands, FP32 MFMA products      */
     BORN_PRECISION_SPLIT_BF16 = 1,/* hi+lo BF16 operands, FP32 accumulation       */
@@ -312,8 +313,8 @@ int born_plan_force_general(born_plan_t plan, int32_t on);
  * all 0 exactly 0.  A program whose results hang on outputs far below the
  * others (channels that do not see a scatterer 100 dB above the rest, one
  * active element) switches it off, and so may one that has no use for forward
- * and adjoint: the spectra of h_ref, about twice its size, are
- * given back.  The next call builds the workspace of the other kernels. */
+ * and adjoint: the spectra of h_ref, about twice its size, are given back.  The
+ * next call builds the workspace of the other kernels. */
 int born_plan_set_correlation(born_plan_t plan, int32_t on);
 
 /* Which kernels a plan's calls take: kernels[0] forward and adjoint, [1]
